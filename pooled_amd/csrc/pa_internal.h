@@ -117,6 +117,9 @@ struct GemmParams {
   int acc; int kind;
 };
 hipError_t pa_launch_gemm(const GemmParams& p, int n_cu, hipStream_t s);
+// a few columns of quantised weights (proj_gemm_skinny.hip)
+bool pa_gemm_skinny_serves(const GemmParams& p);
+hipError_t pa_launch_gemm_skinny(const GemmParams& p, int n_cu, hipStream_t s);
 // large chunks (proj_gemm_wide.hip): the weights widened once into w16 (f16 in fragment order, the caller's staging), then a
 // GEMM over two f16 operands; pa_gemm_wide_serves tells whether a call qualifies
 bool pa_gemm_wide_serves(const GemmParams& p, int n_cu);

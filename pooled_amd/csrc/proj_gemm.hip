@@ -206,179 +206,6 @@ __global__ __launch_bounds__(256, XT == 2 ? 2 : 1) void pa_gemm_kernel(GemmParam
     }
 }
 
-// ---- skinny chunks (a verify block, the reference's 16-column passes: engine/wgsl/coop.js batched matvec) ----
-// With a handful of columns the tiled kernel leaves the chip empty (d_out / 128 workgroups, each walking all of K)
-// while the work is one pass over the weights.  This kernel streams the weights GEMV-style -- a wave owns RW rows, a
-// lane the 32-value blocks lane + 64 i of each -- widens them once into f16 pairs in registers, stages all the
-// chunk's columns in LDS (80-byte block stride: conflict-free 128-bit reads) and runs one v_dot2_f32_f16 per two
-// weights and column.  Same operand precision as the tiled kernel (weights and activations f16, sums f32), so a
-// result does not depend on which kernel served the chunk beyond the order of the sums.  The lanes' partial sums go
-// through LDS (the staging area, free by then): lane t of a wave adds up the 64 partials of its (row, column).
-#define SK_NC 16        // columns a launch serves at most
-template <int KIND, int BPL, int RW>
-__global__ __launch_bounds__(256)
-void pa_gemm_skinny_kernel(const uint16_t* a_x, const void* a_w, const uint16_t* a_scales, uint32_t a_x_stride, uint32_t a_d_out, uint32_t a_d_in, uint32_t a_n_cols,
-                           GemmParams p_in) {
-  static_assert(KIND == PA_W_Q4_0 || KIND == PA_W_Q8_0, "quantised weights");
-  // (the leading arguments repeat fields of p_in: they are preloaded into scalar registers, so the loads below need no
-  // scalar-load round trip; the other arguments are fetched in one batch behind them)
-  GemmParams p = p_in;
-  p.x = a_x; p.w = a_w; p.scales = a_scales; p.x_stride = a_x_stride; p.d_out = a_d_out; p.d_in = a_d_in; p.n_cols = a_n_cols;
-  extern __shared__ __attribute__((aligned(16))) unsigned char sk_lds[];
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t nb = p.d_in / GK, ncol = p.n_cols;
-  const uint32_t xcol = nb * GROW;                                    // bytes of a staged column
-  const size_t row0 = ((size_t)blockIdx.x * 4 + wave) * RW;
-  // The first eight 16-byte pieces a thread stages of the chunk's columns (all of them for 8 columns of 2048) are
-  // requested FIRST, the wave's weight rows right behind them: a wave's loads complete in order, the columns come from
-  // L2 in a fraction of the time the weight stream takes from HBM, and their trip into LDS then runs under the latency
-  // of the weights instead of after it.
-  const uint32_t cpc = p.d_in / 8;                                    // 16-byte pieces of a column
-  const uint32_t pieces = ncol * cpc;
-  u4 xv0[8];
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const uint32_t e = min(tid + 256 * j, pieces - 1), c = e / cpc, k8 = e % cpc;
-    xv0[j] = *(const u4*)((const unsigned char*)(p.x + (size_t)c * p.x_stride) + k8 * 16);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  constexpr int WQ = KIND == PA_W_Q4_0 ? 1 : 2;                       // 16-byte words of a packed block
-  u4 wq[RW][BPL][WQ];
-  uint16_t wsc[RW][BPL];
-#pragma unroll
-  for (int r = 0; r < RW; r++) {
-    const size_t row = min(row0 + r, (size_t)p.d_out - 1);            // rows past the end repeat the last one (not stored)
-#pragma unroll
-    for (int i = 0; i < BPL; i++) {
-      const uint32_t b = min(lane + 64 * i, nb - 1);                   // blocks past the end likewise (scale forced to 0)
-      const u4* src = (const u4*)((const unsigned char*)p.w + (row * nb + b) * (16 * WQ));
-#pragma unroll
-      for (int w = 0; w < WQ; w++) wq[r][i][w] = src[w];
-      wsc[r][i] = p.scales[row * nb + b];
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" :: "s"(p.y), "s"(p.y_stride), "s"(p.acc));
-  // the chunk's columns -> LDS, 16 bytes a thread and turn: the pieces requested above, ...
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const uint32_t e = tid + 256 * j, c = e / cpc, k8 = e % cpc;
-    if (e < pieces) *(u4*)(sk_lds + c * xcol + (k8 >> 2) * GROW + (k8 & 3) * 16) = xv0[j];
-  }
-  // ... then any further turns (eight loads a thread go out before the first is stored -- unconditional, a turn past the
-  // end re-reads the last piece: one load a loop turn is one round trip a turn)
-  for (uint32_t e0 = tid + 256 * 8; e0 < pieces; e0 += 256 * 8) {
-    u4 v[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const uint32_t e = min(e0 + 256 * j, pieces - 1), c = e / cpc, k8 = e % cpc;
-      v[j] = *(const u4*)((const unsigned char*)(p.x + (size_t)c * p.x_stride) + k8 * 16);
-    }
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const uint32_t e = e0 + 256 * j, c = e / cpc, k8 = e % cpc;
-      if (e < pieces) *(u4*)(sk_lds + c * xcol + (k8 >> 2) * GROW + (k8 & 3) * 16) = v[j];
-    }
-  }
-  // widen: pair k of a block = elements 2k, 2k + 1
-  h2 wv[RW][BPL][16];
-#pragma unroll
-  for (int r = 0; r < RW; r++)
-#pragma unroll
-    for (int i = 0; i < BPL; i++) {
-      const _Float16 s1 = __ushort_as_half(lane + 64 * i < nb ? wsc[r][i] : (uint16_t)0);
-      const h2 sc = { s1, s1 };
-      if constexpr (KIND == PA_W_Q4_0) {
-        const h2 bias = { (_Float16)1032.f, (_Float16)1032.f };
-#pragma unroll
-        for (int d = 0; d < 4; d++) {
-          const uint32_t l = wq[r][i][0][d] & 0x0F0F0F0Fu, h = (wq[r][i][0][d] >> 4) & 0x0F0F0F0Fu;
-          wv[r][i][2 * d] = bytes_to_h2(l, 0x04010400u, bias, sc); wv[r][i][2 * d + 1] = bytes_to_h2(l, 0x04030402u, bias, sc);
-          wv[r][i][8 + 2 * d] = bytes_to_h2(h, 0x04010400u, bias, sc); wv[r][i][8 + 2 * d + 1] = bytes_to_h2(h, 0x04030402u, bias, sc);
-        }
-      } else {
-        const h2 bias = { (_Float16)1152.f, (_Float16)1152.f };
-#pragma unroll
-        for (int w = 0; w < 2; w++)
-#pragma unroll
-          for (int d = 0; d < 4; d++) {
-            const uint32_t x = wq[r][i][w][d] ^ 0x80808080u;
-            wv[r][i][8 * w + 2 * d] = bytes_to_h2(x, 0x04010400u, bias, sc); wv[r][i][8 * w + 2 * d + 1] = bytes_to_h2(x, 0x04030402u, bias, sc);
-          }
-      }
-    }
-  __syncthreads();
-  float part[SK_NC][RW];
-#pragma unroll
-  for (int c = 0; c < SK_NC; c++) {
-#pragma unroll
-    for (int r = 0; r < RW; r++) part[c][r] = 0.f;
-    if ((uint32_t)c < ncol) {
-#pragma unroll
-      for (int i = 0; i < BPL; i++) {
-        const unsigned char* xb = sk_lds + c * xcol + min(lane + 64 * i, nb - 1) * GROW;
-        h2 xv[16];
-#pragma unroll
-        for (int q = 0; q < 4; q++) { const h8 v = *(const h8*)(xb + 16 * q); xv[4 * q] = (h2){ v[0], v[1] }; xv[4 * q + 1] = (h2){ v[2], v[3] }; xv[4 * q + 2] = (h2){ v[4], v[5] }; xv[4 * q + 3] = (h2){ v[6], v[7] }; }
-#pragma unroll
-        for (int r = 0; r < RW; r++)
-#pragma unroll
-          for (int k = 0; k < 16; k++) part[c][r] = __builtin_amdgcn_fdot2(wv[r][i][k], xv[k], part[c][r], false);
-      }
-    }
-  }
-  __syncthreads();                                                    // every wave is done with the staged columns
-  // partials -> LDS [wave][lane][SK_NC * RW + 1], then lane t sums column t of its wave's 64 x (SK_NC * RW) table
-  constexpr int PV = SK_NC * RW, PS = PV + 1;
-  float* ps = (float*)sk_lds + (size_t)wave * 64 * PS;
-#pragma unroll
-  for (int c = 0; c < SK_NC; c++)
-    if ((uint32_t)c < ncol)
-#pragma unroll
-      for (int r = 0; r < RW; r++) ps[lane * PS + c * RW + r] = part[c][r];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  for (uint32_t t = lane; t < ncol * RW; t += 64) {
-    const uint32_t c = t / RW, r = t % RW;
-    float* y = p.y + (size_t)c * p.y_stride + min(row0 + r, (size_t)p.d_out - 1);
-    const float yo = p.acc ? *y : 0.f;                                // on its way while the partials are added up
-    float a = 0.f;
-    for (int l = 0; l < 64; l++) a += ps[l * PS + t];
-    if (row0 + r < p.d_out) *y = p.acc ? yo + a : a;
-  }
-}
-
-// LDS the skinny kernel needs: the staged columns, or the four waves' partial tables if those are larger
-static size_t skinny_lds(const GemmParams& p, int rw) {
-  const size_t x = (size_t)p.n_cols * (p.d_in / GK) * GROW, ps = (size_t)4 * 64 * (SK_NC * rw + 1) * sizeof(float);
-  return x > ps ? x : ps;
-}
-template <int KIND, int BPL, int RW>
-static hipError_t launch_skinny(const GemmParams& p, hipStream_t s) {
-  const size_t lds = skinny_lds(p, RW);
-  static size_t attr = 0;
-  if (lds > attr) {
-    hipError_t e = hipFuncSetAttribute((const void*)pa_gemm_skinny_kernel<KIND, BPL, RW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    attr = lds;
-  }
-  hipLaunchKernelGGL((pa_gemm_skinny_kernel<KIND, BPL, RW>), dim3((p.d_out + 4 * RW - 1) / (4 * RW)), dim3(256), lds, s, p.x, p.w, p.scales, p.x_stride, p.d_out, p.d_in,
-                     p.n_cols, p);
-  return hipGetLastError();
-}
-template <int KIND>
-static hipError_t launch_skinny_kind(const GemmParams& p, int n_cu, hipStream_t s) {
-  if (p.d_in <= 2048) {
-    // (three rows a wave where that lowers the rows of the busiest SIMD -- 9216 rows: 2304 waves at 2.25 a SIMD, or 3072
-    // at three -- as the one-token GEMV chooses)
-    const uint32_t simds = 4u * (uint32_t)(n_cu > 0 ? n_cu : 256);
-    auto busiest = [&](uint32_t r) { const uint32_t waves = (p.d_out + r - 1) / r; return ((waves + simds - 1) / simds) * r; };
-    if (busiest(3) < busiest(4)) return launch_skinny<KIND, 1, 3>(p, s);
-    return launch_skinny<KIND, 1, 4>(p, s);
-  }
-  if (p.d_in <= 4096) return launch_skinny<KIND, 2, 2>(p, s);
-  return launch_skinny<KIND, 4, 1>(p, s);
-}
-
 template <int XT>
 static hipError_t launch_gemm_xt(const GemmParams& p, hipStream_t s) {
   const dim3 grid((p.d_out + GT - 1) / GT, (p.n_cols + GT * XT - 1) / (GT * XT)), block(256);
@@ -393,22 +220,6 @@ static hipError_t launch_gemm_xt(const GemmParams& p, hipStream_t s) {
 
 hipError_t pa_launch_gemm(const GemmParams& p, int n_cu, hipStream_t s) {
   if (p.d_out == 0 || p.d_in == 0 || (p.d_in & 31) || p.n_cols == 0) return hipErrorInvalidValue;
-  // a handful of columns: a pass over the weights per launch of up to 16 columns (as many as fit the LDS staging),
-  // up to 32 columns in all -- past that the tiled kernel wins
-  if (p.kind != PA_W_F32 && p.n_cols <= 2 * SK_NC && p.d_in <= 8192 && (p.x_stride & 7) == 0) {
-    const uint32_t fit = (uint32_t)((144 * 1024) / ((size_t)(p.d_in / GK) * GROW));
-    const uint32_t per = fit < SK_NC ? fit : SK_NC;
-    if (per >= 1) {
-      for (uint32_t c0 = 0; c0 < p.n_cols; c0 += per) {
-        GemmParams q = p;
-        q.x = p.x + (size_t)c0 * p.x_stride; q.y = p.y + (size_t)c0 * p.y_stride;
-        q.n_cols = p.n_cols - c0 < per ? p.n_cols - c0 : per;
-        const hipError_t e = p.kind == PA_W_Q4_0 ? launch_skinny_kind<PA_W_Q4_0>(q, n_cu, s) : launch_skinny_kind<PA_W_Q8_0>(q, n_cu, s);
-        if (e != hipSuccess) return e;
-      }
-      return hipSuccess;
-    }
-  }
   // 256-column workgroups (two fit a CU) when they still give every CU four: otherwise 128-column ones (three a CU)
   const size_t wgs2 = (size_t)((p.d_out + GT - 1) / GT) * ((p.n_cols + 2 * GT - 1) / (2 * GT));
   const bool xt2 = wgs2 >= (size_t)4 * (n_cu > 0 ? n_cu : 256);

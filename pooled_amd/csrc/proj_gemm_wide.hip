@@ -491,10 +491,7 @@ bool pa_gemm_wide_serves(const GemmParams& p, int n_cu) {
   return wgs >= (uint64_t)(n_cu > 0 ? n_cu : 256);
 }
 
-// chunks of more than 16 columns that the large-chunk kernel does not serve.  Measured with cold weights (Q4_0, 32 to
-// 64 weights in rotation): [q|k|v] 9216 x 2048 13.0 - 13.5 us for 8 to 32 columns against 12.9 / 17.9 / 28 / 34 us at 8 /
-// 16 / 24 / 32 columns on the skinny kernel (which reads the packed weights, a quarter of the bytes, but one launch
-// per 16 columns); wo 2048 x 4096 16.7 us against 8.5 / 15.9 / 19.9 / 27.6
+// chunks that neither the large-chunk kernel nor the one for a few columns (proj_gemm_skinny.hip) serves
 bool pa_gemm_mid_serves(const GemmParams& p) {
   return p.n_cols > 16 && p.d_in % GM_KS == 0 && (p.x_stride & 7) == 0 && ((uintptr_t)p.x & 15) == 0;
 }

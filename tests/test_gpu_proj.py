@@ -173,6 +173,32 @@ def test_gemm_large_chunks(kind, d_out, d_in, n):
 
 
 @pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])
+@pytest.mark.parametrize("d_out,d_in,n", [(16, 32, 1), (17, 256, 2), (31, 288, 15), (4096, 4096, 16), (4100, 4128, 8), (4130, 8192, 9), (8200, 512, 17),
+                                          (8193, 2080, 32), (8192, 5120, 16), (4111, 6144, 31), (2048, 4096, 33), (600, 7968, 32)])
+def test_gemm_few_columns(kind, d_out, d_in, n):
+    """Up to 32 columns straight from the packed planes: one, two and four 16-row groups a workgroup (fewer and more of them
+    than CUs, d_in either side of 4096, what fits the LDS), one and two column blocks, chunks of 8 and 16 blocks that d_in
+    fills or not, ragged rows, and the first column counts of the next kernel.  The sums are f32 in another order than the
+    f64 oracle's: 2e-5 of the largest output is some 300 roundings at most."""
+    rng = np.random.default_rng(d_out + 7 * d_in + n + kind)
+    w, sc = _weights(kind, d_out, d_in, rng)
+    x16 = rng.standard_normal((n, d_in)).astype(np.float16)
+    ref = O.gemm_f16(kind, w, sc, x16.astype(np.float32))
+    xs, ys = d_in + 8, d_out + 3
+    xpad = np.full((n, xs), np.float16(np.nan)); xpad[:, :d_in] = x16
+    y0 = rng.standard_normal((n, ys)).astype(np.float32)
+    with PooledAttn(SHAPES["qwen36_moe"], 64, n_layers=1, max_cols=1) as pa:
+        wh = pa.weight(kind, w, sc)
+        dx = pa.to_device(xpad.view(np.uint16)); dy = pa.to_device(y0)
+        pa.gemm(wh, dx, xs, n, dy, ys); pa.sync()
+        got = dy.download(np.float32, n * ys).reshape(n, ys)
+        assert _rel(got[:, :d_out], ref) < 2e-5, "plain"
+        assert np.array_equal(got[:, d_out:], y0[:, d_out:]), "the stride padding of y must stay untouched"
+        pa.gemm(wh, dx, xs, n, dy, ys, acc=True); pa.sync()
+        assert _rel(dy.download(np.float32, n * ys).reshape(n, ys)[:, :d_out], 2.0 * ref) < 2e-5, "accumulate"
+
+
+@pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])
 def test_gemm_weight_cache_budget(kind):
     """The kept f16 copy and the per-call staging hold the same values: a context with no budget (every call widens into
     the context's staging), one whose budget holds the first weight only, and the default give the same bits, also
