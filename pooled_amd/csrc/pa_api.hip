@@ -1046,22 +1046,33 @@ static int slot_make(pa_ctx* ctx, const char* who, uint32_t slot, uint32_t pos) 
   return PA_OK;
 }
 
-// rows [0, pos) of one tensor between the cache ([nKV][max_seq + 32][hd]) and a slot ([nKV][pos][hd]): one pitched copy
-static hipError_t slot_copy(const pa_ctx* ctx, int which, void* cache, void* slot_buf, uint32_t pos, bool to_slot) {
-  const size_t plane = (size_t)pos * head_row_bytes(ctx, which), cache_pitch = ((size_t)ctx->cfg.max_seq + 32) * head_row_bytes(ctx, which);
-  return to_slot ? hipMemcpy2DAsync(slot_buf, plane, cache, cache_pitch, plane, ctx->cfg.n_kv_heads, hipMemcpyDeviceToDevice, ctx->stream)
-                 : hipMemcpy2DAsync(cache, cache_pitch, slot_buf, plane, plane, ctx->cfg.n_kv_heads, hipMemcpyDeviceToDevice, ctx->stream);
+// rows [0, pos) of every tensor of the slot's layers between the caches ([nKV][max_seq + 32][row]) and the slot ([nKV][pos][row])
+static hipError_t slot_copy(const pa_ctx* ctx, const pa_slot& sl, bool to_slot) {
+  PaCopyParams p;
+  p.n = 0;
+  for (size_t l = 0; l < ctx->layers.size() && l < sl.t[0].size(); l++) {
+    if (!sl.t[0][l]) continue;
+    for (int w = 0; w < n_tensors(ctx); w++) {
+      const size_t row = head_row_bytes(ctx, w), slot_pitch = (size_t)sl.pos * row, cache_pitch = ((size_t)ctx->cfg.max_seq + 32) * row;
+      void* cache = ctx->layers[l].tensor(w);
+      p.src[p.n] = to_slot ? cache : sl.t[w][l]; p.dst[p.n] = to_slot ? sl.t[w][l] : cache;
+      p.src_pitch[p.n] = to_slot ? cache_pitch : slot_pitch; p.dst_pitch[p.n] = to_slot ? slot_pitch : cache_pitch;
+      p.units[p.n] = (uint32_t)(slot_pitch / 16);
+      if (++p.n == PA_COPY_TENSORS) {
+        const hipError_t e = pa_launch_copy_planes(p, ctx->cfg.n_kv_heads, ctx->stream);
+        if (e != hipSuccess) return e;
+        p.n = 0;
+      }
+    }
+  }
+  return pa_launch_copy_planes(p, ctx->cfg.n_kv_heads, ctx->stream);
 }
 
 extern "C" int pa_slot_save(pa_ctx* ctx, uint32_t slot, uint32_t pos) {
   if (!ctx) return PA_ERR_INVALID;
   int rc = slot_make(ctx, "pa_slot_save", slot, pos);
   if (rc) return rc;
-  pa_slot& sl = ctx->slots[slot];
-  for (size_t l = 0; l < ctx->layers.size(); l++) {
-    if (!sl.t[0][l]) continue;
-    for (int w = 0; w < n_tensors(ctx); w++) HIPCHK(ctx, slot_copy(ctx, w, ctx->layers[l].tensor(w), sl.t[w][l], pos, true));
-  }
+  HIPCHK(ctx, slot_copy(ctx, ctx->slots[slot], true));
   return PA_OK;
 }
 
@@ -1070,11 +1081,9 @@ extern "C" int pa_slot_load(pa_ctx* ctx, uint32_t slot, uint32_t* pos) {
   auto it = ctx->slots.find(slot);
   if (it == ctx->slots.end()) return fail(ctx, PA_ERR_INVALID, "pa_slot_load: no saved slot " + std::to_string(slot));
   pa_slot& sl = it->second;
-  for (size_t l = 0; l < ctx->layers.size(); l++) {
-    if (l >= sl.t[0].size() || !sl.t[0][l]) continue;
-    if (!ctx->layers[l].k) return fail(ctx, PA_ERR_INVALID, "pa_slot_load: the slot holds a layer that has no cache now");
-    for (int w = 0; w < n_tensors(ctx); w++) HIPCHK(ctx, slot_copy(ctx, w, ctx->layers[l].tensor(w), sl.t[w][l], sl.pos, false));
-  }
+  for (size_t l = 0; l < sl.t[0].size() && l < ctx->layers.size(); l++)
+    if (sl.t[0][l] && !ctx->layers[l].k) return fail(ctx, PA_ERR_INVALID, "pa_slot_load: the slot holds a layer that has no cache now");
+  HIPCHK(ctx, slot_copy(ctx, sl, false));
   *pos = sl.pos;
   return PA_OK;
 }

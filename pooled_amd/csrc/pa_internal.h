@@ -134,6 +134,17 @@ hipError_t pa_launch_rmsnorm_f16(const float* x, uint32_t x_stride, const float*
 hipError_t pa_launch_widen_q8(const void* k8, const void* v8, const float* ks, const float* vs, uint16_t* ko, uint16_t* vo,
                               uint32_t n_kv_heads, uint32_t hd, uint32_t head_rows, uint32_t n_live, uint32_t n_rows, hipStream_t s);
 
+// cache planes between two places, several tensors a launch (kv_copy.hip)
+#define PA_COPY_TENSORS 40u
+struct PaCopyParams {
+  const void* src[PA_COPY_TENSORS]; void* dst[PA_COPY_TENSORS];
+  size_t src_pitch[PA_COPY_TENSORS], dst_pitch[PA_COPY_TENSORS];   // bytes between planes
+  uint32_t units[PA_COPY_TENSORS];                                 // 16-byte units of a plane (rows are multiples of 16 bytes)
+  uint32_t first[PA_COPY_TENSORS];                                 // a tensor's first workgroup (set by the launcher)
+  uint32_t n;
+};
+hipError_t pa_launch_copy_planes(PaCopyParams& p, uint32_t n_planes, hipStream_t s);
+
 // ---- context -----------------------------------------------------------------------------------
 
 // One layer's caches.  f16 caches: k, v.  int8 caches (PA_FLAG_KV_Q8): k, v hold int8 values (hd bytes a row), ks, vs

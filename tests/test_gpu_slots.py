@@ -41,6 +41,34 @@ def test_save_overwrite_load_is_byte_exact(shape, pos):
             assert np.array_equal(pa.slot_export(7, l, 1), caches[l][1][:pos])
 
 
+@pytest.mark.parametrize("shape,layers,pos,q8", [("qwen36_moe", 21, 64, False), ("qwen36_moe", 20, 65, False), ("qwen3_1p7b", 11, 1, True),
+                                                 ("qwen38_27b", 10, 127, True), ("qwen3_1p7b", 2, 129, False)])
+def test_save_load_of_many_tensors(shape, layers, pos, q8):
+    """Just as many tensors as one launch of the copy kernel takes, and more; planes of a piece, one row less and one more:
+    the saved rows come back bit for bit, later rows and the rows between two planes stay as they are."""
+    cfg = dict(SHAPES[shape], kv_q8=q8)
+    nkv, hd, max_seq = cfg["n_kv_heads"], cfg["head_dim"], pos + 3
+    rng = np.random.default_rng(pos)
+    dts = [(np.int8, hd)] * 2 + [(np.float32, hd // 32)] * 2 if q8 else [(np.uint16, hd)] * 2
+    draw = lambda dt, n: rng.standard_normal((max_seq, nkv * n)).astype(dt) if dt is np.float32 else rng.integers(-100 if dt is np.int8 else 0, 100, (max_seq, nkv * n)).astype(dt)
+    with PooledAttn(cfg, max_seq, n_layers=layers, max_cols=1) as pa:
+        first = [[draw(dt, n) for dt, n in dts] for _ in range(layers)]
+        second = [[draw(dt, n) for dt, n in dts] for _ in range(layers)]
+        for l in range(layers):
+            pa.layer_alloc(l)
+            for w in range(len(dts)):
+                pa.kv_write(l, w, 0, first[l][w])
+        pa.slot_save(1, pos)
+        for l in range(layers):
+            for w in range(len(dts)):
+                pa.kv_write(l, w, 0, second[l][w])
+        assert pa.slot_load(1) == pos
+        for l in range(layers):
+            for w in range(len(dts)):
+                got = pa.kv_read(l, w, 0, max_seq).reshape(max_seq, -1)
+                assert np.array_equal(got[:pos], first[l][w][:pos]) and np.array_equal(got[pos:], second[l][w][pos:])
+
+
 def test_slot_semantics():
     cfg = SHAPES["qwen36_moe"]
     with PooledAttn(cfg, 200, n_layers=1, max_cols=1) as pa:
