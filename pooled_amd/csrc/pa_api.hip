@@ -843,8 +843,7 @@ extern "C" int pa_gemm(pa_ctx* ctx, const pa_weight* w, const void* d_x_f16, uin
     HIPCHK(ctx, pa_launch_gemm_skinny(p, ctx->n_cu, ctx->stream));
     return PA_OK;
   }
-  const bool wide = pa_gemm_wide_serves(p, ctx->n_cu);
-  if (wide || pa_gemm_mid_serves(p)) {
+  if (pa_gemm_wide_serves(p)) {
     // the weights as f16 in fragment order: a copy kept with the weight from its first large chunk on, while the
     // context's budget lasts (the handle's contents never change); past the budget, or where the allocation fails,
     // widened per call into the context's staging
@@ -867,7 +866,7 @@ extern "C" int pa_gemm(pa_ctx* ctx, const pa_weight* w, const void* d_x_f16, uin
       (void)hipEventDestroy(wm->w16_ready);
       wm->w16_ready = nullptr; wm->w16_stream = nullptr;
     }
-    hipError_t e = pa_launch_gemm_wide(p, w16, widen, !wide, ctx->n_cu, ctx->stream);
+    hipError_t e = pa_launch_gemm_wide(p, w16, widen, ctx->n_cu, ctx->stream);
     if (fresh) {
       hipEvent_t ready = nullptr;
       if (e == hipSuccess) e = hipEventCreateWithFlags(&ready, hipEventDisableTiming);

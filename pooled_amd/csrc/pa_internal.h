@@ -120,12 +120,14 @@ hipError_t pa_launch_gemm(const GemmParams& p, int n_cu, hipStream_t s);
 // a few columns of quantised weights (proj_gemm_skinny.hip)
 bool pa_gemm_skinny_serves(const GemmParams& p);
 hipError_t pa_launch_gemm_skinny(const GemmParams& p, int n_cu, hipStream_t s);
-// large chunks (proj_gemm_wide.hip): the weights widened once into w16 (f16 in fragment order, the caller's staging), then a
+// wider chunks (proj_gemm_wide.hip): the weights widened once into w16 (f16 in fragment order, the caller's staging), then a
 // GEMM over two f16 operands; pa_gemm_wide_serves tells whether a call qualifies
-bool pa_gemm_wide_serves(const GemmParams& p, int n_cu);
+bool pa_gemm_wide_serves(const GemmParams& p);
 size_t pa_gemm_wide_staging_bytes(uint32_t d_out, uint32_t d_in);
-bool pa_gemm_mid_serves(const GemmParams& p);
-hipError_t pa_launch_gemm_wide(const GemmParams& p, uint16_t* w16, bool widen, bool mid, int n_cu, hipStream_t s);
+hipError_t pa_launch_gemm_wide(const GemmParams& p, uint16_t* w16, bool widen, int n_cu, hipStream_t s);
+// its kernel for larger tiles (proj_gemm_tile.hip), and what a call would take there
+float pa_gemm_tile_us(const GemmParams& p, int n_cu);
+hipError_t pa_launch_gemm_tile(const GemmParams& p, const uint16_t* w16, int n_cu, hipStream_t s);
 // rmsnorm of n_cols f32 columns, written as f16 (the GEMM's activation operand)
 hipError_t pa_launch_rmsnorm_f16(const float* x, uint32_t x_stride, const float* w, uint32_t dim, float eps, uint32_t n_cols,
                                  uint16_t* out, uint32_t out_stride, hipStream_t s);

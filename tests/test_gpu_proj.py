@@ -198,6 +198,30 @@ def test_gemm_few_columns(kind, d_out, d_in, n):
         assert _rel(dy.download(np.float32, n * ys).reshape(n, ys)[:, :d_out], 2.0 * ref) < 2e-5, "accumulate"
 
 
+@pytest.mark.parametrize("d_out,d_in,n", [(8074, 256, 454), (8824, 256, 451), (8594, 256, 528), (7884, 128, 834), (8208, 128, 900), (8972, 128, 1028),
+                                          (7342, 128, 1544), (8561, 128, 1544), (4090, 2048, 500), (2040, 384, 3000)])
+def test_gemm_tile_shapes(d_out, d_in, n):
+    """The larger tiles of wide chunks: sizes that take each of 128 columns x 128 / 160 / 192 / 256 / 320 / 384 / 448 rows, 256 x
+    256 and 64 x 128 on a 256-CU part (and 128 x 256 again), one to sixteen stages, ragged on both axes.  Sums in f32 in
+    another order than the f64 oracle's, products of f16 exact: 2e-5 of the largest output as above."""
+    rng = np.random.default_rng(d_out + d_in + n)
+    w, sc = _weights(PA_W_Q8_0, d_out, d_in, rng)
+    x16 = rng.standard_normal((n, d_in)).astype(np.float16)
+    ref = O.gemm_f16(PA_W_Q8_0, w, sc, x16.astype(np.float32))
+    xs, ys = d_in + 8, d_out + 5
+    xpad = np.full((n, xs), np.float16(np.nan)); xpad[:, :d_in] = x16
+    y0 = rng.standard_normal((n, ys)).astype(np.float32)
+    with PooledAttn(SHAPES["qwen36_moe"], 64, n_layers=1, max_cols=1) as pa:
+        wh = pa.weight(PA_W_Q8_0, w, sc)
+        dx = pa.to_device(xpad.view(np.uint16)); dy = pa.to_device(y0)
+        pa.gemm(wh, dx, xs, n, dy, ys); pa.sync()
+        got = dy.download(np.float32, n * ys).reshape(n, ys)
+        assert _rel(got[:, :d_out], ref) < 2e-5, "plain"
+        assert np.array_equal(got[:, d_out:], y0[:, d_out:]), "the stride padding of y must stay untouched"
+        pa.gemm(wh, dx, xs, n, dy, ys, acc=True); pa.sync()
+        assert _rel(dy.download(np.float32, n * ys).reshape(n, ys)[:, :d_out], 2.0 * ref) < 2e-5, "accumulate"
+
+
 @pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])
 def test_gemm_weight_cache_budget(kind):
     """The kept f16 copy and the per-call staging hold the same values: a context with no budget (every call widens into
