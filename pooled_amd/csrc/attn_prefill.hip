@@ -26,6 +26,11 @@
 //     in f16) and takes the 128-register O rescale off the common path.
 //   * Workgroup ids are remapped so that each XCD (ids are dealt round-robin to the 8 XCDs) works on one
 //     contiguous range of (kv head, column block): the K/V stream of a kv head is fetched into one L2.
+//   * Unsplit passes are paired: waves 0-3 take a half block of columns from the front of the chunk, waves 4-7 the one as
+//     far from its back, so that every workgroup has the same work and the causal triangle of a chunk at the start of a
+//     prompt does not leave most CUs idle behind the last columns' workgroups (with one block of neighbouring columns a
+//     workgroup, 4096 columns from 0 of the MoE shape 225 us, paired 180 us: 128 steps at the pace of one wave a SIMD, which
+//     is 0.72 of two waves').  Where half blocks would need a workgroup more than whole ones, the blocks stay whole.
 //   * Optional split over the context (short chunks on long contexts would otherwise leave CUs idle): partial
 //     (m, l, O) go to the same buffers the decode kernel uses and the same merge kernel finishes them.
 #include "pf_common.h"
@@ -43,7 +48,7 @@ template <int HD, int W> struct PfShape {
 };
 
 template <int HD, int QB, int W>
-__global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p, uint32_t n_col_blocks) {
+__global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p, uint32_t n_col_blocks, uint32_t half_cols) {
   typedef PfShape<HD, W> S;
   // four separate LDS objects (two K, two V buffers): the compiler then orders an LDS read only after the
   // LDS-direct loads into the *same* buffer, and the prefetch into the other buffer stays in flight
@@ -67,10 +72,21 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform (scalar) so per-wave branches are scalar branches
   const uint32_t ln = lane & 31, hb = lane >> 5;   // MFMA row / column index, k half
   const uint32_t G = p.group, nH = p.n_heads;
-  const uint32_t c0 = cb * p.cols_per_group;
-  const uint32_t ncl = min(p.cols_per_group, p.n_cols - c0);
+  // columns of this WAVE [c0, c0 + R / G): the workgroup's block, or (half_cols) its half's block: waves of the lower half
+  // take block cb from the front, the others the one as far from the back, so that every workgroup has the same work
+  uint32_t c0 = cb * p.cols_per_group, wrow0 = wave * QB * 32;       // wrow0: the wave's first row in its block
+  uint32_t ncl = min(p.cols_per_group, p.n_cols - c0), c_end = c0 + ncl;
+  if (half_cols) {
+    const uint32_t n_half = (p.n_cols + half_cols - 1) / half_cols, far = n_half - 1 - cb;
+    const bool lower = wave < W / 2;
+    c0 = (lower ? cb : far) * half_cols;
+    if (!lower) wrow0 -= W / 2 * QB * 32;
+    c_end = min((far + 1) * half_cols, p.n_cols);
+    ncl = min(half_cols, p.n_cols - c0);
+    if (far == cb && lower) ncl = 0;               // an odd number of blocks: the middle one is alone
+  }
   const uint32_t R = ncl * G;                      // live rows (<= W * QB * 32)
-  const uint32_t seq_max = p.base_pos + c0 + ncl;  // rows visible to the block's last column
+  const uint32_t seq_max = p.base_pos + c_end;     // rows visible to the workgroup's last column
   const uint32_t t_begin = sp * p.split_len;
   if (t_begin >= seq_max) return;
   const uint32_t t_end = min(t_begin + p.split_len, seq_max);
@@ -113,16 +129,15 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
 
   // ---- per-lane rows: query row of block qb is wave*QB*32 + qb*32 + ln = (column r / G, head r % G) ----
   uint32_t end_pos[QB], row_id[QB];
-  uint32_t w_min_end = 0xffffffffu;
+  uint32_t w_min_end = 0xffffffffu, w_max_end = 0;                // positions seen by the wave's first row, by its last one
 #pragma unroll
   for (int qb = 0; qb < QB; qb++) {
-    const uint32_t r = wave * QB * 32 + qb * 32 + ln;
-    row_id[qb] = min(r, R - 1);
+    const uint32_t r = wrow0 + qb * 32 + ln;
+    row_id[qb] = R ? min(r, R - 1) : 0;
     end_pos[qb] = r < R ? p.base_pos + c0 + r / G + 1 : 0u;
   }
   {
-    const uint32_t r_first = wave * QB * 32;
-    if (r_first < R) w_min_end = p.base_pos + c0 + r_first / G + 1;
+    if (wrow0 < R) { w_min_end = p.base_pos + c0 + wrow0 / G + 1; w_max_end = p.base_pos + c0 + min(wrow0 + QB * 32 - 1, R - 1) / G + 1; }
   }
 
   // ---- Q fragments (B operand of S^T = K Q^T): row ln of block qb, dims 16 ks + 8 hb .. + 7, as f16 ----
@@ -308,9 +323,11 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
       constexpr int par = decltype(PAR)::value;
       const uint32_t tp = t_begin + i * PF_TN;
       if (i + 1 < n_steps) { issue_k(par ? kbuf0 : kbuf1, tp + PF_TN); issue_v(par ? vbuf0 : vbuf1, tp + PF_TN); }
-      qk(par ? kbuf1 : kbuf0, tp);
-      sm(tp);
-      pv(par ? vbuf1 : vbuf0, tp);
+      if (tp < w_max_end) {                         // past it every row of the wave is masked
+        qk(par ? kbuf1 : kbuf0, tp);
+        sm(tp);
+        pv(par ? vbuf1 : vbuf0, tp);
+      }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
     };
@@ -325,7 +342,7 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
 #pragma unroll
   for (int qb = 0; qb < QB; qb++) {
     l_run[qb] += __shfl_xor(l_run[qb], 32, 64);
-    const uint32_t r = wave * QB * 32 + qb * 32 + ln;
+    const uint32_t r = wrow0 + qb * 32 + ln;
     if (r >= R) continue;
     const uint32_t col = c0 + r / G, hq = g * G + r % G;
     if (p.n_splits == 1) {
@@ -380,9 +397,11 @@ static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, hip
     if (e != hipSuccess) return e;
     attr_set = true;
   }
+  const uint32_t half = W / 2 * QB * 32 / p.group;
+  const bool paired = p.n_splits == 1 && half > 0 && ((p.n_cols + half - 1) / half + 1) / 2 == col_groups;
   const uint32_t total = col_groups * p.n_kv_heads * p.n_splits;
   const uint32_t gx = ((total + 7) / 8) * 8;       // whole rounds of the 8 XCDs
-  PA_LAUNCH((pa_prefill_kernel<HD, QB, W>), dim3(gx), dim3(W * 64), lds, s, t, p, col_groups);
+  PA_LAUNCH((pa_prefill_kernel<HD, QB, W>), dim3(gx), dim3(W * 64), lds, s, t, p, col_groups, paired ? half : 0u);
   return hipGetLastError();
 }
 

@@ -47,6 +47,16 @@ def test_prefill_small(shape, base, n):
     assert_parity(got, ref, "%s base %d n %d" % (shape, base, n))
 
 
+@pytest.mark.parametrize("shape", ["qwen36_moe", "qwen38_27b", "qwen3_1p7b"])
+@pytest.mark.parametrize("base,n", [(0, 37), (0, 129), (33, 200), (3, 449)])
+def test_prefill_paired_halves(shape, base, n):
+    """An unsplit pass gives a workgroup a half block of columns from the front and one from the back: one half block alone,
+    odd and even numbers of them, a ragged last one, halves whose row ends are hundreds of positions apart."""
+    got, ref, plan = _prefill(SHAPES[shape], base, n, seed=base + n + 3)
+    assert plan["kernel"] == 1 and plan["n_splits"] == 1
+    assert_parity(got, ref, "paired %s base %d n %d" % (shape, base, n))
+
+
 def test_prefill_equals_decode_columns():
     """Every prefill column equals a single-token decode at the same position (tolerance)."""
     cfg = SHAPES["qwen36_moe"]
