@@ -295,6 +295,61 @@ def test_attn_layer_prefill_matches_oracle(shape, dim, kind, base, n):
         assert np.abs(a - ref).max() <= np.abs(ref).max() * 2.0 ** -9
 
 
+@pytest.mark.parametrize("shape,more,base,n", [
+    ("qwen36_moe", {}, 0, 129),                                   # unsplit halves, last block ragged
+    ("qwen36_moe", dict(kv_q8=True), 700, 70),                    # split over the context (merge kernel), int8 caches
+    ("qwen38_27b", {}, 33, 65),                                   # six heads a kv head
+    ("qwen3_1p7b", {}, 5, 200),                                   # rotation of the whole head (pairs 64 apart), no gate
+    ("qwen3_1p7b", dict(qk_norm=False), 0, 97),
+    ("qwen36_moe", dict(n_rot=256), 40, 48),                      # pairs 128 apart
+    ("qwen36_moe", dict(n_rot=128, qk_norm=False, gate=False), 3, 61),
+    ("qwen36_moe", dict(n_rot=48), 20, 50),                       # pairs inside a k-step: q through the pre-step
+    ("qwen3_1p7b", dict(n_rot=32, gate=True), 0, 80),
+])
+def test_layer_prefill_from_raw_q_columns(shape, more, base, n):
+    """The attention kernel takes q and gate from where the projection left them: the same residual as the stages one by one.
+    The norm's f64 sum runs in another order, so a roped q value may move by one f32 ulp, and its f16 operand by one f16 ulp
+    where that crosses a rounding boundary: 2^-10 of one product of a row's score."""
+    from pooled_amd.capi import PA_OUT_F16
+    cfg = dict(SHAPES[shape], **more)
+    nH, nKV, hd = cfg["n_heads"], cfg["n_kv_heads"], cfg["head_dim"]
+    qd, kvd, dim = nH * hd, nKV * hd, 256
+    q_rows = qd * (2 if cfg["gate"] else 1)
+    rows = q_rows + 2 * kvd
+    rng = np.random.default_rng(base * 1000 + n)
+    w_qkv, s_qkv = _weights(PA_W_Q4_0, rows, dim, rng, scale=0.05)
+    w_o, s_o = _weights(PA_W_Q4_0, dim, qd, rng, scale=0.005)
+    nw = (1 + 0.1 * rng.standard_normal(dim)).astype(np.float32)
+    hw = (1 + 0.1 * rng.standard_normal(hd)).astype(np.float32); hk = (1 + 0.1 * rng.standard_normal(hd)).astype(np.float32)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    outs, caches = [], []
+    with PooledAttn(cfg, base + n + 1, n_layers=2, max_cols=max(base, n)) as pa:
+        pa.set_prefill_tile(1)
+        wq = pa.weight(PA_W_Q4_0, w_qkv, s_qkv); wo = pa.weight(PA_W_Q4_0, w_o, s_o)
+        dnw = pa.to_device(nw); dqw = pa.to_device(hw); dkw = pa.to_device(hk)
+        kraw, vraw = (pa.to_device(rng.standard_normal((max(base, 1), kvd)).astype(np.float32)) for _ in range(2))
+        for layer in (0, 1):
+            pa.layer_alloc(layer)
+            if base:
+                pa.kv_store(layer, kraw, kvd, vraw, kvd, 0, base)
+            dx = pa.to_device(x)
+            if layer == 0:
+                pa.attn_layer_prefill(layer, wq, wo, dnw, dqw, dkw, dx, dim, base, n)
+            else:
+                dxn = pa.alloc(n * dim * 2); dqkv = pa.alloc(n * rows * 4); dat = pa.alloc(n * qd * 2)
+                pa.rmsnorm_f16(dx, dim, dnw, dim, n, dxn, dim)
+                pa.gemm(wq, dxn, dim, n, dqkv, rows)
+                pa.L.pa_glue_kv(pa.ctx, layer, dqkv.ptr, rows, dqkv.ptr + q_rows * 4, rows, dqkv.ptr + (q_rows + kvd) * 4, rows, dqw.ptr, dkw.ptr, base, n)
+                pa.attn("prefill", layer, None, 0, pa.gate_buffer_ptr() if cfg["gate"] else None, qd, base, n, dat, qd, PA_OUT_F16)
+                pa.gemm(wo, dat, qd, n, dx, dim, acc=True)
+            pa.sync()
+            outs.append(dx.download(np.float32, n * dim))
+            caches.append([pa.kv_read(layer, w, base, n) for w in range(4 if cfg.get("kv_q8") else 2)])
+    for a, b in zip(*caches):
+        assert np.array_equal(np.asarray(a), np.asarray(b))
+    assert np.abs(outs[0] - outs[1]).max() <= 2.0 ** -10 * np.abs(outs[1]).max()
+
+
 def test_layer_calls_on_int8_caches_equal_their_stages():
     """pa_attn_layer_decode / pa_attn_layer_prefill on int8 caches: the same bits as their stages called one by one
     (each stage has its own parity test)."""
