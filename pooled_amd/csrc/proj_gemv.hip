@@ -242,27 +242,59 @@ static hipError_t launch_k(const GemvParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
+// rw of 1 .. R rows per wave
+template <int KIND, int BPL, bool NORM, int R>
+static hipError_t launch_rows(uint32_t rw, const GemvParams& p, hipStream_t s) {
+  if constexpr (R > 1) { if (rw < (uint32_t)R) return launch_rows<KIND, BPL, NORM, R - 1>(rw, p, s); }
+  return launch_k<KIND, BPL, R, NORM>(p, s);
+}
+
+// Rows per wave past 4096 inputs (quantised weights).  Every workgroup fetches, norms and stages all of x -- 20 KB and the norm's
+// 20 KB at 5120 inputs, twice the weights of its eight rows at two rows a wave -- so few large workgroups are faster as long as
+// every SIMD keeps two waves and they come out even.  Time follows the rows of the busiest SIMD plus about 1.6 rows' worth for every
+// wave it is dealt; measured at 1 .. 8 rows a wave (us, cold weights, Q4_0): 14336 x 5120 20.6 15.1 14.4 13.6 13.2 13.9 12.5 13.1;
+// 10240 x 5120 16.0 11.8 12.0 11.1 9.9 10.9 11.8 12.9; 8192 x 5120 13.4 10.7 10.1 8.7 9.5 10.6 11.8 9.6; 17000 x 4608 20.5 16.8 13.9
+// 15.0 14.2 13.9 15.0 22.3; Q8_0 14336 x 5120 21.3 20.7 19.9 18.8 18.0 25.6.  With fewer than six rows a SIMD two rows a wave are as
+// good as any (5120 x 6144: 7.3, 7.4 at three, 7.3 at five).  RMAX: what fits the registers of two waves a SIMD.
+static uint32_t wide_rows(uint32_t d_out, int n_cu, uint32_t rmax) {
+  const uint32_t simds = 4u * (uint32_t)n_cu;
+  if (d_out < 6 * simds) return d_out >= 4 * simds ? 2 : 1;
+  uint32_t best = 1;
+  float cost = 1e30f;
+  for (uint32_t r = 1; r <= rmax; r++) {
+    const uint32_t waves = (d_out + r - 1) / r, per_simd = (waves + simds - 1) / simds;
+    const float c = per_simd * (r + 1.6f);
+    if (per_simd >= 2 && c < cost) { best = r; cost = c; }
+  }
+  return best;
+}
+
 template <int KIND, int BPL, bool NORM>
 static hipError_t launch_rw(const GemvParams& p, int n_cu, hipStream_t s) {
-  // rows per wave: as many as still leave about two 4-wave workgroups per CU, within the registers that RW x BPL
-  // blocks of weights take (f32: 32 registers a block, Q8_0: 8, Q4_0: 4)
-  constexpr int RWMAX = (KIND == PA_W_F32 ? 2 : 8) / BPL > 0 ? (KIND == PA_W_F32 ? 2 : 8) / BPL : 1;
-  const uint32_t waves_wanted = 8u * (uint32_t)n_cu;
-  uint32_t rw = p.d_out >= 8 * waves_wanted ? 8 : p.d_out >= 4 * waves_wanted ? 4 : p.d_out >= 2 * waves_wanted ? 2 : 1;
-  if (rw > (uint32_t)RWMAX) rw = RWMAX;
-  // Once the weights are there the kernel is VALU work, and the SIMD with the most rows sets the time: with four rows a
-  // wave the MoE model's 9216 [q|k|v] rows are 2304 waves, 2.25 a SIMD -- some SIMDs work through three waves (12 rows),
-  // most through two.  Three rows a wave are 3072 waves, three on every SIMD (9 rows).  Taken when it lowers the busiest
-  // SIMD's rows.
-  if constexpr (RWMAX >= 4) {
-    const uint32_t simds = 4u * (uint32_t)n_cu;
-    auto busiest = [&](uint32_t r) { const uint32_t waves = (p.d_out + r - 1) / r; return ((waves + simds - 1) / simds) * r; };
-    if (rw == 4 && busiest(3) < busiest(4)) return launch_k<KIND, BPL, 3, NORM>(p, s);
+  if constexpr (BPL >= 3) {
+    constexpr int RMAX = KIND == PA_W_Q4_0 ? (BPL == 3 ? 7 : 4) : (BPL == 3 ? 5 : 3);
+    return launch_rows<KIND, BPL, NORM, RMAX>(wide_rows(p.d_out, n_cu, RMAX), p, s);
+  } else {
+    // rows per wave: as many as still leave about two 4-wave workgroups per CU, within the registers that RW x BPL
+    // blocks of weights take (f32: 32 registers a block, Q8_0: 8, Q4_0: 4)
+    constexpr int RWMAX = (KIND == PA_W_F32 ? 2 : 8) / BPL > 0 ? (KIND == PA_W_F32 ? 2 : 8) / BPL : 1;
+    const uint32_t waves_wanted = 8u * (uint32_t)n_cu;
+    uint32_t rw = p.d_out >= 8 * waves_wanted ? 8 : p.d_out >= 4 * waves_wanted ? 4 : p.d_out >= 2 * waves_wanted ? 2 : 1;
+    if (rw > (uint32_t)RWMAX) rw = RWMAX;
+    // Once the weights are there the kernel is VALU work, and the SIMD with the most rows sets the time: with four rows a
+    // wave the MoE model's 9216 [q|k|v] rows are 2304 waves, 2.25 a SIMD -- some SIMDs work through three waves (12 rows),
+    // most through two.  Three rows a wave are 3072 waves, three on every SIMD (9 rows).  Taken when it lowers the busiest
+    // SIMD's rows.
+    if constexpr (RWMAX >= 4) {
+      const uint32_t simds = 4u * (uint32_t)n_cu;
+      auto busiest = [&](uint32_t r) { const uint32_t waves = (p.d_out + r - 1) / r; return ((waves + simds - 1) / simds) * r; };
+      if (rw == 4 && busiest(3) < busiest(4)) return launch_k<KIND, BPL, 3, NORM>(p, s);
+    }
+    if constexpr (RWMAX >= 8) { if (rw == 8) return launch_k<KIND, BPL, 8, NORM>(p, s); }
+    if constexpr (RWMAX >= 4) { if (rw >= 4) return launch_k<KIND, BPL, 4, NORM>(p, s); }
+    if constexpr (RWMAX >= 2) { if (rw >= 2) return launch_k<KIND, BPL, 2, NORM>(p, s); }
+    return launch_k<KIND, BPL, 1, NORM>(p, s);
   }
-  if constexpr (RWMAX >= 8) { if (rw == 8) return launch_k<KIND, BPL, 8, NORM>(p, s); }
-  if constexpr (RWMAX >= 4) { if (rw >= 4) return launch_k<KIND, BPL, 4, NORM>(p, s); }
-  if constexpr (RWMAX >= 2) { if (rw >= 2) return launch_k<KIND, BPL, 2, NORM>(p, s); }
-  return launch_k<KIND, BPL, 1, NORM>(p, s);
 }
 
 template <int KIND, bool NORM>

@@ -49,6 +49,31 @@ def test_gemv_matches_oracle(kind, d_out, d_in):
         assert np.array_equal(dy.download(np.float32, d_out), got)
 
 
+@pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])
+@pytest.mark.parametrize("d_out,d_in", [(6143, 4128), (6145, 4128), (8191, 5120), (11265, 4160), (14337, 6144), (9001, 6176), (6150, 8192)])
+def test_gemv_many_rows_a_wave(kind, d_out, d_in):
+    """Past 4096 inputs: one to seven rows a wave (d_out over the SIMDs picks), the last wave's rows past the end repeating the last
+    one.  Every tenth row and the last ones are checked."""
+    rng = np.random.default_rng(d_out + d_in + kind)
+    w, sc = _weights(kind, d_out, d_in, rng)
+    x = rng.standard_normal(d_in).astype(np.float32)
+    nw = (1 + 0.1 * rng.standard_normal(d_in)).astype(np.float32)
+    y0 = rng.standard_normal(d_out).astype(np.float32)
+    rows = np.unique(np.r_[0:d_out:10, d_out - 9:d_out])
+    cfg = SHAPES["qwen36_moe"]
+    ref = O.gemv(kind, w[rows], sc[rows], x)
+    ref_n = O.gemv(kind, w[rows], sc[rows], O.rmsnorm(x, nw, cfg["eps"]).astype(np.float32))
+    with PooledAttn(cfg, 64, n_layers=1, max_cols=1) as pa:
+        wh = pa.weight(kind, w, sc)
+        dx = pa.to_device(x); dn = pa.to_device(nw); dy = pa.to_device(np.r_[y0, np.float32(7)])
+        pa.gemv(wh, dx, dy, acc=True); pa.sync()
+        got = dy.download(np.float32, d_out + 1)
+        assert got[d_out] == 7 and _rel(got[rows], ref + y0[rows]) < 2e-5
+        pa.gemv_norm(wh, dx, dn, dy); pa.sync()
+        got = dy.download(np.float32, d_out + 1)
+        assert got[d_out] == 7 and _rel(got[rows], ref_n) < 2e-5
+
+
 @pytest.mark.parametrize("kind", [PA_W_F32, PA_W_Q4_0])
 def test_gemv_norm_matches_rmsnorm_then_gemv(kind):
     cfg = SHAPES["qwen36_moe"]
