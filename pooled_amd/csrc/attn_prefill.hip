@@ -31,6 +31,10 @@
 //     prompt does not leave most CUs idle behind the last columns' workgroups (with one block of neighbouring columns a
 //     workgroup, 4096 columns from 0 of the MoE shape 225 us, paired 180 us: 128 steps at the pace of one wave a SIMD, which
 //     is 0.72 of two waves').  Where half blocks would need a workgroup more than whole ones, the blocks stay whole.
+//   * Unsplit passes of more workgroups than CUs keep whole blocks (halves that end apart run one wave a SIMD for a while: more work
+//     in all), dealt over the XCDs of a kv head in turn, the longest first.  In order of position, one XCD of a head had the front of the
+//     triangle and another the back, the longest blocks last: 4096 columns of the 24 / 4-head shape from 0 420 -> 315 us, 3000 at
+//     3000 567 -> 454.
 //   * Optional split over the context (short chunks on long contexts would otherwise leave CUs idle): partial
 //     (m, l, O) go to the same buffers the decode kernel uses and the same merge kernel finishes them.
 //   * RAW (the layer call): q arrives as the projection left it and is normed and roped on its way into the fragments, with
@@ -105,7 +109,7 @@ static __device__ __attribute__((always_inline)) inline void pf_raw_row(const fl
 
 // RAW: 0, or the rotated dims of the raw q columns (RAW / 32 k-steps between the partners of a pair)
 template <int HD, int QB, int W, int RAW>
-__global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p, uint32_t n_col_blocks, uint32_t half_cols) {
+__global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p, uint32_t n_col_blocks, uint32_t half_cols, uint32_t head_xcds) {
   typedef PfShape<HD, W> S;
   // four separate LDS objects (two K, two V buffers): the compiler then orders an LDS read only after the
   // LDS-direct loads into the *same* buffer, and the prefetch into the other buffer stays in flight
@@ -119,11 +123,19 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   // the same K/V rows.  The grid is one-dimensional; dispatch id i runs on XCD i % 8, and XCD k owns the contiguous
   // item range [k per_xcd, (k + 1) per_xcd): every XCD gets the same number of workgroups whatever the split count,
   // and the workgroups that share a K/V stream share an L2.
-  const uint32_t total = n_col_blocks * p.n_kv_heads * p.n_splits;
-  const uint32_t per_xcd = (total + 7) / 8;
-  const uint32_t lid = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-  if (lid >= total) return;
-  const uint32_t cb = lid % n_col_blocks, sp = (lid / n_col_blocks) % p.n_splits, g = lid / (n_col_blocks * p.n_splits);
+  // head_xcds (unsplit passes of whole blocks): the XCDs of a kv head take its column blocks in turn, the longest first.
+  uint32_t cb, sp, g;
+  if (head_xcds) {
+    const uint32_t xcd = blockIdx.x % 8, i = blockIdx.x / 8 * head_xcds + xcd % head_xcds;
+    if (i >= n_col_blocks) return;
+    cb = n_col_blocks - 1 - i; sp = 0; g = xcd / head_xcds;
+  } else {
+    const uint32_t total = n_col_blocks * p.n_kv_heads * p.n_splits;
+    const uint32_t per_xcd = (total + 7) / 8;
+    const uint32_t lid = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (lid >= total) return;
+    cb = lid % n_col_blocks; sp = (lid / n_col_blocks) % p.n_splits; g = lid / (n_col_blocks * p.n_splits);
+  }
 
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform (scalar) so per-wave branches are scalar branches
@@ -454,7 +466,7 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
 }
 
 template <int HD, int QB, int W, int RAW>
-static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, hipStream_t s, const PaTiming* t) {
+static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t) {
   typedef PfShape<HD, W> S;
   const size_t lds = (size_t)W * QB * (S::KS - S::QR) * 1024;     // Q fragments parked in LDS (dynamic part)
   static bool attr_set = false;
@@ -464,10 +476,13 @@ static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, hip
     attr_set = true;
   }
   const uint32_t half = W / 2 * QB * 32 / p.group;
-  const bool paired = p.n_splits == 1 && half > 0 && ((p.n_cols + half - 1) / half + 1) / 2 == col_groups;
   const uint32_t total = col_groups * p.n_kv_heads * p.n_splits;
-  const uint32_t gx = ((total + 7) / 8) * 8;       // whole rounds of the 8 XCDs
-  PA_LAUNCH((pa_prefill_kernel<HD, QB, W, RAW>), dim3(gx), dim3(W * 64), lds, s, t, p, col_groups, paired ? half : 0u);
+  // Halves of a workgroup that end apart run one wave a SIMD for a while, so pairing costs work to save the wait for the longest
+  // block: it pays while the chip holds all workgroups at once.  More of them: whole blocks, the longest first.
+  const bool paired = p.n_splits == 1 && half > 0 && total <= n_cu && ((p.n_cols + half - 1) / half + 1) / 2 == col_groups;
+  const uint32_t head_xcds = p.n_splits == 1 && !paired && 8 % p.n_kv_heads == 0 ? 8 / p.n_kv_heads : 0;
+  const uint32_t gx = 8 * (head_xcds ? (col_groups + head_xcds - 1) / head_xcds : (total + 7) / 8);       // whole rounds of the 8 XCDs
+  PA_LAUNCH((pa_prefill_kernel<HD, QB, W, RAW>), dim3(gx), dim3(W * 64), lds, s, t, p, col_groups, paired ? half : 0u, head_xcds);
   return hipGetLastError();
 }
 
@@ -476,19 +491,19 @@ static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, hip
 bool pa_prefill_raw_serves(uint32_t n_rot) { return n_rot == 64 || n_rot == 128 || n_rot == 256; }
 
 // row_blocks = 32-row query blocks per workgroup (8: one per wavefront)
-hipError_t pa_launch_prefill(const AttnParams& p, uint32_t hd, uint32_t row_blocks, uint32_t col_groups, hipStream_t s, const PaTiming* t) {
+hipError_t pa_launch_prefill(const AttnParams& p, uint32_t hd, uint32_t row_blocks, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t) {
   if (row_blocks != 8) return hipErrorNotSupported;
   const uint32_t raw = p.f_q_in ? p.n_rot : 0;
   if (hd == 256) switch (raw) {
-    case 0: return launch_prefill_t<256, 1, 8, 0>(p, col_groups, s, t);
-    case 64: return launch_prefill_t<256, 1, 8, 64>(p, col_groups, s, t);
-    case 128: return launch_prefill_t<256, 1, 8, 128>(p, col_groups, s, t);
-    case 256: return launch_prefill_t<256, 1, 8, 256>(p, col_groups, s, t);
+    case 0: return launch_prefill_t<256, 1, 8, 0>(p, col_groups, n_cu, s, t);
+    case 64: return launch_prefill_t<256, 1, 8, 64>(p, col_groups, n_cu, s, t);
+    case 128: return launch_prefill_t<256, 1, 8, 128>(p, col_groups, n_cu, s, t);
+    case 256: return launch_prefill_t<256, 1, 8, 256>(p, col_groups, n_cu, s, t);
   }
   if (hd == 128) switch (raw) {
-    case 0: return launch_prefill_t<128, 1, 8, 0>(p, col_groups, s, t);
-    case 64: return launch_prefill_t<128, 1, 8, 64>(p, col_groups, s, t);
-    case 128: return launch_prefill_t<128, 1, 8, 128>(p, col_groups, s, t);
+    case 0: return launch_prefill_t<128, 1, 8, 0>(p, col_groups, n_cu, s, t);
+    case 64: return launch_prefill_t<128, 1, 8, 64>(p, col_groups, n_cu, s, t);
+    case 128: return launch_prefill_t<128, 1, 8, 128>(p, col_groups, n_cu, s, t);
   }
   return hipErrorNotSupported;
 }

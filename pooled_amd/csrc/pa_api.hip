@@ -662,7 +662,7 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
   PaTiming tm;
   if ((rc = prof_pair(ctx, &tm))) return rc;
   if (pl.kernel == 0) HIPCHK(ctx, pa_launch_decode(p, c.head_dim, pl.row_blocks, pl.waves, pl.col_groups, ctx->stream, &tm));
-  else HIPCHK(ctx, pa_launch_prefill(p, c.head_dim, pl.row_blocks, pl.col_groups, ctx->stream, &tm));
+  else HIPCHK(ctx, pa_launch_prefill(p, c.head_dim, pl.row_blocks, pl.col_groups, ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u, ctx->stream, &tm));
   if (!direct) {
     PaTiming tm2;
     if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;

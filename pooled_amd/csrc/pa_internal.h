@@ -97,7 +97,7 @@ hipError_t pa_launch_combine(const AttnParams& p, uint32_t hd, hipStream_t s, co
 // whether the MFMA prefill kernel takes raw q columns of this rotation
 bool pa_prefill_raw_serves(uint32_t n_rot);
 // MFMA prefill; returns hipErrorNotSupported for shapes it does not cover
-hipError_t pa_launch_prefill(const AttnParams& p, uint32_t hd, uint32_t row_blocks, uint32_t col_groups, hipStream_t s, const PaTiming* t = nullptr);
+hipError_t pa_launch_prefill(const AttnParams& p, uint32_t hd, uint32_t row_blocks, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t = nullptr);
 
 // one-token projection y = W x (proj_gemv.hip): kind PA_W_*, w = f32 [d_out][d_in] / int8 [d_out][d_in] / nibbles
 // [d_out][d_in / 2], scales = f16 bits [d_out][d_in / 32] (quantised kinds); norm_w != nullptr: x is the raw vector and

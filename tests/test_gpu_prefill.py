@@ -57,6 +57,18 @@ def test_prefill_paired_halves(shape, base, n):
     assert_parity(got, ref, "paired %s base %d n %d" % (shape, base, n))
 
 
+@pytest.mark.parametrize("n_kv,n", [(4, 260), (4, 257), (8, 133), (1, 1027), (3, 345)])
+def test_prefill_more_workgroups_than_cus(n_kv, n):
+    """An unsplit pass of more workgroups than the chip holds takes whole blocks of columns, the longest first, dealt over the
+    XCDs of a kv head: one, two or eight of them, numbers of blocks that do not come out even, and (three kv heads) the
+    general mapping."""
+    cfg = dict(SHAPES["qwen3_1p7b"], n_heads=64 * n_kv, n_kv_heads=n_kv)           # 64 heads a kv head: blocks of four columns
+    rows = sorted(set(range(0, n, max(1, n // 60))) | set(range(8)) | set(range(n - 8, n)))
+    got, ref, plan = _prefill(cfg, 21, n, seed=n, check_rows=rows)
+    assert plan["kernel"] == 1 and plan["n_splits"] == 1 and plan["col_groups"] * n_kv > 256
+    assert_parity(got, ref, "whole blocks, %d kv heads n %d" % (n_kv, n))
+
+
 def test_prefill_equals_decode_columns():
     """Every prefill column equals a single-token decode at the same position (tolerance)."""
     cfg = SHAPES["qwen36_moe"]
