@@ -930,11 +930,16 @@ extern "C" int pa_attn_layer_prefill(pa_ctx* ctx, uint32_t layer, const pa_weigh
   uint16_t* at = (uint16_t*)((unsigned char*)ctx->chunk_buf + b_xn + b_qkv);
   if ((rc = pa_rmsnorm_f16(ctx, d_x, x_stride, d_attn_norm_w, dim, n_cols, xn, dim))) return rc;
   if ((rc = pa_gemm(ctx, w_qkv, xn, dim, n_cols, qkv, rows, 0))) return rc;
-  // The gate is read in place by whichever kernel writes the output.  A chunk on the MFMA kernel takes its q columns as they are, too;
-  // the split-K kernel's groups of a few columns would each norm and rope them again, so there the pre-step does it once.
+  // The gate is read in place by whichever kernel writes the output.  A wide chunk on the MFMA kernel takes its q columns as they are,
+  // too: that kernel then starts 4.5 us (head_dim 128: 2.1 us) later, and the pre-step saves 8 bytes a q value, next to nothing while it
+  // is latency-bound.  Measured (us a layer, raw / through the pre-step): 16 heads x 60 columns 72.5 / 68.5, x 200 102.9 / 101.4,
+  // x 900 153 / 155, 24 x 400 212.7 / 212.8, 24 x 680 278 / 280, head_dim 128 16 x 100 51.1 / 49.3, x 1000 111.8 / 113.0: the line is at
+  // about 10000 (column, head) rows.  pa_set_prefill_tile 1: always.
+  // The split-K kernel's groups of a few columns would each norm and rope them again, so there the pre-step does it once.
   const uint32_t head_stride = c.head_dim * (gated ? 2 : 1);
   pa_plan pl;
-  const bool raw_q = ctx->rope_tab && pa_prefill_raw_serves(c.n_rot) && plan_prefill(ctx, base_pos, n_cols, &pl) == PA_OK && pl.kernel == 1;
+  const bool wide = (uint64_t)n_cols * c.n_heads >= 10240 || ctx->prefill_tile_mode == 1;
+  const bool raw_q = wide && ctx->rope_tab && pa_prefill_raw_serves(c.n_rot) && plan_prefill(ctx, base_pos, n_cols, &pl) == PA_OK && pl.kernel == 1;
   const RawQ raw = { qkv, (c.flags & PA_FLAG_QK_NORM) ? d_qw : nullptr, head_stride };
   if ((rc = glue_kv_common(ctx, layer, qkv, rows, qkv + q_rows, rows, qkv + q_rows + kvd, rows, d_qw, d_kw, base_pos, n_cols, !raw_q, false))) return rc;
   if ((rc = attn_common(ctx, "pa_attn_prefill", 1, layer, raw_q ? qkv : nullptr, rows, gated ? qkv + c.head_dim : nullptr, rows, base_pos, n_cols,

@@ -320,6 +320,7 @@ def test_attn_layer_prefill_matches_oracle(shape, dim, kind, base, n):
         assert np.abs(a - ref).max() <= np.abs(ref).max() * 2.0 ** -9
 
 
+@pytest.mark.parametrize("tile", [1, 0])                          # 1: raw q columns; 0: the table, where these few go through the pre-step
 @pytest.mark.parametrize("shape,more,base,n", [
     ("qwen36_moe", {}, 0, 129),                                   # unsplit halves, last block ragged
     ("qwen36_moe", dict(kv_q8=True), 700, 70),                    # split over the context (merge kernel), int8 caches
@@ -331,7 +332,7 @@ def test_attn_layer_prefill_matches_oracle(shape, dim, kind, base, n):
     ("qwen36_moe", dict(n_rot=48), 20, 50),                       # pairs inside a k-step: q through the pre-step
     ("qwen3_1p7b", dict(n_rot=32, gate=True), 0, 80),
 ])
-def test_layer_prefill_from_raw_q_columns(shape, more, base, n):
+def test_layer_prefill_from_raw_q_columns(shape, more, base, n, tile):
     """The attention kernel takes q and gate from where the projection left them: the same residual as the stages one by one.
     The norm's f64 sum runs in another order, so a roped q value may move by one f32 ulp, and its f16 operand by one f16 ulp
     where that crosses a rounding boundary: 2^-10 of one product of a row's score."""
@@ -349,7 +350,7 @@ def test_layer_prefill_from_raw_q_columns(shape, more, base, n):
     x = rng.standard_normal((n, dim)).astype(np.float32)
     outs, caches = [], []
     with PooledAttn(cfg, base + n + 1, n_layers=2, max_cols=max(base, n)) as pa:
-        pa.set_prefill_tile(1)
+        pa.set_prefill_tile(tile)
         wq = pa.weight(PA_W_Q4_0, w_qkv, s_qkv); wo = pa.weight(PA_W_Q4_0, w_o, s_o)
         dnw = pa.to_device(nw); dqw = pa.to_device(hw); dkw = pa.to_device(hk)
         kraw, vraw = (pa.to_device(rng.standard_normal((max(base, 1), kvd)).astype(np.float32)) for _ in range(2))
