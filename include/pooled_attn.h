@@ -317,8 +317,7 @@ int pa_set_weight_cache(pa_ctx* ctx, size_t max_bytes);
  * pre-step + cache write -> causal attention -> gate -> wo GEMM accumulated into the residual columns d_x
  * [n_cols][x_stride] (f32, read and updated in place).  Weights as pa_attn_layer_decode.  Five launches (six when
  * the attention pass is split).  n_cols <= max_cols.  On int8 caches one more launch widens the visible rows for the
- * prefill kernel (as pa_attn_prefill on such caches).  pa_q_buffer / pa_gate_buffer hold nothing of use afterwards: the
- * attention kernel takes the gate, and on wide chunks the raw q columns, from where the projection left them. */
+ * prefill kernel (as pa_attn_prefill on such caches). */
 int pa_attn_layer_prefill(pa_ctx* ctx, uint32_t layer, const pa_weight* w_qkv, const pa_weight* w_o, const float* d_attn_norm_w,
                           const float* d_qw, const float* d_kw, float* d_x, uint32_t x_stride, uint32_t base_pos, uint32_t n_cols);
 

@@ -37,14 +37,7 @@
 //     3000 567 -> 454.
 //   * Optional split over the context (short chunks on long contexts would otherwise leave CUs idle): partial
 //     (m, l, O) go to the same buffers the decode kernel uses and the same merge kernel finishes them.
-//   * RAW (the layer call): q arrives as the projection left it and is normed and roped on its way into the fragments, with
-//     the pre-step's operations on the same values.  A lane of the Q fragment holds half of a row (dims 16 ks + 8 hb .. + 7) and,
-//     with rotation distances of whole k-steps, both partners of every pair, so the head never leaves its registers: one
-//     exchange between the two halves for the sum of squares.  The gate is read in place from the same columns.  That takes the
-//     chunk's q and gate out of the pre-step, which is HBM-bound (four f32 planes in and out): 4096 columns of the MoE shape
-//     53.7 -> 7.2 us, 777 of the 27B shape 19.2 -> 5.7 us; this kernel 174 -> 181 and 118 -> 124 us.
 #include "pf_common.h"
-#include "glue_math.h"
 
 template <int HD, int W> struct PfShape {
   static constexpr int ROWB = HD * 2;             // bytes of one kv head's row
@@ -58,57 +51,7 @@ template <int HD, int W> struct PfShape {
   static_assert(NLD >= 1 && NLD * W * RPB == PF_TN, "tile must divide evenly over the waves");
 };
 
-// One query row as the projection left it, normed and roped (the arithmetic of glue_math.h): x[ks][e] is dim 16 ks + 8 hb + e,
-// lanes l and l ^ 32 hold the two halves of a row.  src and w point at the lane's first dim, tab at its first pair's (cos, sin).
-template <int KS, int HS>
-static __device__ __attribute__((always_inline)) inline void pf_rope(const float2* tab, float (&x)[KS][8]) {
-#pragma clang fp contract(off)
-#pragma unroll
-  for (int ks = 0; ks < HS; ks++) {
-    f4 cs[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) cs[i] = ((const f4*)(tab + 16 * ks))[i];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const float c = cs[e / 2][2 * (e & 1)], s = cs[e / 2][2 * (e & 1) + 1];
-      const float a = x[ks][e], b = x[ks + HS][e];
-      const float ac = a * c, bs = b * s, bc = b * c, as = a * s;       // rounded one by one
-      x[ks][e] = ac - bs;
-      x[ks + HS][e] = bc + as;
-    }
-  }
-}
-template <int KS, int HS>
-static __device__ __attribute__((always_inline)) inline void pf_raw_row(const float* src, const float* w, const float2* tab, float eps, float (&x)[KS][8]) {
-#pragma clang fp contract(off)
-#pragma unroll
-  for (int ks = 0; ks < KS; ks++) {
-    const f4 a = *(const f4*)(src + 16 * ks), b = *(const f4*)(src + 16 * ks + 4);
-#pragma unroll
-    for (int e = 0; e < 4; e++) { x[ks][e] = a[e]; x[ks][4 + e] = b[e]; }
-  }
-  if (w) {
-    double ss = 0.0;
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++)
-#pragma unroll
-      for (int e = 0; e < 8; e++) ss += (double)x[ks][e] * (double)x[ks][e];
-    ss += __shfl_xor(ss, 32, 64);
-    const float inv = rms_inv(ss, 16 * KS, eps);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      const f4 a = *(const f4*)(w + 16 * ks), b = *(const f4*)(w + 16 * ks + 4);
-#pragma unroll
-      for (int e = 0; e < 8; e++) { const float sw = inv * (e < 4 ? a[e & 3] : b[e & 3]); x[ks][e] = x[ks][e] * sw; }
-      if (ks % 4 == 3) __builtin_amdgcn_sched_barrier(0);              // the weights of four k-steps at a time: all at once do not fit
-    }
-  }
-  pf_rope<KS, HS>(tab, x);
-}
-
-// RAW: 0, or the rotated dims of the raw q columns (RAW / 32 k-steps between the partners of a pair)
-template <int HD, int QB, int W, int RAW>
+template <int HD, int QB, int W>
 __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p, uint32_t n_col_blocks, uint32_t half_cols, uint32_t head_xcds) {
   typedef PfShape<HD, W> S;
   // four separate LDS objects (two K, two V buffers): the compiler then orders an LDS read only after the
@@ -220,19 +163,10 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   h8 qf[QB][QR];
 #pragma unroll
   for (int qb = 0; qb < QB; qb++) {
-    const uint32_t q_col = c0 + row_id[qb] / G, q_head = g * G + row_id[qb] % G;
-    const float* qrow = (RAW ? p.f_q_in + (size_t)q_col * p.q_stride + (size_t)q_head * p.f_q_head_stride
-                             : p.q + (size_t)q_col * p.q_stride + (size_t)q_head * HD) + 8 * hb;
-    float x[RAW ? S::KS : 1][8];
-    if constexpr (RAW != 0) pf_raw_row<S::KS, RAW / 32>(qrow, p.f_qw ? p.f_qw + 8 * hb : nullptr, p.rope_tab + (size_t)(p.base_pos + q_col) * (RAW / 2) + 8 * hb, p.eps, x);
+    const float* qrow = p.q + (size_t)(c0 + row_id[qb] / G) * p.q_stride + (size_t)(g * G + row_id[qb] % G) * HD + 8 * hb;
 #pragma unroll
     for (int ks = 0; ks < S::KS; ks++) {
-      f4 a, b;
-      if constexpr (RAW != 0) {
-        a = (f4){ x[ks][0], x[ks][1], x[ks][2], x[ks][3] }; b = (f4){ x[ks][4], x[ks][5], x[ks][6], x[ks][7] };
-      } else {
-        a = *(const f4*)(qrow + 16 * ks); b = *(const f4*)(qrow + 16 * ks + 4);
-      }
+      const f4 a = *(const f4*)(qrow + 16 * ks), b = *(const f4*)(qrow + 16 * ks + 4);
       const h8 f = { (_Float16)a[0], (_Float16)a[1], (_Float16)a[2], (_Float16)a[3],
                      (_Float16)b[0], (_Float16)b[1], (_Float16)b[2], (_Float16)b[3] };
       if (ks < QR) qf[qb][ks] = f;
@@ -426,7 +360,7 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
     if (p.n_splits == 1) {
       // the whole context was seen: normalise, gate, convert, store
       const float inv_l = 1.f / l_run[qb];
-      const float* gate = p.gate ? p.gate + (size_t)col * p.gate_stride + (size_t)hq * p.gate_head_stride : nullptr;
+      const float* gate = p.gate ? p.gate + (size_t)col * p.gate_stride + (size_t)hq * HD : nullptr;
 #pragma unroll
       for (int db = 0; db < S::DB; db++) {
 #pragma unroll
@@ -465,13 +399,13 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   }
 }
 
-template <int HD, int QB, int W, int RAW>
+template <int HD, int QB, int W>
 static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t) {
   typedef PfShape<HD, W> S;
   const size_t lds = (size_t)W * QB * (S::KS - S::QR) * 1024;     // Q fragments parked in LDS (dynamic part)
   static bool attr_set = false;
   if (!attr_set && lds > 0) {
-    hipError_t e = hipFuncSetAttribute((const void*)pa_prefill_kernel<HD, QB, W, RAW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = hipFuncSetAttribute((const void*)pa_prefill_kernel<HD, QB, W>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     attr_set = true;
   }
@@ -482,28 +416,14 @@ static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, uin
   const bool paired = p.n_splits == 1 && half > 0 && total <= n_cu && ((p.n_cols + half - 1) / half + 1) / 2 == col_groups;
   const uint32_t head_xcds = p.n_splits == 1 && !paired && 8 % p.n_kv_heads == 0 ? 8 / p.n_kv_heads : 0;
   const uint32_t gx = 8 * (head_xcds ? (col_groups + head_xcds - 1) / head_xcds : (total + 7) / 8);       // whole rounds of the 8 XCDs
-  PA_LAUNCH((pa_prefill_kernel<HD, QB, W, RAW>), dim3(gx), dim3(W * 64), lds, s, t, p, col_groups, paired ? half : 0u, head_xcds);
+  PA_LAUNCH((pa_prefill_kernel<HD, QB, W>), dim3(gx), dim3(W * 64), lds, s, t, p, col_groups, paired ? half : 0u, head_xcds);
   return hipGetLastError();
 }
-
-// raw q columns: the partners of a rotation pair must sit in the same lane of the Q fragment, whole k-steps (16 dims) apart;
-// instantiated for the usual partial and full rotations
-bool pa_prefill_raw_serves(uint32_t n_rot) { return n_rot == 64 || n_rot == 128 || n_rot == 256; }
 
 // row_blocks = 32-row query blocks per workgroup (8: one per wavefront)
 hipError_t pa_launch_prefill(const AttnParams& p, uint32_t hd, uint32_t row_blocks, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t) {
   if (row_blocks != 8) return hipErrorNotSupported;
-  const uint32_t raw = p.f_q_in ? p.n_rot : 0;
-  if (hd == 256) switch (raw) {
-    case 0: return launch_prefill_t<256, 1, 8, 0>(p, col_groups, n_cu, s, t);
-    case 64: return launch_prefill_t<256, 1, 8, 64>(p, col_groups, n_cu, s, t);
-    case 128: return launch_prefill_t<256, 1, 8, 128>(p, col_groups, n_cu, s, t);
-    case 256: return launch_prefill_t<256, 1, 8, 256>(p, col_groups, n_cu, s, t);
-  }
-  if (hd == 128) switch (raw) {
-    case 0: return launch_prefill_t<128, 1, 8, 0>(p, col_groups, n_cu, s, t);
-    case 64: return launch_prefill_t<128, 1, 8, 64>(p, col_groups, n_cu, s, t);
-    case 128: return launch_prefill_t<128, 1, 8, 128>(p, col_groups, n_cu, s, t);
-  }
+  if (hd == 256) return launch_prefill_t<256, 1, 8>(p, col_groups, n_cu, s, t);
+  if (hd == 128) return launch_prefill_t<128, 1, 8>(p, col_groups, n_cu, s, t);
   return hipErrorNotSupported;
 }

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(64) void pa_glue_kernel(GlueParams p) {
   float x[4], gt[4] = {0.f, 0.f, 0.f, 0.f}, w[4] = {0.f, 0.f, 0.f, 0.f};
   float2 vv[2] = { make_float2(0.f, 0.f), make_float2(0.f, 0.f) };
   float2 cs[2] = { make_float2(1.f, 0.f), make_float2(1.f, 0.f) };
-  const bool gate_copy = isQ && gated && p.gate_out;
+  const bool gate_copy = isQ && gated;
   const bool v_copy = !isQ && p.k_cache && !p.ks_cache;
   const uint32_t half = math ? p.n_rot / 2 : 0;
   const bool norm = math && (p.flags & PA_FLAG_QK_NORM);

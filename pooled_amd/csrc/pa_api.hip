@@ -248,11 +248,9 @@ static void fill_glue(const pa_ctx* ctx, GlueParams& p) {
   p.head_rows = c.max_seq + 32;
 }
 
-// with_q false: key and value rows only (the attention kernel takes the raw q columns itself); with_gate false: the gate stays
-// where it is, for a reader that takes it in place
-static int glue_kv_common(pa_ctx* ctx, uint32_t layer, const float* d_q_in, uint32_t q_stride, const float* d_k, uint32_t k_stride,
-                          const float* d_v, uint32_t v_stride, const float* d_qw, const float* d_kw, uint32_t base_pos, uint32_t n_cols,
-                          bool with_q, bool with_gate) {
+extern "C" int pa_glue_kv(pa_ctx* ctx, uint32_t layer, const float* d_q_in, uint32_t q_stride, const float* d_k,
+                          uint32_t k_stride, const float* d_v, uint32_t v_stride, const float* d_qw, const float* d_kw,
+                          uint32_t base_pos, uint32_t n_cols) {
   if (!ctx) return PA_ERR_INVALID;
   int rc = check_cols(ctx, "pa_glue_kv", layer, true, base_pos, n_cols);
   if (rc) return rc;
@@ -266,16 +264,8 @@ static int glue_kv_common(pa_ctx* ctx, uint32_t layer, const float* d_q_in, uint
   p.k_cache = ctx->layers[layer].k; p.v_cache = ctx->layers[layer].v; p.ks_cache = ctx->layers[layer].ks; p.vs_cache = ctx->layers[layer].vs;
   p.q_stride = q_stride; p.k_stride = k_stride; p.v_stride = v_stride;
   p.base_pos = base_pos; p.n_cols = n_cols;
-  if (!with_q) p.n_heads = 0;
-  if (!with_gate) p.gate_out = nullptr;
   HIPCHK(ctx, pa_launch_glue(p, ctx->stream));
   return PA_OK;
-}
-
-extern "C" int pa_glue_kv(pa_ctx* ctx, uint32_t layer, const float* d_q_in, uint32_t q_stride, const float* d_k,
-                          uint32_t k_stride, const float* d_v, uint32_t v_stride, const float* d_qw, const float* d_kw,
-                          uint32_t base_pos, uint32_t n_cols) {
-  return glue_kv_common(ctx, layer, d_q_in, q_stride, d_k, k_stride, d_v, v_stride, d_qw, d_kw, base_pos, n_cols, true, true);
 }
 
 extern "C" int pa_glue(pa_ctx* ctx, const float* d_q_in, uint32_t q_stride, float* d_k, uint32_t k_stride,
@@ -540,13 +530,9 @@ static int prof_aux_pair(pa_ctx* ctx, const PaTiming& main, PaTiming* t) {
   return PA_OK;
 }
 
-// q columns as the projection left them (heads head_stride floats apart), for a plan on the MFMA prefill kernel
-struct RawQ { const float* q_in; const float* qw; uint32_t head_stride; };
-
-// gate_head_stride: floats between the heads of a gate column (0: head_dim); raw: d_q is not read
 static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, const float* d_q, uint32_t q_stride,
                        const float* d_gate, uint32_t gate_stride, uint32_t base_pos, uint32_t n_cols, void* d_out,
-                       uint32_t out_stride, int out_dtype, uint32_t gate_head_stride = 0, const RawQ* raw = nullptr) {
+                       uint32_t out_stride, int out_dtype) {
   if (!ctx) return PA_ERR_INVALID;
   int rc = check_cols(ctx, who, layer, true, base_pos, n_cols);
   if (rc) return rc;
@@ -653,12 +639,7 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
   p.single_round2 = plan_single_round2(pl);
   p.max_seq = c.max_seq; p.out_f16 = out_dtype == PA_OUT_F16;
   p.scale = (float)(1.0 / std::sqrt((double)c.head_dim));
-  p.gate_head_stride = gate_head_stride ? gate_head_stride : c.head_dim;
-  if (raw) {
-    if (pl.kernel != 1) return fail(ctx, PA_ERR_UNSUPPORTED, std::string(who) + ": raw q columns outside the prefill kernel");
-    p.f_q_in = raw->q_in; p.f_qw = raw->qw; p.f_q_head_stride = raw->head_stride;
-    p.rope_tab = ctx->rope_tab; p.n_rot = c.n_rot; p.eps = c.eps;
-  }
+  p.gate_head_stride = c.head_dim;
   PaTiming tm;
   if ((rc = prof_pair(ctx, &tm))) return rc;
   if (pl.kernel == 0) HIPCHK(ctx, pa_launch_decode(p, c.head_dim, pl.row_blocks, pl.waves, pl.col_groups, ctx->stream, &tm));
@@ -930,20 +911,8 @@ extern "C" int pa_attn_layer_prefill(pa_ctx* ctx, uint32_t layer, const pa_weigh
   uint16_t* at = (uint16_t*)((unsigned char*)ctx->chunk_buf + b_xn + b_qkv);
   if ((rc = pa_rmsnorm_f16(ctx, d_x, x_stride, d_attn_norm_w, dim, n_cols, xn, dim))) return rc;
   if ((rc = pa_gemm(ctx, w_qkv, xn, dim, n_cols, qkv, rows, 0))) return rc;
-  // The gate is read in place by whichever kernel writes the output.  A wide chunk on the MFMA kernel takes its q columns as they are,
-  // too: that kernel then starts 4.5 us (head_dim 128: 2.1 us) later, and the pre-step saves 8 bytes a q value, next to nothing while it
-  // is latency-bound.  Measured (us a layer, raw / through the pre-step): 16 heads x 60 columns 72.5 / 68.5, x 200 102.9 / 101.4,
-  // x 900 153 / 155, 24 x 400 212.7 / 212.8, 24 x 680 278 / 280, head_dim 128 16 x 100 51.1 / 49.3, x 1000 111.8 / 113.0: the line is at
-  // about 10000 (column, head) rows.  pa_set_prefill_tile 1: always.
-  // The split-K kernel's groups of a few columns would each norm and rope them again, so there the pre-step does it once.
-  const uint32_t head_stride = c.head_dim * (gated ? 2 : 1);
-  pa_plan pl;
-  const bool wide = (uint64_t)n_cols * c.n_heads >= 10240 || ctx->prefill_tile_mode == 1;
-  const bool raw_q = wide && ctx->rope_tab && pa_prefill_raw_serves(c.n_rot) && plan_prefill(ctx, base_pos, n_cols, &pl) == PA_OK && pl.kernel == 1;
-  const RawQ raw = { qkv, (c.flags & PA_FLAG_QK_NORM) ? d_qw : nullptr, head_stride };
-  if ((rc = glue_kv_common(ctx, layer, qkv, rows, qkv + q_rows, rows, qkv + q_rows + kvd, rows, d_qw, d_kw, base_pos, n_cols, !raw_q, false))) return rc;
-  if ((rc = attn_common(ctx, "pa_attn_prefill", 1, layer, raw_q ? qkv : nullptr, rows, gated ? qkv + c.head_dim : nullptr, rows, base_pos, n_cols,
-                        at, qd, PA_OUT_F16, head_stride, raw_q ? &raw : nullptr))) return rc;
+  if ((rc = pa_glue_kv(ctx, layer, qkv, rows, qkv + q_rows, rows, qkv + q_rows + kvd, rows, d_qw, d_kw, base_pos, n_cols))) return rc;
+  if ((rc = pa_attn_prefill(ctx, layer, nullptr, 0, gated ? ctx->gate_buf : nullptr, qd, base_pos, n_cols, at, qd, PA_OUT_F16))) return rc;
   return pa_gemm(ctx, w_o, at, qd, n_cols, d_x, x_stride, 1);
 }
 

@@ -50,8 +50,7 @@ struct AttnParams {
                                               // when gate is read in place from an interleaved [q | gate] column)
   uint32_t part_f16;                          // 1: the O partials in part_o are f16 rows [slot][hd] (single-round decode splits
                                               // merged by the wavefront kernel); 0: f32
-  // fused pre-step of pa_attn_decode_step (one column at base_pos; f_q_in == nullptr otherwise): raw projections.
-  // The MFMA prefill kernel takes raw q columns the same way (f_q_in with q_stride floats between columns, q unused; the table set)
+  // fused pre-step of pa_attn_decode_step (one column at base_pos; f_q_in == nullptr otherwise): raw projections
   const float* f_q_in; const float* f_k_in; const float* f_v_in;   // [nH][q_head_stride], [nKV][hd], [nKV][hd]
   const float* f_qw; const float* f_kw;       // norm weights [hd] or nullptr
   const float2* rope_tab; const float* inv_freq;
@@ -94,8 +93,6 @@ hipError_t pa_launch_decode_gather(const AttnParams& p, uint32_t hd, hipStream_t
 hipError_t pa_launch_decode_step(const AttnParams& p, uint32_t hd, hipStream_t s, const PaTiming* t = nullptr);
 hipError_t pa_prepare_decode_step(uint32_t hd, bool q8);
 hipError_t pa_launch_combine(const AttnParams& p, uint32_t hd, hipStream_t s, const PaTiming* t = nullptr);
-// whether the MFMA prefill kernel takes raw q columns of this rotation
-bool pa_prefill_raw_serves(uint32_t n_rot);
 // MFMA prefill; returns hipErrorNotSupported for shapes it does not cover
 hipError_t pa_launch_prefill(const AttnParams& p, uint32_t hd, uint32_t row_blocks, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t = nullptr);
 

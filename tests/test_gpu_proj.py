@@ -320,7 +320,7 @@ def test_attn_layer_prefill_matches_oracle(shape, dim, kind, base, n):
         assert np.abs(a - ref).max() <= np.abs(ref).max() * 2.0 ** -9
 
 
-@pytest.mark.parametrize("tile", [1, 0])                          # 1: raw q columns; 0: the table, where these few go through the pre-step
+@pytest.mark.parametrize("tile", [1, 0])                          # 1: always the matrix-core attention kernel; 0: the table
 @pytest.mark.parametrize("shape,more,base,n", [
     ("qwen36_moe", {}, 0, 129),                                   # unsplit halves, last block ragged
     ("qwen36_moe", dict(kv_q8=True), 700, 70),                    # split over the context (merge kernel), int8 caches
@@ -329,13 +329,15 @@ def test_attn_layer_prefill_matches_oracle(shape, dim, kind, base, n):
     ("qwen3_1p7b", dict(qk_norm=False), 0, 97),
     ("qwen36_moe", dict(n_rot=256), 40, 48),                      # pairs 128 apart
     ("qwen36_moe", dict(n_rot=128, qk_norm=False, gate=False), 3, 61),
-    ("qwen36_moe", dict(n_rot=48), 20, 50),                       # pairs inside a k-step: q through the pre-step
+    ("qwen36_moe", dict(n_rot=48), 20, 50),
     ("qwen3_1p7b", dict(n_rot=32, gate=True), 0, 80),
+    ("qwen36_moe", {}, 0, 5),                                     # a verify block: projections and attention of a few columns
+    ("qwen36_moe", {}, 0, 660),                                   # 10560 (column, head) rows
+    ("qwen3_1p7b", {}, 17, 700),
 ])
-def test_layer_prefill_from_raw_q_columns(shape, more, base, n, tile):
-    """The attention kernel takes q and gate from where the projection left them: the same residual as the stages one by one.
-    The norm's f64 sum runs in another order, so a roped q value may move by one f32 ulp, and its f16 operand by one f16 ulp
-    where that crosses a rounding boundary: 2^-10 of one product of a row's score."""
+def test_layer_prefill_equals_its_stages(shape, more, base, n, tile):
+    """The layer call leaves the bits of its stages called one by one: the residual, the cache rows, and the q and gate buffers,
+    which hold the pre-step's results after either."""
     from pooled_amd.capi import PA_OUT_F16
     cfg = dict(SHAPES[shape], **more)
     nH, nKV, hd = cfg["n_heads"], cfg["n_kv_heads"], cfg["head_dim"]
@@ -348,9 +350,10 @@ def test_layer_prefill_from_raw_q_columns(shape, more, base, n, tile):
     nw = (1 + 0.1 * rng.standard_normal(dim)).astype(np.float32)
     hw = (1 + 0.1 * rng.standard_normal(hd)).astype(np.float32); hk = (1 + 0.1 * rng.standard_normal(hd)).astype(np.float32)
     x = rng.standard_normal((n, dim)).astype(np.float32)
-    outs, caches = [], []
+    outs, caches, pre = [], [], []
     with PooledAttn(cfg, base + n + 1, n_layers=2, max_cols=max(base, n)) as pa:
         pa.set_prefill_tile(tile)
+        stale = np.full(n * qd, np.nan, np.float32)
         wq = pa.weight(PA_W_Q4_0, w_qkv, s_qkv); wo = pa.weight(PA_W_Q4_0, w_o, s_o)
         dnw = pa.to_device(nw); dqw = pa.to_device(hw); dkw = pa.to_device(hk)
         kraw, vraw = (pa.to_device(rng.standard_normal((max(base, 1), kvd)).astype(np.float32)) for _ in range(2))
@@ -359,6 +362,8 @@ def test_layer_prefill_from_raw_q_columns(shape, more, base, n, tile):
             if base:
                 pa.kv_store(layer, kraw, kvd, vraw, kvd, 0, base)
             dx = pa.to_device(x)
+            for buf in (pa.q_buffer_ptr(), pa.gate_buffer_ptr()):
+                pa.L.pa_upload(pa.ctx, buf, stale.ctypes.data, stale.nbytes)
             if layer == 0:
                 pa.attn_layer_prefill(layer, wq, wo, dnw, dqw, dkw, dx, dim, base, n)
             else:
@@ -370,10 +375,13 @@ def test_layer_prefill_from_raw_q_columns(shape, more, base, n, tile):
                 pa.gemm(wo, dat, qd, n, dx, dim, acc=True)
             pa.sync()
             outs.append(dx.download(np.float32, n * dim))
+            pre.append((pa.read_q_buffer(n), pa.read_gate_buffer(n) if cfg["gate"] else np.zeros(0)))
             caches.append([pa.kv_read(layer, w, base, n) for w in range(4 if cfg.get("kv_q8") else 2)])
     for a, b in zip(*caches):
         assert np.array_equal(np.asarray(a), np.asarray(b))
-    assert np.abs(outs[0] - outs[1]).max() <= 2.0 ** -10 * np.abs(outs[1]).max()
+    assert np.isfinite(outs[0]).all() and np.array_equal(outs[0], outs[1])
+    for a, b in zip(*pre):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
 
 
 def test_layer_calls_on_int8_caches_equal_their_stages():
