@@ -115,11 +115,12 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   //      is wave-uniform (scalar registers) ----
   static_assert((W * S::RPB) % 16 == 0, "the swizzle must not depend on the load index");
   const uint32_t ld_row0 = wave * S::RPB + lane / S::CPR, ld_slot = lane % S::CPR;
-  const uint32_t k_off = ld_row0 * (uint32_t)row_bytes + (ld_slot ^ (ld_row0 & 15)) * 16;
-  const uint32_t v_off = ld_row0 * (uint32_t)row_bytes + (ld_slot ^ (4 * (ld_row0 & 3))) * 16;
+  auto k_off_of = [&](uint32_t row0, uint32_t slot) { return row0 * (uint32_t)row_bytes + (slot ^ (row0 & 15)) * 16; };
+  auto v_off_of = [&](uint32_t row0, uint32_t slot) { return row0 * (uint32_t)row_bytes + (slot ^ (4 * (row0 & 3))) * 16; };
+  const uint32_t k_off = k_off_of(ld_row0, ld_slot), v_off = v_off_of(ld_row0, ld_slot);
   constexpr uint32_t LD_STRIDE = W * S::RPB * S::ROWB;           // bytes between the rows of consecutive loads
   // rows at or past t_end (only in the last tile of the context) come from the zero padding row max_seq
-  auto issue_t = [&](const unsigned char* g_base, const uint32_t off, unsigned char* dst, uint32_t tpos) {
+  auto issue_t = [&](const unsigned char* g_base, const uint32_t off, const uint32_t row0, unsigned char* dst, uint32_t tpos) {
     const unsigned char* t0p = g_base + (size_t)tpos * row_bytes;
     if (tpos + PF_TN <= t_end) {
 #pragma unroll
@@ -127,19 +128,19 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
     } else {
 #pragma unroll
       for (int i = 0; i < S::NLD; i++) {
-        const uint32_t row = i * W * S::RPB + ld_row0;
+        const uint32_t row = i * W * S::RPB + row0;
         const unsigned char* src = tpos + row < t_end ? t0p + i * LD_STRIDE + off
-                                                      : g_base + (size_t)p.max_seq * row_bytes + (off - ld_row0 * (uint32_t)row_bytes);
+                                                      : g_base + (size_t)p.max_seq * row_bytes + (off - row0 * (uint32_t)row_bytes);
         PF_GLL(src, dst + (i * W + wave) * 1024);
       }
     }
   };
-  auto issue_k = [&](unsigned char* kdst, uint32_t tpos) { issue_t(kg_base, k_off, kdst, tpos); };
-  auto issue_v = [&](unsigned char* vdst, uint32_t tpos) { issue_t(vg_base, v_off, vdst, tpos); };
+  auto issue_k = [&](unsigned char* kdst, uint32_t tpos) { issue_t(kg_base, k_off, ld_row0, kdst, tpos); };
+  auto issue_v = [&](unsigned char* vdst, uint32_t tpos) { issue_t(vg_base, v_off, ld_row0, vdst, tpos); };
   issue_k(kbuf0, t_begin);
   issue_v(vbuf0, t_begin);
 
-  // ---- per-lane rows: query row of block qb is wave*QB*32 + qb*32 + ln = (column r / G, head r % G) ----
+  // ---- per-lane rows: row r = wrow0 + qb*32 + ln of the wave's block of columns = (column c0 + r / G, head r % G) ----
   uint32_t end_pos[QB], row_id[QB];
   uint32_t w_min_end = 0xffffffffu, w_max_end = 0;                // positions seen by the wave's first row, by its last one
 #pragma unroll
@@ -328,14 +329,24 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   };
 
   // ---- main loop ----
-  const uint32_t n_even = n_steps & ~1u;
+  // A wave's rows are all masked from its step n_live on (the near half of a pair, the upper waves of the last column block): there
+  // it only stages its share of the remaining tiles.  Every wave passes n_steps barriers, whichever loop it is in.
+  // At head_dim 256 that is a loop of its own: with the compute under a branch instead, the loop's blocks end where the compiler
+  // overlaps the end of a tile with the start of the next (us, whole blocks / pairs with the branch / pairs with two loops, medians
+  // over many placements of the caches, which alone move a pass by 1 %: 4096 columns at 124K 6964 / 6996 / 6952, at 64K 3687 / 3702 /
+  // 3685, 2500 at 32K 1382 / 1387 / 1374; from one placement to the next the branch cost up to 1.7 %).  At 128 the branch is the
+  // cheaper form (4096 columns at 28K 946 against 951, 2500 at 8192 253 against 257).
+  constexpr bool TWO_LOOPS = HD == 256;
+  const uint32_t n_live = !TWO_LOOPS ? n_steps : w_max_end > t_begin ? min((w_max_end - t_begin + PF_TN - 1) / PF_TN, n_steps) : 0u;
+  const uint32_t n_even = n_live & ~1u;
+  uint32_t lane_e = lane;
   {
     // all waves in phase: QK, softmax, PV of a tile between two barriers (tile i + 1 of both K and V in flight)
     auto step_s = [&](auto PAR, const uint32_t i) {
       constexpr int par = decltype(PAR)::value;
       const uint32_t tp = t_begin + i * PF_TN;
       if (i + 1 < n_steps) { issue_k(par ? kbuf0 : kbuf1, tp + PF_TN); issue_v(par ? vbuf0 : vbuf1, tp + PF_TN); }
-      if (tp < w_max_end) {                         // past it every row of the wave is masked
+      if (TWO_LOOPS || tp < w_max_end) {
         qk(par ? kbuf1 : kbuf0, tp);
         sm(tp);
         pv(par ? vbuf1 : vbuf0, tp);
@@ -347,14 +358,30 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
       step_s(std::integral_constant<int, 0>{}, i);
       step_s(std::integral_constant<int, 1>{}, i + 1);
     }
-    if (n_steps & 1) step_s(std::integral_constant<int, 0>{}, n_even);
+    if (n_live & 1) step_s(std::integral_constant<int, 0>{}, n_even);
+    if constexpr (TWO_LOOPS) {
+      // the lane, counted anew: what depends on it from here on is not kept in registers through the loop above
+      lane_e = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+      asm volatile("" : "+v"(lane_e));
+      const uint32_t d_row0 = wave * S::RPB + lane_e / S::CPR, d_slot = lane_e % S::CPR;
+      for (uint32_t i = n_live; i < n_steps; i++) {
+        const uint32_t tp = t_begin + i * PF_TN;
+        if (i + 1 < n_steps) {
+          issue_t(kg_base, k_off_of(d_row0, d_slot), d_row0, i & 1 ? kbuf0 : kbuf1, tp + PF_TN);
+          issue_t(vg_base, v_off_of(d_row0, d_slot), d_row0, i & 1 ? vbuf0 : vbuf1, tp + PF_TN);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+      }
+    }
   }
 
   // ---- epilogue ----
+  const uint32_t ln_e = lane_e & 31, hb_e = lane_e >> 5;
 #pragma unroll
   for (int qb = 0; qb < QB; qb++) {
     l_run[qb] += __shfl_xor(l_run[qb], 32, 64);
-    const uint32_t r = wrow0 + qb * 32 + ln;
+    const uint32_t r = wrow0 + qb * 32 + ln_e;
     if (r >= R) continue;
     const uint32_t col = c0 + r / G, hq = g * G + r % G;
     if (p.n_splits == 1) {
@@ -365,7 +392,7 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
       for (int db = 0; db < S::DB; db++) {
 #pragma unroll
         for (int q4 = 0; q4 < 4; q4++) {
-          const uint32_t d = 32 * db + 8 * q4 + 4 * hb;
+          const uint32_t d = 32 * db + 8 * q4 + 4 * hb_e;
           f4 o = { acc[db][qb][4 * q4] * inv_l, acc[db][qb][4 * q4 + 1] * inv_l, acc[db][qb][4 * q4 + 2] * inv_l, acc[db][qb][4 * q4 + 3] * inv_l };
           if (gate) {
             const f4 gt = *(const f4*)(gate + d);
@@ -387,11 +414,11 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
       for (int db = 0; db < S::DB; db++)
 #pragma unroll
         for (int q4 = 0; q4 < 4; q4++) {
-          const uint32_t d = 32 * db + 8 * q4 + 4 * hb;
+          const uint32_t d = 32 * db + 8 * q4 + 4 * hb_e;
           const f4 o = { acc[db][qb][4 * q4], acc[db][qb][4 * q4 + 1], acc[db][qb][4 * q4 + 2], acc[db][qb][4 * q4 + 3] };
           *(f4*)(p.part_o + slot * HD + d) = o;
         }
-      if (hb == 0) {
+      if (hb_e == 0) {
         p.part_ml[slot * 2] = m_ref[qb] * 0.6931471805599453f;
         p.part_ml[slot * 2 + 1] = l_run[qb];
       }

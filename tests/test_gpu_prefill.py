@@ -57,6 +57,16 @@ def test_prefill_paired_halves(shape, base, n):
     assert_parity(got, ref, "paired %s base %d n %d" % (shape, base, n))
 
 
+@pytest.mark.parametrize("shape,base,n", [("qwen36_moe", 0, 33), ("qwen36_moe", 31, 17), ("qwen36_moe", 64, 514), ("qwen38_27b", 10, 106),
+                                          ("qwen38_27b", 1500, 43), ("qwen36_moe", 900, 33)])
+def test_prefill_waves_done_early(shape, base, n):
+    """Waves whose rows end before the workgroup's last tile only stage what is left: none, one and many such steps, an odd and an
+    even number of computed ones, waves without any row, with the context whole and split."""
+    got, ref, plan = _prefill(SHAPES[shape], base, n, seed=base + 3 * n)
+    assert plan["kernel"] == 1
+    assert_parity(got, ref, "waves done early %s base %d n %d" % (shape, base, n))
+
+
 @pytest.mark.parametrize("n_kv,n", [(4, 260), (4, 257), (8, 133), (1, 1027), (3, 345)])
 def test_prefill_more_workgroups_than_cus(n_kv, n):
     """An unsplit pass of more workgroups than the chip holds takes whole blocks of columns, the longest first, dealt over the
