@@ -26,11 +26,12 @@
 //     in f16) and takes the 128-register O rescale off the common path.
 //   * Workgroup ids are remapped so that each XCD (ids are dealt round-robin to the 8 XCDs) works on one
 //     contiguous range of (kv head, column block): the K/V stream of a kv head is fetched into one L2.
-//   * Unsplit passes are paired: waves 0-3 take a half block of columns from the front of the chunk, waves 4-7 the one as
-//     far from its back, so that every workgroup has the same work and the causal triangle of a chunk at the start of a
-//     prompt does not leave most CUs idle behind the last columns' workgroups (with one block of neighbouring columns a
-//     workgroup, 4096 columns from 0 of the MoE shape 225 us, paired 180 us: 128 steps at the pace of one wave a SIMD, which
-//     is 0.72 of two waves').  Where half blocks would need a workgroup more than whole ones, the blocks stay whole.
+//   * PAIRED (unsplit passes of one round whose chunk is a material part of the context, the rule at pairs_pay): waves 0-3 take a
+//     half block of columns from the front of the chunk, waves 4-7 the one as far from its back, so that every workgroup has the same
+//     work and the causal triangle of a chunk at the start of a prompt does not leave most CUs idle behind the last columns'
+//     workgroups (with one block of neighbouring columns a workgroup, 4096 columns from 0 of the MoE shape 225 us, paired 180 us: 128
+//     steps at the pace of one wave a SIMD, which is 0.72 of two waves').  Where half blocks would need a workgroup more than whole
+//     ones, the blocks stay whole.
 //   * Unsplit passes of more workgroups than CUs keep whole blocks (halves that end apart run one wave a SIMD for a while: more work
 //     in all), dealt over the XCDs of a kv head in turn, the longest first.  In order of position, one XCD of a head had the front of the
 //     triangle and another the back, the longest blocks last: 4096 columns of the 24 / 4-head shape from 0 420 -> 315 us, 3000 at
@@ -51,7 +52,7 @@ template <int HD, int W> struct PfShape {
   static_assert(NLD >= 1 && NLD * W * RPB == PF_TN, "tile must divide evenly over the waves");
 };
 
-template <int HD, int QB, int W>
+template <int HD, int QB, int W, bool PAIRED>
 __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p, uint32_t n_col_blocks, uint32_t half_cols, uint32_t head_xcds) {
   typedef PfShape<HD, W> S;
   // four separate LDS objects (two K, two V buffers): the compiler then orders an LDS read only after the
@@ -84,11 +85,11 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform (scalar) so per-wave branches are scalar branches
   const uint32_t ln = lane & 31, hb = lane >> 5;   // MFMA row / column index, k half
   const uint32_t G = p.group, nH = p.n_heads;
-  // columns of this WAVE [c0, c0 + R / G): the workgroup's block, or (half_cols) its half's block: waves of the lower half
+  // columns of this WAVE [c0, c0 + R / G): the workgroup's block, or (PAIRED) its half's block: waves of the lower half
   // take block cb from the front, the others the one as far from the back, so that every workgroup has the same work
   uint32_t c0 = cb * p.cols_per_group, wrow0 = wave * QB * 32;       // wrow0: the wave's first row in its block
   uint32_t ncl = min(p.cols_per_group, p.n_cols - c0), c_end = c0 + ncl;
-  if (half_cols) {
+  if constexpr (PAIRED) {
     const uint32_t n_half = (p.n_cols + half_cols - 1) / half_cols, far = n_half - 1 - cb;
     const bool lower = wave < W / 2;
     c0 = (lower ? cb : far) * half_cols;
@@ -146,7 +147,7 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
 #pragma unroll
   for (int qb = 0; qb < QB; qb++) {
     const uint32_t r = wrow0 + qb * 32 + ln;
-    row_id[qb] = R ? min(r, R - 1) : 0;
+    row_id[qb] = !PAIRED || R ? min(r, R - 1) : 0;
     end_pos[qb] = r < R ? p.base_pos + c0 + r / G + 1 : 0u;
   }
   {
@@ -329,14 +330,13 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   };
 
   // ---- main loop ----
-  // A wave's rows are all masked from its step n_live on (the near half of a pair, the upper waves of the last column block): there
-  // it only stages its share of the remaining tiles.  Every wave passes n_steps barriers, whichever loop it is in.
-  // At head_dim 256 that is a loop of its own: with the compute under a branch instead, the loop's blocks end where the compiler
-  // overlaps the end of a tile with the start of the next (us, whole blocks / pairs with the branch / pairs with two loops, medians
-  // over many placements of the caches, which alone move a pass by 1 %: 4096 columns at 124K 6964 / 6996 / 6952, at 64K 3687 / 3702 /
-  // 3685, 2500 at 32K 1382 / 1387 / 1374; from one placement to the next the branch cost up to 1.7 %).  At 128 the branch is the
-  // cheaper form (4096 columns at 28K 946 against 951, 2500 at 8192 253 against 257).
-  constexpr bool TWO_LOOPS = HD == 256;
+  // PAIRED: the near half's rows are all masked from its step n_live on; there its waves only stage their share of the remaining tiles.
+  // Every wave passes n_steps barriers, whichever loop it is in.  At head_dim 256 that is a loop of its own: with the compute under a
+  // branch instead, the loop's blocks end where the compiler overlaps the end of a tile with the start of the next (us, branch / two
+  // loops: 4096 columns at 8192 666 / 665, at 16384 1113 / 1108, at 64K 3833 / 3811).  At 128 the branch is the cheaper form (4096 columns
+  // at 28K 946 against 951, 2500 at 8192 253 against 257).  Whole blocks (a wave's last row sees at most a tile less than the
+  // workgroup's) compute every step: either form of skipping there costs 0.3 % of a long pass.
+  constexpr bool TWO_LOOPS = PAIRED && HD == 256;
   const uint32_t n_live = !TWO_LOOPS ? n_steps : w_max_end > t_begin ? min((w_max_end - t_begin + PF_TN - 1) / PF_TN, n_steps) : 0u;
   const uint32_t n_even = n_live & ~1u;
   uint32_t lane_e = lane;
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
       constexpr int par = decltype(PAR)::value;
       const uint32_t tp = t_begin + i * PF_TN;
       if (i + 1 < n_steps) { issue_k(par ? kbuf0 : kbuf1, tp + PF_TN); issue_v(par ? vbuf0 : vbuf1, tp + PF_TN); }
-      if (TWO_LOOPS || tp < w_max_end) {
+      if (TWO_LOOPS || !PAIRED || tp < w_max_end) {
         qk(par ? kbuf1 : kbuf0, tp);
         sm(tp);
         pv(par ? vbuf1 : vbuf0, tp);
@@ -359,10 +359,12 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
       step_s(std::integral_constant<int, 1>{}, i + 1);
     }
     if (n_live & 1) step_s(std::integral_constant<int, 0>{}, n_even);
-    if constexpr (TWO_LOOPS) {
+    if constexpr (HD == 256) {
       // the lane, counted anew: what depends on it from here on is not kept in registers through the loop above
       lane_e = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
       asm volatile("" : "+v"(lane_e));
+    }
+    if constexpr (TWO_LOOPS) {
       const uint32_t d_row0 = wave * S::RPB + lane_e / S::CPR, d_slot = lane_e % S::CPR;
       for (uint32_t i = n_live; i < n_steps; i++) {
         const uint32_t tp = t_begin + i * PF_TN;
@@ -426,25 +428,44 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   }
 }
 
-template <int HD, int QB, int W>
-static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t) {
+template <int HD, int QB, int W, bool PAIRED>
+static hipError_t launch_prefill_k(const AttnParams& p, uint32_t col_groups, uint32_t half, uint32_t head_xcds, hipStream_t s, const PaTiming* t) {
   typedef PfShape<HD, W> S;
   const size_t lds = (size_t)W * QB * (S::KS - S::QR) * 1024;     // Q fragments parked in LDS (dynamic part)
   static bool attr_set = false;
   if (!attr_set && lds > 0) {
-    hipError_t e = hipFuncSetAttribute((const void*)pa_prefill_kernel<HD, QB, W>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = hipFuncSetAttribute((const void*)pa_prefill_kernel<HD, QB, W, PAIRED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     attr_set = true;
   }
+  const uint32_t total = col_groups * p.n_kv_heads * p.n_splits;
+  const uint32_t gx = 8 * (head_xcds ? (col_groups + head_xcds - 1) / head_xcds : (total + 7) / 8);       // whole rounds of the 8 XCDs
+  PA_LAUNCH((pa_prefill_kernel<HD, QB, W, PAIRED>), dim3(gx), dim3(W * 64), lds, s, t, p, col_groups, half, head_xcds);
+  return hipGetLastError();
+}
+
+// Whether an unsplit pass of one round is paired.  Pairing takes the wait for the longest block away (n_cols / 2 positions at
+// most) and pays for it in energy: every pair stages tiles up to its far half's end, and halves that end apart run one wave a SIMD
+// for a while.  At head_dim 256 a full chip runs at the power limit, so once the triangle is a small part of the context pairs are the
+// slower form; a chip that is not full holds its clock longer.  Measured (us, whole blocks / pairs): 256 workgroups, 4096 columns of
+// the 16 / 2-head shape at 0 262 / 225, at 8192 677 / 665, at 16384 1109 / 1108, at 64K 3803 / 3811, at 124K 7130 / 7162; 2650 columns of the
+// 24 / 4-head shape at 4096 409 / 402, at 8192 623 / 624, at 16384 1054 / 1070; 158 workgroups, 2500 columns of the first at 8192
+// 473 / 467, at 16384 778 / 768, at 32768 1421 / 1417, at 64K 2696 / 2707.  Head_dim 128 stays ahead (4096 columns at 28672 1039 / 1016).
+template <int HD>
+static bool pairs_pay(const AttnParams& p, uint32_t total, uint32_t n_cu) {
+  return HD == 128 || (uint64_t)p.base_pos * total <= 3ull * p.n_cols * n_cu;
+}
+
+template <int HD, int QB, int W>
+static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t) {
   const uint32_t half = W / 2 * QB * 32 / p.group;
   const uint32_t total = col_groups * p.n_kv_heads * p.n_splits;
-  // Halves of a workgroup that end apart run one wave a SIMD for a while, so pairing costs work to save the wait for the longest
-  // block: it pays while the chip holds all workgroups at once.  More of them: whole blocks, the longest first.
-  const bool paired = p.n_splits == 1 && half > 0 && total <= n_cu && ((p.n_cols + half - 1) / half + 1) / 2 == col_groups;
-  const uint32_t head_xcds = p.n_splits == 1 && !paired && 8 % p.n_kv_heads == 0 ? 8 / p.n_kv_heads : 0;
-  const uint32_t gx = 8 * (head_xcds ? (col_groups + head_xcds - 1) / head_xcds : (total + 7) / 8);       // whole rounds of the 8 XCDs
-  PA_LAUNCH((pa_prefill_kernel<HD, QB, W>), dim3(gx), dim3(W * 64), lds, s, t, p, col_groups, paired ? half : 0u, head_xcds);
-  return hipGetLastError();
+  const bool one_round = total <= n_cu;
+  if (p.n_splits == 1 && half > 0 && one_round && ((p.n_cols + half - 1) / half + 1) / 2 == col_groups && pairs_pay<HD>(p, total, n_cu))
+    return launch_prefill_k<HD, QB, W, true>(p, col_groups, half, 0, s, t);
+  // more workgroups than the chip holds at once: the longest blocks first
+  const uint32_t head_xcds = p.n_splits == 1 && !one_round && 8 % p.n_kv_heads == 0 ? 8 / p.n_kv_heads : 0;
+  return launch_prefill_k<HD, QB, W, false>(p, col_groups, 0, head_xcds, s, t);
 }
 
 // row_blocks = 32-row query blocks per workgroup (8: one per wavefront)

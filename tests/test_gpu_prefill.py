@@ -57,6 +57,17 @@ def test_prefill_paired_halves(shape, base, n):
     assert_parity(got, ref, "paired %s base %d n %d" % (shape, base, n))
 
 
+@pytest.mark.parametrize("base,n", [(3000, 1000), (3200, 1000), (3300, 1010), (9000, 1024)])
+def test_prefill_long_context_keeps_whole_blocks(base, n):
+    """At head_dim 256 an unsplit pass that fills the chip pairs half blocks only while base_pos x workgroups is within 3 x n_cols x
+    CUs (the first case on a 256-CU part); past that the blocks stay whole: either side of the line, a ragged last block."""
+    cfg = dict(SHAPES["qwen36_moe"], n_heads=64, n_kv_heads=2)                      # 32 heads a kv head: blocks of eight columns
+    rows = sorted(set(range(0, n, 50)) | set(range(5)) | set(range(n - 5, n)))
+    got, ref, plan = _prefill(cfg, base, n, seed=base + n, check_rows=rows)
+    assert plan["kernel"] == 1 and plan["n_splits"] == 1 and plan["col_groups"] * 2 == 2 * -(-n // 8) <= 256
+    assert_parity(got, ref, "whole blocks at base %d n %d" % (base, n))
+
+
 @pytest.mark.parametrize("shape,base,n", [("qwen36_moe", 0, 33), ("qwen36_moe", 31, 17), ("qwen36_moe", 64, 514), ("qwen38_27b", 10, 106),
                                           ("qwen38_27b", 1500, 43), ("qwen36_moe", 900, 33)])
 def test_prefill_waves_done_early(shape, base, n):
