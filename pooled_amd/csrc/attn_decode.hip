@@ -1302,18 +1302,12 @@ static constexpr size_t decode_lds_bytes() {
   // P region of the single-round kernel with two row blocks
   return 16 * NB * S::QROW + (size_t)W * S::STAGE + 3 * W * 16 * NB * sizeof(float) + 2 * 16 * NB * sizeof(uint32_t) + (NB == 2 && W == 4 ? (size_t)W * NB * 1024 : 0);
 }
-// the kernel's dynamic LDS limit, raised once per instantiation (at its first launch, or ahead of it by
+// the kernel's dynamic LDS limit, raised once per instantiation and device (at its first launch, or ahead of it by
 // pa_prepare_decode_step)
 template <int HD, int NB, int W, bool FUSED, bool GATHER, bool Q8, bool SR>
 static hipError_t decode_lds_attr() {
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)pa_decode_kernel<HD, NB, W, FUSED, GATHER, Q8, SR>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)decode_lds_bytes<HD, NB, W>());
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
-  return hipSuccess;
+  static PaPerDevice lds_set;
+  return pa_lds_limit(lds_set, (const void*)pa_decode_kernel<HD, NB, W, FUSED, GATHER, Q8, SR>, decode_lds_bytes<HD, NB, W>());
 }
 
 template <int HD, int NB, int W, bool FUSED, bool GATHER, bool Q8, bool SR>

@@ -432,11 +432,10 @@ template <int HD, int QB, int W, bool PAIRED>
 static hipError_t launch_prefill_k(const AttnParams& p, uint32_t col_groups, uint32_t half, uint32_t head_xcds, hipStream_t s, const PaTiming* t) {
   typedef PfShape<HD, W> S;
   const size_t lds = (size_t)W * QB * (S::KS - S::QR) * 1024;     // Q fragments parked in LDS (dynamic part)
-  static bool attr_set = false;
-  if (!attr_set && lds > 0) {
-    hipError_t e = hipFuncSetAttribute((const void*)pa_prefill_kernel<HD, QB, W, PAIRED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (lds > 0) {
+    static PaPerDevice lds_set;
+    const hipError_t e = pa_lds_limit(lds_set, (const void*)pa_prefill_kernel<HD, QB, W, PAIRED>, lds);
     if (e != hipSuccess) return e;
-    attr_set = true;
   }
   const uint32_t total = col_groups * p.n_kv_heads * p.n_splits;
   const uint32_t gx = 8 * (head_xcds ? (col_groups + head_xcds - 1) / head_xcds : (total + 7) / 8);       // whole rounds of the 8 XCDs

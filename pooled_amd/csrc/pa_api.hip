@@ -15,7 +15,6 @@ static thread_local std::string g_create_err;
 // device address up once per device (hipGetSymbolAddress with that device current) and everything -- kernel
 // arguments included -- goes through that pointer.
 #define PA_STATIC_SCRATCH_BYTES (8u << 20)
-#define PA_MAX_DEVICES 64
 static __device__ __align__(256) unsigned char scratch[PA_STATIC_SCRATCH_BYTES];
 static void* g_scratch_ptr[PA_MAX_DEVICES];
 static std::mutex g_scratch_mutex;

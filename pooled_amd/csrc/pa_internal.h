@@ -7,6 +7,7 @@
 #include <vector>
 #include <map>
 #include "../../include/pooled_attn.h"
+#include "pa_per_device.h"
 
 // ---- kernel-side parameter blocks -------------------------------------------------------------
 
@@ -82,6 +83,14 @@ struct PaTiming { hipEvent_t start = nullptr, stop = nullptr; };
     if ((timing) && (timing)->start) hipExtLaunchKernelGGL(kernel, grid, block, lds, stream, (timing)->start, (timing)->stop, 0, __VA_ARGS__); \
     else hipLaunchKernelGGL(kernel, grid, block, lds, stream, __VA_ARGS__);                                               \
   } while (0)
+
+// raises a kernel's dynamic LDS limit on the current device, where the attribute belongs: once per device, `set` being the kernel's own
+inline hipError_t pa_lds_limit(PaPerDevice& set, const void* kernel, size_t bytes) {
+  int device;
+  const hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return e;
+  return set.once(device, [&] { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes); });
+}
 
 hipError_t pa_launch_glue(const GlueParams& p, hipStream_t s);
 hipError_t pa_launch_rope_table(float2* tab, const float* inv_freq, uint32_t half, uint32_t n_pos, hipStream_t s);

@@ -167,11 +167,10 @@ static hipError_t sk_launch(const GemmParams& p, hipStream_t s) {
   const uint32_t stage = RG * 16 * CH * (KIND == PA_W_Q4_0 ? 16 : 32), red = RG * NB * 1024;
   const size_t lds = (size_t)nw * (stage > red ? stage : red);
   if (nw > SK_MAXW || lds > 160 * 1024) return hipErrorNotSupported;
-  static bool attr_set = false;
-  if (!attr_set && lds > 65536) {
-    hipError_t e = hipFuncSetAttribute((const void*)pa_gemm_skinny_kernel<KIND, RG, NB, CH, WHOLE>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  if (lds > 65536) {
+    static PaPerDevice lds_set;
+    const hipError_t e = pa_lds_limit(lds_set, (const void*)pa_gemm_skinny_kernel<KIND, RG, NB, CH, WHOLE>, 160 * 1024);
     if (e != hipSuccess) return e;
-    attr_set = true;
   }
   hipLaunchKernelGGL((pa_gemm_skinny_kernel<KIND, RG, NB, CH, WHOLE>), dim3((p.d_out + 16 * RG - 1) / (16 * RG)), dim3(nw * 64), lds, s, p.w, p.scales, p.x, p.x_stride,
                      p.d_out, p.d_in, p.n_cols, p);

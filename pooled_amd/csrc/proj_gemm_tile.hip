@@ -198,16 +198,11 @@ static hipError_t gt_launch(const GemmTileParams& q, int acc, hipStream_t s) {
   constexpr int lds_st = S * (BM + BN) * BK * 2, lds_red = KG > 1 ? KG * BM * BN * 4 : 0, lds = lds_st > lds_red ? lds_st : lds_red;
   static_assert(lds <= 160 * 1024, "LDS");
   const uint32_t total = ((q.n_cols + BM - 1) / BM) * ((q.d_out + BN - 1) / BN);
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
-  const dim3 block(512);
-  if (acc) hipLaunchKernelGGL((pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, true>), dim3((total + 7) / 8 * 8), block, lds, s, q);
-  else hipLaunchKernelGGL((pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, false>), dim3((total + 7) / 8 * 8), block, lds, s, q);
+  static PaPerDevice lds_set[2];
+  const auto kernel = acc ? pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, true> : pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, false>;
+  const hipError_t e = pa_lds_limit(lds_set[acc ? 1 : 0], (const void*)kernel, lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3((total + 7) / 8 * 8), dim3(512), lds, s, q);
   return hipGetLastError();
 }
 
