@@ -134,8 +134,12 @@ hipError_t pa_launch_gemm_skinny(const GemmParams& p, int n_cu, hipStream_t s);
 bool pa_gemm_wide_serves(const GemmParams& p);
 size_t pa_gemm_wide_staging_bytes(uint32_t d_out, uint32_t d_in);
 hipError_t pa_launch_gemm_wide(const GemmParams& p, uint16_t* w16, bool widen, int n_cu, hipStream_t s);
-// its kernel for larger tiles (proj_gemm_tile.hip), and what a call would take there
-float pa_gemm_tile_us(const GemmParams& p, int n_cu);
+// its kernel for larger tiles (proj_gemm_tile.hip), and what a call would take there, on which tile (columns << 16 | rows)
+float pa_gemm_tile_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, uint32_t* shape);
+// the rules that pick an instance by size, in plain C: the tests ask them which instances their sizes take
+extern "C" uint32_t pa_rule_gemv_wide_rows(uint32_t d_out, int n_cu, uint32_t rmax);
+extern "C" int pa_rule_gemm_few_groups(int kind, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu);
+extern "C" uint32_t pa_rule_gemm_wide_tile(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t x_stride, int n_cu);
 hipError_t pa_launch_gemm_tile(const GemmParams& p, const uint16_t* w16, int n_cu, hipStream_t s);
 // rmsnorm of n_cols f32 columns, written as f16 (the GEMM's activation operand)
 hipError_t pa_launch_rmsnorm_f16(const float* x, uint32_t x_stride, const float* w, uint32_t dim, float eps, uint32_t n_cols,

@@ -186,20 +186,26 @@ static hipError_t sk_cols(const GemmParams& p, hipStream_t s) {
 // few columns, they only leave CUs idle.  Measured (us, 1 / 2 / 4 groups): 9216 x 2048 Q4_0 2 columns 6.3 / 6.8 / 7.4, 8
 // columns 7.3 / 7.4 / 7.6, 16 columns 9.2 / 9.0 / 8.3, 32 columns 14.7 / 12.7 / 10.6; 2048 x 4096 16 columns 7.1 / 8.5 / 11.2;
 // 14336 x 5120 8 columns 18.0 / 15.3 / 15.7, 16 columns 25.1 / 18.6 / 17.3; 5120 x 6144 16 columns 16.4 / 12.0 / -.
-static int sk_row_groups(const GemmParams& p, int n_cu) {
-  const uint32_t groups = (p.d_out + 15) / 16, cus = n_cu > 0 ? (uint32_t)n_cu : 256u;
+static int sk_row_groups(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu) {
+  const uint32_t groups = (d_out + 15) / 16, cus = n_cu > 0 ? (uint32_t)n_cu : 256u;
   if (groups <= cus) return 1;
-  if (p.n_cols <= 8) return p.d_in > 4096 ? 2 : 1;
+  if (n_cols <= 8) return d_in > 4096 ? 2 : 1;
   return groups >= 2 * cus ? 4 : 2;
+}
+// chunks of 8 blocks (twice the waves) while 16 waves cover d_in
+static int sk_chunk(uint32_t d_in) { return d_in <= 4096 ? 8 : 16; }
+// ... as many of them as the staged weights of a workgroup leave room for in its LDS
+extern "C" int pa_rule_gemm_few_groups(int kind, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu) {
+  const int ch = sk_chunk(d_in);
+  int rg = sk_row_groups(d_out, d_in, n_cols, n_cu);
+  const uint32_t bytes = (d_in / 32 + ch - 1) / ch * ch * 16 * (kind == PA_W_Q4_0 ? 16 : 32);
+  while (rg > 1 && rg * bytes > 160 * 1024) rg /= 2;
+  return rg;
 }
 template <int KIND>
 static hipError_t sk_shape(const GemmParams& p, int n_cu, hipStream_t s) {
-  // chunks of 8 blocks (twice the waves) while 16 waves cover d_in; the staged weights of a workgroup within its LDS
-  const int ch = p.d_in <= 4096 ? 8 : 16;
-  int rg = sk_row_groups(p, n_cu);
-  const uint32_t bytes = (p.d_in / 32 + ch - 1) / ch * ch * 16 * (KIND == PA_W_Q4_0 ? 16 : 32);
-  while (rg > 1 && rg * bytes > 160 * 1024) rg /= 2;
-  if (ch == 16) return rg == 1 ? sk_cols<KIND, 1, 16>(p, s) : rg == 2 ? sk_cols<KIND, 2, 16>(p, s) : sk_cols<KIND, 4, 16>(p, s);
+  const int rg = pa_rule_gemm_few_groups(KIND, p.d_out, p.d_in, p.n_cols, n_cu);
+  if (sk_chunk(p.d_in) == 16) return rg == 1 ? sk_cols<KIND, 1, 16>(p, s) : rg == 2 ? sk_cols<KIND, 2, 16>(p, s) : sk_cols<KIND, 4, 16>(p, s);
   return rg == 1 ? sk_cols<KIND, 1, 8>(p, s) : rg == 2 ? sk_cols<KIND, 2, 8>(p, s) : sk_cols<KIND, 4, 8>(p, s);
 }
 

@@ -236,9 +236,10 @@ static int pa_pick_tile(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu
   return best;
 }
 
-float pa_gemm_tile_us(const GemmParams& p, int n_cu) {
+float pa_gemm_tile_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, uint32_t* shape) {
   float us;
-  pa_pick_tile(p.d_out, p.d_in, p.n_cols, n_cu, &us);
+  const TileShape& t = tile_shapes[pa_pick_tile(d_out, d_in, n_cols, n_cu, &us)];
+  *shape = (uint32_t)t.bm << 16 | t.bn;
   return us;
 }
 

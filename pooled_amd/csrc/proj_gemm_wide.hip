@@ -257,6 +257,21 @@ bool pa_gemm_wide_serves(const GemmParams& p) {
 // bytes of the staging matrix of a weight: whole 32-row blocks
 size_t pa_gemm_wide_staging_bytes(uint32_t d_out, uint32_t d_in) { return (size_t)((d_out + 31) / 32) * 32 * d_in * sizeof(uint16_t); }
 
+// The 64 x 64 kernel runs two workgroups a CU and its time follows their number: about 4 us and 4.6 ns per k and workgroup a
+// CU (4096 x 2048: 256 / 512 / 777 columns 13.4 / 22.0 / 34 us).  The larger tiles where their rounds come out cheaper, and their
+// kernel takes the stride.
+// Fewer 64 x 64 tiles than half the CUs: 32-row tiles (twice the workgroups) with twice the stages in flight (2048 x 4096 on up to
+// 64 columns, cold: 20 -> 16.7 us; with 144 tiles, 9216 x 2048, it is 2 us slower).
+// Columns << 16 | rows of the tile a call takes; 64-column tiles of up to 64 rows are this file's kernel.
+extern "C" uint32_t pa_rule_gemm_wide_tile(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t x_stride, int n_cu) {
+  const uint32_t cus = n_cu > 0 ? (uint32_t)n_cu : 256u;
+  const uint64_t tiles64 = (uint64_t)((n_cols + GM_T - 1) / GM_T) * ((d_out + 63) / 64);
+  const float mid_us = 4.f + 4.6e-3f * d_in * std::max(1.f, (float)tiles64 / cus);
+  uint32_t shape;
+  if (x_stride <= (1u << 22) && pa_gemm_tile_us(d_out, d_in, n_cols, n_cu, &shape) < mid_us) return shape;
+  return (uint32_t)GM_T << 16 | (tiles64 * 2 < cus ? 32u : 64u);
+}
+
 // w16: staging of pa_gemm_wide_staging_bytes (the caller's, 16-byte aligned); widen = false: it already holds these weights
 hipError_t pa_launch_gemm_wide(const GemmParams& p, uint16_t* w16, bool widen, int n_cu, hipStream_t s) {
   if (widen) {
@@ -272,16 +287,10 @@ hipError_t pa_launch_gemm_wide(const GemmParams& p, uint16_t* w16, bool widen, i
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  // The 64 x 64 kernel runs two workgroups a CU and its time follows their number: about 4 us and 4.6 ns per k and workgroup a
-  // CU (4096 x 2048: 256 / 512 / 777 columns 13.4 / 22.0 / 34 us).  The larger tiles where their rounds come out cheaper.
-  const uint32_t cus = n_cu > 0 ? (uint32_t)n_cu : 256u;
-  const uint64_t tiles64 = (uint64_t)((p.n_cols + GM_T - 1) / GM_T) * ((p.d_out + 63) / 64);
-  const float mid_us = 4.f + 4.6e-3f * p.d_in * std::max(1.f, (float)tiles64 / cus);
-  if (p.x_stride <= (1u << 22) && pa_gemm_tile_us(p, n_cu) < mid_us) return pa_launch_gemm_tile(p, w16, n_cu, s);
+  const uint32_t tile = pa_rule_gemm_wide_tile(p.d_out, p.d_in, p.n_cols, p.x_stride, n_cu);
+  if (tile >> 16 != GM_T || (tile & 0xffff) > 64) return pa_launch_gemm_tile(p, w16, n_cu, s);
   Gemm16Params q;
   q.x = p.x; q.w16 = w16; q.y = p.y; q.x_stride = p.x_stride; q.y_stride = p.y_stride;
   q.d_out = p.d_out; q.d_in = p.d_in; q.n_cols = p.n_cols; q.acc = p.acc;
-  // fewer 64 x 64 tiles than half the CUs: 32-row tiles (twice the workgroups) with twice the stages in flight
-  // (2048 x 4096 on up to 64 columns, cold: 20 -> 16.7 us; with 144 tiles, 9216 x 2048, it is 2 us slower)
-  return tiles64 * 2 < cus ? launch_gemm16_mid<1, 8>(q, s) : launch_gemm16_mid<2, 4>(q, s);
+  return (tile & 0xffff) == 32 ? launch_gemm16_mid<1, 8>(q, s) : launch_gemm16_mid<2, 4>(q, s);
 }

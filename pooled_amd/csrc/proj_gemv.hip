@@ -256,7 +256,7 @@ static hipError_t launch_rows(uint32_t rw, const GemvParams& p, hipStream_t s) {
 // 10240 x 5120 16.0 11.8 12.0 11.1 9.9 10.9 11.8 12.9; 8192 x 5120 13.4 10.7 10.1 8.7 9.5 10.6 11.8 9.6; 17000 x 4608 20.5 16.8 13.9
 // 15.0 14.2 13.9 15.0 22.3; Q8_0 14336 x 5120 21.3 20.7 19.9 18.8 18.0 25.6.  With fewer than six rows a SIMD two rows a wave are as
 // good as any (5120 x 6144: 7.3, 7.4 at three, 7.3 at five).  RMAX: what fits the registers of two waves a SIMD.
-static uint32_t wide_rows(uint32_t d_out, int n_cu, uint32_t rmax) {
+extern "C" uint32_t pa_rule_gemv_wide_rows(uint32_t d_out, int n_cu, uint32_t rmax) {
   const uint32_t simds = 4u * (uint32_t)n_cu;
   if (d_out < 6 * simds) return d_out >= 4 * simds ? 2 : 1;
   uint32_t best = 1;
@@ -273,7 +273,7 @@ template <int KIND, int BPL, bool NORM>
 static hipError_t launch_rw(const GemvParams& p, int n_cu, hipStream_t s) {
   if constexpr (BPL >= 3) {
     constexpr int RMAX = KIND == PA_W_Q4_0 ? (BPL == 3 ? 7 : 4) : (BPL == 3 ? 5 : 3);
-    return launch_rows<KIND, BPL, NORM, RMAX>(wide_rows(p.d_out, n_cu, RMAX), p, s);
+    return launch_rows<KIND, BPL, NORM, RMAX>(pa_rule_gemv_wide_rows(p.d_out, n_cu, RMAX), p, s);
   } else {
     // rows per wave: as many as still leave about two 4-wave workgroups per CU, within the registers that RW x BPL
     // blocks of weights take (f32: 32 registers a block, Q8_0: 8, Q4_0: 4)

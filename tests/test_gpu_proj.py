@@ -49,8 +49,14 @@ def test_gemv_matches_oracle(kind, d_out, d_in):
         assert np.array_equal(dy.download(np.float32, d_out), got)
 
 
+# sizes past 4096 inputs that take every number of rows a wave (test_proj_rules.py asks the rule): on a 256-CU part Q4_0 / Q8_0
+# 2 / 2, 4 / 4, 4 / 4, 6 / 4, 5 / 5 rows of three blocks a lane, 3 / 3 and 4 / 3 of four blocks, then 7 / 5, 1 / 1, 3 / 3 and 2 / 2, 1 / 1
+GEMV_WIDE_SIZES = [(6143, 4128), (6145, 4128), (8191, 5120), (11265, 4160), (14337, 6144), (9001, 6176), (6150, 8192),
+                   (14335, 5120), (4000, 4128), (6144, 4128), (4111, 8192), (1000, 7968)]
+
+
 @pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])
-@pytest.mark.parametrize("d_out,d_in", [(6143, 4128), (6145, 4128), (8191, 5120), (11265, 4160), (14337, 6144), (9001, 6176), (6150, 8192)])
+@pytest.mark.parametrize("d_out,d_in", GEMV_WIDE_SIZES)
 def test_gemv_many_rows_a_wave(kind, d_out, d_in):
     """Past 4096 inputs: one to seven rows a wave (d_out over the SIMDs picks), the last wave's rows past the end repeating the last
     one.  Every tenth row and the last ones are checked."""
@@ -145,9 +151,13 @@ def test_attn_layer_decode_matches_oracle(shape, dim, kind, pos):
 
 @pytest.mark.parametrize("kind", [PA_W_F32, PA_W_Q8_0, PA_W_Q4_0])
 @pytest.mark.parametrize("d_out,d_in,n", [(9216, 2048, 300), (2048, 4096, 129), (37, 96, 5), (130, 8192, 40), (256, 32, 128), (384, 96, 700),
-                                          (100, 384, 65), (64, 128, 33), (4096, 2048, 512),      # the 64 x 64 kernel with an odd stage count, one stage, a C2-sized chunk (as are the first two and the fourth)
-                                          (9216, 2048, 8), (2048, 4096, 16), (130, 8192, 3), (70, 64, 1), (2048, 4096, 31), (130, 8192, 17)])   # from (9216, 2048, 8) on: up to 16 columns the skinny-chunk kernel, one or more launches; the last two the 64 x 32 tiles of the mid-size kernel
+                                          (100, 384, 65), (64, 128, 33), (4096, 2048, 512),
+                                          (9216, 2048, 8), (2048, 4096, 16), (130, 8192, 3), (70, 64, 1), (2048, 4096, 31), (130, 8192, 17)])
 def test_gemm_matches_oracle(kind, d_out, d_in, n):
+    """One size or more of every kernel (on a 256-CU part): 128 x 128 tiles (9216 rows, 300 columns) and 64 x 128 ones (4096 rows, 512
+    columns); 64 columns x 32 rows with many stages, three and one (129, 40, 65 and 33 columns); d_in not a multiple of 128 past the few
+    columns, and f32 weights up to 16 columns, on the kernel that widens in its loop; quantised weights from (37, 96, 5) and
+    (9216, 2048, 8) on from the packed planes, but 17 columns of 8192 Q8_0 inputs on 64 x 32 tiles."""
     rng = np.random.default_rng(d_out + 3 * d_in + n + kind)
     w, sc = _weights(kind, d_out, d_in, rng)
     x16 = rng.standard_normal((n, d_in)).astype(np.float16)
@@ -171,11 +181,10 @@ def test_gemm_matches_oracle(kind, d_out, d_in, n):
                                           (2048, 4096, 600), (130, 8192, 513), (1000, 64, 1100)])
 def test_gemm_large_chunks(kind, d_out, d_in, n):
     """Chunks of 512 columns and more over d_in a multiple of 128: the weights are widened to f16 in fragment order (a
-    copy kept with the weight handle) and the GEMM runs over two f16 operands (128-column wave tiles, 256 to 512 weight
-    rows a workgroup: the first four shapes take 384, 256, 512 and 384 on a 256-CU part; the last three stay on the
-    tiled kernel, too few workgroups or d_in not a multiple of 128).  Ragged edges on both axes, padded strides that
-    must stay untouched, the accumulating form (the second call on a handle, which finds the kept copy), and a second
-    weight."""
+    copy kept with the weight handle) and the GEMM runs over two f16 operands.  On a 256-CU part the sizes take tiles of 128 columns x
+    384 rows, 128 x 256, 256 x 256, three times the 64-column kernel (64 rows, 64 and 32); d_in 64 stays on the kernel that widens
+    in its loop, 256 columns a workgroup.  Ragged edges on both axes, padded strides that must stay untouched, the accumulating form (the
+    second call on a handle, which finds the kept copy), and a second weight."""
     rng = np.random.default_rng(d_out + d_in + n + kind)
     w, sc = _weights(kind, d_out, d_in, rng)
     x16 = rng.standard_normal((n, d_in)).astype(np.float16)
@@ -197,9 +206,17 @@ def test_gemm_large_chunks(kind, d_out, d_in, n):
         assert _rel(dy.download(np.float32, n * ys).reshape(n, ys)[:, :d_out], O.gemm_f16(kind, w2, sc2, x16.astype(np.float32))) < 2e-5, "second weight"
 
 
+# with the next list every instance of the few-column kernel that a 256-CU part takes (test_proj_rules.py asks the rule)
+GEMM_FEW_SIZES = [(16, 32, 1), (17, 256, 2), (31, 288, 15), (4096, 4096, 16), (4100, 4128, 8), (4130, 8192, 9), (8200, 512, 17),
+                  (8193, 2080, 32), (8192, 5120, 16), (4111, 6144, 31), (2048, 4096, 33), (600, 7968, 32),
+                  (33, 4128, 5), (70, 2080, 19), (33, 256, 20), (40, 4608, 11), (48, 5120, 31),   # one row group
+                  (5000, 2048, 12), (5000, 2080, 16), (5000, 2048, 24), (4111, 1056, 32),   # two of chunks of 8 blocks
+                  (9216, 2048, 16), (8201, 1056, 13),                                    # four, one column block
+                  (4111, 4128, 31), (8193, 4128, 9), (8200, 4128, 20), (8200, 5120, 32)]   # Q4_0: two and four of chunks of 16
+
+
 @pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])
-@pytest.mark.parametrize("d_out,d_in,n", [(16, 32, 1), (17, 256, 2), (31, 288, 15), (4096, 4096, 16), (4100, 4128, 8), (4130, 8192, 9), (8200, 512, 17),
-                                          (8193, 2080, 32), (8192, 5120, 16), (4111, 6144, 31), (2048, 4096, 33), (600, 7968, 32)])
+@pytest.mark.parametrize("d_out,d_in,n", GEMM_FEW_SIZES)
 def test_gemm_few_columns(kind, d_out, d_in, n):
     """Up to 32 columns straight from the packed planes: one, two and four 16-row groups a workgroup (fewer and more of them
     than CUs, d_in either side of 4096, what fits the LDS), one and two column blocks, chunks of 8 and 16 blocks that d_in
@@ -223,8 +240,12 @@ def test_gemm_few_columns(kind, d_out, d_in, n):
         assert _rel(dy.download(np.float32, n * ys).reshape(n, ys)[:, :d_out], 2.0 * ref) < 2e-5, "accumulate"
 
 
-@pytest.mark.parametrize("d_out,d_in,n", [(8074, 256, 454), (8824, 256, 451), (8594, 256, 528), (7884, 128, 834), (8208, 128, 900), (8972, 128, 1028),
-                                          (7342, 128, 1544), (8561, 128, 1544), (4090, 2048, 500), (2040, 384, 3000)])
+# one size and more for every tile that a 256-CU part takes (test_proj_rules.py asks the rule)
+GEMM_TILE_SIZES = [(8074, 256, 454), (8824, 256, 451), (8594, 256, 528), (7884, 128, 834), (8208, 128, 900), (8972, 128, 1028),
+                   (7342, 128, 1544), (8561, 128, 1544), (4090, 2048, 500), (2040, 384, 3000)]
+
+
+@pytest.mark.parametrize("d_out,d_in,n", GEMM_TILE_SIZES)
 def test_gemm_tile_shapes(d_out, d_in, n):
     """The larger tiles of wide chunks: sizes that take each of 128 columns x 128 / 160 / 192 / 256 / 320 / 384 / 448 rows, 256 x
     256 and 64 x 128 on a 256-CU part (and 128 x 256 again), one to sixteen stages, ragged on both axes.  Sums in f32 in

@@ -1,0 +1,67 @@
+"""No-GPU checks of which kernel instance a projection takes by its sizes: the library's own rules, asked on a 256-CU part, against
+the sizes that the GPU tests run.  A change of a rule that leaves an instance without a tested size fails here."""
+import ctypes
+from pooled_amd import capi
+from pooled_amd.capi import PA_W_Q4_0, PA_W_Q8_0
+from test_gpu_proj import GEMM_FEW_SIZES, GEMM_TILE_SIZES, GEMV_WIDE_SIZES
+
+CUS = 256
+u32 = ctypes.c_uint32
+
+
+def _rule(name, *args):
+    fn = getattr(capi.load(), name)
+    fn.restype = u32
+    return fn(*(a if isinstance(a, ctypes._SimpleCData) else u32(a) for a in args))
+
+
+def _gemv(kind, d_out, d_in):
+    """(kind, blocks a lane, rows a wave) past 4096 inputs"""
+    bpl = 3 if d_in <= 6144 else 4
+    most = {(PA_W_Q4_0, 3): 7, (PA_W_Q4_0, 4): 4, (PA_W_Q8_0, 3): 5, (PA_W_Q8_0, 4): 3}[kind, bpl]
+    return kind, bpl, _rule("pa_rule_gemv_wide_rows", d_out, ctypes.c_int(CUS), most)
+
+
+def test_gemv_sizes_take_every_number_of_rows():
+    got = {_gemv(kind, d_out, d_in) for kind in (PA_W_Q4_0, PA_W_Q8_0) for d_out, d_in in GEMV_WIDE_SIZES}
+    assert got == {(k, b, r) for k, b, most in ((PA_W_Q4_0, 3, 7), (PA_W_Q4_0, 4, 4), (PA_W_Q8_0, 3, 5), (PA_W_Q8_0, 4, 3)) for r in range(1, most + 1)}
+    # a wave whose last rows are past the end, for every instance of two rows and more but one (three rows are taken at one d_out only)
+    ragged = {_gemv(kind, d_out, d_in) for kind in (PA_W_Q4_0, PA_W_Q8_0) for d_out, d_in in GEMV_WIDE_SIZES if d_out % _gemv(kind, d_out, d_in)[2]}
+    assert {g for g in got if g[2] > 1} - ragged <= {(PA_W_Q4_0, 3, 3), (PA_W_Q8_0, 3, 3)}
+
+
+def _few(kind, d_out, d_in, n):
+    """(kind, row groups, column blocks, blocks of a chunk, d_in in whole chunks) of the few-column kernel; None past its range"""
+    if n > 32 or (n > 16 and kind != PA_W_Q4_0 and d_in > 4096):
+        return None
+    ch = 8 if d_in <= 4096 else 16
+    rg = _rule("pa_rule_gemm_few_groups", ctypes.c_int(kind), d_out, d_in, n, ctypes.c_int(CUS))
+    return kind, rg, 1 if n <= 16 else 2, ch, d_in % (32 * ch) == 0
+
+
+def test_few_column_sizes_take_every_instance():
+    kinds = (PA_W_Q4_0, PA_W_Q8_0)
+    tested = {_few(k, *size) for k in kinds for size in GEMM_FEW_SIZES}
+    reached = {_few(k, d_out, d_in, n) for k in kinds for d_out in (16, 4096, 4097, 5000, 8176, 8177, 9216, 20000) for d_in in range(32, 8193, 32)
+               for n in (1, 8, 9, 16, 17, 32)}
+    assert len(reached) > 30 and reached <= tested | {None}
+
+
+def _tile(d_out, d_in, n, x_stride=None):
+    t = _rule("pa_rule_gemm_wide_tile", d_out, d_in, n, x_stride or d_in + 8, ctypes.c_int(CUS))
+    return t >> 16, t & 0xffff
+
+
+def test_tile_sizes_take_every_tile():
+    assert [_tile(*size) for size in GEMM_TILE_SIZES] == [(128, 128), (128, 160), (128, 192), (128, 256), (128, 320), (128, 384), (128, 448),
+                                                          (256, 256), (64, 128), (128, 256)]
+    every = {_tile(d_out, d_in, n) for d_out in range(33, 16000, 331) for d_in in (128, 2048, 5120, 8192) for n in (17, 100, 400, 512, 900, 1544, 2500, 4096)}
+    small = {(64, 64), (64, 32)}
+    assert every <= {_tile(*size) for size in GEMM_TILE_SIZES} | small
+    # both forms of the 64-column kernel, as the docstrings of the other GEMM tests have them
+    assert [_tile(600, 128, 11000), _tile(2048, 4096, 600), _tile(130, 8192, 513)] == [(64, 64), (64, 64), (64, 32)]
+    assert [_tile(9216 - 40, 2048, 4096 - 3), _tile(2048, 4096, 4000), _tile(4090, 256, 4096)] == [(128, 384), (128, 256), (256, 256)]
+    assert [_tile(9216, 2048, 300), _tile(4096, 2048, 512)] == [(128, 128), (64, 128)]
+    assert {_tile(2048, 4096, 129), _tile(130, 8192, 40), _tile(100, 384, 65), _tile(64, 128, 33), _tile(130, 8192, 17)} == {(64, 32)}
+    # rows further apart than the larger tiles' 32-bit offsets reach
+    assert _tile(9216, 2048, 4096, 1 << 22) == (128, 384) and _tile(9216, 2048, 4096, (1 << 22) + 8) == (64, 64)
