@@ -45,7 +45,8 @@ static __device__ inline h8 sk_frag(const u2 q, uint32_t nib, h2 sc) {
 #define SK_MAXW 16       // waves of a workgroup
 
 // RG: 16-row groups of a workgroup; NB: 16-column blocks; CH: quantisation blocks (k-steps) of a wave's chunk; WHOLE: d_in is a
-// multiple of 32 CH (every chunk whole, scales in 16-byte loads)
+// multiple of 32 CH (every chunk whole and its scales on 16 bytes).  Otherwise the last wave's chunk ends with the row: it begins inside
+// the chunk before it, and the blocks they share get scale 0 (fewer blocks than a chunk: its tail past the row's end does).
 template <int KIND, int RG, int NB, int CH, bool WHOLE>
 __global__ __launch_bounds__(SK_MAXW * 64)
 void pa_gemm_skinny_kernel(const void* a_w, const uint16_t* a_scales, const uint16_t* a_x, uint32_t a_x_stride, uint32_t a_d_out, uint32_t a_d_in, uint32_t a_n_cols,
@@ -65,7 +66,8 @@ void pa_gemm_skinny_kernel(const void* a_w, const uint16_t* a_scales, const uint
   extern __shared__ __attribute__((aligned(1024))) unsigned char sk_lds[];   // [wave][RG][16][RB]; at the end [wave][RG NB][4][64] floats
   const uint32_t tid = threadIdx.x, lane = tid & 63, ln = lane & 15, kg = lane >> 4, nw = blockDim.x >> 6;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t nb = p.d_in / 32, b0 = wave * CH;                  // the wave's first block
+  const uint32_t nb = p.d_in / 32, first = wave * CH;               // the first block that the wave counts
+  const uint32_t b0 = WHOLE ? first : nb < CH ? 0u : min(first, nb - CH);   // ... and that it loads
   const uint32_t r0 = blockIdx.x * (16 * RG);
   unsigned char* stage = sk_lds + (size_t)wave * (RG * 16 * RB);
 #pragma unroll
@@ -74,7 +76,7 @@ void pa_gemm_skinny_kernel(const void* a_w, const uint16_t* a_scales, const uint
     for (int i = 0; i < NLD; i++) {
       const uint32_t rl = i * RPL + lane / SPR, piece = (lane % SPR) ^ swz(rl);
       const size_t row = min(r0 + 16 * r + rl, p.d_out - 1);           // rows past the end repeat the last one (not stored)
-      const uint32_t off = WHOLE ? b0 * BB + piece * 16 : min(b0 * BB + piece * 16, nb * BB - 16);    // past the row's end: its last piece, weighted 0
+      const uint32_t off = WHOLE ? b0 * BB + piece * 16 : min(b0 * BB + piece * 16, nb * BB - 16);    // past the row's end (rows of less than a chunk): its last piece, weighted 0
       PF_GLL((const unsigned char*)p.w + row * nb * BB + off, stage + (r * NLD + i) * 1024);
     }
   u4 sc4[RG][CH / 8];                                                     // the 16 scales of the lane's row(s), f16
@@ -85,11 +87,16 @@ void pa_gemm_skinny_kernel(const void* a_w, const uint16_t* a_scales, const uint
 #pragma unroll
       for (int k = 0; k < CH / 8; k++) sc4[r][k] = *(const u4*)(src + b0 + 8 * k);
     } else {
+      // 8 scales a 16-byte load here too, from any even address (vector loads take unaligned dwords); a load each cost 2 - 5 us a round
+      // of the chip (1 column: Q8_0 9488 x 7456 32.0 -> 26.8 us, 4906 x 4864 13.2 -> 9.9, Q4_0 8624 x 7232 30.8 -> 20.4)
       uint16_t t[CH];
+      if (CH == 16 || nb >= CH) __builtin_memcpy(t, src + b0, 2 * CH);     // (chunks of 16: d_in is past 4096)
+      else {
 #pragma unroll
-      for (int k = 0; k < CH; k++) t[k] = src[min(b0 + k, nb - 1)];
+        for (int k = 0; k < CH; k++) t[k] = src[min((uint32_t)k, nb - 1)];
+      }
 #pragma unroll
-      for (int k = 0; k < CH; k++) if (b0 + k >= nb) t[k] = 0;
+      for (int k = 0; k < CH; k++) if ((uint32_t)k < first - b0 || (CH == 8 && (uint32_t)k >= nb - b0)) t[k] = 0;
       __builtin_memcpy(sc4[r], t, 2 * CH);
     }
   }
