@@ -129,6 +129,7 @@ hipError_t pa_launch_gemm(const GemmParams& p, int n_cu, hipStream_t s);
 // a few columns of quantised weights (proj_gemm_skinny.hip)
 bool pa_gemm_skinny_serves(const GemmParams& p);
 hipError_t pa_launch_gemm_skinny(const GemmParams& p, int n_cu, hipStream_t s);
+hipError_t pa_launch_gemm_dot(const GemmParams& p, hipStream_t s);      // ... of up to four columns over long rows (proj_gemm_dot.hip)
 // wider chunks (proj_gemm_wide.hip): the weights widened once into w16 (f16 in fragment order, the caller's staging), then a
 // GEMM over two f16 operands; pa_gemm_wide_serves tells whether a call qualifies
 bool pa_gemm_wide_serves(const GemmParams& p);
@@ -139,6 +140,7 @@ float pa_gemm_tile_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, 
 // the rules that pick an instance by size, in plain C: the tests ask them which instances their sizes take
 extern "C" uint32_t pa_rule_gemv_wide_rows(uint32_t d_out, int n_cu, uint32_t rmax);
 extern "C" int pa_rule_gemm_few_groups(int kind, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu);
+extern "C" int pa_rule_gemm_few_dot(int kind, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu);
 extern "C" uint32_t pa_rule_gemm_wide_tile(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t x_stride, int n_cu);
 hipError_t pa_launch_gemm_tile(const GemmParams& p, const uint16_t* w16, int n_cu, hipStream_t s);
 // rmsnorm of n_cols f32 columns, written as f16 (the GEMM's activation operand)

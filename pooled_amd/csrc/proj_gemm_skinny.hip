@@ -6,7 +6,7 @@
 //
 // The work is one pass over the packed weights.  What bounds it: the latency of that one pass on small matrices, the
 // activations every workgroup pulls from L2 on wide ones, the widening arithmetic (16 VALU instructions for 8 weights) on
-// large ones.  Measured (cold weights; against the dot-product kernel on the VALU that this one replaced): Q4_0 9216 x 2048,
+// large ones.  Measured (cold weights; against dot products on the VALU, kept in proj_gemm_dot.hip for where they are ahead): Q4_0 9216 x 2048,
 // 8 / 16 columns 8.9 / 14.8 -> 7.3 / 8.3 us; 2048 x 4096 7.2 / 14.8 -> 6.1 / 7.1; 14336 x 5120 101 / 170 -> 15.3 / 17.3; 5120 x 6144
 // 38 / 79 -> 10.0 / 12.0; Q8_0 4096 x 2048 6.3 / 8.3 -> 4.9 / 5.5.
 //   * a workgroup is 16 RG weight rows; K is cut into chunks of CH = 8 or 16 quantisation blocks, one per wave, so every
@@ -18,6 +18,7 @@
 //   * the activations of a k-step are 16 contiguous bytes a lane, straight from L2 into the registers the MFMA reads;
 //   * the waves' partial tiles meet in LDS and are added up in wave order: deterministic, no partial sums in memory.
 #include "pf_common.h"
+#include <algorithm>
 typedef unsigned int u2 __attribute__((ext_vector_type(2)));
 
 static __device__ inline h2 sk_as_h2(uint32_t u) { h2 r; __builtin_memcpy(&r, &u, 4); return r; }
@@ -209,6 +210,25 @@ extern "C" int pa_rule_gemm_few_groups(int kind, uint32_t d_out, uint32_t d_in, 
   while (rg > 1 && rg * bytes > 160 * 1024) rg /= 2;
   return rg;
 }
+// Whether one to four columns over long rows go to the dot-product kernel (proj_gemm_dot.hip) instead.  This kernel costs whole rounds of
+// the workgroups that the CUs' LDS and waves hold, the other follows rows x columns; both estimates in us were fitted to 604 measured
+// calls (50 sizes of each kind, 1 to 6 columns, cold weights) and are within 6 % of most.  Always this kernel there: up to 1.65 times the other's time
+// (Q8_0 885 x 6240), Q8_0 5120 x 6144 1 / 2 columns 13.7 / 14.2 us against 10.3 / 11.4; by the rule 0.3 % behind the better one on average,
+// 17 % at worst.  Up to 2048 inputs the other kernel was never ahead; past two columns of more than 2048 rows by 10 % at most, past four by 15 %.
+extern "C" int pa_rule_gemm_few_dot(int kind, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu) {
+  if (d_in <= 2048 || n_cols > 4 || (n_cols > 2 && d_out > 2048)) return 0;
+  const bool q4 = kind == PA_W_Q4_0, longer = d_in > 4096;
+  const uint32_t cus = n_cu > 0 ? (uint32_t)n_cu : 256u, ch = sk_chunk(d_in), nw = (d_in / 32 + ch - 1) / ch, rg = pa_rule_gemm_few_groups(kind, d_out, d_in, n_cols, n_cu);
+  const uint32_t lds = nw * rg * std::max(16 * ch * (q4 ? 16u : 32u), 1024u), wgs = (d_out + 16 * rg - 1) / (16 * rg);
+  const uint32_t held = std::max(1u, std::min(160u * 1024 / lds, 32u / nw)), rounds = (wgs + cus * held - 1) / (cus * held);
+  const float mb = 1e-6f * d_out * d_in * (q4 ? 0.5625f : 1.0625f), rows = 1e-3f * d_out, n = (float)n_cols;
+  const float dot = longer ? 3.25f + 0.41f * n + (0.44f + 0.27f * n) * rows + 0.091f * mb : 3.5f + 0.23f * n + (0.34f + 0.05f * n) * rows + 0.086f * mb;
+  // start, a round, a round of ragged rows on top, a MB of weights, 100 KB of LDS a workgroup
+  static const float cost[2][2][5] = { { { 1.8f, 0.f, 0.42f, 0.19f, 3.6f }, { 0.f, 3.8f, 0.64f, 0.13f, 1.9f } },          // Q8_0: up to 4096 inputs, longer
+                                       { { 1.4f, 0.73f, 0.68f, 0.234f, 4.9f }, { 0.f, 2.9f, 0.97f, 0.206f, 3.2f } } };    // Q4_0
+  const float* c = cost[q4][longer];
+  return dot < c[0] + (c[1] + (d_in % (32 * ch) ? c[2] : 0.f)) * rounds + c[3] * mb + c[4] * 1e-5f * lds;
+}
 template <int KIND>
 static hipError_t sk_shape(const GemmParams& p, int n_cu, hipStream_t s) {
   const int rg = pa_rule_gemm_few_groups(KIND, p.d_out, p.d_in, p.n_cols, n_cu);
@@ -225,5 +245,6 @@ bool pa_gemm_skinny_serves(const GemmParams& p) {
 }
 hipError_t pa_launch_gemm_skinny(const GemmParams& p, int n_cu, hipStream_t s) {
   if (p.d_out == 0 || p.d_in == 0 || (p.d_in & 31) || p.n_cols == 0) return hipErrorInvalidValue;
+  if (pa_rule_gemm_few_dot(p.kind, p.d_out, p.d_in, p.n_cols, n_cu)) return pa_launch_gemm_dot(p, s);
   return p.kind == PA_W_Q4_0 ? sk_shape<PA_W_Q4_0>(p, n_cu, s) : sk_shape<PA_W_Q8_0>(p, n_cu, s);
 }

@@ -212,15 +212,17 @@ GEMM_FEW_SIZES = [(16, 32, 1), (17, 256, 2), (31, 288, 15), (4096, 4096, 16), (4
                   (33, 4128, 5), (70, 2080, 19), (33, 256, 20), (40, 4608, 11), (48, 5120, 31),   # one row group
                   (5000, 2048, 12), (5000, 2080, 16), (5000, 2048, 24), (4111, 1056, 32),   # two of chunks of 8 blocks
                   (9216, 2048, 16), (8201, 1056, 13),                                    # four, one column block
-                  (4111, 4128, 31), (8193, 4128, 9), (8200, 4128, 20), (8200, 5120, 32)]   # Q4_0: two and four of chunks of 16
+                  (4111, 4128, 31), (8193, 4128, 9), (8200, 4128, 20), (8200, 5120, 32),   # Q4_0: two and four of chunks of 16
+                  (5120, 6144, 1), (5119, 6144, 2), (1001, 8192, 4), (999, 7968, 3), (9216, 4064, 1), (3, 4128, 2), (6001, 4096, 2)]   # dot products
 
 
 @pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])
 @pytest.mark.parametrize("d_out,d_in,n", GEMM_FEW_SIZES)
 def test_gemm_few_columns(kind, d_out, d_in, n):
-    """Up to 32 columns straight from the packed planes: one, two and four 16-row groups a workgroup (fewer and more of them
+    """Up to 32 columns straight from the packed planes, on the matrix cores: one, two and four 16-row groups a workgroup (fewer and more of them
     than CUs, d_in either side of 4096, what fits the LDS), one and two column blocks, chunks of 8 and 16 blocks that d_in
-    fills or not, ragged rows, and the first column counts of the next kernel.  The sums are f32 in another order than the
+    fills or not, ragged rows, and the first column counts of the next kernel; one to four columns over long rows on the VALU's dot
+    products.  The sums are f32 in another order than the
     f64 oracle's: 2e-5 of the largest output is some 300 roundings at most."""
     rng = np.random.default_rng(d_out + 7 * d_in + n + kind)
     w, sc = _weights(kind, d_out, d_in, rng)

@@ -31,9 +31,12 @@ def test_gemv_sizes_take_every_number_of_rows():
 
 
 def _few(kind, d_out, d_in, n):
-    """(kind, row groups, column blocks, blocks of a chunk, d_in in whole chunks) of the few-column kernel; None past its range"""
+    """(kind, row groups, column blocks, blocks of a chunk, d_in in whole chunks) of the few-column kernel, (kind, blocks a lane) of the
+    dot-product one; None past their range"""
     if n > 32 or (n > 16 and kind != PA_W_Q4_0 and d_in > 4096):
         return None
+    if _rule("pa_rule_gemm_few_dot", ctypes.c_int(kind), d_out, d_in, n, ctypes.c_int(CUS)):
+        return kind, 2 if d_in <= 4096 else 4
     ch = 8 if d_in <= 4096 else 16
     rg = _rule("pa_rule_gemm_few_groups", ctypes.c_int(kind), d_out, d_in, n, ctypes.c_int(CUS))
     return kind, rg, 1 if n <= 16 else 2, ch, d_in % (32 * ch) == 0
@@ -43,8 +46,13 @@ def test_few_column_sizes_take_every_instance():
     kinds = (PA_W_Q4_0, PA_W_Q8_0)
     tested = {_few(k, *size) for k in kinds for size in GEMM_FEW_SIZES}
     reached = {_few(k, d_out, d_in, n) for k in kinds for d_out in (16, 4096, 4097, 5000, 8176, 8177, 9216, 20000) for d_in in range(32, 8193, 32)
-               for n in (1, 8, 9, 16, 17, 32)}
-    assert len(reached) > 30 and reached <= tested | {None}
+               for n in (1, 2, 4, 8, 9, 16, 17, 32)}
+    assert len(reached) > 40 and reached <= tested | {None}
+    # the dot-product kernel takes up to four columns over rows of more than 2048 inputs, two of them past 2048 rows
+    dot = {(k, d_out, d_in, n) for k in kinds for d_out in (16, 1000, 2048, 2049, 5120, 9216, 20000) for d_in in range(32, 8193, 32) for n in (1, 2, 3, 4, 5)
+           if len(_few(k, d_out, d_in, n)) == 2}
+    assert {n for _, _, _, n in dot} == {1, 2, 3, 4} and all(d_in > 2048 and (n <= 2 or d_out <= 2048) for _, d_out, d_in, n in dot)
+    assert all((PA_W_Q8_0, 5120, 6144, n) in dot for n in (1, 2)) and not any((PA_W_Q4_0, 20000, 5120, n) in dot for n in (1, 2))
 
 
 def _tile(d_out, d_in, n, x_stride=None):
