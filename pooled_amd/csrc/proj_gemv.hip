@@ -250,15 +250,23 @@ static hipError_t launch_rows(uint32_t rw, const GemvParams& p, hipStream_t s) {
 }
 
 // Rows per wave past 4096 inputs (quantised weights).  Every workgroup fetches, norms and stages all of x -- 20 KB and the norm's
-// 20 KB at 5120 inputs, twice the weights of its eight rows at two rows a wave -- so few large workgroups are faster as long as
+// 20 KB at 5120 inputs, twice the Q4_0 weights of its eight rows at two rows a wave -- so few large workgroups are faster as long as
 // every SIMD keeps two waves and they come out even.  Time follows the rows of the busiest SIMD plus about 1.6 rows' worth for every
-// wave it is dealt; measured at 1 .. 8 rows a wave (us, cold weights, Q4_0): 14336 x 5120 20.6 15.1 14.4 13.6 13.2 13.9 12.5 13.1;
-// 10240 x 5120 16.0 11.8 12.0 11.1 9.9 10.9 11.8 12.9; 8192 x 5120 13.4 10.7 10.1 8.7 9.5 10.6 11.8 9.6; 17000 x 4608 20.5 16.8 13.9
-// 15.0 14.2 13.9 15.0 22.3; Q8_0 14336 x 5120 21.3 20.7 19.9 18.8 18.0 25.6.  With fewer than six rows a SIMD two rows a wave are as
-// good as any (5120 x 6144: 7.3, 7.4 at three, 7.3 at five).  RMAX: what fits the registers of two waves a SIMD.
-extern "C" uint32_t pa_rule_gemv_wide_rows(uint32_t d_out, int n_cu, uint32_t rmax) {
+// wave it is dealt; measured at 1 .. 7 rows a wave with the norm (us, cold weights, Q4_0): 14336 x 5120 18.5 13.5 13.3 13.1 12.9 13.6 12.3;
+// 10240 x 5120 14.6 11.3 11.3 10.7 9.7 10.5 11.6; 8192 x 5120 12.5 9.1 9.7 8.6 9.4 10.6 11.7; 17000 x 4608 20.8 15.5 15.0 14.7 14.8
+// 14.0 15.0.  With fewer than six rows a SIMD two rows a wave are as good as any (5120 x 6144: 7.3, 7.4 at three, 7.3 at five).
+// Q8_0 rows are twice the bytes to the same x: two rows a wave are ahead everywhere without the norm (14336 x 5120 18.9 16.4 16.9 17.5 17.6,
+// accumulating 18.3 15.9 17.3 17.8 17.6; 17000 x 4608 21.6 17.4 18.5 18.9 20.1) and with it past 12 rows a SIMD or four blocks a lane
+// (17000 x 4608 22.0 19.2 20.0 20.6 20.5; 16000 x 7168 35.9 26.9 28.1); below, the rule's choice (7168 x 5120 12.4 11.1 11.6 10.7 12.1; 9000 x 6016
+// 15.6 14.4 13.8 15.4 13.9).  At most what fits the registers of two waves a SIMD.
+static constexpr uint32_t wide_rows_max(int kind, int bpl, bool norm) {
+  return kind == PA_W_Q4_0 ? (bpl == 3 ? 7 : 4) : norm && bpl == 3 ? 5 : 2;
+}
+extern "C" uint32_t pa_rule_gemv_wide_rows(int kind, uint32_t d_out, uint32_t d_in, int norm, int n_cu) {
   const uint32_t simds = 4u * (uint32_t)n_cu;
   if (d_out < 6 * simds) return d_out >= 4 * simds ? 2 : 1;
+  const uint32_t rmax = wide_rows_max(kind, d_in <= 6144 ? 3 : 4, norm != 0);
+  if (rmax == 2 || (kind == PA_W_Q8_0 && d_out > 12 * simds)) return 2;
   uint32_t best = 1;
   float cost = 1e30f;
   for (uint32_t r = 1; r <= rmax; r++) {
@@ -272,8 +280,7 @@ extern "C" uint32_t pa_rule_gemv_wide_rows(uint32_t d_out, int n_cu, uint32_t rm
 template <int KIND, int BPL, bool NORM>
 static hipError_t launch_rw(const GemvParams& p, int n_cu, hipStream_t s) {
   if constexpr (BPL >= 3) {
-    constexpr int RMAX = KIND == PA_W_Q4_0 ? (BPL == 3 ? 7 : 4) : (BPL == 3 ? 5 : 3);
-    return launch_rows<KIND, BPL, NORM, RMAX>(pa_rule_gemv_wide_rows(p.d_out, n_cu, RMAX), p, s);
+    return launch_rows<KIND, BPL, NORM, wide_rows_max(KIND, BPL, NORM)>(pa_rule_gemv_wide_rows(KIND, p.d_out, p.d_in, NORM, n_cu), p, s);
   } else {
     // rows per wave: as many as still leave about two 4-wave workgroups per CU, within the registers that RW x BPL
     // blocks of weights take (f32: 32 registers a block, Q8_0: 8, Q4_0: 4)

@@ -49,10 +49,9 @@ def test_gemv_matches_oracle(kind, d_out, d_in):
         assert np.array_equal(dy.download(np.float32, d_out), got)
 
 
-# sizes past 4096 inputs that take every number of rows a wave (test_proj_rules.py asks the rule): on a 256-CU part Q4_0 / Q8_0
-# 2 / 2, 4 / 4, 4 / 4, 6 / 4, 5 / 5 rows of three blocks a lane, 3 / 3 and 4 / 3 of four blocks, then 7 / 5, 1 / 1, 3 / 3 and 2 / 2, 1 / 1
+# sizes past 4096 inputs that take every number of rows a wave with and without the norm (test_proj_rules.py asks the rule)
 GEMV_WIDE_SIZES = [(6143, 4128), (6145, 4128), (8191, 5120), (11265, 4160), (14337, 6144), (9001, 6176), (6150, 8192),
-                   (14335, 5120), (4000, 4128), (6144, 4128), (4111, 8192), (1000, 7968)]
+                   (14335, 5120), (4000, 4128), (6144, 4128), (4111, 8192), (1000, 7968), (9003, 6016)]
 
 
 @pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])

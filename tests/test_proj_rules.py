@@ -15,19 +15,22 @@ def _rule(name, *args):
     return fn(*(a if isinstance(a, ctypes._SimpleCData) else u32(a) for a in args))
 
 
-def _gemv(kind, d_out, d_in):
-    """(kind, blocks a lane, rows a wave) past 4096 inputs"""
-    bpl = 3 if d_in <= 6144 else 4
-    most = {(PA_W_Q4_0, 3): 7, (PA_W_Q4_0, 4): 4, (PA_W_Q8_0, 3): 5, (PA_W_Q8_0, 4): 3}[kind, bpl]
-    return kind, bpl, _rule("pa_rule_gemv_wide_rows", d_out, ctypes.c_int(CUS), most)
+def _gemv(kind, d_out, d_in, norm):
+    """(kind, blocks a lane, norm, rows a wave) past 4096 inputs"""
+    return kind, 3 if d_in <= 6144 else 4, norm, _rule("pa_rule_gemv_wide_rows", ctypes.c_int(kind), d_out, d_in, ctypes.c_int(norm), ctypes.c_int(CUS))
 
 
 def test_gemv_sizes_take_every_number_of_rows():
-    got = {_gemv(kind, d_out, d_in) for kind in (PA_W_Q4_0, PA_W_Q8_0) for d_out, d_in in GEMV_WIDE_SIZES}
-    assert got == {(k, b, r) for k, b, most in ((PA_W_Q4_0, 3, 7), (PA_W_Q4_0, 4, 4), (PA_W_Q8_0, 3, 5), (PA_W_Q8_0, 4, 3)) for r in range(1, most + 1)}
+    forms = [(k, norm) for k in (PA_W_Q4_0, PA_W_Q8_0) for norm in (False, True)]
+    got = {_gemv(k, d_out, d_in, norm) for k, norm in forms for d_out, d_in in GEMV_WIDE_SIZES}
+    most = {(PA_W_Q4_0, 3, True): 7, (PA_W_Q4_0, 3, False): 7, (PA_W_Q4_0, 4, True): 4, (PA_W_Q4_0, 4, False): 4,
+            (PA_W_Q8_0, 3, True): 5, (PA_W_Q8_0, 3, False): 2, (PA_W_Q8_0, 4, True): 2, (PA_W_Q8_0, 4, False): 2}
+    assert got == {(k, b, norm, r) for (k, b, norm), m in most.items() for r in range(1, m + 1)}
     # a wave whose last rows are past the end, for every instance of two rows and more but one (three rows are taken at one d_out only)
-    ragged = {_gemv(kind, d_out, d_in) for kind in (PA_W_Q4_0, PA_W_Q8_0) for d_out, d_in in GEMV_WIDE_SIZES if d_out % _gemv(kind, d_out, d_in)[2]}
-    assert {g for g in got if g[2] > 1} - ragged <= {(PA_W_Q4_0, 3, 3), (PA_W_Q8_0, 3, 3)}
+    ragged = {_gemv(k, d_out, d_in, norm) for k, norm in forms for d_out, d_in in GEMV_WIDE_SIZES if d_out % _gemv(k, d_out, d_in, norm)[3]}
+    assert all(b == 3 and r == 3 for _, b, _, r in {g for g in got if g[3] > 1} - ragged)
+    # Q8_0: two rows without the norm, and on tall weights
+    assert _gemv(PA_W_Q8_0, 14336, 5120, False)[3] == 2 and _gemv(PA_W_Q8_0, 14336, 5120, True)[3] == 2 and _gemv(PA_W_Q8_0, 7168, 5120, True)[3] == 4
 
 
 def _few(kind, d_out, d_in, n):
