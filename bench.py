@@ -212,7 +212,7 @@ def prefill_leg(steps, with_cpu, kv_q8=False):
                min_ms_per_step=round(min(step_ms), 4), max_ms_per_step=round(max(step_ms), 4), cold_first_ms=round(cold_first_ms, 4),
                step_ms=[round(x, 3) for x in step_ms], flops_per_step=flops, plan=pa.plan("prefill", base, n),
                roofline=dict(bound="mfma", achieved=round(tf_kernel, 1), peak=MFMA_F16_PEAK_TFLOPS, unit="TFLOP/s", frac=round(tf_kernel / MFMA_F16_PEAK_TFLOPS, 4),
-                             traffic=None, kernel="pa_prefill_kernel<256, 1, 8>", kernel_ms=round(k_ms, 4), kernel_ms_mean=round(k_mean, 4),
+                             traffic=None, kernel="pa_prefill_kernel<256, 1, 8, false>", kernel_ms=round(k_ms, 4), kernel_ms_mean=round(k_mean, 4),
                              kernel_ms_min=round(min(kern_ms), 4), kernel_ms_max=round(max(kern_ms), 4), reported="median launch",
                              algorithmic_flops_per_launch=flops, launches=len(kern_ms)))
     if with_cpu:
@@ -384,7 +384,7 @@ def layer_leg(pa, cfg, ctx, steps, warmup, attn_ms, n_rot, rng):
                 gemv_o_acc=dict(us=round(t_o * 1e3, 2), weight_bytes=b_o, gbs=round(b_o / t_o / 1e6, 1)),
                 bytes_per_step=kv_bytes + b_qkv + b_o, gbs=round((kv_bytes + b_qkv + b_o) / t_layer / 1e6, 1),
                 pct_hbm_peak=round(100 * (kv_bytes + b_qkv + b_o) / t_layer / 1e6 / HBM_PEAK_GBS, 2),
-                verify_block=dict(workload="%d tokens at positions %d .. %d through the same half of the layer (pa_attn_layer_prefill: rmsnorm, skinny-chunk "
+                verify_block=dict(workload="%d tokens at positions %d .. %d through the same half of the layer (pa_attn_layer_prefill: rmsnorm, few-column "
                                            "projections, pre-step, split-K attention in column groups, merge/gate)" % (nv, ctx - nv + 1, ctx),
                                   us_per_step=round(t_verify * 1e3, 2), us_per_token=round(t_verify * 1e3 / nv, 2)))
 

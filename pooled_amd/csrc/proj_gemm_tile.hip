@@ -17,9 +17,9 @@
 // What bounds it: on full rounds of the chip the MFMA rate the power limit allows and the rounds' own ends (4096 columns:
 // 14336 x 5120 1090 - 1130 TFLOP/s, 9216 x 2048 1000); on one round or less the LDS-direct loads' latency (a tile's 96 - 120 KB
 // in flight a CU).  Measured against the kernel it replaced (128 columns x 256 / 384 / 512 rows, four waves, weight fragments
-// from memory straight to registers) and the 64 x 64 kernel: 777 columns of 5120 x 6144 106 -> 73 us, of 14336 x 5120 144 -> 132, of
-// 9216 x 2048 67 -> 42; 2048 columns of 2048 x 4096 82 -> 47; 512 of 14336 x 5120 142 -> 94, of 4096 x 2048 22.0 -> 19.4; 4096 of
-// 9216 x 2048 163 -> 155.  Not kept: a ninth wave that prefetches the weight stream into L2 (slower on every shape), activation
+// from memory straight to registers) and the 64 x 64 kernel, Q8_0, five weights in rotation: 777 columns of 5120 x 6144 100 -> 64 us, of
+// 14336 x 5120 143 -> 133, of 9216 x 2048 59 -> 36; 2048 columns of 2048 x 4096 76 -> 40; 512 of 14336 x 5120 141 -> 92, of 4096 x 2048
+// 16.8 -> 15.0; 4096 of 9216 x 2048 161 -> 154, of 14336 x 5120 609 -> 568.  Not kept: a ninth wave that prefetches the weight stream into L2 (slower on every shape), activation
 // rows at a padded stride (no change).
 #include "pf_common.h"
 
@@ -223,7 +223,10 @@ static const TileShape tile_shapes[] = {
 
 // One workgroup is resident per CU, so a call costs whole rounds of n_cu workgroups: the shape with the cheapest rounds, and
 // its estimate in us.  Larger tiles pay less traffic per product but are coarser: which one wins changes with every
-// multiple of a tile edge (777 columns of 5120 x 6144: 128 x 160, 224 workgroups, 73 us; 128 x 128, 280 workgroups, 87 us).
+// multiple of a tile edge (777 columns of 5120 x 6144: 128 x 160, 224 workgroups, 63 us; 128 x 128, 280 workgroups, 87 us).  Of
+// 104 sizes measured on every tile and on the 64 x 64 kernel (8 weight shapes x 13 column counts, cold weights) the choice between
+// all of them is the fastest at 84 and within 6 % at 8; it is 9 - 33 % behind at 12, most where one round of few workgroups (which
+// costs less than a full one) is set against the 64 x 64 kernel: 9216 x 2048, 200 columns 27.9 us, on 128 x 128 21.1.
 static int pa_pick_tile(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, float* us) {
   int best = 0;
   *us = 1e30f;

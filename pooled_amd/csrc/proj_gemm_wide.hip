@@ -258,7 +258,7 @@ bool pa_gemm_wide_serves(const GemmParams& p) {
 size_t pa_gemm_wide_staging_bytes(uint32_t d_out, uint32_t d_in) { return (size_t)((d_out + 31) / 32) * 32 * d_in * sizeof(uint16_t); }
 
 // The 64 x 64 kernel runs two workgroups a CU and its time follows their number: about 4 us and 4.6 ns per k and workgroup a
-// CU (4096 x 2048: 256 / 512 / 777 columns 13.4 / 22.0 / 34 us).  The larger tiles where their rounds come out cheaper, and their
+// CU (cold weights, 4096 x 2048: 256 / 512 / 777 columns 13.0 / 19.8 / 32.3 us; past one a CU it is some 10 % longer on 9216 rows).  The larger tiles where their rounds come out cheaper, and their
 // kernel takes the stride.
 // Fewer 64 x 64 tiles than half the CUs: 32-row tiles (twice the workgroups) with twice the stages in flight (2048 x 4096 on up to
 // 64 columns, cold: 20 -> 16.7 us; with 144 tiles, 9216 x 2048, it is 2 us slower).
