@@ -330,14 +330,15 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   };
 
   // ---- main loop ----
-  // PAIRED: the near half's rows are all masked from its step n_live on; there its waves only stage their share of the remaining tiles.
-  // Every wave passes n_steps barriers, whichever loop it is in.  At head_dim 256 that is a loop of its own: with the compute under a
-  // branch instead, the loop's blocks end where the compiler overlaps the end of a tile with the start of the next (us, branch / two
-  // loops: 4096 columns at 8192 666 / 665, at 16384 1113 / 1108, at 64K 3833 / 3811).  At 128 the branch is the cheaper form (4096 columns
-  // at 28K 946 against 951, 2500 at 8192 253 against 257).  Whole blocks (a wave's last row sees at most a tile less than the
-  // workgroup's) compute every step: either form of skipping there costs 0.3 % of a long pass.
-  constexpr bool TWO_LOOPS = PAIRED && HD == 256;
-  const uint32_t n_live = !TWO_LOOPS ? n_steps : w_max_end > t_begin ? min((w_max_end - t_begin + PF_TN - 1) / PF_TN, n_steps) : 0u;
+  // From its step n_live on a wave has no row left: it only stages its share of the remaining tiles.  Every wave passes n_steps barriers,
+  // whichever loop it is in.  PAIRED: that is the near half of a pair.  Whole blocks: the waves past the last block's rows, from the start
+  // (split passes, those waves computing / not: 24 / 4-head shape at 50000, 130 columns 214 / 205 us, 88 columns 170 / 160); a wave whose
+  // rows end a tile before the workgroup's computes it, as an end of its own costs 0.3 % of a long pass.
+  // It is a loop of its own: with the compute under a branch instead, the loop's blocks end where the compiler overlaps the end of a tile
+  // with the start of the next (us, branch / two loops, pairs: 4096 columns at 8192 666 / 665, at 16384 1113 / 1108, at 64K 3833 / 3811).
+  // For pairs at head_dim 128 the branch is the cheaper form (4096 columns at 28K 946 against 951, 2500 at 8192 253 against 257).
+  constexpr bool TWO_LOOPS = !PAIRED || HD == 256;
+  const uint32_t n_live = !PAIRED ? (wrow0 < R ? n_steps : 0u) : !TWO_LOOPS ? n_steps : w_max_end > t_begin ? min((w_max_end - t_begin + PF_TN - 1) / PF_TN, n_steps) : 0u;
   const uint32_t n_even = n_live & ~1u;
   uint32_t lane_e = lane;
   {
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
       constexpr int par = decltype(PAR)::value;
       const uint32_t tp = t_begin + i * PF_TN;
       if (i + 1 < n_steps) { issue_k(par ? kbuf0 : kbuf1, tp + PF_TN); issue_v(par ? vbuf0 : vbuf1, tp + PF_TN); }
-      if (TWO_LOOPS || !PAIRED || tp < w_max_end) {
+      if (TWO_LOOPS || tp < w_max_end) {
         qk(par ? kbuf1 : kbuf0, tp);
         sm(tp);
         pv(par ? vbuf1 : vbuf0, tp);
