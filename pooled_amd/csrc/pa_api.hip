@@ -247,10 +247,9 @@ static void fill_glue(const pa_ctx* ctx, GlueParams& p) {
   p.head_rows = c.max_seq + 32;
 }
 
-extern "C" int pa_glue_kv(pa_ctx* ctx, uint32_t layer, const float* d_q_in, uint32_t q_stride, const float* d_k,
-                          uint32_t k_stride, const float* d_v, uint32_t v_stride, const float* d_qw, const float* d_kw,
-                          uint32_t base_pos, uint32_t n_cols) {
-  if (!ctx) return PA_ERR_INVALID;
+// a chunk's pre-step and cache write: what it is given checked, and the kernel's parameters
+static int glue_kv_params(pa_ctx* ctx, uint32_t layer, const float* d_q_in, uint32_t q_stride, const float* d_k, uint32_t k_stride, const float* d_v,
+                          uint32_t v_stride, const float* d_qw, const float* d_kw, uint32_t base_pos, uint32_t n_cols, GlueParams& p) {
   int rc = check_cols(ctx, "pa_glue_kv", layer, true, base_pos, n_cols);
   if (rc) return rc;
   const pa_config& c = ctx->cfg;
@@ -258,11 +257,21 @@ extern "C" int pa_glue_kv(pa_ctx* ctx, uint32_t layer, const float* d_q_in, uint
   if (!d_q_in || !d_k || !d_v) return fail(ctx, PA_ERR_INVALID, "pa_glue_kv: null input");
   if ((c.flags & PA_FLAG_QK_NORM) && (!d_qw || !d_kw)) return fail(ctx, PA_ERR_INVALID, "pa_glue_kv: norm weights required");
   if (q_stride < qcol || k_stride < kvd || v_stride < kvd) return fail(ctx, PA_ERR_INVALID, "pa_glue_kv: column stride shorter than a column");
-  GlueParams p; fill_glue(ctx, p);
+  fill_glue(ctx, p);
   p.q_in = d_q_in; p.k_in = d_k; p.v_in = d_v; p.qw = d_qw; p.kw = d_kw;
   p.k_cache = ctx->layers[layer].k; p.v_cache = ctx->layers[layer].v; p.ks_cache = ctx->layers[layer].ks; p.vs_cache = ctx->layers[layer].vs;
   p.q_stride = q_stride; p.k_stride = k_stride; p.v_stride = v_stride;
   p.base_pos = base_pos; p.n_cols = n_cols;
+  return PA_OK;
+}
+
+extern "C" int pa_glue_kv(pa_ctx* ctx, uint32_t layer, const float* d_q_in, uint32_t q_stride, const float* d_k,
+                          uint32_t k_stride, const float* d_v, uint32_t v_stride, const float* d_qw, const float* d_kw,
+                          uint32_t base_pos, uint32_t n_cols) {
+  if (!ctx) return PA_ERR_INVALID;
+  GlueParams p;
+  int rc = glue_kv_params(ctx, layer, d_q_in, q_stride, d_k, k_stride, d_v, v_stride, d_qw, d_kw, base_pos, n_cols, p);
+  if (rc) return rc;
   HIPCHK(ctx, pa_launch_glue(p, ctx->stream));
   return PA_OK;
 }
@@ -829,60 +838,68 @@ extern "C" int pa_rmsnorm_f16(pa_ctx* ctx, const float* d_x, uint32_t x_stride, 
   return PA_OK;
 }
 
+// a wide chunk's projection; heads: with the pre-step as its end (pa_gemm_heads_serves)
+static int gemm_wide(pa_ctx* ctx, const pa_weight* w, const GemmParams& p, const GlueParams* heads) {
+  // the weights as f16 in fragment order: a copy kept with the weight from its first large chunk on, while the
+  // context's budget lasts (the handle's contents never change); past the budget, or where the allocation fails,
+  // widened per call into the context's staging
+  const size_t need = pa_gemm_wide_staging_bytes(w->d_out, w->d_in);
+  pa_weight* wm = const_cast<pa_weight*>(w);
+  void* fresh = nullptr;                        // a copy to keep, allocated by this call; attached only once its fill is queued
+  if (!wm->w16 && ctx->weight_cache_used + need <= ctx->weight_cache_limit) {
+    if (hipMalloc(&fresh, need) != hipSuccess) { fresh = nullptr; (void)hipGetLastError(); }
+  }
+  uint16_t* w16 = wm->w16 ? wm->w16 : (uint16_t*)fresh;
+  bool widen = fresh != nullptr;
+  if (!w16) {
+    int rc = grow_scratch(ctx, &ctx->w16_buf, &ctx->w16_buf_bytes, need);
+    if (rc) return rc;
+    w16 = (uint16_t*)ctx->w16_buf; widen = true;
+  }
+  if (wm->w16 && wm->w16_ready && wm->w16_stream != ctx->stream) {
+    // the kept copy was filled on another stream: wait for that fill once, on the host; from then on any stream may read it
+    HIPCHK(ctx, hipEventSynchronize(wm->w16_ready));
+    (void)hipEventDestroy(wm->w16_ready);
+    wm->w16_ready = nullptr; wm->w16_stream = nullptr;
+  }
+  hipError_t e = pa_launch_gemm_wide(p, w16, widen, heads, ctx->n_cu, ctx->stream);
+  if (fresh) {
+    hipEvent_t ready = nullptr;
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ready, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(ready, ctx->stream);
+    if (e != hipSuccess) {
+      // the fill did not go out (or cannot be tracked): the handle keeps no copy, so a later call widens again
+      (void)hipStreamSynchronize(ctx->stream);
+      if (ready) (void)hipEventDestroy(ready);
+      (void)hipFree(fresh);
+      return fail_hip(ctx, e, "pa_gemm: widening the weights");
+    }
+    wm->w16 = (uint16_t*)fresh; wm->w16_bytes = need; wm->w16_ready = ready; wm->w16_stream = ctx->stream;
+    ctx->weight_cache_used += need;
+  }
+  HIPCHK(ctx, e);
+  return PA_OK;
+}
+
+static GemmParams gemm_params(const pa_weight* w, const void* d_x_f16, uint32_t x_stride, uint32_t n_cols, float* d_y, uint32_t y_stride, int acc) {
+  GemmParams p; memset(&p, 0, sizeof p);
+  p.w = w->w; p.scales = w->scales; p.x = (const uint16_t*)d_x_f16; p.y = d_y; p.x_stride = x_stride; p.y_stride = y_stride;
+  p.d_out = w->d_out; p.d_in = w->d_in; p.n_cols = n_cols; p.acc = acc; p.kind = w->kind;
+  return p;
+}
+
 extern "C" int pa_gemm(pa_ctx* ctx, const pa_weight* w, const void* d_x_f16, uint32_t x_stride, uint32_t n_cols, float* d_y, uint32_t y_stride, int acc) {
   const char* who = "pa_gemm";
   if (!ctx) return PA_ERR_INVALID;
   if (!w || !d_x_f16 || !d_y) return fail(ctx, PA_ERR_INVALID, std::string(who) + ": null argument");
   if (n_cols == 0 || x_stride < w->d_in || (x_stride & 7) || y_stride < w->d_out || ((uintptr_t)d_x_f16 & 15) || ((uintptr_t)d_y & 3))
     return fail(ctx, PA_ERR_INVALID, std::string(who) + ": x stride must be a multiple of 8 halves and >= d_in, y stride >= d_out, x 16-byte aligned");
-  GemmParams p; memset(&p, 0, sizeof p);
-  p.w = w->w; p.scales = w->scales; p.x = (const uint16_t*)d_x_f16; p.y = d_y; p.x_stride = x_stride; p.y_stride = y_stride;
-  p.d_out = w->d_out; p.d_in = w->d_in; p.n_cols = n_cols; p.acc = acc; p.kind = w->kind;
+  const GemmParams p = gemm_params(w, d_x_f16, x_stride, n_cols, d_y, y_stride, acc);
   if (pa_gemm_skinny_serves(p)) {
     HIPCHK(ctx, pa_launch_gemm_skinny(p, ctx->n_cu, ctx->stream));
     return PA_OK;
   }
-  if (pa_gemm_wide_serves(p)) {
-    // the weights as f16 in fragment order: a copy kept with the weight from its first large chunk on, while the
-    // context's budget lasts (the handle's contents never change); past the budget, or where the allocation fails,
-    // widened per call into the context's staging
-    const size_t need = pa_gemm_wide_staging_bytes(w->d_out, w->d_in);
-    pa_weight* wm = const_cast<pa_weight*>(w);
-    void* fresh = nullptr;                        // a copy to keep, allocated by this call; attached only once its fill is queued
-    if (!wm->w16 && ctx->weight_cache_used + need <= ctx->weight_cache_limit) {
-      if (hipMalloc(&fresh, need) != hipSuccess) { fresh = nullptr; (void)hipGetLastError(); }
-    }
-    uint16_t* w16 = wm->w16 ? wm->w16 : (uint16_t*)fresh;
-    bool widen = fresh != nullptr;
-    if (!w16) {
-      int rc = grow_scratch(ctx, &ctx->w16_buf, &ctx->w16_buf_bytes, need);
-      if (rc) return rc;
-      w16 = (uint16_t*)ctx->w16_buf; widen = true;
-    }
-    if (wm->w16 && wm->w16_ready && wm->w16_stream != ctx->stream) {
-      // the kept copy was filled on another stream: wait for that fill once, on the host; from then on any stream may read it
-      HIPCHK(ctx, hipEventSynchronize(wm->w16_ready));
-      (void)hipEventDestroy(wm->w16_ready);
-      wm->w16_ready = nullptr; wm->w16_stream = nullptr;
-    }
-    hipError_t e = pa_launch_gemm_wide(p, w16, widen, ctx->n_cu, ctx->stream);
-    if (fresh) {
-      hipEvent_t ready = nullptr;
-      if (e == hipSuccess) e = hipEventCreateWithFlags(&ready, hipEventDisableTiming);
-      if (e == hipSuccess) e = hipEventRecord(ready, ctx->stream);
-      if (e != hipSuccess) {
-        // the fill did not go out (or cannot be tracked): the handle keeps no copy, so a later call widens again
-        (void)hipStreamSynchronize(ctx->stream);
-        if (ready) (void)hipEventDestroy(ready);
-        (void)hipFree(fresh);
-        return fail_hip(ctx, e, "pa_gemm: widening the weights");
-      }
-      wm->w16 = (uint16_t*)fresh; wm->w16_bytes = need; wm->w16_ready = ready; wm->w16_stream = ctx->stream;
-      ctx->weight_cache_used += need;
-    }
-    HIPCHK(ctx, e);
-    return PA_OK;
-  }
+  if (pa_gemm_wide_serves(p)) return gemm_wide(ctx, w, p, nullptr);
   HIPCHK(ctx, pa_launch_gemm(p, ctx->n_cu, ctx->stream));
   return PA_OK;
 }
@@ -909,8 +926,15 @@ extern "C" int pa_attn_layer_prefill(pa_ctx* ctx, uint32_t layer, const pa_weigh
   float* qkv = (float*)((unsigned char*)ctx->chunk_buf + b_xn);
   uint16_t* at = (uint16_t*)((unsigned char*)ctx->chunk_buf + b_xn + b_qkv);
   if ((rc = pa_rmsnorm_f16(ctx, d_x, x_stride, d_attn_norm_w, dim, n_cols, xn, dim))) return rc;
-  if ((rc = pa_gemm(ctx, w_qkv, xn, dim, n_cols, qkv, rows, 0))) return rc;
-  if ((rc = pa_glue_kv(ctx, layer, qkv, rows, qkv + q_rows, rows, qkv + q_rows + kvd, rows, d_qw, d_kw, base_pos, n_cols))) return rc;
+  GlueParams heads;
+  const GemmParams proj = gemm_params(w_qkv, xn, dim, n_cols, qkv, rows, 0);
+  if ((rc = glue_kv_params(ctx, layer, qkv, rows, qkv + q_rows, rows, qkv + q_rows + kvd, rows, d_qw, d_kw, base_pos, n_cols, heads))) return rc;
+  if (pa_gemm_heads_serves(proj, heads, ctx->n_cu)) {
+    if ((rc = gemm_wide(ctx, w_qkv, proj, &heads))) return rc;
+  } else {
+    if ((rc = pa_gemm(ctx, w_qkv, xn, dim, n_cols, qkv, rows, 0))) return rc;
+    HIPCHK(ctx, pa_launch_glue(heads, ctx->stream));
+  }
   if ((rc = pa_attn_prefill(ctx, layer, nullptr, 0, gated ? ctx->gate_buf : nullptr, qd, base_pos, n_cols, at, qd, PA_OUT_F16))) return rc;
   return pa_gemm(ctx, w_o, at, qd, n_cols, d_x, x_stride, 1);
 }

@@ -134,13 +134,18 @@ hipError_t pa_launch_gemm_dot(const GemmParams& p, hipStream_t s);      // ... o
 // GEMM over two f16 operands; pa_gemm_wide_serves tells whether a call qualifies
 bool pa_gemm_wide_serves(const GemmParams& p);
 size_t pa_gemm_wide_staging_bytes(uint32_t d_out, uint32_t d_in);
-hipError_t pa_launch_gemm_wide(const GemmParams& p, uint16_t* w16, bool widen, int n_cu, hipStream_t s);
+hipError_t pa_launch_gemm_wide(const GemmParams& p, uint16_t* w16, bool widen, const GlueParams* heads, int n_cu, hipStream_t s);
+// a chunk's [q | k | v] projection that ends with the pre-step and the cache write instead of storing p.y: whether a call takes that form
+bool pa_gemm_heads_serves(const GemmParams& p, const GlueParams& heads, int n_cu);
+float pa_gemm_heads_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t head_dim, uint32_t kg, int n_cu, uint32_t* shape);
+hipError_t pa_launch_gemm_heads(const GemmParams& p, const uint16_t* w16, const GlueParams& heads, uint32_t kg, int n_cu, hipStream_t s);
 // its kernel for larger tiles (proj_gemm_tile.hip), and what a call would take there, on which tile (columns << 16 | rows)
-float pa_gemm_tile_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, uint32_t* shape);
+float pa_gemm_tile_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, uint32_t* shape, uint32_t* kg);
 // the rules that pick an instance by size, in plain C: the tests ask them which instances their sizes take
 extern "C" uint32_t pa_rule_gemv_wide_rows(int kind, uint32_t d_out, uint32_t d_in, int norm, int n_cu);
 extern "C" int pa_rule_gemm_few_groups(int kind, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu);
 extern "C" int pa_rule_gemm_few_dot(int kind, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu);
+extern "C" uint32_t pa_rule_gemm_heads(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t n_heads, uint32_t head_dim, int gated, int n_cu);
 extern "C" uint32_t pa_rule_gemm_wide_tile(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t x_stride, int n_cu);
 hipError_t pa_launch_gemm_tile(const GemmParams& p, const uint16_t* w16, int n_cu, hipStream_t s);
 // rmsnorm of n_cols f32 columns, written as f16 (the GEMM's activation operand)

@@ -22,14 +22,182 @@
 // 16.8 -> 15.0; 4096 of 9216 x 2048 161 -> 154, of 14336 x 5120 609 -> 568.  Not kept: a ninth wave that prefetches the weight stream into L2 (slower on every shape), activation
 // rows at a padded stride (no change).
 #include "pf_common.h"
+#include "glue_math.h"
+#include <algorithm>
 
 struct GemmTileParams {
   const uint16_t* x; const uint16_t* w16; float* y;
   uint32_t x_stride, y_stride, d_out, d_in, n_cols;
 };
 
-template <int WM, int WN, int KG, int TM, int TN, int S, bool ACC>
-__global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p) {
+// ---- the pre-step as the end of the [q | k | v] projection: whole heads in a workgroup's rows ----
+// What the tile holds leaves as the pre-step would leave it (glue_kv.hip; the same arithmetic on the same f32 values, a head's sum of squares
+// in f64 in another order), and the f32 projections themselves are never stored: a launch less, and for 4096 columns of the gated 16 / 2-head
+// shape 150 MB less written and as much less read.  It is LDS, VALU and store work behind a tile's products, with nothing to hide under, so it is dealt
+// by what it is: columns on lanes for the sums of squares, rotation pairs on lanes for the rotation (both elements of a pair in one lane),
+// the other dims a column at a time, everything read before the first store.  Layer pass, apart / so (us a layer): 4096 columns
+// of that shape 499 / 459, 2048 282 / 243, 300 71 / 66; 777 of the 24 / 4-head shape 292 / 280; 512 and 1024 of the 16 / 8-head shape 53 / 48 and 82 / 73.
+enum { GT_STORE = 0, GT_ACC = 1, GT_HEADS = 2 };
+
+// what a block of head_dim weight rows is: [q | gate] or q heads, then k, then v heads
+enum { HB_Q = 0, HB_GATE = 1, HB_K = 2, HB_V = 3 };
+static __device__ inline uint32_t head_block(const GlueParams& g, uint32_t b, uint32_t& h) {
+  const uint32_t gated = g.flags & PA_FLAG_GATE ? 1 : 0, nq = g.n_heads << gated;
+  if (b < nq) { h = b >> gated; return gated && (b & 1) ? HB_GATE : HB_Q; }
+  h = b - nq;
+  if (h < g.n_kv_heads) return HB_K;
+  h -= g.n_kv_heads;
+  return HB_V;
+}
+
+// four consecutive values of a finished k or v row (dims d0 ..; 8 lanes = 32 dims) to an f16 or int8 cache; every lane of the wave calls
+static __device__ inline void cache_store4(const GlueParams& g, bool v, uint32_t h, uint32_t pos, uint32_t d0, const float (&x)[4], bool on) {
+  const size_t row = (size_t)h * g.head_rows + pos;
+  uint16_t* cache = v ? g.v_cache : g.k_cache;
+  if (g.ks_cache) {
+    uint32_t w; float sc;
+    quant4_q8(x, w, sc);
+    if (on) {
+      *(uint32_t*)((unsigned char*)cache + row * g.head_dim + d0) = w;
+      if (d0 % 32 == 0) (v ? g.vs_cache : g.ks_cache)[row * (g.head_dim / 32) + d0 / 32] = sc;
+    }
+  } else if (on) {
+    *(h4*)((_Float16*)cache + row * g.head_dim + d0) = (h4){ (_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3] };
+  }
+}
+
+// LDS of it: CP columns x BN rows ([CP][BN + 4] f32), the slices' sums of squares, the heads' factors, the norm weights, then the (cos, sin)
+// rows of the tile's BM columns where they fit.  Nothing is loaded from memory between the stores: loads and stores share one counter, and a
+// wait for a loaded value with stores pending waits for those as well.
+#define GT_LDS (160 * 1024)
+template <int CP, int BN> struct HeadsLds {
+  static constexpr int LR = BN + 4;
+  static constexpr int part = CP * LR * 4, inv = part + 512 * 8, nw = inv + (BN / 128) * CP * 4, cs = nw + 2 * 256 * 4;
+};
+static __device__ __host__ inline bool cs_in_lds(uint32_t fixed, uint32_t bm, uint32_t half) { return fixed + bm * half * 8 <= GT_LDS; }
+
+static __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// requests the norm weights and the (cos, sin) rows of columns c0 .. c0 + BM; they are there behind the caller's wait and barrier
+template <int CP, int BN, int BM>
+static __device__ inline void heads_request(const GlueParams& g, unsigned char* lds, uint32_t c0) {
+  typedef HeadsLds<CP, BN> H;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = g.n_rot / 2;
+  if (g.flags & PA_FLAG_QK_NORM) ((float*)(lds + H::nw))[tid] = (tid < 256 ? g.qw : g.kw)[min(tid & 255, g.head_dim - 1)];
+  if (cs_in_lds(H::cs, BM, half)) {
+    const unsigned char* src = (const unsigned char*)(g.rope_tab + (size_t)(g.base_pos + c0) * half);
+    const uint32_t last = (g.n_cols - c0) * half * 8 - 16;
+    for (uint32_t q = wave; q * 1024 < BM * half * 8; q += 8) PF_GLL_S(src, min(q * 1024 + lane * 16, last), lds + H::cs + q * 1024);
+  }
+}
+
+// global column of local column c: col_of(c); rows r0 ..  All 512 threads call, behind a barrier.
+template <int HD, int CP, int BN, int BM, class ColOf>
+static __device__ inline void finish_heads(const GlueParams& g, unsigned char* lds, uint32_t c0, uint32_t r0, uint32_t d_out, ColOf col_of) {
+#pragma clang fp contract(off)
+  typedef HeadsLds<CP, BN> H;
+  constexpr int LR = H::LR, NS = 512 / CP, RS = BN / NS;               // slices a column, rows a slice
+  constexpr int NHB = BN / HD, CPW = CP / 8;                           // heads of the tile, columns of a wave (consecutive ones)
+  static_assert(RS % 16 == 0 && RS <= 128, "a slice is inside a head");
+  const float* hx = (const float*)lds;
+  double* part = (double*)(lds + H::part);                             // [NS][CP]
+  float* inv = (float*)(lds + H::inv);                                 // [NHB][CP], a wave's columns its own
+  uint32_t tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));                                        // (no lane's addresses are kept from phase to phase beside the accumulators)
+  const uint32_t lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = g.n_rot / 2, lw = wave * CPW;
+  const bool norm = (g.flags & PA_FLAG_QK_NORM) != 0, cs_lds = cs_in_lds(H::cs, BM, half);
+  if (norm) {
+    const uint32_t c = tid % CP, sl = tid / CP;
+    uint32_t h;
+    const uint32_t kind = head_block(g, (r0 + sl * RS) / HD, h);
+    if (kind == HB_Q || kind == HB_K) {
+      double ss[4] = { 0.0, 0.0, 0.0, 0.0 };
+#pragma unroll
+      for (int k = 0; k < RS; k += 4) {
+        const f4 v = *(const f4*)(hx + c * LR + sl * RS + k);
+#pragma unroll
+        for (int i = 0; i < 4; i++) ss[i] = __builtin_fma((double)v[i], (double)v[i], ss[i]);
+      }
+      part[sl * CP + c] = (ss[0] + ss[1]) + (ss[2] + ss[3]);
+    }
+    lds_barrier();
+    if (lane < NHB * CPW) {
+      const uint32_t cc = lw + lane % CPW, hb = lane / CPW;
+      double t[NS / NHB];
+#pragma unroll
+      for (int k = 0; k < NS / NHB; k++) t[k] = part[(hb * (NS / NHB) + k) * CP + cc];
+      double s = t[0];
+#pragma unroll
+      for (int k = 1; k < NS / NHB; k++) s += t[k];
+      inv[hb * CP + cc] = rms_inv(s, HD, g.eps);
+    }
+    wave_lds_fence();
+  }
+  const uint32_t qd = g.n_heads * HD;
+  constexpr uint32_t Q4 = HD / 4, CPI = 64 / Q4, NI = CPW / CPI;       // quads of a head, columns an instruction, instructions
+  const uint32_t cl = lane / Q4, d = 4 * (lane % Q4);
+  for (int hb = 0; hb < NHB; hb++) {
+    uint32_t h;
+    const uint32_t row = r0 + hb * HD;
+    if (row < d_out) {
+    const uint32_t kind = head_block(g, row / HD, h);
+    const float* hx0 = hx + hb * HD;
+    const bool plain = kind == HB_GATE || kind == HB_V;
+    const float* wp = (const float*)(lds + H::nw) + (kind == HB_Q ? 0 : 256);
+    auto store4 = [&](uint32_t col, uint32_t dd, const float (&x)[4], bool on) __attribute__((always_inline)) {
+      if (kind == HB_Q || kind == HB_GATE) { if (on) *(f4*)((kind == HB_Q ? g.q_out : g.gate_out) + (size_t)col * qd + h * HD + dd) = (f4){ x[0], x[1], x[2], x[3] }; }
+      else cache_store4(g, kind == HB_V, h, g.base_pos + col, dd, x, on);
+    };
+    if (!plain) {
+      // rotated dims: a lane holds elements da .. da + 3 and their partners
+      const uint32_t U = half / 4, lgU = 31 - __builtin_clz(U), u = lane & (U - 1), da = 4 * u, db = da + half;
+      f4 wa = { 1.f, 1.f, 1.f, 1.f }, wb = wa;
+      if (norm) { wa = *(const f4*)(wp + da); wb = *(const f4*)(wp + db); }
+      for (uint32_t e = lane; e < (CPW << lgU); e += 64) {
+        const uint32_t c = lw + (e >> lgU), col = col_of(c);
+        const bool on = col < g.n_cols;
+        f4 t0, t1;
+        if (cs_lds) { const f4* t = (const f4*)(lds + H::cs + ((col - c0) * half + da) * 8); t0 = t[0]; t1 = t[1]; }
+        else { const f4* t = (const f4*)(g.rope_tab + (size_t)(g.base_pos + (on ? col : c0)) * half + da); t0 = t[0]; t1 = t[1]; }
+        const float cs[4] = { t0[0], t0[2], t1[0], t1[2] }, sn[4] = { t0[1], t0[3], t1[1], t1[3] };
+        const f4 va = *(const f4*)(hx0 + c * LR + da), vb = *(const f4*)(hx0 + c * LR + db);
+        const float iv = norm ? inv[hb * CP + c] : 1.f;
+        float oa[4], ob[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          float a = va[i], b = vb[i];
+          if (norm) { const float sa = iv * wa[i], sb = iv * wb[i]; a = a * sa; b = b * sb; }
+          const float ac = a * cs[i], bs = b * sn[i], bc = b * cs[i], as = a * sn[i];    // rounded one by one
+          oa[i] = ac - bs; ob[i] = bc + as;
+        }
+        store4(col, da, oa, on);
+        store4(col, db, ob, on);
+      }
+    }
+    // the rest (gate and v heads: all), a column or two an instruction; everything read before the first store
+    if (plain || 2 * half < HD) {
+      const bool scale = norm && !plain;
+      f4 w = { 1.f, 1.f, 1.f, 1.f }, v[NI];
+      float iv[NI];
+      if (scale) w = *(const f4*)(wp + d);
+#pragma unroll
+      for (uint32_t k = 0; k < NI; k++) { v[k] = *(const f4*)(hx0 + (lw + k * CPI + cl) * LR + d); iv[k] = scale ? inv[hb * CP + lw + k * CPI + cl] : 1.f; }
+#pragma unroll
+      for (uint32_t k = 0; k < NI; k++) {
+        const uint32_t col = col_of(lw + k * CPI + cl);
+        float x[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) { x[i] = v[k][i]; if (scale) { const float sw = iv[k] * w[i]; x[i] = x[i] * sw; } }
+        store4(col, d, x, col < g.n_cols && (plain || d >= 2 * half));
+      }
+    }
+    }
+  }
+}
+
+template <int WM, int WN, int KG, int TM, int TN, int S, int EPI>
+__global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p, GlueParams gp) {
+  constexpr bool ACC = EPI == GT_ACC;
   static_assert(WM * WN * KG == 8, "eight waves");
   constexpr int KS = 2;                                  // k-steps of a stage per wave
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BK = 16 * KG * KS;
@@ -142,7 +310,36 @@ __global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p) 
   // accumulator i of a tile: column 8 (i / 4) + 4 fk + i % 4, row fl.  Accumulating calls: loads and stores share one counter,
   // and a wait for a loaded value with stores pending waits for those as well, so the old values are fetched several
   // tiles at a time, unconditionally (clamped addresses: a guarded load is a branch, one load a basic block), then added.
-  if constexpr (KG == 1) {
+  if constexpr (EPI == GT_HEADS && KG == 1) {
+    float* hx = (float*)gt_lds;
+    constexpr int LR = BN + 4;
+    lds_barrier();
+    heads_request<WM * 32, BN, BM>(gp, gt_lds, c0);
+    auto dump = [&](auto A) __attribute__((always_inline)) {
+#pragma unroll
+      for (int b = 0; b < TN; b++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) hx[(wm * 32 + 8 * (i / 4) + 4 * fk + (i % 4)) * LR + (wn * TN + b) * 32 + fl] = acc[decltype(A)::value][b][i];
+      asm volatile("; block %0" :: "n"(decltype(A)::value) : "memory");   // (the blocks' stores are not merged into one on selected registers)
+    };
+#pragma nounroll
+    for (int a = 0; a < TM; a++) {                                       // a phase: block a of every wave's columns
+      static_assert(TM <= 7, "blocks of a wave");
+      if (a == 0) dump(std::integral_constant<int, 0>{});
+      if constexpr (TM > 1) if (a == 1) dump(std::integral_constant<int, 1>{});
+      if constexpr (TM > 2) if (a == 2) dump(std::integral_constant<int, 2>{});
+      if constexpr (TM > 3) if (a == 3) dump(std::integral_constant<int, 3>{});
+      if constexpr (TM > 4) if (a == 4) dump(std::integral_constant<int, 4>{});
+      if constexpr (TM > 5) if (a == 5) dump(std::integral_constant<int, 5>{});
+      if constexpr (TM > 6) if (a == 6) dump(std::integral_constant<int, 6>{});
+      if (a == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // what heads_request asked for
+      lds_barrier();
+      const auto col = [&](uint32_t c) { return c0 + (c / 32 * TM + a) * 32 + c % 32; };
+      if (gp.head_dim == 256) finish_heads<256, WM * 32, BN, BM>(gp, gt_lds, c0, r0, p.d_out, col);
+      else finish_heads<128, WM * 32, BN, BM>(gp, gt_lds, c0, r0, p.d_out, col);
+      lds_barrier();
+    }
+  } else if constexpr (KG == 1) {
     constexpr int D = TN <= 5 ? TN : 4;                                  // tiles of a phase: what fits next to the accumulators
 #pragma unroll
     for (int m0 = 0; m0 < NM; m0 += D) {
@@ -182,6 +379,26 @@ __global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p) 
       for (int k = 0; k < SPW; k++) old[k] = p.y[(size_t)min(col_s(k), p.n_cols - 1) * p.y_stride + min(row_s(k), p.d_out - 1)];
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if constexpr (EPI == GT_HEADS) {
+      float sum[SPW];
+#pragma unroll
+      for (int k = 0; k < SPW; k++) {
+        sum[k] = 0.f;
+#pragma unroll
+        for (int g = 0; g < KG; g++) sum[k] += red[((g * (WM * WN) + wt) * NT * 16 + kgrp * SPW + k) * 64 + lane];
+      }
+      lds_barrier();
+      heads_request<BM, BN, BM>(gp, gt_lds, c0);
+      float* hx = (float*)gt_lds;
+#pragma unroll
+      for (int k = 0; k < SPW; k++) hx[(col_s(k) - c0) * (BN + 4) + row_s(k) - r0] = sum[k];
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();
+      const auto col = [&](uint32_t c) { return c0 + c; };
+      if constexpr (BN % 256 == 0) { if (gp.head_dim == 256) finish_heads<256, BM, BN, BM>(gp, gt_lds, c0, r0, p.d_out, col); }
+      if (gp.head_dim == 128) finish_heads<128, BM, BN, BM>(gp, gt_lds, c0, r0, p.d_out, col);
+      return;
+    }
 #pragma unroll
     for (int k = 0; k < SPW; k++) {
       float s = 0.f;
@@ -192,33 +409,52 @@ __global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p) 
   }
 }
 
-template <int WM, int WN, int KG, int TM, int TN, int S>
-static hipError_t gt_launch(const GemmTileParams& q, int acc, hipStream_t s) {
+template <int WM, int WN, int KG, int TM, int TN, int S, bool HEADS>
+static hipError_t gt_launch(const GemmTileParams& q, int acc, const GlueParams* heads, hipStream_t s) {
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BK = 32 * KG;
-  constexpr int lds_st = S * (BM + BN) * BK * 2, lds_red = KG > 1 ? KG * BM * BN * 4 : 0, lds = lds_st > lds_red ? lds_st : lds_red;
-  static_assert(lds <= 160 * 1024, "LDS");
+  constexpr int lds_st = S * (BM + BN) * BK * 2, lds_red = KG > 1 ? KG * BM * BN * 4 : 0, lds_fixed = lds_st > lds_red ? lds_st : lds_red;
+  typedef HeadsLds<(KG > 1 ? BM : WM * 32), BN> H;
+  static_assert(lds_fixed <= GT_LDS && (!HEADS || H::cs <= GT_LDS), "LDS");
+  int lds = lds_fixed;
+  if (HEADS) lds = std::max(lds, H::cs + (cs_in_lds(H::cs, BM, heads->n_rot / 2) ? BM * (int)heads->n_rot * 4 : 0));
   const uint32_t total = ((q.n_cols + BM - 1) / BM) * ((q.d_out + BN - 1) / BN);
   static PaPerDevice lds_set[2];
-  const auto kernel = acc ? pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, true> : pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, false>;
-  const hipError_t e = pa_lds_limit(lds_set[acc ? 1 : 0], (const void*)kernel, lds);
+  GlueParams none{};
+  const auto kernel = HEADS ? pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, HEADS ? GT_HEADS : GT_STORE>
+                            : acc ? pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, HEADS ? GT_HEADS : GT_ACC> : pa_gemm_tile_kernel<WM, WN, KG, TM, TN, S, HEADS ? GT_HEADS : GT_STORE>;
+  const hipError_t e = pa_lds_limit(lds_set[acc ? 1 : 0], (const void*)kernel, HEADS ? GT_LDS : lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, dim3((total + 7) / 8 * 8), dim3(512), lds, s, q);
+  hipLaunchKernelGGL(kernel, dim3((total + 7) / 8 * 8), dim3(512), lds, s, q, heads ? *heads : none);
   return hipGetLastError();
 }
 
 // The tile shapes, with what a round of the chip costs: ns per k of d_in (measured on rounds of 200 - 256 workgroups) on top
 // of about 6 us for a round's first loads and last stores.
-struct TileShape { uint16_t bm, bn; float ns_k; hipError_t (*launch)(const GemmTileParams&, int, hipStream_t); };
+struct TileShape { uint16_t bm, bn, kg; float us, ns_k; hipError_t (*launch)(const GemmTileParams&, int, const GlueParams*, hipStream_t); };
 static const TileShape tile_shapes[] = {
-  { 64, 128, 6.5f, gt_launch<1, 2, 4, 2, 2, 3> },
-  { 128, 128, 10.3f, gt_launch<2, 2, 2, 2, 2, 4> },
-  { 128, 160, 11.8f, gt_launch<4, 1, 2, 1, 5, 4> },
-  { 128, 192, 14.0f, gt_launch<4, 2, 1, 1, 3, 6> },
-  { 128, 256, 15.5f, gt_launch<2, 4, 1, 2, 2, 6> },
-  { 128, 320, 19.0f, gt_launch<4, 2, 1, 1, 5, 5> },
-  { 128, 384, 21.5f, gt_launch<2, 4, 1, 2, 3, 4> },
-  { 128, 448, 25.0f, gt_launch<4, 2, 1, 1, 7, 4> },
-  { 256, 256, 27.0f, gt_launch<2, 4, 1, 4, 2, 4> },
+  { 64, 128, 4, 6.f, 6.5f, gt_launch<1, 2, 4, 2, 2, 3, false> },
+  { 128, 128, 2, 6.f, 10.3f, gt_launch<2, 2, 2, 2, 2, 4, false> },
+  { 128, 160, 2, 6.f, 11.8f, gt_launch<4, 1, 2, 1, 5, 4, false> },
+  { 128, 192, 1, 6.f, 14.0f, gt_launch<4, 2, 1, 1, 3, 6, false> },
+  { 128, 256, 1, 6.f, 15.5f, gt_launch<2, 4, 1, 2, 2, 6, false> },
+  { 128, 320, 1, 6.f, 19.0f, gt_launch<4, 2, 1, 1, 5, 5, false> },
+  { 128, 384, 1, 6.f, 21.5f, gt_launch<2, 4, 1, 2, 3, 4, false> },
+  { 128, 448, 1, 6.f, 25.0f, gt_launch<4, 2, 1, 1, 7, 4, false> },
+  { 256, 256, 1, 6.f, 27.0f, gt_launch<2, 4, 1, 4, 2, 4, false> },
+};
+// ... and those that hold whole heads (128 rows: of head_dim 128) and can end with the pre-step, whose work is part of a round's start here.
+// Fitted to 75 sizes (the three model shapes, 33 to 4096 columns): of the shapes with the call's kg, the one taken is the fastest or within 0.6 % of it.
+static const TileShape head_shapes[] = {
+  { 64, 128, 4, 3.5f, 7.1f, gt_launch<1, 2, 4, 2, 2, 3, true> },
+  { 128, 128, 2, 4.3f, 8.9f, gt_launch<2, 2, 2, 2, 2, 4, true> },
+  { 64, 256, 2, 5.6f, 11.8f, gt_launch<1, 4, 2, 2, 2, 3, true> },
+  { 96, 256, 1, 5.f, 12.8f, gt_launch<1, 8, 1, 3, 1, 6, true> },
+  { 128, 256, 1, 3.7f, 14.5f, gt_launch<2, 4, 1, 2, 2, 6, true> },
+  { 160, 256, 1, 9.2f, 15.9f, gt_launch<1, 8, 1, 5, 1, 5, true> },
+  { 192, 256, 1, 10.3f, 16.1f, gt_launch<2, 4, 1, 3, 2, 5, true> },
+  { 224, 256, 1, 17.2f, 17.4f, gt_launch<1, 8, 1, 7, 1, 4, true> },
+  { 256, 256, 1, 16.5f, 17.8f, gt_launch<2, 4, 1, 4, 2, 4, true> },
+  { 320, 256, 1, 24.2f, 20.7f, gt_launch<2, 4, 1, 5, 2, 4, true> },
 };
 
 // One workgroup is resident per CU, so a call costs whole rounds of n_cu workgroups: the shape with the cheapest rounds, and
@@ -227,22 +463,24 @@ static const TileShape tile_shapes[] = {
 // 104 sizes measured on every tile and on the 64 x 64 kernel (8 weight shapes x 13 column counts, cold weights) the choice between
 // all of them is the fastest at 84 and within 6 % at 8; it is 9 - 33 % behind at 12, most where one round of few workgroups (which
 // costs less than a full one) is set against the 64 x 64 kernel: 9216 x 2048, 200 columns 27.9 us, on 128 x 128 21.1.
+static float rounds_us(const TileShape& t, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu) {
+  const uint64_t wgs = (uint64_t)((n_cols + t.bm - 1) / t.bm) * ((d_out + t.bn - 1) / t.bn), cus = n_cu > 0 ? n_cu : 256;
+  return (float)((wgs + cus - 1) / cus) * (t.us + t.ns_k * 1e-3f * d_in);
+}
 static int pa_pick_tile(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, float* us) {
   int best = 0;
   *us = 1e30f;
   for (int i = 0; i < (int)(sizeof tile_shapes / sizeof tile_shapes[0]); i++) {
-    const TileShape& t = tile_shapes[i];
-    const uint64_t wgs = (uint64_t)((n_cols + t.bm - 1) / t.bm) * ((d_out + t.bn - 1) / t.bn), cus = n_cu > 0 ? n_cu : 256;
-    const float c = (float)((wgs + cus - 1) / cus) * (6.f + t.ns_k * 1e-3f * d_in);
+    const float c = rounds_us(tile_shapes[i], d_out, d_in, n_cols, n_cu);
     if (c < *us) { *us = c; best = i; }
   }
   return best;
 }
 
-float pa_gemm_tile_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, uint32_t* shape) {
+float pa_gemm_tile_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, uint32_t* shape, uint32_t* kg) {
   float us;
   const TileShape& t = tile_shapes[pa_pick_tile(d_out, d_in, n_cols, n_cu, &us)];
-  *shape = (uint32_t)t.bm << 16 | t.bn;
+  *shape = (uint32_t)t.bm << 16 | t.bn; *kg = t.kg;
   return us;
 }
 
@@ -251,5 +489,34 @@ hipError_t pa_launch_gemm_tile(const GemmParams& p, const uint16_t* w16, int n_c
   GemmTileParams q;
   q.x = p.x; q.w16 = w16; q.y = p.y; q.x_stride = p.x_stride; q.y_stride = p.y_stride; q.d_out = p.d_out; q.d_in = p.d_in; q.n_cols = p.n_cols;
   float us;
-  return tile_shapes[pa_pick_tile(p.d_out, p.d_in, p.n_cols, n_cu, &us)].launch(q, p.acc, s);
+  return tile_shapes[pa_pick_tile(p.d_out, p.d_in, p.n_cols, n_cu, &us)].launch(q, p.acc, nullptr, s);
+}
+
+// kg: the groups of waves that a stage's k-steps are split over, which fixes the order of an element's sum
+static int pick_heads(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t head_dim, uint32_t kg, int n_cu, float* us) {
+  int best = -1;
+  *us = 1e30f;
+  for (int i = 0; i < (int)(sizeof head_shapes / sizeof head_shapes[0]); i++) {
+    if (head_shapes[i].bn % head_dim || head_shapes[i].kg != kg) continue;
+    const float c = rounds_us(head_shapes[i], d_out, d_in, n_cols, n_cu);
+    if (c < *us) { *us = c; best = i; }
+  }
+  return best;
+}
+
+float pa_gemm_heads_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t head_dim, uint32_t kg, int n_cu, uint32_t* shape) {
+  float us;
+  const int i = pick_heads(d_out, d_in, n_cols, head_dim, kg, n_cu, &us);
+  *shape = i < 0 ? 0 : (uint32_t)head_shapes[i].bm << 16 | head_shapes[i].bn;
+  return us;
+}
+
+hipError_t pa_launch_gemm_heads(const GemmParams& p, const uint16_t* w16, const GlueParams& heads, uint32_t kg, int n_cu, hipStream_t s) {
+  const uint32_t half = heads.n_rot / 2;
+  if (p.d_out == 0 || p.d_in == 0 || p.d_in % 128 != 0 || p.n_cols == 0 || p.x_stride > (1u << 22) || p.d_out % heads.head_dim || half < (heads.ks_cache ? 32u : 4u) || (half & (half - 1)) || !heads.rope_tab) return hipErrorInvalidValue;
+  GemmTileParams q;
+  q.x = p.x; q.w16 = w16; q.y = nullptr; q.x_stride = p.x_stride; q.y_stride = 0; q.d_out = p.d_out; q.d_in = p.d_in; q.n_cols = p.n_cols;
+  float us;
+  const int i = pick_heads(p.d_out, p.d_in, p.n_cols, heads.head_dim, kg, n_cu, &us);
+  return i < 0 ? hipErrorNotSupported : head_shapes[i].launch(q, 0, &heads, s);
 }

@@ -262,18 +262,42 @@ size_t pa_gemm_wide_staging_bytes(uint32_t d_out, uint32_t d_in) { return (size_
 // kernel takes the stride.
 // Fewer 64 x 64 tiles than half the CUs: 32-row tiles (twice the workgroups) with twice the stages in flight (2048 x 4096 on up to
 // 64 columns, cold: 20 -> 16.7 us; with 144 tiles, 9216 x 2048, it is 2 us slower).
+static float mid_tile_us(uint32_t d_in, uint64_t tiles64, uint32_t cus) { return 4.f + 4.6e-3f * d_in * std::max(1.f, (float)tiles64 / cus); }
 // Columns << 16 | rows of the tile a call takes; 64-column tiles of up to 64 rows are this file's kernel.
 extern "C" uint32_t pa_rule_gemm_wide_tile(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t x_stride, int n_cu) {
   const uint32_t cus = n_cu > 0 ? (uint32_t)n_cu : 256u;
   const uint64_t tiles64 = (uint64_t)((n_cols + GM_T - 1) / GM_T) * ((d_out + 63) / 64);
-  const float mid_us = 4.f + 4.6e-3f * d_in * std::max(1.f, (float)tiles64 / cus);
-  uint32_t shape;
-  if (x_stride <= (1u << 22) && pa_gemm_tile_us(d_out, d_in, n_cols, n_cu, &shape) < mid_us) return shape;
+  const float mid_us = mid_tile_us(d_in, tiles64, cus);
+  uint32_t shape, kg;
+  if (x_stride <= (1u << 22) && pa_gemm_tile_us(d_out, d_in, n_cols, n_cu, &shape, &kg) < mid_us) return shape;
   return (uint32_t)GM_T << 16 | (tiles64 * 2 < cus ? 32u : 64u);
 }
 
+// How a chunk's [q | k | v] projection that ends with the pre-step runs (proj_gemm_tile.hip): k groups << 28 | columns << 16 | rows of its tile, or 0
+// where the two apart are the faster form -- the tiles that hold whole heads are few, and below some 200 - 300 columns (64-column tiles of too
+// few workgroups) they cost more than the pre-step's launch, 3.5 us and the f32 projections through memory at 6 TB/s (16 columns 3.9 us, 512 of
+// the 16 / 8-head shape 6.5, 777 of the 24 / 4-head shape 19.6, 4096 of the 16 / 2-head shape 53.5).  Only tiles that split K as the call apart does:
+// the results are its bits.  On 75 sizes the choice is 4 % ahead of always apart (best 14 %), at no size more than 1 % behind.
+extern "C" uint32_t pa_rule_gemm_heads(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t n_heads, uint32_t head_dim, int gated, int n_cu) {
+  const uint32_t cus = n_cu > 0 ? (uint32_t)n_cu : 256u;
+  uint32_t shape, kg, whole;
+  const uint64_t tiles64 = (uint64_t)((n_cols + GM_T - 1) / GM_T) * ((d_out + 63) / 64);
+  float apart = pa_gemm_tile_us(d_out, d_in, n_cols, n_cu, &shape, &kg);
+  const float mid = mid_tile_us(d_in, tiles64, cus);
+  if (mid <= apart) { apart = mid; kg = 4; }                            // (the 64-column kernel's four waves: k-steps w and w + 4 of eight)
+  apart += 3.5f + 0.166e-6f * 4.f * n_cols * ((float)d_out + n_heads * head_dim * (gated ? 2.f : 1.f));
+  return pa_gemm_heads_us(d_out, d_in, n_cols, head_dim, kg, n_cu, &whole) < apart ? kg << 28 | whole : 0;
+}
+// ... whose arithmetic takes rotation tables of a power of two of pairs, on int8 caches whole blocks of them
+bool pa_gemm_heads_serves(const GemmParams& p, const GlueParams& g, int n_cu) {
+  const uint32_t half = g.n_rot / 2;
+  if (!pa_gemm_wide_serves(p) || pa_gemm_skinny_serves(p) || p.x_stride > (1u << 22) || !g.rope_tab) return false;
+  if ((half & (half - 1)) || half < (g.ks_cache ? 32u : 4u)) return false;
+  return pa_rule_gemm_heads(p.d_out, p.d_in, p.n_cols, g.n_heads, g.head_dim, (g.flags & PA_FLAG_GATE) != 0, n_cu) != 0;
+}
+
 // w16: staging of pa_gemm_wide_staging_bytes (the caller's, 16-byte aligned); widen = false: it already holds these weights
-hipError_t pa_launch_gemm_wide(const GemmParams& p, uint16_t* w16, bool widen, int n_cu, hipStream_t s) {
+hipError_t pa_launch_gemm_wide(const GemmParams& p, uint16_t* w16, bool widen, const GlueParams* heads, int n_cu, hipStream_t s) {
   if (widen) {
     const uint32_t nb = p.d_in / 32;
     const size_t n_threads = (size_t)((p.d_out + 31) / 32) * 32 * nb;
@@ -287,6 +311,7 @@ hipError_t pa_launch_gemm_wide(const GemmParams& p, uint16_t* w16, bool widen, i
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
+  if (heads) return pa_launch_gemm_heads(p, w16, *heads, pa_rule_gemm_heads(p.d_out, p.d_in, p.n_cols, heads->n_heads, heads->head_dim, (heads->flags & PA_FLAG_GATE) != 0, n_cu) >> 28, n_cu, s);
   const uint32_t tile = pa_rule_gemm_wide_tile(p.d_out, p.d_in, p.n_cols, p.x_stride, n_cu);
   if (tile >> 16 != GM_T || (tile & 0xffff) > 64) return pa_launch_gemm_tile(p, w16, n_cu, s);
   Gemm16Params q;

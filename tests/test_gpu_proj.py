@@ -459,3 +459,56 @@ def test_layer_calls_on_int8_caches_equal_their_stages():
             assert np.all(np.isfinite(a))
         for w in range(4):
             assert np.array_equal(pa.kv_read(0, w, 0, base + n + 1), pa.kv_read(1, w, 0, base + n + 1))
+
+
+# (n_heads, n_kv_heads, head_dim, gate), model width, columns, tile: every tile that ends with the pre-step, ragged in columns
+HEADS_SIZES = [((24, 4, 256, True), 1024, 292, (1, 96, 256)), ((32, 8, 128, True), 128, 662, (1, 128, 256)), ((32, 2, 256, True), 256, 403, (1, 160, 256)),
+               ((32, 2, 256, True), 256, 514, (1, 192, 256)), ((32, 2, 256, True), 2048, 588, (1, 224, 256)), ((32, 2, 256, True), 1024, 588, (1, 256, 256)),
+               ((32, 8, 128, True), 1024, 1550, (1, 320, 256)), ((16, 2, 256, True), 2048, 300, (2, 64, 256)), ((16, 8, 128, False), 256, 995, (2, 128, 128)),
+               ((16, 8, 128, False), 128, 33, (4, 64, 128)), ((17, 17, 128, False), 128, 40, (4, 64, 128)), ((21, 7, 128, False), 128, 1550, (1, 128, 256))]
+
+
+@pytest.mark.parametrize("more", [{}, dict(kv_q8=True), dict(qk_norm=False, n_rot=8), dict(n_rot=-1), dict(n_rot=-1, kv_q8=True, qk_norm=False)])
+@pytest.mark.parametrize("heads,dim,n,tile", HEADS_SIZES)
+def test_projection_that_ends_with_the_pre_step_equals_the_two(heads, dim, n, tile, more):
+    """What the layer call's [q | k | v] projection leaves in the q and gate buffers and in the caches is, bit for bit, what pa_gemm and
+    pa_glue_kv leave: the same sums in the same order, the same arithmetic behind them.  n_rot: a quarter of the head, the least that is
+    served, and the whole head (whose rotation tables are past the LDS of the wider tiles); rows around the chunk stay as they were."""
+    nH, nKV, hd, gate = heads
+    cfg = dict(n_heads=nH, n_kv_heads=nKV, head_dim=hd, n_rot=hd // 4 if hd == 256 else 64, rope_theta=1e6, eps=1e-6, qk_norm=True, gate=gate)
+    cfg.update(more)
+    if cfg["n_rot"] < 0:
+        cfg["n_rot"] = hd
+    qd, kvd = nH * hd, nKV * hd
+    q_rows = qd * (2 if gate else 1)
+    rows, base = q_rows + 2 * kvd, 7
+    rng = np.random.default_rng(n)
+    w_qkv, s_qkv = _weights(PA_W_Q4_0, rows, dim, rng, scale=0.05)
+    w_o, s_o = _weights(PA_W_Q4_0, dim, qd, rng, scale=0.005)
+    nw = (1 + 0.1 * rng.standard_normal(dim)).astype(np.float32)
+    hw = (1 + 0.1 * rng.standard_normal(hd)).astype(np.float32); hk = (1 + 0.1 * rng.standard_normal(hd)).astype(np.float32)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    pre, caches = [], []
+    with PooledAttn(cfg, base + n + 2, n_layers=2, max_cols=n) as pa:
+        wq = pa.weight(PA_W_Q4_0, w_qkv, s_qkv); wo = pa.weight(PA_W_Q4_0, w_o, s_o)
+        dnw = pa.to_device(nw); dqw = pa.to_device(hw); dkw = pa.to_device(hk)
+        stale = np.full(n * qd, np.nan, np.float32)
+        for layer in (0, 1):
+            pa.layer_alloc(layer)
+            dx = pa.to_device(x)
+            for buf in (pa.q_buffer_ptr(), pa.gate_buffer_ptr()):
+                pa.L.pa_upload(pa.ctx, buf, stale.ctypes.data, stale.nbytes)
+            if layer == 0:
+                pa.attn_layer_prefill(layer, wq, wo, dnw, dqw, dkw, dx, dim, base, n)
+            else:
+                dxn = pa.alloc(n * dim * 2); dqkv = pa.alloc(n * rows * 4)
+                pa.rmsnorm_f16(dx, dim, dnw, dim, n, dxn, dim)
+                pa.gemm(wq, dxn, dim, n, dqkv, rows)
+                pa.L.pa_glue_kv(pa.ctx, layer, dqkv.ptr, rows, dqkv.ptr + q_rows * 4, rows, dqkv.ptr + (q_rows + kvd) * 4, rows, dqw.ptr, dkw.ptr, base, n)
+            pa.sync()
+            pre.append((pa.read_q_buffer(n), pa.read_gate_buffer(n) if gate else np.zeros(0)))
+            caches.append([pa.kv_read(layer, w, 0, base + n + 2) for w in range(4 if cfg.get("kv_q8") else 2)])
+    for a, b in zip(*pre):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+    for a, b in zip(*caches):
+        assert np.array_equal(np.asarray(a), np.asarray(b))

@@ -3,7 +3,7 @@ the sizes that the GPU tests run.  A change of a rule that leaves an instance wi
 import ctypes
 from pooled_amd import capi
 from pooled_amd.capi import PA_W_Q4_0, PA_W_Q8_0
-from test_gpu_proj import GEMM_FEW_SIZES, GEMM_TILE_SIZES, GEMV_WIDE_SIZES
+from test_gpu_proj import GEMM_FEW_SIZES, GEMM_TILE_SIZES, GEMV_WIDE_SIZES, HEADS_SIZES
 
 CUS = 256
 u32 = ctypes.c_uint32
@@ -76,3 +76,17 @@ def test_tile_sizes_take_every_tile():
     assert {_tile(2048, 4096, 129), _tile(130, 8192, 40), _tile(100, 384, 65), _tile(64, 128, 33), _tile(130, 8192, 17)} == {(64, 32)}
     # rows further apart than the larger tiles' 32-bit offsets reach
     assert _tile(9216, 2048, 4096, 1 << 22) == (128, 384) and _tile(9216, 2048, 4096, (1 << 22) + 8) == (64, 64)
+
+
+def test_pre_step_sizes_take_every_tile():
+    def tile(heads, dim, n):
+        nH, nKV, hd, gate = heads
+        v = _rule("pa_rule_gemm_heads", nH * hd * (2 if gate else 1) + 2 * nKV * hd, dim, n, nH, hd, ctypes.c_int(gate), ctypes.c_int(CUS))
+        return v >> 28, v >> 16 & 0xfff, v & 0xffff
+    assert [tile(*size[:3]) for size in HEADS_SIZES] == [size[3] for size in HEADS_SIZES]
+    models = [((16, 8, 128, False), 2048), ((16, 2, 256, True), 2048), ((24, 4, 256, True), 5120)]
+    every = {tile(heads, dim, n) for heads, d in models for dim in (d, 256, 1024, 8192) for n in range(33, 4097, 13)}
+    assert every <= {size[3] for size in HEADS_SIZES} | {(0, 0, 0)}
+    assert [tile(*models[0], 512), tile(*models[1], 4096), tile(*models[2], 777)] == [(4, 64, 128), (1, 320, 256), (1, 224, 256)]
+    # a few columns, and sizes whose sums are split as no tile of whole heads splits them: apart
+    assert [tile(*models[0], 100), tile(*models[1], 100), tile(*models[1], 256)] == [(0, 0, 0)] * 3
