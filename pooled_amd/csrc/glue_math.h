@@ -219,11 +219,11 @@ static __device__ inline void glue_head_wave(const float (&x_in)[4], const float
 // int8 cache row, the lane's 4 consecutive values of a 32-value block (8 lanes = one block; the reference's
 // kv_store_q8, engine/wgsl/qwen35.js:908-946): scale = max|x| / 127 over the block, inv = 1 / scale (0 for an all-zero
 // block), value = clamp(round-half-even(x * inv), -127, 127), every operation a separately rounded f32 one.  Returns
-// the 4 values packed low byte first and the block's scale (the same in its 8 lanes).  All 64 lanes must call.
+// the 4 values packed low byte first and the block's scale (the same in its 8 lanes).  The 8 lanes of a block must call together.
 static __device__ inline void quant4_q8(const float (&x)[4], uint32_t& w, float& sc) {
 #pragma clang fp contract(off)
   float a = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
-  a = fmaxf(a, __shfl_xor(a, 1, 64)); a = fmaxf(a, __shfl_xor(a, 2, 64)); a = fmaxf(a, __shfl_xor(a, 4, 64));
+  a = fmaxf(a, dpp_f32<0xB1>(a)); a = fmaxf(a, dpp_f32<0x4E>(a)); a = fmaxf(a, dpp_f32<0x141>(a));    // (permutations inside the 8 lanes; through the LDS crossbar: three dependent round trips)
   sc = a / 127.0f;
   const float inv = sc > 0.f ? 1.0f / sc : 0.f;
   w = 0;
