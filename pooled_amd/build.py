@@ -70,5 +70,5 @@ def build_all(verbose=False, extra=()):
 
 
 if __name__ == "__main__":
-    # -DNAME=VALUE arguments go to hipcc (the prefill kernel's PF_QR / PF_KD / PF_VD constants)
+    # -DNAME=VALUE arguments go to hipcc (the prefill kernel's PF_KD / PF_VD constants)
     print(build_all(verbose="-v" in sys.argv, extra=tuple(a for a in sys.argv[1:] if a.startswith("-D"))))

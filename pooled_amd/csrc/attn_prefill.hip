@@ -15,15 +15,21 @@
 //     An LDS-direct load writes 64 lanes x 16 B contiguously, so rows cannot be padded; bank conflicts are
 //     avoided by an XOR swizzle applied on the *global* side (lane i fetches the chunk that belongs at its LDS
 //     slot): K chunk c of row r sits at slot c ^ (r & 15) (conflict-free ds_read_b128 fragments), V chunk c at
-//     c ^ 4 (r & 3) (2-way = optimal ds_read_b64_tr_b16).  Rows at or past the end of the context are fetched
+//     c ^ 4 (r & 3) ^ 2 (r / 4 & 1) (2-way = optimal ds_read_b64_tr_b16).  Rows at or past the end of the context are fetched
 //     from the cache's zero padding row instead, so 0 x stale bits never reaches O.
-//   * S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16_f16.  Q fragments stay in registers for the whole
-//     kernel (at hd 256 half of them, the other half is parked in LDS); K fragments are ds_read_b128, V^T fragments come from the gfx950 LDS transpose read
-//     (ds_read_b64_tr_b16).  The S^T accumulator layout (lane = query row, 16 positions) is the B-operand
-//     layout of the PV product, so P never leaves registers.
-//   * Online softmax in f32 in the exp2 domain with a lazily updated reference maximum: O and l are rescaled
-//     only when some row's maximum grows by more than 2^8, which keeps exp2(x - m_ref) <= 256 (exact enough
-//     in f16) and takes the 128-register O rescale off the common path.
+//   * S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_16x16x32_f16, a wave's 32 rows as two blocks of 16.  Q fragments stay in registers for the
+//     whole kernel; K fragments are ds_read_b128, V^T fragments come from the gfx950 LDS transpose read (ds_read_b64_tr_b16), each feeding
+//     both blocks.  The S^T accumulator layout (lane = query row, 4 + 4 positions) is the B-operand layout of the PV product, so P never leaves
+//     registers.  On a full chip of head_dim 256 the kernel runs at the power limit, where this shape has the better rate (products alone
+//     on random operands: 1.73 - 1.80 PFLOP/s against 1.65 on 32 x 32 x 16), as long as the softmax's two rows a lane cost no
+//     more than one did:
+//   * Online softmax in f32 in the exp2 domain with a lazily updated reference maximum: O and l are rescaled only when a P comes out above 2^8
+//     (exact enough in f16), which takes the 128-register O rescale, and with it every row maximum, off the common path: what is
+//     looked at is the packed P itself, seven maxima a tile, and a tile that fails is taken again with raised references.  Row maxima of
+//     every tile: 4 % slower at head_dim 256, 7 - 10 % at 128.
+//     Both steps together against 32 x 32 x 16 with row maxima (us, 16 / 2-head shape): 4096 columns at 64K 3708 -> 3325, at 8192 658 -> 598, 2500
+//     at 16384 (158 workgroups: below the limit) 778 -> 761; 16 / 8-head shape, 4096 at 28000 972 -> 878, 2500 at 8192 276 -> 272; 777 of the 24 / 4-head
+//     shape at 5003, split, 142 -> 133.  Fragments three ahead in both products: two of K are 1 - 2 % slower, four spill.
 //   * Workgroup ids are remapped so that each XCD (ids are dealt round-robin to the 8 XCDs) works on one
 //     contiguous range of (kv head, column block): the K/V stream of a kv head is fetched into one L2.
 //   * PAIRED (unsplit passes of one round whose chunk is a material part of the context, the rule at pairs_pay): waves 0-3 take a
@@ -43,18 +49,18 @@
 template <int HD, int W> struct PfShape {
   static constexpr int ROWB = HD * 2;             // bytes of one kv head's row
   static constexpr int TILE = PF_TN * ROWB;       // bytes of one staged tile (K or V)
-  static constexpr int KS = HD / 16;              // k-steps of QK^T
-  static constexpr int DB = HD / 32;              // 32-dim blocks of the output
-  static constexpr int QR = HD == 256 ? PF_QR : KS;   // k-steps whose Q fragments stay in registers
+  static constexpr int KS = HD / 32;              // k-steps of QK^T
+  static constexpr int DB = HD / 16;              // 16-dim blocks of the output
   static constexpr int CPR = HD / 8;              // 16-byte chunks per row
   static constexpr int RPB = 64 / CPR;            // rows per 1 KB LDS-direct load
   static constexpr int NLD = PF_TN / RPB / W;   // LDS-direct loads per wave, tensor and step
   static_assert(NLD >= 1 && NLD * W * RPB == PF_TN, "tile must divide evenly over the waves");
 };
 
-template <int HD, int QB, int W, bool PAIRED>
+template <int HD, int W, bool PAIRED>
 __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p, uint32_t n_col_blocks, uint32_t half_cols, uint32_t head_xcds) {
   typedef PfShape<HD, W> S;
+  constexpr int NB = 2;                            // 16-row blocks of a wave
   // four separate LDS objects (two K, two V buffers): the compiler then orders an LDS read only after the
   // LDS-direct loads into the *same* buffer, and the prefetch into the other buffer stays in flight
   __shared__ __attribute__((aligned(1024))) unsigned char kbuf0[S::TILE];
@@ -83,22 +89,31 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
 
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform (scalar) so per-wave branches are scalar branches
-  const uint32_t ln = lane & 31, hb = lane >> 5;   // MFMA row / column index, k half
+  const uint32_t ln = lane & 15, kg = lane >> 4;    // MFMA row / column index, k group
   const uint32_t G = p.group, nH = p.n_heads;
+  // r / G as a multiply and a shift (exact for r < 1024 and G <= 64)
+  const uint32_t g_magic = (65536u + G - 1u) / G;
+  auto div_g = [&](uint32_t r) __attribute__((always_inline)) -> uint32_t { return (r * g_magic) >> 16; };
+  // the lane, counted anew: what depends on it is not kept in registers across the code before
+  auto fresh_lane = []() __attribute__((always_inline)) -> uint32_t {
+    uint32_t l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+  };
   // columns of this WAVE [c0, c0 + R / G): the workgroup's block, or (PAIRED) its half's block: waves of the lower half
   // take block cb from the front, the others the one as far from the back, so that every workgroup has the same work
-  uint32_t c0 = cb * p.cols_per_group, wrow0 = wave * QB * 32;       // wrow0: the wave's first row in its block
+  uint32_t c0 = cb * p.cols_per_group, wrow0 = wave * 32;       // wrow0: the wave's first row in its block
   uint32_t ncl = min(p.cols_per_group, p.n_cols - c0), c_end = c0 + ncl;
   if constexpr (PAIRED) {
     const uint32_t n_half = (p.n_cols + half_cols - 1) / half_cols, far = n_half - 1 - cb;
     const bool lower = wave < W / 2;
     c0 = (lower ? cb : far) * half_cols;
-    if (!lower) wrow0 -= W / 2 * QB * 32;
+    if (!lower) wrow0 -= W / 2 * 32;
     c_end = min((far + 1) * half_cols, p.n_cols);
     ncl = min(half_cols, p.n_cols - c0);
     if (far == cb && lower) ncl = 0;               // an odd number of blocks: the middle one is alone
   }
-  const uint32_t R = ncl * G;                      // live rows (<= W * QB * 32)
+  const uint32_t R = ncl * G;                      // live rows (<= 32 W)
   const uint32_t seq_max = p.base_pos + c_end;     // rows visible to the workgroup's last column
   const uint32_t t_begin = sp * p.split_len;
   if (t_begin >= seq_max) return;
@@ -116,216 +131,204 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   //      is wave-uniform (scalar registers) ----
   static_assert((W * S::RPB) % 16 == 0, "the swizzle must not depend on the load index");
   const uint32_t ld_row0 = wave * S::RPB + lane / S::CPR, ld_slot = lane % S::CPR;
-  auto k_off_of = [&](uint32_t row0, uint32_t slot) { return row0 * (uint32_t)row_bytes + (slot ^ (row0 & 15)) * 16; };
-  auto v_off_of = [&](uint32_t row0, uint32_t slot) { return row0 * (uint32_t)row_bytes + (slot ^ (4 * (row0 & 3))) * 16; };
+  auto k_slot = [&](uint32_t row, uint32_t slot) { return slot ^ (row & 15); };
+  auto v_slot = [&](uint32_t row, uint32_t slot) { return slot ^ (4 * (row & 3)) ^ (2 * ((row >> 2) & 1)); };
+  auto k_off_of = [&](uint32_t row0, uint32_t slot) { return row0 * (uint32_t)row_bytes + k_slot(row0, slot) * 16; };
+  auto v_off_of = [&](uint32_t row0, uint32_t slot) { return row0 * (uint32_t)row_bytes + v_slot(row0, slot) * 16; };
   const uint32_t k_off = k_off_of(ld_row0, ld_slot), v_off = v_off_of(ld_row0, ld_slot);
   constexpr uint32_t LD_STRIDE = W * S::RPB * S::ROWB;           // bytes between the rows of consecutive loads
-  // rows at or past t_end (only in the last tile of the context) come from the zero padding row max_seq
-  auto issue_t = [&](const unsigned char* g_base, const uint32_t off, const uint32_t row0, unsigned char* dst, uint32_t tpos) {
-    const unsigned char* t0p = g_base + (size_t)tpos * row_bytes;
+  // Rows at or past t_end (only in the last tile of the context) come from the zero padding row max_seq; their addresses are worked out
+  // there and one load at a time, so that nothing of them takes registers in the loop.
+  auto issue = [&](unsigned char* kdst, unsigned char* vdst, const uint32_t tpos, const uint32_t ko, const uint32_t vo) __attribute__((always_inline)) {
     if (tpos + PF_TN <= t_end) {
+      const unsigned char* kt = kg_base + (size_t)tpos * row_bytes;
+      const unsigned char* vt = vg_base + (size_t)tpos * row_bytes;
 #pragma unroll
-      for (int i = 0; i < S::NLD; i++) PF_GLL_S(t0p + i * LD_STRIDE, off, dst + (i * W + wave) * 1024);
+      for (int i = 0; i < S::NLD; i++) PF_GLL_S(kt + i * LD_STRIDE, ko, kdst + (i * W + wave) * 1024);
+#pragma unroll
+      for (int i = 0; i < S::NLD; i++) PF_GLL_S(vt + i * LD_STRIDE, vo, vdst + (i * W + wave) * 1024);
     } else {
+      const uint32_t l = fresh_lane(), row0 = wave * S::RPB + l / S::CPR, slot = l % S::CPR;
 #pragma unroll
       for (int i = 0; i < S::NLD; i++) {
-        const uint32_t row = i * W * S::RPB + row0;
-        const unsigned char* src = tpos + row < t_end ? t0p + i * LD_STRIDE + off
-                                                      : g_base + (size_t)p.max_seq * row_bytes + (off - row0 * (uint32_t)row_bytes);
-        PF_GLL(src, dst + (i * W + wave) * 1024);
+        const uint32_t row = tpos + i * W * S::RPB + row0;
+        const size_t at = (size_t)(row < t_end ? row : p.max_seq) * row_bytes;
+        PF_GLL(kg_base + at + k_slot(row0, slot) * 16, kdst + (i * W + wave) * 1024);
+        PF_GLL(vg_base + at + v_slot(row0, slot) * 16, vdst + (i * W + wave) * 1024);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
-  auto issue_k = [&](unsigned char* kdst, uint32_t tpos) { issue_t(kg_base, k_off, ld_row0, kdst, tpos); };
-  auto issue_v = [&](unsigned char* vdst, uint32_t tpos) { issue_t(vg_base, v_off, ld_row0, vdst, tpos); };
-  issue_k(kbuf0, t_begin);
-  issue_v(vbuf0, t_begin);
+  issue(kbuf0, vbuf0, t_begin, k_off, v_off);
 
-  // ---- per-lane rows: row r = wrow0 + qb*32 + ln of the wave's block of columns = (column c0 + r / G, head r % G) ----
-  uint32_t end_pos[QB], row_id[QB];
+  // ---- per-lane rows: row r = wrow0 + 16 nb + ln of the wave's block of columns = (column c0 + r / G, head r % G) ----
   uint32_t w_min_end = 0xffffffffu, w_max_end = 0;                // positions seen by the wave's first row, by its last one
-#pragma unroll
-  for (int qb = 0; qb < QB; qb++) {
-    const uint32_t r = wrow0 + qb * 32 + ln;
-    row_id[qb] = !PAIRED || R ? min(r, R - 1) : 0;
-    end_pos[qb] = r < R ? p.base_pos + c0 + r / G + 1 : 0u;
-  }
-  {
-    if (wrow0 < R) { w_min_end = p.base_pos + c0 + wrow0 / G + 1; w_max_end = p.base_pos + c0 + min(wrow0 + QB * 32 - 1, R - 1) / G + 1; }
-  }
+  if (wrow0 < R) { w_min_end = p.base_pos + c0 + div_g(wrow0) + 1; w_max_end = p.base_pos + c0 + div_g(min(wrow0 + NB * 16 - 1, R - 1)) + 1; }
 
-  // ---- Q fragments (B operand of S^T = K Q^T): row ln of block qb, dims 16 ks + 8 hb .. + 7, as f16 ----
-  // The first QR k-steps stay in registers for the whole kernel; the others are parked in LDS in fragment order
-  // ([wave][qb][ks - QR][lane] x 16 B: conflict-free b128 reads of a wave's own region) and re-read every step.
-  // At hd 256 all 16 in registers (64 VGPRs) leave too little room beside the 128 accumulators; a single spill
-  // reload inside the loop would also force the in-order vmcnt to drain the LDS-direct loads in flight.
-  constexpr int QR = S::QR;
-  extern __shared__ __attribute__((aligned(16))) unsigned char q_lds_all[];
-  unsigned char* q_lds = q_lds_all + (size_t)wave * QB * (S::KS - QR) * 1024 + lane * 16;
-  h8 qf[QB][QR];
+  // ---- Q fragments (B operand of S^T = K Q^T): row ln of block nb, dims 32 ks + 8 kg .. + 7, as f16, in registers for the whole kernel ----
+  h8 qf[NB][S::KS];
 #pragma unroll
-  for (int qb = 0; qb < QB; qb++) {
-    const float* qrow = p.q + (size_t)(c0 + row_id[qb] / G) * p.q_stride + (size_t)(g * G + row_id[qb] % G) * HD + 8 * hb;
+  for (int nb = 0; nb < NB; nb++) {
+    const uint32_t r = wrow0 + nb * 16 + ln, rc = !PAIRED || R ? min(r, R - 1) : 0;
+    const uint32_t qc = div_g(rc);
+    const float* qrow = p.q + (size_t)(c0 + qc) * p.q_stride + (size_t)(g * G + rc - qc * G) * HD + 8 * kg;
 #pragma unroll
     for (int ks = 0; ks < S::KS; ks++) {
-      const f4 a = *(const f4*)(qrow + 16 * ks), b = *(const f4*)(qrow + 16 * ks + 4);
-      const h8 f = { (_Float16)a[0], (_Float16)a[1], (_Float16)a[2], (_Float16)a[3],
-                     (_Float16)b[0], (_Float16)b[1], (_Float16)b[2], (_Float16)b[3] };
-      if (ks < QR) qf[qb][ks] = f;
-      else *(h8*)(q_lds + (qb * (S::KS - QR) + (ks - QR)) * 1024) = f;
+      const f4 a = *(const f4*)(qrow + 32 * ks), b = *(const f4*)(qrow + 32 * ks + 4);
+      qf[nb][ks] = (h8){ (_Float16)a[0], (_Float16)a[1], (_Float16)a[2], (_Float16)a[3],
+                         (_Float16)b[0], (_Float16)b[1], (_Float16)b[2], (_Float16)b[3] };
     }
   }
 
-  f16v acc[S::DB][QB];
+  f4 acc[S::DB][NB];
 #pragma unroll
   for (int db = 0; db < S::DB; db++)
 #pragma unroll
-    for (int qb = 0; qb < QB; qb++)
+    for (int nb = 0; nb < NB; nb++) acc[db][nb] = (f4){0.f, 0.f, 0.f, 0.f};
+  float m_ref[NB], l_run[NB];
 #pragma unroll
-      for (int i = 0; i < 16; i++) acc[db][qb][i] = 0.f;
-  float m_ref[QB], l_run[QB];
-#pragma unroll
-  for (int qb = 0; qb < QB; qb++) { m_ref[qb] = NEG_INF; l_run[qb] = 0.f; }
-  const float c1 = p.scale * 1.4426950408889634f;   // scores -> log2 domain
+  for (int nb = 0; nb < NB; nb++) { m_ref[nb] = wrow0 + nb * 16 + ln < R ? NEG_INF : 0.f; l_run[nb] = 0.f; }   // (rows past the last: never counted as unseen)
+  bool unseen = true;
+  const float c1 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(p.scale * 1.4426950408889634f)));   // scores -> log2 domain (scalar)
 
   // per-lane LDS read offsets with the swizzles folded in (buffer bases are 1 KB aligned, so XOR == add on the
-  // swizzled bits): K fragment of k-step ks is at k_rd ^ (ks * 32); V fragment of dim block db at v_rd ^ (db * 64)
-  const uint32_t k_rd = ln * S::ROWB + ((hb ^ (ln & 1)) * 16) + ((ln & 15) >> 1) * 32;
-  const uint32_t b4 = lane >> 4, sl = lane & 15;
-  const uint32_t v_rd = (4 * (b4 >> 1) + (sl >> 2)) * S::ROWB + (2 * (b4 & 1) + ((sl & 3) >> 1)) * 16 + (sl & 1) * 8 + ((sl >> 2) & 3) * 64;
+  // swizzled bits, 256 bytes of a row): K fragment of k-step ks is at k_rd ^ (ks * 64); V fragment of dim block db at v_rd ^ (db * 32)
+  const uint32_t k_rd = ln * S::ROWB + (kg ^ ln) * 16;
+  const uint32_t v_rd = (4 * kg + (ln >> 2)) * S::ROWB + (((ln & 3) >> 1) ^ (4 * (ln >> 2)) ^ (2 * (kg & 1))) * 16 + (ln & 1) * 8;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
   // The three phases of a tile.  s (raw scores) lives from qk to sm, pf (f16 probabilities) from sm to pv.
-  f16v s[QB];
-  h8 pf[QB][2];
-  // ---- S^T = K Q^T : rows = 32 positions, columns = 32 query rows per block ----
+  f4 s[2][NB];
+  h8 pf[NB];
+  // ---- S^T = K Q^T : rows = 2 x 16 positions, columns = 16 query rows per block ----
   auto qk = [&](const unsigned char* kb, const uint32_t tp) {
 #pragma unroll
-    for (int qb = 0; qb < QB; qb++)
+    for (int pb = 0; pb < 2; pb++)
 #pragma unroll
-      for (int i = 0; i < 16; i++) s[qb][i] = 0.f;
-    // K fragments (and the Q fragments parked in LDS) are fetched KD k-steps ahead of the MFMA that consumes them
-    constexpr int KD = PF_KD;
-    h8 ka[KD], qa[QB][KD];
+      for (int nb = 0; nb < NB; nb++) s[pb][nb] = (f4){0.f, 0.f, 0.f, 0.f};
+    // fragment f = positions 16 (f % 2) .., k-step f / 2; fetched KD fragments ahead of the MFMAs that consume them
+    constexpr int KD = PF_KD, NF = 2 * S::KS;
+    h8 ka[KD];
+    auto at = [&](int f) { return kb + (k_rd ^ (f / 2 % 4 * 64)) + f / 8 * 256 + f % 2 * 16 * S::ROWB; };
 #pragma unroll
-    for (int i = 0; i < KD; i++) {
-      ka[i] = *(const h8*)(kb + (k_rd ^ (i * 32)));
-      if (i >= QR) {
+    for (int f = 0; f < KD; f++) ka[f] = *(const h8*)at(f);
 #pragma unroll
-        for (int qb = 0; qb < QB; qb++) qa[qb][i] = *(const h8*)(q_lds + (qb * (S::KS - QR) + (i - QR)) * 1024);
-      }
+    for (int f = 0; f < NF; f++) {
+      const h8 a = ka[f % KD];
+      if (f + KD < NF) ka[f % KD] = *(const h8*)at(f + KD);
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) s[f % 2][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qf[nb][f / 2], s[f % 2][nb], 0, 0, 0);
     }
+    // pin the issue order the source states: the first KD fetches up front, then each fragment's successor behind its MFMAs
 #pragma unroll
-    for (int ks = 0; ks < S::KS; ks++) {
-      const h8 a = ka[ks % KD];
-      h8 b[QB];
+    for (int f = 0; f < KD; f++) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
 #pragma unroll
-      for (int qb = 0; qb < QB; qb++) b[qb] = ks < QR ? qf[qb][ks < QR ? ks : 0] : qa[qb][ks % KD];
-      if (ks + KD < S::KS) {
-        ka[ks % KD] = *(const h8*)(kb + (k_rd ^ ((ks + KD) * 32)));
-        if (ks + KD >= QR) {
-#pragma unroll
-          for (int qb = 0; qb < QB; qb++) qa[qb][ks % KD] = *(const h8*)(q_lds + (qb * (S::KS - QR) + (ks + KD - QR)) * 1024);
-        }
-      }
-#pragma unroll
-      for (int qb = 0; qb < QB; qb++) s[qb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b[qb], s[qb], 0, 0, 0);
-    }
-    // pin the issue order the source states: the first KD fetches up front, then each k-step's fetches behind its MFMAs
-#pragma unroll
-    for (int i = 0; i < KD; i++) { __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); if (i >= QR) __builtin_amdgcn_sched_group_barrier(0x100, QB, 0); }
-#pragma unroll
-    for (int ks = 0; ks < S::KS; ks++) {
-      __builtin_amdgcn_sched_group_barrier(0x008, QB, 0);
-      if (ks + KD < S::KS) { __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); if (ks + KD >= QR) __builtin_amdgcn_sched_group_barrier(0x100, QB, 0); }
+    for (int f = 0; f < NF; f++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, NB, 0);
+      if (f + KD < NF) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
   };
-  // ---- online softmax; lane holds query row ln of each block, positions tp + 8 (i / 4) + 4 hb + i % 4 ----
+  // ---- online softmax; lane holds query row ln of each block, positions tp + 16 pb + 4 kg + i ----
   // Raw scores stay unscaled: the scale rides in the exp2 argument (one fma per element), the row sum is a
   // v_dot2 over the f16-rounded probabilities (the values PV really uses), and the mask is a separate pass
   // that only tiles straddling a row end execute.
   auto sm = [&](const uint32_t tp) {
     if (tp + PF_TN > w_min_end) {
-      asm volatile("; causal tile" ::: "memory");   // keeps this a branch: most tiles skip the 3 ops per element
+      // (volatile: keeps this a branch -- most tiles skip the 3 ops per element -- and what it works out in it)
+      const uint32_t l = fresh_lane();
 #pragma unroll
-      for (int qb = 0; qb < QB; qb++)
+      for (int nb = 0; nb < NB; nb++) {
+        const uint32_t r = wrow0 + nb * 16 + (l & 15), end_pos = r < R ? p.base_pos + c0 + div_g(r) + 1 : 0u;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-          const uint32_t pos = tp + 8 * (i >> 2) + 4 * hb + (i & 3);
-          s[qb][i] = pos < end_pos[qb] ? s[qb][i] : NEG_INF;
-        }
-    }
-    float mt[QB];
+        for (int pb = 0; pb < 2; pb++)
 #pragma unroll
-    for (int qb = 0; qb < QB; qb++) {
-      float mx = fmaxf(s[qb][0], s[qb][1]);
-#pragma unroll
-      for (int i = 2; i < 16; i += 2) mx = fmaxf(fmaxf(mx, s[qb][i]), s[qb][i + 1]);
-      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-      mt[qb] = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * c1;      // both k halves of the row, log2 domain
-    }
-    bool grow = false;
-#pragma unroll
-    for (int qb = 0; qb < QB; qb++) grow |= mt[qb] > m_ref[qb] + PF_RESCALE_TH;
-    if (__any(grow)) {
-#pragma unroll
-      for (int qb = 0; qb < QB; qb++) {
-        const float m_new = fmaxf(m_ref[qb], mt[qb]);
-        const float alpha = m_new == NEG_INF ? 1.f : __builtin_amdgcn_exp2f(m_ref[qb] - m_new);
-        m_ref[qb] = m_new;
-        l_run[qb] *= alpha;
-#pragma unroll
-        for (int db = 0; db < S::DB; db++) acc[db][qb] *= alpha;
+          for (int i = 0; i < 4; i++) {
+            const uint32_t pos = tp + 16 * pb + 4 * (l >> 4) + i;
+            s[pb][nb][i] = pos < end_pos ? s[pb][nb][i] : NEG_INF;
+          }
       }
     }
+    // P against the reference maxima as they are; where one of the wave's comes out above 2^PF_RESCALE_TH (on the packed values, seven maxima
+    // a tile instead of the rows' own), the references are raised and P is taken again, below 1 this time.  So no row maximum is worked out on
+    // the common path -- but on a wave's first tile, and for as long as one of its rows has seen nothing (a split before the row's end).
+    auto raise = [&]() __attribute__((always_inline)) {
+      bool none = false;
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) {
+        float mx = fmaxf(s[0][nb][0], s[0][nb][1]);
+        mx = fmaxf(fmaxf(mx, s[0][nb][2]), s[0][nb][3]);
+        mx = fmaxf(fmaxf(mx, s[1][nb][0]), s[1][nb][1]);
+        mx = fmaxf(fmaxf(mx, s[1][nb][2]), s[1][nb][3]);
+        const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx = fmaxf(__uint_as_float(s16[0]), __uint_as_float(s16[1]));
+        const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        const float m_new = fmaxf(m_ref[nb], fmaxf(__uint_as_float(s32[0]), __uint_as_float(s32[1])) * c1);   // all four position groups of the row, log2 domain
+        const float alpha = m_new == NEG_INF ? 1.f : __builtin_amdgcn_exp2f(m_ref[nb] - m_new);
+        m_ref[nb] = m_new;
+        l_run[nb] *= alpha;
+        none |= m_new == NEG_INF;
+#pragma unroll
+        for (int db = 0; db < S::DB; db++) acc[db][nb] *= alpha;
+      }
+      unseen = __any(none);
+    };
+    auto probs = [&]() __attribute__((always_inline)) -> bool {
+      h2 top = { (_Float16)0.f, (_Float16)0.f };
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) {
+        const float nmr = m_ref[nb] == NEG_INF ? 0.f : -m_ref[nb];
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j / 4][nb][j % 4], c1, nmr));
+          const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j / 4][nb][j % 4 + 1], c1, nmr));
+          const h2 pp = { (_Float16)e0, (_Float16)e1 };
+          top = __builtin_elementwise_max(top, pp);
+          pf[nb][j] = pp[0]; pf[nb][j + 1] = pp[1];
+        }
+      }
+      const _Float16 lim = (_Float16)(float)(1 << PF_RESCALE_TH);
+      return __any(top[0] > lim || top[1] > lim);
+    };
+    if (__builtin_expect(unseen, 0)) raise();
+    if (__builtin_expect(probs(), 0)) { raise(); probs(); }
     const h2 ones = { (_Float16)1.f, (_Float16)1.f };
 #pragma unroll
-    for (int qb = 0; qb < QB; qb++) {
-      const float nmr = m_ref[qb] == NEG_INF ? 0.f : -m_ref[qb];
-      float ps = l_run[qb];
+    for (int nb = 0; nb < NB; nb++) {
 #pragma unroll
-      for (int i = 0; i < 16; i += 2) {
-        const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qb][i], c1, nmr));
-        const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qb][i + 1], c1, nmr));
-        const h2 pp = { (_Float16)e0, (_Float16)e1 };
-        ps = __builtin_amdgcn_fdot2(pp, ones, ps, false);
-        pf[qb][i >> 3][i & 7] = pp[0]; pf[qb][i >> 3][(i & 7) + 1] = pp[1];
-      }
-      l_run[qb] = ps;
+      for (int j = 0; j < 8; j += 2) { const h2 pp = { pf[nb][j], pf[nb][j + 1] }; l_run[nb] = __builtin_amdgcn_fdot2(pp, ones, l_run[nb], false); }
     }
   };
-  // ---- O^T += V^T P^T : rows = 32 dims, contraction over 2 x 16 positions ----
+  // ---- O^T += V^T P^T : rows = 16 dims a block, contraction over the 32 positions (slot 8 kg + j: position 4 kg + j, or 16 + 4 kg + j - 4) ----
   auto pv = [&](const unsigned char* vb, const uint32_t tp) {
-    // fragment f = j DB + db: positions 16 j .., dims 32 db .. (consecutive MFMAs hit different accumulators);
-    // fetched VD fragments ahead
-    constexpr int VD = PF_VD, NF = 2 * S::DB;
+    // dim block db's fragment is fetched VD blocks ahead
+    constexpr int VD = PF_VD;
     h4 vlo[VD], vhi[VD];
+    auto at = [&](int f) { return vb + (v_rd ^ (f % 8 * 32)) + f / 8 * 256; };
 #pragma unroll
     for (int f = 0; f < VD; f++) {
-      const unsigned char* vp = vb + (v_rd ^ ((f % S::DB) * 64)) + (f / S::DB) * 16 * S::ROWB;
+      const unsigned char* vp = at(f);
       vlo[f] = lds_read_tr16(vp);
-      vhi[f] = lds_read_tr16(vp + 8 * S::ROWB);
+      vhi[f] = lds_read_tr16(vp + 16 * S::ROWB);
     }
 #pragma unroll
-    for (int f = 0; f < NF; f++) {
+    for (int f = 0; f < S::DB; f++) {
       const h4 lo = vlo[f % VD], hi = vhi[f % VD];
-      if (f + VD < NF) {
-        const int fn = f + VD;
-        const unsigned char* vp = vb + (v_rd ^ ((fn % S::DB) * 64)) + (fn / S::DB) * 16 * S::ROWB;
+      if (f + VD < S::DB) {
+        const unsigned char* vp = at(f + VD);
         vlo[f % VD] = lds_read_tr16(vp);
-        vhi[f % VD] = lds_read_tr16(vp + 8 * S::ROWB);
+        vhi[f % VD] = lds_read_tr16(vp + 16 * S::ROWB);
       }
       const h8 a = { lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3] };
 #pragma unroll
-      for (int qb = 0; qb < QB; qb++) acc[f % S::DB][qb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pf[qb][f / S::DB], acc[f % S::DB][qb], 0, 0, 0);
+      for (int nb = 0; nb < NB; nb++) acc[f][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pf[nb], acc[f][nb], 0, 0, 0);
     }
 #pragma unroll
     for (int f = 0; f < VD; f++) __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
 #pragma unroll
-    for (int f = 0; f < NF; f++) {
-      __builtin_amdgcn_sched_group_barrier(0x008, QB, 1);
-      if (f + VD < NF) __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
+    for (int f = 0; f < S::DB; f++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, NB, 1);
+      if (f + VD < S::DB) __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
     }
   };
 
@@ -346,7 +349,7 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
     auto step_s = [&](auto PAR, const uint32_t i) {
       constexpr int par = decltype(PAR)::value;
       const uint32_t tp = t_begin + i * PF_TN;
-      if (i + 1 < n_steps) { issue_k(par ? kbuf0 : kbuf1, tp + PF_TN); issue_v(par ? vbuf0 : vbuf1, tp + PF_TN); }
+      if (i + 1 < n_steps) issue(par ? kbuf0 : kbuf1, par ? vbuf0 : vbuf1, tp + PF_TN, k_off, v_off);
       if (TWO_LOOPS || tp < w_max_end) {
         qk(par ? kbuf1 : kbuf0, tp);
         sm(tp);
@@ -361,18 +364,13 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
     }
     if (n_live & 1) step_s(std::integral_constant<int, 0>{}, n_even);
     if constexpr (HD == 256) {
-      // the lane, counted anew: what depends on it from here on is not kept in registers through the loop above
-      lane_e = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-      asm volatile("" : "+v"(lane_e));
+      lane_e = fresh_lane();
     }
     if constexpr (TWO_LOOPS) {
       const uint32_t d_row0 = wave * S::RPB + lane_e / S::CPR, d_slot = lane_e % S::CPR;
       for (uint32_t i = n_live; i < n_steps; i++) {
         const uint32_t tp = t_begin + i * PF_TN;
-        if (i + 1 < n_steps) {
-          issue_t(kg_base, k_off_of(d_row0, d_slot), d_row0, i & 1 ? kbuf0 : kbuf1, tp + PF_TN);
-          issue_t(vg_base, v_off_of(d_row0, d_slot), d_row0, i & 1 ? vbuf0 : vbuf1, tp + PF_TN);
-        }
+        if (i + 1 < n_steps) issue(i & 1 ? kbuf0 : kbuf1, i & 1 ? vbuf0 : vbuf1, tp + PF_TN, k_off_of(d_row0, d_slot), v_off_of(d_row0, d_slot));
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
       }
@@ -380,67 +378,52 @@ __global__ __launch_bounds__(W * 64, W / 4) void pa_prefill_kernel(AttnParams p,
   }
 
   // ---- epilogue ----
-  const uint32_t ln_e = lane_e & 31, hb_e = lane_e >> 5;
+  const uint32_t ln_e = lane_e & 15, kg_e = lane_e >> 4;
 #pragma unroll
-  for (int qb = 0; qb < QB; qb++) {
-    l_run[qb] += __shfl_xor(l_run[qb], 32, 64);
-    const uint32_t r = wrow0 + qb * 32 + ln_e;
+  for (int nb = 0; nb < NB; nb++) {
+    l_run[nb] += __shfl_xor(l_run[nb], 16, 64);
+    l_run[nb] += __shfl_xor(l_run[nb], 32, 64);
+    const uint32_t r = wrow0 + nb * 16 + ln_e;
     if (r >= R) continue;
-    const uint32_t col = c0 + r / G, hq = g * G + r % G;
+    const uint32_t rc = div_g(r), col = c0 + rc, hq = g * G + r - rc * G;
     if (p.n_splits == 1) {
       // the whole context was seen: normalise, gate, convert, store
-      const float inv_l = 1.f / l_run[qb];
+      const float inv_l = 1.f / l_run[nb];
       const float* gate = p.gate ? p.gate + (size_t)col * p.gate_stride + (size_t)hq * HD : nullptr;
 #pragma unroll
       for (int db = 0; db < S::DB; db++) {
+        const uint32_t d = 16 * db + 4 * kg_e;
+        f4 o = acc[db][nb] * inv_l;
+        if (gate) {
+          const f4 gt = *(const f4*)(gate + d);
 #pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-          const uint32_t d = 32 * db + 8 * q4 + 4 * hb_e;
-          f4 o = { acc[db][qb][4 * q4] * inv_l, acc[db][qb][4 * q4 + 1] * inv_l, acc[db][qb][4 * q4 + 2] * inv_l, acc[db][qb][4 * q4 + 3] * inv_l };
-          if (gate) {
-            const f4 gt = *(const f4*)(gate + d);
-#pragma unroll
-            for (int i = 0; i < 4; i++) o[i] *= 1.f / (1.f + __expf(-gt[i]));
-          }
-          if (p.out_f16) {
-            const h4 hv = { (_Float16)o[0], (_Float16)o[1], (_Float16)o[2], (_Float16)o[3] };
-            *(h4*)((_Float16*)p.out + (size_t)col * p.out_stride + (size_t)hq * HD + d) = hv;
-          } else {
-            *(f4*)((float*)p.out + (size_t)col * p.out_stride + (size_t)hq * HD + d) = o;
-          }
+          for (int i = 0; i < 4; i++) o[i] *= 1.f / (1.f + __expf(-gt[i]));
+        }
+        if (p.out_f16) {
+          const h4 hv = { (_Float16)o[0], (_Float16)o[1], (_Float16)o[2], (_Float16)o[3] };
+          *(h4*)((_Float16*)p.out + (size_t)col * p.out_stride + (size_t)hq * HD + d) = hv;
+        } else {
+          *(f4*)((float*)p.out + (size_t)col * p.out_stride + (size_t)hq * HD + d) = o;
         }
       }
     } else {
       // split partial: un-normalised O, m in natural-log units of the scaled scores, l
       const size_t slot = ((size_t)col * nH + hq) * p.slots + sp;
 #pragma unroll
-      for (int db = 0; db < S::DB; db++)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-          const uint32_t d = 32 * db + 8 * q4 + 4 * hb_e;
-          const f4 o = { acc[db][qb][4 * q4], acc[db][qb][4 * q4 + 1], acc[db][qb][4 * q4 + 2], acc[db][qb][4 * q4 + 3] };
-          *(f4*)(p.part_o + slot * HD + d) = o;
-        }
-      if (hb_e == 0) {
-        p.part_ml[slot * 2] = m_ref[qb] * 0.6931471805599453f;
-        p.part_ml[slot * 2 + 1] = l_run[qb];
+      for (int db = 0; db < S::DB; db++) *(f4*)(p.part_o + slot * HD + 16 * db + 4 * kg_e) = acc[db][nb];
+      if (kg_e == 0) {
+        p.part_ml[slot * 2] = m_ref[nb] * 0.6931471805599453f;
+        p.part_ml[slot * 2 + 1] = l_run[nb];
       }
     }
   }
 }
 
-template <int HD, int QB, int W, bool PAIRED>
+template <int HD, int W, bool PAIRED>
 static hipError_t launch_prefill_k(const AttnParams& p, uint32_t col_groups, uint32_t half, uint32_t head_xcds, hipStream_t s, const PaTiming* t) {
-  typedef PfShape<HD, W> S;
-  const size_t lds = (size_t)W * QB * (S::KS - S::QR) * 1024;     // Q fragments parked in LDS (dynamic part)
-  if (lds > 0) {
-    static PaPerDevice lds_set;
-    const hipError_t e = pa_lds_limit(lds_set, (const void*)pa_prefill_kernel<HD, QB, W, PAIRED>, lds);
-    if (e != hipSuccess) return e;
-  }
   const uint32_t total = col_groups * p.n_kv_heads * p.n_splits;
   const uint32_t gx = 8 * (head_xcds ? (col_groups + head_xcds - 1) / head_xcds : (total + 7) / 8);       // whole rounds of the 8 XCDs
-  PA_LAUNCH((pa_prefill_kernel<HD, QB, W, PAIRED>), dim3(gx), dim3(W * 64), lds, s, t, p, col_groups, half, head_xcds);
+  PA_LAUNCH((pa_prefill_kernel<HD, W, PAIRED>), dim3(gx), dim3(W * 64), 0, s, t, p, col_groups, half, head_xcds);
   return hipGetLastError();
 }
 
@@ -456,22 +439,22 @@ static bool pairs_pay(const AttnParams& p, uint32_t total, uint32_t n_cu) {
   return HD == 128 || (uint64_t)p.base_pos * total <= 3ull * p.n_cols * n_cu;
 }
 
-template <int HD, int QB, int W>
+template <int HD, int W>
 static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t) {
-  const uint32_t half = W / 2 * QB * 32 / p.group;
+  const uint32_t half = W / 2 * 32 / p.group;
   const uint32_t total = col_groups * p.n_kv_heads * p.n_splits;
   const bool one_round = total <= n_cu;
   if (p.n_splits == 1 && half > 0 && one_round && ((p.n_cols + half - 1) / half + 1) / 2 == col_groups && pairs_pay<HD>(p, total, n_cu))
-    return launch_prefill_k<HD, QB, W, true>(p, col_groups, half, 0, s, t);
+    return launch_prefill_k<HD, W, true>(p, col_groups, half, 0, s, t);
   // more workgroups than the chip holds at once: the longest blocks first
   const uint32_t head_xcds = p.n_splits == 1 && !one_round && 8 % p.n_kv_heads == 0 ? 8 / p.n_kv_heads : 0;
-  return launch_prefill_k<HD, QB, W, false>(p, col_groups, 0, head_xcds, s, t);
+  return launch_prefill_k<HD, W, false>(p, col_groups, 0, head_xcds, s, t);
 }
 
 // row_blocks = 32-row query blocks per workgroup (8: one per wavefront)
 hipError_t pa_launch_prefill(const AttnParams& p, uint32_t hd, uint32_t row_blocks, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t) {
   if (row_blocks != 8) return hipErrorNotSupported;
-  if (hd == 256) return launch_prefill_t<256, 1, 8>(p, col_groups, n_cu, s, t);
-  if (hd == 128) return launch_prefill_t<128, 1, 8>(p, col_groups, n_cu, s, t);
+  if (hd == 256) return launch_prefill_t<256, 8>(p, col_groups, n_cu, s, t);
+  if (hd == 128) return launch_prefill_t<128, 8>(p, col_groups, n_cu, s, t);
   return hipErrorNotSupported;
 }

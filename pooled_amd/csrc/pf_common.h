@@ -14,16 +14,13 @@ typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
 #define NEG_INF (-__builtin_inff())
 #define PF_TN 32                 // positions per step
-#ifndef PF_QR
-#define PF_QR 16                 // head_dim 256: k-steps of Q kept in registers (any others are parked in LDS)
-#endif
 #ifndef PF_KD
-#define PF_KD 2                  // K (and parked Q) fragments fetched this many k-steps ahead
+#define PF_KD 3                  // K fragments (two MFMAs each) fetched ahead
 #endif
 #ifndef PF_VD
-#define PF_VD 2                  // V^T fragments fetched this many MFMAs ahead
+#define PF_VD 3                  // V^T fragments (two MFMAs each) fetched ahead
 #endif
-#define PF_RESCALE_TH 8.0f       // log2 units
+#define PF_RESCALE_TH 8          // log2 units
 
 static __device__ inline h4 lds_read_tr16(const unsigned char* p) {
   hh4 t = __builtin_amdgcn_ds_read_tr16_b64_v4f16((hh4 __attribute__((address_space(3)))*)p);

@@ -193,3 +193,31 @@ def test_c5_prefill_128k_row_sample():
     got, ref, plan = _prefill(cfg, base, n, seed=0x5EED0005, max_seq=base + n, out_dtype=PA_OUT_F16, check_rows=rows)
     assert plan["kernel"] == 1 and plan["n_splits"] == 1
     assert_parity(got, ref, "C5 prefill 128K, column sample", tight=True)
+
+
+@pytest.mark.parametrize("shape,base,n,tile", [("qwen36_moe", 0, 40, 1), ("qwen36_moe", 900, 33, 1), ("qwen3_1p7b", 70, 300, 1), ("qwen38_27b", 5000, 64, 1)])
+@pytest.mark.parametrize("trend", ["up", "down", "jump", "late"])
+def test_prefill_reference_maxima(shape, base, n, tile, trend):
+    """Scores whose maximum rises by a few units a tile, falls, jumps by 60 in the middle of the context (exp2 of it is past the f16
+    range before the references are raised) or only behind the chunk's first columns (rows of a wave that end before the jump must not
+    notice): every row against the oracle, whole and split contexts."""
+    cfg = SHAPES[shape]
+    nH, nKV, hd = cfg["n_heads"], cfg["n_kv_heads"], cfg["head_dim"]
+    rng = np.random.default_rng(base + n)
+    rows = base + n
+    t = np.arange(rows)
+    level = {"up": t / 32 * 0.7 % 40, "down": 30 - 30 * t / rows, "jump": 60.0 * (t >= rows // 2), "late": 60.0 * (t >= base + n // 2)}[trend]
+    k = rng.standard_normal((rows, nKV, hd)).astype(np.float32) * 0.25
+    k[:, :, 0] = level[:, None]                                   # q's first value is sqrt(hd): it adds the level to every score
+    k16 = k.astype(np.float16).view(np.uint16)
+    v16 = rng.standard_normal((rows, nKV, hd)).astype(np.float16).view(np.uint16)
+    q = rng.standard_normal((n, nH, hd)).astype(np.float16).astype(np.float32)
+    q[:, :, 0] = hd ** 0.5
+    q16 = q.astype(np.float16).astype(np.float32)                 # f16 queries: the scores carry no rounding of q
+    ref = C.attention(q16, k16, v16, base, gate=None, rows=list(range(n)))
+    with PooledAttn(cfg, rows + 3, n_layers=1, max_cols=n) as pa:
+        pa.layer_alloc(0); pa.kv_write(0, 0, 0, k16); pa.kv_write(0, 1, 0, v16)
+        pa.set_prefill_tile(tile)
+        assert pa.plan("prefill", base, n)["kernel"] == 1
+        got = pa.run_attn("prefill", 0, q16, base)
+    assert_parity(got.astype(np.float32), ref, "maxima %s %s base %d" % (trend, shape, base))
