@@ -211,12 +211,15 @@ template <int HD> struct DecShape {
 // tile -- int8 -> f16 through the 0x6400 | (v + 128) bit pattern (= 1152 + v exactly), a packed subtract and a
 // packed multiply by the f16-rounded scale.  From there on (MFMA, softmax, merge) it is the f16 kernel.
 //
+// EX2 (a column-exact verify block on single-round splits): a workgroup takes two columns, a row block each, on the splits that are whole for
+// both -- the K/V tiles are loaded and staged once, everything behind them is done per block as the one-column decode does it, bit for bit.
+//
 // SR (single-round splits; one 16-row block, or two of a verify block): splits are one tile per wave (split_len = W x
 // 32); the product O^T = V^T P^T of a split is divided over the waves by output dims, see the code.  Without SR every wave
 // loops over its own tiles: contiguous splits of any length, or (AttnParams::tile_ilv) a kv head's tiles dealt round robin
 // to the waves of all its splits.
-template <int HD, int NB, int W, bool FUSED, bool GATHER, bool Q8, bool SR>
-__global__ __launch_bounds__(W * 64, ((NB == 1 && !GATHER && W <= 4) || (SR && NB == 2 && HD == 128) ? 2 : 1))
+template <int HD, int NB, int W, bool FUSED, bool GATHER, bool Q8, bool SR, bool EX2>
+__global__ __launch_bounds__(W * 64, ((NB == 1 && !GATHER && W <= 4) || (SR && NB == 2 && HD == 128) || EX2 ? 2 : 1))
 void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a_max_seq, uint32_t a_n_splits, uint32_t a_self_row,
                       uint32_t a_grid_x, const float* a_f_q_in, uint32_t a_group, uint32_t a_f_q_head_stride, AttnParams p_in) {
   // The leading arguments repeat fields of p_in: the first twelve dwords of a kernel's arguments are preloaded into
@@ -225,6 +228,7 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
   AttnParams p = p_in;
   p.k_cache = a_k_cache; p.base_pos = a_base_pos; p.max_seq = a_max_seq; p.n_splits = a_n_splits; p.self_row = a_self_row & 1u;
   const bool cols_adjacent = (a_self_row & 2u) != 0;                 // (rides in a preloaded argument: see the workgroup mapping below)
+  static_assert(!EX2 || (SR && NB == 2 && !FUSED && !GATHER), "two columns of a column-exact block: two row blocks of single-round splits");
   p.f_q_in = a_f_q_in; p.group = a_group; p.f_q_head_stride = a_f_q_head_stride;
   const uint32_t grid_x = a_grid_x;
   static_assert(!SR || NB == 1 || (NB == 2 && W == 4 && !FUSED && !GATHER), "single-round splits: one 16-row block, or two of a verify block");
@@ -233,8 +237,11 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
   static_assert(!Q8 || !GATHER, "int8 caches: no gather mode");
   typedef DecShape<HD> S;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  unsigned char* q_lds = smem;                                       // [16*NB][QROW]
-  unsigned char* stage_all = smem + 16 * NB * S::QROW;               // [W][STAGE]
+  // q rows [16*NB][QROW]: a region of their own, or (EX2: two workgroups of head_dim 256 a CU leave none) wave 0's staging region, read into
+  // registers before that wave's K tile goes there
+  unsigned char* q_lds = smem;
+  static_assert(!EX2 || 16 * NB * S::QROW <= S::STAGE, "the q rows fit a staging region");
+  unsigned char* stage_all = smem + (EX2 ? 0 : 16 * NB * S::QROW);   // [W][STAGE]
   float* mex = (float*)(stage_all + W * S::STAGE);                   // [W][16*NB]
   float* lex = mex + W * 16 * NB;                                    // [W][16*NB]
   float* sct = lex + W * 16 * NB;                                    // [W][16*NB]: the tile loop's merge, a wave's weight exp(m_w - M) per row
@@ -279,8 +286,21 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
   // G <= 64; a division by a run-time G is some thirty instructions, and the q loads' addresses wait for four of them a row block)
   const uint32_t g_magic = (65536u + G - 1u) / G;
   auto div_g = [&](uint32_t r) __attribute__((always_inline)) -> uint32_t { return (r * g_magic) >> 16; };
-  const uint32_t c0 = FUSED ? 0u : cg * p.cols_per_group;            // (the fused step serves one column)
-  const uint32_t ncl = FUSED ? 1u : min(p.cols_per_group, p.n_cols - c0);
+  uint32_t c0 = FUSED ? 0u : cg * p.cols_per_group;                  // (the fused step serves one column)
+  uint32_t ncl = FUSED ? 1u : min(p.cols_per_group, p.n_cols - c0);
+  // Two columns of a column-exact block: a row block each, which does what the one-column decode's row block does on the rows that
+  // both see -- the whole splits.  The split after those ends at another row for each: a workgroup a column, the second one's at index
+  // n_splits.  (Bit 2 of the self_row argument: the pass's last column has whole splits only, and is a group of its own.)
+  if constexpr (EX2) {
+    const uint32_t together = p.n_cols - ((a_self_row >> 2) & 1u);
+    c0 = min(c0, together);
+    ncl = c0 == together ? 1u : min(2u, together - c0);
+    const uint32_t whole = (p.base_pos + c0) / (W * TILE);
+    if (sp >= whole) {
+      if (sp - whole >= ncl) return;
+      c0 += sp - whole; ncl = 1; sp = whole;
+    }
+  }
   const uint32_t R = ncl * G;                                        // live rows (<= 16*NB)
   const uint32_t sel_base = GATHER ? c0 * p.sel_stride + 1 : 0;      // gather: first list entry of this column
   // rows visible to the group's last column (gather: the column's list length)
@@ -288,7 +308,7 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
   const uint32_t seq_max = GATHER ? min(p.sel[c0 * p.sel_stride], p.sel_max) : p.base_pos + c0 + ncl - p.self_row;
   // rows 8 .. 15 of the q tile hold the low halves of rows 0 .. 7 (q_lo_row): every one-column decode with G <= 8, and
   // blocks of at most eight stacked rows
-  const bool qsplit = NB == 1 && R <= 8;
+  const bool qsplit = (NB == 1 && R <= 8) || (EX2 && G <= 8);
   const uint32_t split_len = SR ? (uint32_t)(W * TILE) : p.split_len;   // single-round splits: one tile per wave
   // TILV (tile loop on a contiguous cache, p.tile_ilv): the tiles of a kv head are dealt round robin to the waves of
   // all its splits -- wave v of the n_splits x W takes tiles v, v + n_splits W, ... -- so the loads in flight on the chip
@@ -372,24 +392,33 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
 
   // the column's own K / V row, 4 dims a lane: loaded here (the pre-step wrote it), or made below by the fused pre-step
   const bool self_wave = self_wg && wave == 0;
-  h4 kx = {0, 0, 0, 0}, vx = {0, 0, 0, 0};
+  constexpr int SC = EX2 ? 2 : 1;
+  h4 kx[SC], vx[SC];
+#pragma unroll
+  for (int j = 0; j < SC; j++) { kx[j] = (h4){0, 0, 0, 0}; vx[j] = kx[j]; }
   if constexpr (!FUSED && !GATHER && !Q8) {
     if (self_wave) {
-      const size_t ro = (size_t)(p.base_pos + c0) * row_bytes + min(lane, (uint32_t)HD / 4 - 1) * 8;
-      kx = *(const h4*)(kbase + ro);
-      vx = *(const h4*)(vbase + ro);
+#pragma unroll
+      for (int j = 0; j < SC; j++) {
+        const size_t ro = (size_t)(p.base_pos + c0 + min((uint32_t)j, ncl - 1)) * row_bytes + min(lane, (uint32_t)HD / 4 - 1) * 8;
+        kx[j] = *(const h4*)(kbase + ro);
+        vx[j] = *(const h4*)(vbase + ro);
+      }
     }
   }
   if constexpr (Q8 && !FUSED) {         // int8 row: widened as the tile path widens it (exact integer x f16-rounded scale, one rounding)
     if (self_wave) {
       const uint32_t l4 = min(lane, (uint32_t)HD / 4 - 1);
-      const size_t ro = (size_t)(p.base_pos + c0) * HD + 4 * l4, so = ((size_t)(p.base_pos + c0) * S::SPR + l4 / 8) * 4;
+#pragma unroll
+      for (int j = 0; j < SC; j++) {
+      const size_t row = p.base_pos + c0 + min((uint32_t)j, ncl - 1), ro = row * HD + 4 * l4, so = (row * S::SPR + l4 / 8) * 4;
       const uint32_t kq = *(const uint32_t*)(kbase8 + ro), vq = *(const uint32_t*)(vbase8 + ro);
       const _Float16 ksc = (_Float16)*(const float*)(ksbase + so), vsc = (_Float16)*(const float*)(vsbase + so);
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        kx[i] = (_Float16)(int)(signed char)(kq >> (8 * i)) * ksc;
-        vx[i] = (_Float16)(int)(signed char)(vq >> (8 * i)) * vsc;
+        kx[j][i] = (_Float16)(int)(signed char)(kq >> (8 * i)) * ksc;
+        vx[j][i] = (_Float16)(int)(signed char)(vq >> (8 * i)) * vsc;
+      }
       }
     }
   }
@@ -449,9 +478,10 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
     for (int j = 0; j < QPT; j++) {
       const uint32_t e = tid + j * W * 64;
       const uint32_t r = e / (HD / 4), d4 = e % (HD / 4);
-      const uint32_t rc = min(qsplit && r >= 8 ? r - 8 : r, R - 1);  // padding rows copy the last live row (masked out later)
-      const uint32_t qc = div_g(rc);
-      qv[j] = *(const f4*)(p.q + (size_t)(c0 + qc) * p.q_stride + (size_t)(g * G + rc - qc * G) * HD + 4 * d4);
+      uint32_t rc = min(qsplit && r >= 8 ? r - 8 : r, R - 1);        // padding rows copy the last live row (masked out later)
+      uint32_t qc = div_g(rc), qh = rc - qc * G;
+      if (EX2) { rc = r & 15; qc = min(r >> 4, ncl - 1); qh = min(qsplit && rc >= 8 ? rc - 8 : rc, G - 1); }
+      qv[j] = *(const f4*)(p.q + (size_t)(c0 + qc) * p.q_stride + (size_t)(g * G + qh) * HD + 4 * d4);
     }
   }
   // Loads are unconditional: the caches carry TILE rows of padding past max_seq, so a tile that straddles the
@@ -547,16 +577,16 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
         const _Float16 ks16 = (_Float16)ksc, vs16 = (_Float16)vsc;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          kx[i] = (_Float16)(int)(signed char)(kw8 >> (8 * i)) * ks16;
-          vx[i] = (_Float16)(int)(signed char)(vw8 >> (8 * i)) * vs16;
+          kx[0][i] = (_Float16)(int)(signed char)(kw8 >> (8 * i)) * ks16;
+          vx[0][i] = (_Float16)(int)(signed char)(vw8 >> (8 * i)) * vs16;
         }
       } else if (lane < HD / 4) {
         const f4 v = *(const f4*)(xs + 4 * lane);
-        kx = (h4){ (_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3] };
-        vx = (h4){ (_Float16)xv4[0], (_Float16)xv4[1], (_Float16)xv4[2], (_Float16)xv4[3] };
+        kx[0] = (h4){ (_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3] };
+        vx[0] = (h4){ (_Float16)xv4[0], (_Float16)xv4[1], (_Float16)xv4[2], (_Float16)xv4[3] };
         const size_t ro = ((size_t)g * head_rows + p.base_pos) * HD + 4 * lane;
-        *(h4*)((_Float16*)const_cast<uint16_t*>(p.k_cache) + ro) = kx;
-        *(h4*)((_Float16*)const_cast<uint16_t*>(p.v_cache) + ro) = vx;
+        *(h4*)((_Float16*)const_cast<uint16_t*>(p.k_cache) + ro) = kx[0];
+        *(h4*)((_Float16*)const_cast<uint16_t*>(p.v_cache) + ro) = vx[0];
       }
       wave_lds_fence();
     }
@@ -566,7 +596,7 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
       const uint32_t e = tid + j * W * 64;
       const uint32_t r = e / (HD / 4), d4 = e % (HD / 4);
       const h4 hv = { (_Float16)qv[j][0], (_Float16)qv[j][1], (_Float16)qv[j][2], (_Float16)qv[j][3] };
-      *(h4*)(q_lds + r * S::QROW + d4 * 8) = qsplit && r >= 8 ? q_lo_row(qv[j], hv) : hv;
+      *(h4*)(q_lds + r * S::QROW + d4 * 8) = qsplit && (EX2 ? r & 15 : r) >= 8 ? q_lo_row(qv[j], hv) : hv;
     }
   }
   if (FUSED && !v_late) {
@@ -580,40 +610,53 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
   for (int nb = 0; nb < NB; nb++) {
     const uint32_t r = nb * 16 + ln;
     end_pos[nb] = r < R ? (GATHER ? seq_max : p.base_pos + c0 + div_g(r) + 1 - p.self_row) : 0u;
+    if (EX2) end_pos[nb] = ln < G && (uint32_t)nb < ncl ? p.base_pos + c0 + nb : 0u;
   }
   __syncthreads();
+  h8 qf[EX2 ? S::KS : 1][NB];
+  if constexpr (EX2) {
+#pragma unroll
+    for (int ks = 0; ks < S::KS; ks++)
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) qf[ks][nb] = *(const h8*)(q_lds + (nb * 16 + ln) * S::QROW + ks * 64 + kg * 16);
+    __syncthreads();                                                 // (wave 0's K tile goes there; its own-row scores below are in front of that)
+  }
   // ---- the column's own row as a partial of its own (slot = number of splits that hold rows): m = its score,
   // l = 1, O = its value row.  The scores run on the VALU over the f16 operands the MFMA path would see, f32 sums in a
   // fixed order; the work hides under the latency of the tile loads.  Decoding a token at a position that is a
   // multiple of the split length therefore streams whole tiles only.
   if (self_wave) {
     const uint32_t live_len = tilv ? (uint32_t)(W * TILE) : split_len;     // rows from one split's first row to the next one's
-    const uint32_t self_slot = min((seq_max + live_len - 1) / live_len, p.n_splits);
     const bool on = lane < HD / 4;
-    const f4 vxf = { (float)vx[0], (float)vx[1], (float)vx[2], (float)vx[3] };
+#pragma unroll
+    for (int j = 0; j < SC; j++) {
+    if (j > 0 && (uint32_t)j >= ncl) break;
+    const uint32_t self_slot = min(((SC == 1 ? seq_max : p.base_pos + c0 + j) + live_len - 1) / live_len, p.n_splits);
+    const f4 vxf = { (float)vx[j][0], (float)vx[j][1], (float)vx[j][2], (float)vx[j][3] };
     // No store inside the loop: while the chip streams, the memory pipeline accepts a store as slowly as a load, and
     // with a partial row and an (m, l) pair stored per head this one wave -- the last of the kernel to start on its tile
     // -- ran microseconds behind the rest and set the end of the kernel.  The G heads of a kv head share the value row, so
     // it is stored once, under the kv head's first head (the merge reads it there for every head), up front; lane r keeps
     // head r's score and the G (m, l) pairs leave in one store behind the loop.
-    const size_t slot0 = ((size_t)c0 * nH + g * G) * p.slots + self_slot;
+    const size_t slot0 = ((size_t)(c0 + j) * nH + g * G) * p.slots + self_slot;
     if (on) {
-      if (p.part_f16) *(h4*)((_Float16*)p.part_o + slot0 * HD + 4 * lane) = vx;
+      if (p.part_f16) *(h4*)((_Float16*)p.part_o + slot0 * HD + 4 * lane) = vx[j];
       else *(f4*)(p.part_o + slot0 * HD + 4 * lane) = vxf;
     }
     float dv = 0.f;
     for (uint32_t r = 0; r < G; r++) {                                 // one column: row r is head g * G + r
-      const h4 qv = *(const h4*)(q_lds + r * S::QROW + min(lane, (uint32_t)HD / 4 - 1) * 8);
+      const h4 qv = *(const h4*)(q_lds + (16 * j + r) * S::QROW + min(lane, (uint32_t)HD / 4 - 1) * 8);
       h4 ql = {0, 0, 0, 0};
-      if (qsplit) ql = *(const h4*)(q_lds + (r + 8) * S::QROW + min(lane, (uint32_t)HD / 4 - 1) * 8);
+      if (qsplit) ql = *(const h4*)(q_lds + (16 * j + r + 8) * S::QROW + min(lane, (uint32_t)HD / 4 - 1) * 8);
       float d = 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; i++) d = __builtin_fmaf((float)qv[i] + (float)ql[i], (float)kx[i], d);
+      for (int i = 0; i < 4; i++) d = __builtin_fmaf((float)qv[i] + (float)ql[i], (float)kx[j][i], d);
       if (!on) d = 0.f;
       d = wave_sum_f32(d);
       if (lane == r) dv = d;
     }
     if (lane < G) *(float2*)(p.part_ml + (slot0 + (size_t)lane * p.slots) * 2) = make_float2(dv * p.scale, 1.f);
+    }
   }
   if (!has_rows) return;
 
@@ -669,8 +712,10 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
       auto fetch = [&](int ks, int slot) __attribute__((always_inline)) {
         a0r[slot] = *(const h8*)(stage + ln * S::KROW + ks * 64 + kg * 16);
         a1r[slot] = *(const h8*)(stage + (16 + ln) * S::KROW + ks * 64 + kg * 16);
+        if constexpr (!EX2) {
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) br[slot][nb] = *(const h8*)(q_lds + (nb * 16 + ln) * S::QROW + ks * 64 + kg * 16);
+          for (int nb = 0; nb < NB; nb++) br[slot][nb] = *(const h8*)(q_lds + (nb * 16 + ln) * S::QROW + ks * 64 + kg * 16);
+        }
       };
 #pragma unroll
       for (int ks = 0; ks < FD; ks++) fetch(ks, ks);
@@ -679,7 +724,7 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
         const h8 a0 = a0r[ks % FD], a1 = a1r[ks % FD];
         h8 b[NB];
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) b[nb] = br[ks % FD][nb];
+        for (int nb = 0; nb < NB; nb++) { if constexpr (EX2) b[nb] = qf[ks][nb]; else b[nb] = br[ks % FD][nb]; }
         if (ks + FD < S::KS) fetch(ks + FD, ks % FD);
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) {
@@ -688,19 +733,21 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
         }
       }
 #pragma unroll
-      for (int ks = 0; ks < FD; ks++) __builtin_amdgcn_sched_group_barrier(0x100, 2 + NB, 0);
+      for (int ks = 0; ks < FD; ks++) __builtin_amdgcn_sched_group_barrier(0x100, EX2 ? 2 : 2 + NB, 0);
 #pragma unroll
       for (int ks = 0; ks < S::KS; ks++) {
-        if (ks + FD < S::KS) __builtin_amdgcn_sched_group_barrier(0x100, 2 + NB, 0);
+        if (ks + FD < S::KS) __builtin_amdgcn_sched_group_barrier(0x100, EX2 ? 2 : 2 + NB, 0);
         __builtin_amdgcn_sched_group_barrier(0x008, 2 * NB, 0);
       }
     }
-    if constexpr (NB == 1) {
+    if constexpr (NB == 1 || EX2) {
       if (qsplit) {                      // K q_lo^T sits in the lanes of rows 8 .. 15: rows 0 .. 7 take it from there
 #pragma unroll
-        for (int pb = 0; pb < 2; pb++)
+        for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-          for (int i = 0; i < 4; i++) s[pb][0][i] += row_ror<8>(s[pb][0][i]);
+          for (int pb = 0; pb < 2; pb++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) s[pb][nb][i] += row_ror<8>(s[pb][nb][i]);
       }
     }
     wave_lds_fence();
@@ -860,8 +907,8 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
             for (int j = 0; j < DBW; j++) o[j] += (dead ? (f4){0.f, 0.f, 0.f, 0.f} : pr[w2][j][nb]) * c;
           }
           const uint32_t r = nb * 16 + ln;
-          if (r < R) {
-            const uint32_t rc = div_g(r), col = c0 + rc, hq = g * G + r - rc * G;
+          if (EX2 ? ln < G && (uint32_t)nb < ncl : r < R) {
+            const uint32_t rc = EX2 ? (uint32_t)nb : div_g(r), col = c0 + rc, hq = g * G + (EX2 ? ln : r - rc * G);
             const size_t slot = ((size_t)col * nH + hq) * p.slots + sp;
             // f16 partials (|O| <= 128 rows x |v|: far inside the range; the merge adds them up in f32): half the bytes this
             // kernel writes at its very end and half of what the merge kernel waits for
@@ -1295,37 +1342,39 @@ __global__ __launch_bounds__(256) void pa_combine_wide_kernel(AttnParams p) {
   }
 }
 
-template <int HD, int NB, int W>
+template <int HD, int NB, int W, bool EX2>
 static constexpr size_t decode_lds_bytes() {
   typedef DecShape<HD> S;
   // q rows, the waves' staging regions, the (m, l) exchange and the merge's weight table, its two row tables, and the
   // P region of the single-round kernel with two row blocks
-  return 16 * NB * S::QROW + (size_t)W * S::STAGE + 3 * W * 16 * NB * sizeof(float) + 2 * 16 * NB * sizeof(uint32_t) + (NB == 2 && W == 4 ? (size_t)W * NB * 1024 : 0);
+  return (EX2 ? 0 : 16 * NB * S::QROW) + (size_t)W * S::STAGE + 3 * W * 16 * NB * sizeof(float) + 2 * 16 * NB * sizeof(uint32_t) + (NB == 2 && W == 4 ? (size_t)W * NB * 1024 : 0);
 }
 // the kernel's dynamic LDS limit, raised once per instantiation and device (at its first launch, or ahead of it by
 // pa_prepare_decode_step)
-template <int HD, int NB, int W, bool FUSED, bool GATHER, bool Q8, bool SR>
+template <int HD, int NB, int W, bool FUSED, bool GATHER, bool Q8, bool SR, bool EX2 = false>
 static hipError_t decode_lds_attr() {
   static PaPerDevice lds_set;
-  return pa_lds_limit(lds_set, (const void*)pa_decode_kernel<HD, NB, W, FUSED, GATHER, Q8, SR>, decode_lds_bytes<HD, NB, W>());
+  return pa_lds_limit(lds_set, (const void*)pa_decode_kernel<HD, NB, W, FUSED, GATHER, Q8, SR, EX2>, decode_lds_bytes<HD, NB, W, EX2>());
 }
 
-template <int HD, int NB, int W, bool FUSED, bool GATHER, bool Q8, bool SR>
+template <int HD, int NB, int W, bool FUSED, bool GATHER, bool Q8, bool SR, bool EX2 = false>
 static hipError_t launch_decode_k(const AttnParams& p, uint32_t col_groups, hipStream_t s, const PaTiming* t) {
-  const size_t lds = decode_lds_bytes<HD, NB, W>();
-  hipError_t e = decode_lds_attr<HD, NB, W, FUSED, GATHER, Q8, SR>();
+  const size_t lds = decode_lds_bytes<HD, NB, W, EX2>();
+  hipError_t e = decode_lds_attr<HD, NB, W, FUSED, GATHER, Q8, SR, EX2>();
   if (e != hipSuccess) return e;
   if (!SR && col_groups != (p.n_cols + p.cols_per_group - 1) / p.cols_per_group) return hipErrorInvalidValue;
-  const dim3 grid = SR ? dim3(p.n_splits, p.n_kv_heads, col_groups) : dim3((p.n_splits * p.n_kv_heads * col_groups + 7) / 8 * 8);
+  static_assert(!EX2 || 2 * decode_lds_bytes<HD, NB, W, EX2>() <= 160 * 1024, "two workgroups a CU");
+  // EX2: a workgroup more, for the second column's last split
+  const dim3 grid = SR ? dim3(p.n_splits + (EX2 ? 1 : 0), p.n_kv_heads, col_groups) : dim3((p.n_splits * p.n_kv_heads * col_groups + 7) / 8 * 8);
   AttnParams pk = p;
   {
     const uint64_t total = (uint64_t)p.n_splits * p.n_kv_heads * col_groups;
     auto magic = [&](uint32_t d) -> uint32_t { return d > 1 && total * d < (1ull << 32) ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; };
     pk.col_groups = col_groups; pk.ncg_magic = magic(col_groups); pk.ns_magic = magic(p.n_splits);
   }
-  // (bit 1 of the self_row argument: the columns of a column-exact block on adjacent dispatch ids of an XCD)
-  const uint32_t self_arg = p.self_row | (SR && p.exact_cols ? 2u : 0u);
-  PA_LAUNCH((pa_decode_kernel<HD, NB, W, FUSED, GATHER, Q8, SR>), grid, dim3(W * 64), lds, s, t, p.k_cache, p.base_pos, p.max_seq, p.n_splits, self_arg,
+  // (bit 1 of the self_row argument: the columns of a column-exact block on adjacent dispatch ids of an XCD; bit 2: its last column alone)
+  const uint32_t self_arg = p.self_row | (SR && p.exact_cols ? 2u : 0u) | (EX2 && p.exact_cols == 2 ? 4u : 0u);
+  PA_LAUNCH((pa_decode_kernel<HD, NB, W, FUSED, GATHER, Q8, SR, EX2>), grid, dim3(W * 64), lds, s, t, p.k_cache, p.base_pos, p.max_seq, p.n_splits, self_arg,
             (uint32_t)grid.x, p.f_q_in, p.group, p.f_q_head_stride, pk);
   return hipGetLastError();
 }
@@ -1338,6 +1387,7 @@ static hipError_t launch_decode_t(const AttnParams& p, uint32_t col_groups, hipS
     if (p.split_len == W * TILE) return launch_decode_k<HD, NB, W, FUSED, GATHER, Q8, true>(p, col_groups, s, t);
   }
   if constexpr (NB == 2 && W == 4 && !FUSED && !GATHER) {
+    if (p.exact_cols) return launch_decode_k<HD, NB, W, FUSED, GATHER, Q8, true, true>(p, col_groups, s, t);
     if (p.single_round2 && p.split_len == W * TILE) return launch_decode_k<HD, NB, W, FUSED, GATHER, Q8, true>(p, col_groups, s, t);
   }
   return launch_decode_k<HD, NB, W, FUSED, GATHER, Q8, false>(p, col_groups, s, t);

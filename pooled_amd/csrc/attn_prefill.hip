@@ -35,8 +35,8 @@
 //   * PAIRED (unsplit passes of one round whose chunk is a material part of the context, the rule at pairs_pay): waves 0-3 take a
 //     half block of columns from the front of the chunk, waves 4-7 the one as far from its back, so that every workgroup has the same
 //     work and the causal triangle of a chunk at the start of a prompt does not leave most CUs idle behind the last columns'
-//     workgroups (with one block of neighbouring columns a workgroup, 4096 columns from 0 of the MoE shape 225 us, paired 180 us: 128
-//     steps at the pace of one wave a SIMD, which is 0.72 of two waves').  Where half blocks would need a workgroup more than whole
+//     workgroups (with one block of neighbouring columns a workgroup, 4096 columns from 0 of the 16 / 2-head shape 190 us, paired 155 us: 128
+//     steps at the pace of one wave a SIMD, which is some 0.7 of two waves').  Where half blocks would need a workgroup more than whole
 //     ones, the blocks stay whole.
 //   * Unsplit passes of more workgroups than CUs keep whole blocks (halves that end apart run one wave a SIMD for a while: more work
 //     in all), dealt over the XCDs of a kv head in turn, the longest first.  In order of position, one XCD of a head had the front of the
@@ -429,14 +429,14 @@ static hipError_t launch_prefill_k(const AttnParams& p, uint32_t col_groups, uin
 
 // Whether an unsplit pass of one round is paired.  Pairing takes the wait for the longest block away (n_cols / 2 positions at
 // most) and pays for it in energy: every pair stages tiles up to its far half's end, and halves that end apart run one wave a SIMD
-// for a while.  At head_dim 256 a full chip runs at the power limit, so once the triangle is a small part of the context pairs are the
-// slower form; a chip that is not full holds its clock longer.  Measured (us, whole blocks / pairs): 256 workgroups, 4096 columns of
-// the 16 / 2-head shape at 0 262 / 225, at 8192 677 / 665, at 16384 1109 / 1108, at 64K 3803 / 3811, at 124K 7130 / 7162; 2650 columns of the
-// 24 / 4-head shape at 4096 409 / 402, at 8192 623 / 624, at 16384 1054 / 1070; 158 workgroups, 2500 columns of the first at 8192
-// 473 / 467, at 16384 778 / 768, at 32768 1421 / 1417, at 64K 2696 / 2707.  Head_dim 128 stays ahead (4096 columns at 28672 1039 / 1016).
+// for a while.  At head_dim 256 a full chip runs at the power limit, so once the triangle is a small part of the context pairs are at
+// most as fast.  Measured (us, whole blocks / pairs, with the pre-step): 256 workgroups, 4096 columns of the 16 / 2-head shape at 0 244 / 209, at 8192
+// 614 / 587, at 16384 979 / 965, at 32768 1748 / 1733, at 124K 6286 / 6269; 2650 columns of the 24 / 4-head shape at 4096 370 / 356, at 8192 555 / 551, at
+// 16384 927 / 929; 158 workgroups, 2500 columns of the first at 8192 456 / 440, at 16384 763 / 754, at 32768 1387 / 1386, at 64K 2618 / 2646.
+// Head_dim 128 stays ahead (4096 columns at 28672 920 / 888).
 template <int HD>
 static bool pairs_pay(const AttnParams& p, uint32_t total, uint32_t n_cu) {
-  return HD == 128 || (uint64_t)p.base_pos * total <= 3ull * p.n_cols * n_cu;
+  return HD == 128 || (uint64_t)p.base_pos * total <= 6ull * p.n_cols * n_cu;
 }
 
 template <int HD, int W>

@@ -590,14 +590,24 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
         p.q_stride = q_stride; p.gate_stride = gate_stride; p.out_stride = out_stride;
         p.n_heads = c.n_heads; p.n_kv_heads = c.n_kv_heads; p.group = c.n_heads / c.n_kv_heads;
         p.base_pos = base_pos + col; p.n_cols = run;
-        p.split_len = p0.split_len; p.n_splits = p0.n_splits; p.slots = p0.slots; p.cols_per_group = 1;
-        p.self_row = 1; p.part_f16 = plan_f16_partials(p0, 1); p.exact_cols = 1; p.tile_ilv = plan_tile_ilv(p0);
+        // On single-round plans a workgroup may take two columns (a row block each) of those splits that are whole for both: the columns of a
+        // run agree on them, but for a last one whose rows are whole splits.  Such a workgroup takes 1.3 - 1.5 times as long, so it pays where
+        // the chip holds them in fewer rounds, and not for a second round of few.  Measured (us a layer, one column / two, two workgroups a CU
+        // either way): 16 / 2-head shape at 12001, 4 columns (752 / 380 workgroups) 18.7 / 18.7, 8 (1504 / 760) 26.7 / 23.9, 15 42.2 / 36.4; at 30000, 2
+        // (940 / 472) 23.3 / 21.1, 8 57.2 / 46.5; at 20000, 3 (942 / 632) 21.7 / 23.8; 24 / 4-head shape at 12000, 8 46.3 / 37.3; 16 / 8-head shape at 6000,
+        // 2 (752 / 384) 13.1 / 15.0, 4 (1504 / 768) 17.1 / 15.9.
+        const bool alone = (base_pos + col + run - 1) % 128 == 0;
+        const uint32_t pairs = ceil_div(run - alone, 2) + alone, held = 2u * (uint32_t)ctx->n_cu;
+        const uint64_t wgs1 = (uint64_t)p0.n_splits * c.n_kv_heads * run, wgs2 = ((uint64_t)p0.n_splits + 1) * c.n_kv_heads * pairs;
+        const bool two = p0.split_len == 128 && wgs1 * 4 > held * 7ull && (wgs2 + held - 1) / held < (wgs1 + held - 1) / held;
+        p.split_len = p0.split_len; p.n_splits = p0.n_splits; p.slots = p0.slots; p.cols_per_group = two ? 2 : 1;
+        p.self_row = 1; p.part_f16 = plan_f16_partials(p0, 1); p.exact_cols = two && alone ? 2 : 1; p.tile_ilv = plan_tile_ilv(p0);
         p.max_seq = c.max_seq; p.out_f16 = out_dtype == PA_OUT_F16;
         p.scale = (float)(1.0 / std::sqrt((double)c.head_dim));
         p.gate_head_stride = c.head_dim;
         PaTiming tm, tm2;
         if ((rc = prof_pair(ctx, &tm))) return rc;
-        HIPCHK(ctx, pa_launch_decode(p, c.head_dim, 1, 4, run, ctx->stream, &tm));
+        HIPCHK(ctx, pa_launch_decode(p, c.head_dim, two ? 2 : 1, 4, two ? pairs : run, ctx->stream, &tm));
         if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;
         HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream, &tm2));
       }

@@ -61,7 +61,7 @@ struct AttnParams {
   // sel_max: the longest list the pass was sized for; a longer length word is read as sel_max (the list cannot run
   // into the next column's), a length of 0 gives a column of zeros
   const uint32_t* sel; uint32_t sel_stride, sel_max;
-  uint32_t exact_cols;                        // 1: a column-exact verify block in one launch: every column is a column group of its
+  uint32_t exact_cols;                        // 1 (2: and its last column alone, cols_per_group being two): a column-exact verify block in one launch: every column is a column group of its
                                               // own under the plan of a one-column decode (the merge must be the wavefront kernel)
   uint32_t col_groups, ncg_magic, ns_magic;   // tile loop (set by its launcher): the column groups of the pass and ceil(2^32 / d) for d = col_groups
                                               // and d = n_splits, so that the kernel maps its dispatch id to (column group, split, kv head) with

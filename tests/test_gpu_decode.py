@@ -234,6 +234,35 @@ def test_verify_exact_flag_gives_the_sequential_decodes_bits(shape, n_cols, base
             assert np.array_equal(single[0].view(np.uint32), multi[c].view(np.uint32)), "column %d differs from its decode" % c
 
 
+@pytest.mark.parametrize("shape,n_cols,base,more", [("qwen36_moe", 8, 9209, {}), ("qwen36_moe", 9, 9209, dict(kv_q8=True)), ("qwen38_27b", 15, 12000, {}),
+                                                    ("qwen38_27b", 7, 12154, dict(kv_q8=True)), ("qwen3_1p7b", 9, 6137, {}), ("qwen36_moe", 2, 30001, {}),
+                                                    ("qwen36_moe", 16, 16380, {}), ("qwen3_1p7b", 5, 7005, dict(n_heads=80, n_kv_heads=8))])
+def test_verify_exact_two_columns_a_workgroup(shape, n_cols, base, more):
+    """Column-exact blocks of more workgroups than the chip holds twice share their whole splits between two columns: odd and even
+    numbers of columns, a last column that ends with a whole split (9216, 12160, 6144, 16384 rows) alone or before a change of plan, f16 and f32
+    partials, more than eight heads a kv head, int8 caches.  Rows behind a column are infinite: no column may see them."""
+    cfg = dict(SHAPES[shape], verify_exact=True, **more)
+    rng = np.random.default_rng(base + n_cols)
+    L = base + n_cols
+    q = rng.standard_normal((n_cols, cfg["n_heads"], cfg["head_dim"]), dtype=np.float32)
+    with PooledAttn(cfg, L + 5, n_layers=1, max_cols=2048) as pa:
+        pa.layer_alloc(0)
+        kvd = pa.kv_dim
+        for r in range(0, L, 2048):
+            n = min(2048, L - r)
+            k, v = rng.standard_normal((2, n, kvd), dtype=np.float32)
+            if not cfg.get("kv_q8"):
+                v[max(0, base + 1 - r):] = np.inf
+            dk, dv = pa.to_device(k), pa.to_device(v)
+            pa.kv_store(0, dk, kvd, dv, kvd, r, n)
+            pa.sync()
+        multi = pa.run_attn("decode", 0, q, base)
+        assert np.isfinite(multi[0]).all()
+        for c in range(n_cols):
+            single = pa.run_attn("decode", 0, q[c:c + 1], base + c)
+            assert np.array_equal(single[0].view(np.uint32), multi[c].view(np.uint32)), "column %d differs from its decode" % c
+
+
 def test_decode_f16_output_and_strides():
     cfg = SHAPES["qwen36_moe"]
     rng = np.random.default_rng(14)

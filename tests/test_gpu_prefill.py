@@ -59,8 +59,8 @@ def test_prefill_paired_halves(shape, base, n):
 
 @pytest.mark.parametrize("base,n", [(3000, 1000), (3200, 1000), (3300, 1010), (9000, 1024)])
 def test_prefill_long_context_keeps_whole_blocks(base, n):
-    """At head_dim 256 an unsplit pass that fills the chip pairs half blocks only while base_pos x workgroups is within 3 x n_cols x
-    CUs (the first case on a 256-CU part); past that the blocks stay whole: either side of the line, a ragged last block."""
+    """At head_dim 256 an unsplit pass that fills the chip pairs half blocks only while base_pos x workgroups is within 6 x n_cols x
+    CUs (all but the last case on a 256-CU part); past that the blocks stay whole: either side of the line, a ragged last block."""
     cfg = dict(SHAPES["qwen36_moe"], n_heads=64, n_kv_heads=2)                      # 32 heads a kv head: blocks of eight columns
     rows = sorted(set(range(0, n, 50)) | set(range(5)) | set(range(n - 5, n)))
     got, ref, plan = _prefill(cfg, base, n, seed=base + n, check_rows=rows)
