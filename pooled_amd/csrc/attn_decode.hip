@@ -214,6 +214,9 @@ template <int HD> struct DecShape {
 // EX2 (a column-exact verify block on single-round splits): a workgroup takes two columns, a row block each, on the splits that are whole for
 // both -- the K/V tiles are loaded and staged once, everything behind them is done per block as the one-column decode does it, bit for bit.
 //
+// SR with eight waves (a one-column decode of at most 256 rows): the kv head's whole context in one workgroup, which also merges the column's own
+// row, normalises, gates and stores the output: no partials, no merge launch.
+//
 // SR (single-round splits; one 16-row block, or two of a verify block): splits are one tile per wave (split_len = W x
 // 32); the product O^T = V^T P^T of a split is divided over the waves by output dims, see the code.  Without SR every wave
 // loops over its own tiles: contiguous splits of any length, or (AttnParams::tile_ilv) a kv head's tiles dealt round robin
@@ -228,6 +231,7 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
   AttnParams p = p_in;
   p.k_cache = a_k_cache; p.base_pos = a_base_pos; p.max_seq = a_max_seq; p.n_splits = a_n_splits; p.self_row = a_self_row & 1u;
   const bool cols_adjacent = (a_self_row & 2u) != 0;                 // (rides in a preloaded argument: see the workgroup mapping below)
+  constexpr bool ONE = SR && NB == 1 && W == 8;                       // the whole context of a one-column decode
   static_assert(!EX2 || (SR && NB == 2 && !FUSED && !GATHER), "two columns of a column-exact block: two row blocks of single-round splits");
   p.f_q_in = a_f_q_in; p.group = a_group; p.f_q_head_stride = a_f_q_head_stride;
   const uint32_t grid_x = a_grid_x;
@@ -248,6 +252,8 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
   uint32_t* rowcol = (uint32_t*)(sct + W * 16 * NB);                 // [16*NB]: the column of a stacked row ...
   uint32_t* rowhq = rowcol + 16 * NB;                                // [16*NB]: ... and its query head (same merge)
   unsigned char* p_lds = (unsigned char*)(rowhq + 16 * NB);          // [W][NB][64 x 16 B]: the tiles' P, single-round kernel with two row blocks
+  float* own_s = sct;                                                // ONE: the own row's scores ...
+  _Float16* own_v = (_Float16*)(rowhq + 16 * NB);                    // ... and values, [HD]
 
   uint32_t bx = blockIdx.x, by = blockIdx.y, cg = blockIdx.z;
   if constexpr (SR && !FUSED && !GATHER) {
@@ -639,7 +645,8 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
     // it is stored once, under the kv head's first head (the merge reads it there for every head), up front; lane r keeps
     // head r's score and the G (m, l) pairs leave in one store behind the loop.
     const size_t slot0 = ((size_t)(c0 + j) * nH + g * G) * p.slots + self_slot;
-    if (on) {
+    if constexpr (ONE) { if (on) *(h4*)(own_v + 4 * lane) = vx[j]; }
+    else if (on) {
       if (p.part_f16) *(h4*)((_Float16*)p.part_o + slot0 * HD + 4 * lane) = vx[j];
       else *(f4*)(p.part_o + slot0 * HD + 4 * lane) = vxf;
     }
@@ -655,10 +662,11 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
       d = wave_sum_f32(d);
       if (lane == r) dv = d;
     }
-    if (lane < G) *(float2*)(p.part_ml + (slot0 + (size_t)lane * p.slots) * 2) = make_float2(dv * p.scale, 1.f);
+    if constexpr (ONE) { if (lane < G) own_s[lane] = dv * p.scale; }
+    else if (lane < G) *(float2*)(p.part_ml + (slot0 + (size_t)lane * p.slots) * 2) = make_float2(dv * p.scale, 1.f);
     }
   }
-  if (!has_rows) return;
+  if (!ONE && !has_rows) return;
 
   // The three staging / product steps of a tile, shared by the tile loop and the single-round path below.
   // stage_k: the K registers of the tile at position tp -> LDS (int8: widened), then the loads of the wave's next tile.
@@ -806,7 +814,7 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
     constexpr int DBW = S::DB / W;                                      // 16-dim output blocks per wave
     {
       const bool has_tile = wave < n_tiles;
-      const uint32_t tp = t_begin + min(wave, n_tiles - 1) * TILE;      // the tile this wave holds in registers
+      const uint32_t tp = t_begin + min(wave, ONE ? max(n_tiles, 1u) - 1 : n_tiles - 1) * TILE;      // the tile this wave holds in registers
       stage_k(tp, false, 0);
       f4 s[2][NB];
       qk(s);
@@ -887,12 +895,22 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
           if (st + VD < NS) __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
           __builtin_amdgcn_sched_group_barrier(0x008, NB, 1);
         }
+        // ONE: the gate of the wave's slice of a row, requested ahead of the sums
+        f4 gtv[ONE ? DBW : 1];
+        const uint32_t o_row = min(ln, G - 1);
+        if constexpr (ONE) {
+#pragma unroll
+          for (int j = 0; j < DBW; j++)
+            gtv[j] = p.gate ? *(const f4*)(p.gate + (size_t)c0 * p.gate_stride + (size_t)(g * G + o_row) * p.gate_head_stride + (wave * DBW + j) * 16 + 4 * kg) : (f4){0.f, 0.f, 0.f, 0.f};
+        }
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) {
           // a wave without a tile staged stale rows: its m is -inf, and its products must not reach O even as 0 x NaN
           float mw[W], lw[W], M = NEG_INF;
 #pragma unroll
           for (int w2 = 0; w2 < W; w2++) { mw[w2] = mex[w2 * 16 * NB + nb * 16 + ln]; lw[w2] = lex[w2 * 16 * NB + nb * 16 + ln]; M = fmaxf(M, mw[w2]); }
+          const float own = ONE ? own_s[o_row] : NEG_INF;
+          if constexpr (ONE) M = fmaxf(M, own);
           const float m_safe = M == NEG_INF ? 0.f : M;
           float Lr = 0.f;
           f4 o[DBW];
@@ -905,6 +923,28 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
             Lr += lw[w2] * c;
 #pragma unroll
             for (int j = 0; j < DBW; j++) o[j] += (dead ? (f4){0.f, 0.f, 0.f, 0.f} : pr[w2][j][nb]) * c;
+          }
+          if constexpr (ONE) {
+            const float c = __expf(own - m_safe);
+            Lr += c;
+            const float inv = __builtin_amdgcn_rcpf(Lr);               // (v_rcp_f32, 1 ulp, as in the merge kernels)
+#pragma unroll
+            for (int j = 0; j < DBW; j++) {
+              const uint32_t d = (wave * DBW + j) * 16 + 4 * kg;
+              const h4 v = *(const h4*)(own_v + d);
+              f4 r;
+#pragma unroll
+              for (int i = 0; i < 4; i++) {
+                r[i] = (o[j][i] + (float)v[i] * c) * inv;
+                if (p.gate) r[i] *= __builtin_amdgcn_rcpf(1.f + __expf(-gtv[j][i]));
+              }
+              if (ln < G) {
+                const size_t at = (size_t)c0 * p.out_stride + (size_t)(g * G + ln) * HD + d;
+                if (p.out_f16) *(h4*)((_Float16*)p.out + at) = (h4){ (_Float16)r[0], (_Float16)r[1], (_Float16)r[2], (_Float16)r[3] };
+                else *(f4*)((float*)p.out + at) = r;
+              }
+            }
+            return;
           }
           const uint32_t r = nb * 16 + ln;
           if (EX2 ? ln < G && (uint32_t)nb < ncl : r < R) {
@@ -1347,7 +1387,7 @@ static constexpr size_t decode_lds_bytes() {
   typedef DecShape<HD> S;
   // q rows, the waves' staging regions, the (m, l) exchange and the merge's weight table, its two row tables, and the
   // P region of the single-round kernel with two row blocks
-  return (EX2 ? 0 : 16 * NB * S::QROW) + (size_t)W * S::STAGE + 3 * W * 16 * NB * sizeof(float) + 2 * 16 * NB * sizeof(uint32_t) + (NB == 2 && W == 4 ? (size_t)W * NB * 1024 : 0);
+  return (EX2 ? 0 : 16 * NB * S::QROW) + (size_t)W * S::STAGE + 3 * W * 16 * NB * sizeof(float) + 2 * 16 * NB * sizeof(uint32_t) + (NB == 2 && W == 4 ? (size_t)W * NB * 1024 : 0) + (NB == 1 && W == 8 ? HD * 2 : 0);
 }
 // the kernel's dynamic LDS limit, raised once per instantiation and device (at its first launch, or ahead of it by
 // pa_prepare_decode_step)
@@ -1398,6 +1438,7 @@ static hipError_t launch_decode_hd(const AttnParams& p, uint32_t nb, uint32_t wa
   // eight waves: the one-launch path for small chunks at head_dim 128 with two row blocks (its 250 registers a wave
   // leave room for two waves a SIMD, and a tile's softmax and LDS work is what the loop waits for)
   if (waves == 8) {
+    if (nb == 1 && p.direct_out) return p.k_scale ? launch_decode_k<HD, 1, 8, false, false, true, true>(p, col_groups, s, t) : launch_decode_k<HD, 1, 8, false, false, false, true>(p, col_groups, s, t);
     if constexpr (HD == 128) { if (nb == 2 && !p.k_scale) return launch_decode_t<HD, 2, 8, false>(p, col_groups, s, t); }
     return hipErrorInvalidValue;
   }
@@ -1428,6 +1469,12 @@ hipError_t pa_launch_decode(const AttnParams& p, uint32_t hd, uint32_t nb, uint3
 
 hipError_t pa_launch_decode_step(const AttnParams& p, uint32_t hd, hipStream_t s, const PaTiming* t) {
   if (!p.f_q_in || p.n_cols != 1 || p.group > 16 || !p.self_row) return hipErrorInvalidValue;
+  if (p.direct_out) {                             // at most 256 rows: the whole context in one workgroup
+    if (p.split_len != 8 * TILE) return hipErrorInvalidValue;
+    if (hd == 256) return p.k_scale ? launch_decode_k<256, 1, 8, true, false, true, true>(p, 1, s, t) : launch_decode_k<256, 1, 8, true, false, false, true>(p, 1, s, t);
+    if (hd == 128) return p.k_scale ? launch_decode_k<128, 1, 8, true, false, true, true>(p, 1, s, t) : launch_decode_k<128, 1, 8, true, false, false, true>(p, 1, s, t);
+    return hipErrorInvalidValue;
+  }
   if (p.k_scale) {                                // int8 caches
     if (hd == 256) return launch_decode_t<256, 1, 4, true, false, true>(p, 1, s, t);
     if (hd == 128) return launch_decode_t<128, 1, 4, true, false, true>(p, 1, s, t);
@@ -1444,9 +1491,11 @@ hipError_t pa_prepare_decode_step(uint32_t hd, bool q8) {
   if (hd == 256) {
     e = q8 ? decode_lds_attr<256, 1, 4, true, false, true, true>() : decode_lds_attr<256, 1, 4, true, false, false, true>();
     if (e == hipSuccess) e = q8 ? decode_lds_attr<256, 1, 4, true, false, true, false>() : decode_lds_attr<256, 1, 4, true, false, false, false>();
+    if (e == hipSuccess) e = q8 ? decode_lds_attr<256, 1, 8, true, false, true, true>() : decode_lds_attr<256, 1, 8, true, false, false, true>();
   } else if (hd == 128) {
     e = q8 ? decode_lds_attr<128, 1, 4, true, false, true, true>() : decode_lds_attr<128, 1, 4, true, false, false, true>();
     if (e == hipSuccess) e = q8 ? decode_lds_attr<128, 1, 4, true, false, true, false>() : decode_lds_attr<128, 1, 4, true, false, false, false>();
+    if (e == hipSuccess) e = q8 ? decode_lds_attr<128, 1, 8, true, false, true, true>() : decode_lds_attr<128, 1, 8, true, false, false, true>();
   }
   return e;
 }

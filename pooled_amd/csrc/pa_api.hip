@@ -338,6 +338,8 @@ static bool plan_single_round2(const pa_plan& pl) {
 static uint32_t plan_tile_ilv(const pa_plan& pl) {
   return pl.kernel == 0 && pl.split_len != 32 * pl.waves && pl.n_splits > 1 ? 32 * pl.waves : 0;
 }
+// a one-column decode of at most 256 rows: one workgroup a kv head, which writes the output itself
+static bool plan_one_wg(const pa_plan& pl) { return plan_self_row(pl) && pl.row_blocks == 1 && pl.waves == 8 && pl.n_splits == 1 && pl.split_len == 256; }
 #define PA_F16_PARTIALS_MIN_SPLITS 64u
 static bool plan_f16_partials(const pa_plan& pl, uint32_t n_cols) {
   return pl.kernel == 0 && pl.row_blocks == 1 && pl.split_len == 32 * pl.waves && n_cols < 16 && pl.n_splits >= PA_F16_PARTIALS_MIN_SPLITS;
@@ -373,8 +375,14 @@ static int plan_decode(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa
   const uint32_t occ = nb == 1 ? 2 : 1;
   const uint32_t target = ctx->decode_splits_override ? ctx->decode_splits_override
                                                       : std::max(1u, (occ * (uint32_t)ctx->n_cu) / (c.n_kv_heads * groups));
-  uint32_t sl, ns;
-  if (one_split || ctx->decode_splits_override) {
+  uint32_t sl, ns, waves = W;
+  if (self && nb == 1 && !one_split && !ctx->decode_splits_override && seq_max <= 256) {
+    // A token over so few rows: one workgroup of eight waves a kv head, a tile a wave, which finishes the output itself.  The merge launch that it
+    // saves (2.5 us) is more than the second workgroup of a kv head would bring: us a step, two launches / one, dense hd-128 shape at 20, 130 and
+    // 250 rows 7.5 / 5.9, 7.4 / 5.8, 7.4 / 6.0, MoE shape 9.5 / 8.2, 9.2 / 8.3, 9.1 / 8.1, 27B shape 9.5 / 8.1, 9.5 / 8.3, 9.3 / 8.1.  (Eight tiles are what a
+    // CU's LDS holds at hd 256.)
+    waves = 8; sl = 256; ns = 1;
+  } else if (one_split || ctx->decode_splits_override) {
     // a given number of splits (a tuning override; its splits are contiguous ranges, the last one open-ended), or one
     const uint32_t tpw = one_split ? std::max(ceil_div(tiles, W), 1u) : std::max(ceil_div(tiles, target * W), 1u);
     sl = 32 * W * tpw; ns = ceil_div(seq_max, sl);
@@ -408,7 +416,7 @@ static int plan_decode(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa
     sl = 32 * W * tpw;
   }
   pl->kernel = 0; pl->split_len = sl; pl->n_splits = ns;
-  pl->col_groups = groups; pl->cols_per_group = cw; pl->waves = W; pl->row_blocks = nb; pl->slots = pl->n_splits + self;
+  pl->col_groups = groups; pl->cols_per_group = cw; pl->waves = waves; pl->row_blocks = nb; pl->slots = pl->n_splits + self;
   return PA_OK;
 }
 
@@ -563,12 +571,12 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
     // The plan moves at few positions (a split more on the single-round kernel every 128 rows, a tile per wave more
     // on the tile loop every few thousand), so a block is one run, or two.
     auto one_col_plan = [&](uint32_t pos, pa_plan* pl) -> bool {
-      return plan_decode(ctx, pos, 1, pl, true) == PA_OK && pl->kernel == 0 && pl->row_blocks == 1 && pl->waves == 4 && plan_self_row(*pl) &&
+      return plan_decode(ctx, pos, 1, pl, true) == PA_OK && pl->kernel == 0 && pl->row_blocks == 1 && (pl->waves == 4 || plan_one_wg(*pl)) && plan_self_row(*pl) &&
              pl->slots <= 8192;
     };
     // (round-robin tiles: the split length is nominal, the splits are the same whenever their number is)
     auto same_plan = [&](const pa_plan& a, const pa_plan& b) -> bool {
-      return (a.split_len == b.split_len || (plan_tile_ilv(a) && plan_tile_ilv(b))) && a.n_splits == b.n_splits && a.slots == b.slots;
+      return (a.split_len == b.split_len || (plan_tile_ilv(a) && plan_tile_ilv(b))) && a.n_splits == b.n_splits && a.slots == b.slots && a.waves == b.waves;
     };
     const size_t osz = out_dtype == PA_OUT_F16 ? 2 : 4;
     for (uint32_t col = 0; col < n_cols;) {
@@ -582,7 +590,8 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
       if (run == 1) {                 // a column on its own: the one-column decode itself
         if ((rc = attn_common(ctx, who, 0, layer, q_c, q_stride, gate_c, gate_stride, base_pos + col, 1, out_c, out_stride, out_dtype))) return rc;
       } else {
-        if ((rc = ensure_partials(ctx, run, p0.slots))) return rc;
+        const bool one = plan_one_wg(p0);
+        if (!one && (rc = ensure_partials(ctx, run, p0.slots))) return rc;
         AttnParams p; memset(&p, 0, sizeof p);
         p.q = q_c; p.gate = gate_c; p.k_cache = ctx->layers[layer].k; p.v_cache = ctx->layers[layer].v;
         p.k_scale = ctx->layers[layer].ks; p.v_scale = ctx->layers[layer].vs;
@@ -607,9 +616,12 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
         p.gate_head_stride = c.head_dim;
         PaTiming tm, tm2;
         if ((rc = prof_pair(ctx, &tm))) return rc;
-        HIPCHK(ctx, pa_launch_decode(p, c.head_dim, two ? 2 : 1, 4, two ? pairs : run, ctx->stream, &tm));
-        if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;
-        HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream, &tm2));
+        p.direct_out = one;
+        HIPCHK(ctx, pa_launch_decode(p, c.head_dim, two ? 2 : 1, p0.waves, two ? pairs : run, ctx->stream, &tm));
+        if (!one) {
+          if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;
+          HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream, &tm2));
+        }
       }
       col += run;
     }
@@ -621,7 +633,7 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
   if (pl.slots > 8192) return fail(ctx, PA_ERR_UNSUPPORTED, std::string(who) + ": too many splits");
   // one split and no own-row partial: the kernel writes the output itself (the prefill kernel, or the split-K kernel's
   // tile loop: its single-round form always leaves a partial)
-  const bool direct = pl.n_splits == 1 && !plan_self_row(pl) && (pl.kernel == 1 || pl.split_len != 32 * pl.waves || pl.row_blocks > 1);
+  const bool direct = plan_one_wg(pl) || (pl.n_splits == 1 && !plan_self_row(pl) && (pl.kernel == 1 || pl.split_len != 32 * pl.waves || pl.row_blocks > 1));
   if (!direct && (rc = ensure_partials(ctx, n_cols, pl.slots))) return rc;
   AttnParams p; memset(&p, 0, sizeof p);
   p.q = d_q; p.gate = d_gate; p.k_cache = ctx->layers[layer].k; p.v_cache = ctx->layers[layer].v;
@@ -699,7 +711,8 @@ static int decode_step_common(pa_ctx* ctx, const char* who, bool static_scratch,
   rc = plan_decode(ctx, pos, 1, &pl, true);
   if (rc) return fail(ctx, rc, std::string(who) + ": shape outside the gfx950 table");
   if (pl.slots > 8192) return fail(ctx, PA_ERR_UNSUPPORTED, std::string(who) + ": too many splits");
-  if (pl.row_blocks != 1 || pl.waves != 4 || pl.col_groups != 1 || !plan_self_row(pl)) return fail(ctx, PA_ERR_UNSUPPORTED, std::string(who) + ": plan is not a one-block decode");
+  const bool one = plan_one_wg(pl);
+  if (pl.row_blocks != 1 || (pl.waves != 4 && !one) || pl.col_groups != 1 || !plan_self_row(pl)) return fail(ctx, PA_ERR_UNSUPPORTED, std::string(who) + ": plan is not a one-block decode");
   float* part_o = nullptr; float* part_ml = nullptr;
   if (static_scratch) {
     const size_t need_o = ((size_t)c.n_heads * pl.slots * c.head_dim * sizeof(float) + 255) & ~(size_t)255;
@@ -719,7 +732,7 @@ static int decode_step_common(pa_ctx* ctx, const char* who, bool static_scratch,
   p.n_heads = c.n_heads; p.n_kv_heads = c.n_kv_heads; p.group = c.n_heads / c.n_kv_heads;
   p.base_pos = pos; p.n_cols = 1;
   p.split_len = pl.split_len; p.n_splits = pl.n_splits; p.slots = pl.slots; p.cols_per_group = pl.cols_per_group;
-  p.self_row = 1; p.part_f16 = plan_f16_partials(pl, 1); p.tile_ilv = plan_tile_ilv(pl);
+  p.self_row = 1; p.part_f16 = plan_f16_partials(pl, 1); p.tile_ilv = plan_tile_ilv(pl); p.direct_out = one;
   p.max_seq = c.max_seq; p.out_f16 = out_dtype == PA_OUT_F16;
   p.scale = (float)(1.0 / std::sqrt((double)c.head_dim));
   // the pre-step inputs; the gate is read in place from the interleaved [q | gate] heads
@@ -732,6 +745,7 @@ static int decode_step_common(pa_ctx* ctx, const char* who, bool static_scratch,
   PaTiming tm;                                        // profiling may create events: not on the allocation-free path
   if (!static_scratch && (rc = prof_pair(ctx, &tm))) return rc;
   HIPCHK(ctx, pa_launch_decode_step(p, c.head_dim, ctx->stream, &tm));
+  if (one) return PA_OK;
   PaTiming tm2;
   if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;
   HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream, &tm2));

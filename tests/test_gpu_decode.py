@@ -236,11 +236,13 @@ def test_verify_exact_flag_gives_the_sequential_decodes_bits(shape, n_cols, base
 
 @pytest.mark.parametrize("shape,n_cols,base,more", [("qwen36_moe", 8, 9209, {}), ("qwen36_moe", 9, 9209, dict(kv_q8=True)), ("qwen38_27b", 15, 12000, {}),
                                                     ("qwen38_27b", 7, 12154, dict(kv_q8=True)), ("qwen3_1p7b", 9, 6137, {}), ("qwen36_moe", 2, 30001, {}),
-                                                    ("qwen36_moe", 16, 16380, {}), ("qwen3_1p7b", 5, 7005, dict(n_heads=80, n_kv_heads=8))])
+                                                    ("qwen36_moe", 16, 16380, {}), ("qwen3_1p7b", 5, 7005, dict(n_heads=80, n_kv_heads=8)),
+                                                    ("qwen36_moe", 10, 250, {}), ("qwen3_1p7b", 7, 253, dict(kv_q8=True))])
 def test_verify_exact_two_columns_a_workgroup(shape, n_cols, base, more):
     """Column-exact blocks of more workgroups than the chip holds twice share their whole splits between two columns: odd and even
     numbers of columns, a last column that ends with a whole split (9216, 12160, 6144, 16384 rows) alone or before a change of plan, f16 and f32
-    partials, more than eight heads a kv head, int8 caches.  Rows behind a column are infinite: no column may see them."""
+    partials, more than eight heads a kv head, int8 caches; and short blocks of one workgroup a column and kv head up to 256 rows, splits past
+    them.  Rows behind a column are infinite: no column may see them."""
     cfg = dict(SHAPES[shape], verify_exact=True, **more)
     rng = np.random.default_rng(base + n_cols)
     L = base + n_cols

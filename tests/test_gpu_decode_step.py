@@ -52,6 +52,30 @@ def test_decode_step_matches_oracle_and_unfused(shape, pos):
     assert np.array_equal(got.view(np.uint32), unf[0].view(np.uint32)), "fused output differs from pa_glue_kv + pa_attn_decode"
 
 
+@pytest.mark.parametrize("shape,more", [("qwen36_moe", {}), ("qwen38_27b", {}), ("qwen3_1p7b", {}), ("qwen3_1p7b", dict(n_heads=13, n_kv_heads=1, gate=True)),
+                                        ("qwen36_moe", dict(n_kv_heads=1, gate=False))])
+def test_decode_step_in_one_workgroup_and_past_it(shape, more):
+    """Up to 256 streamed rows a kv head's context is one workgroup, which merges the own row and writes the output itself; from 257 on it is
+    splits and a merge: either side of the line, whole and partial tiles, waves without one; the unfused pair's bits; rows behind the token NaN."""
+    cfg = dict(SHAPES[shape], **more)
+    for pos in (0, 1, 32, 33, 224, 255, 256, 257):
+        d, k16, v16, K, V, ref, max_seq = _case(cfg, pos, seed=pos + 11)
+        with PooledAttn(cfg, max_seq, n_layers=1, max_cols=1) as pa:
+            pa.layer_alloc(0)
+            for which, a in ((0, k16), (1, v16)):
+                a = a.copy(); a[pos:] = np.uint16(0x7E00)
+                pa.kv_write(0, which, 0, a)
+            pl = pa.plan("decode", pos, 1)
+            assert (pl["waves"], pl["n_splits"]) == ((8, 1) if pos <= 256 else (4, 3)), pl
+            got = pa.run_decode_step(0, d["qraw"][0], d["kraw"][0], d["vraw"][0], d["qw"], d["kw"], pos)
+            half = pa.run_decode_step(0, d["qraw"][0], d["kraw"][0], d["vraw"][0], d["qw"], d["kw"], pos, out_dtype=PA_OUT_F16)
+            pa.run_glue_kv(0, d["qraw"], d["kraw"], d["vraw"], d["qw"], d["kw"], pos)
+            unf = pa.run_attn("decode", 0, pa.read_q_buffer(1), pos, gate=pa.read_gate_buffer(1) if cfg["gate"] else None)
+        assert_parity(got[None], ref, "%s pos %d" % (shape, pos))
+        assert np.array_equal(got.view(np.uint32), unf[0].view(np.uint32))
+        assert np.array_equal(half, got.astype(np.float16))
+
+
 def test_decode_step_f16_out_and_no_norm():
     cfg = dict(SHAPES["qwen3_1p7b"], qk_norm=False)
     pos = 600

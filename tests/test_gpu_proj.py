@@ -512,3 +512,41 @@ def test_projection_that_ends_with_the_pre_step_equals_the_two(heads, dim, n, ti
         assert np.isfinite(a).all() and np.array_equal(a, b)
     for a, b in zip(*caches):
         assert np.array_equal(np.asarray(a), np.asarray(b))
+
+
+@pytest.mark.parametrize("shape,more,kind", [("qwen3_1p7b", {}, PA_W_Q8_0), ("qwen36_moe", {}, PA_W_Q4_0), ("qwen36_moe", dict(kv_q8=True), PA_W_Q8_0),
+                                             ("qwen3_1p7b", dict(gate=True, n_heads=10, n_kv_heads=2), PA_W_F32), ("qwen36_moe", dict(n_heads=13, n_kv_heads=13, gate=False), PA_W_Q4_0),
+                                             ("qwen38_27b", {}, PA_W_Q4_0)])
+@pytest.mark.parametrize("dim", [64, 2080])
+def test_layer_decode_equals_its_stages(shape, more, kind, dim):
+    """The layer call on short contexts, one workgroup a kv head up to 256 streamed rows and splits past them: the bits of pa_gemv_norm,
+    pa_attn_decode_step and pa_gemv, with no streamed row, one, a whole number of tiles and of splits, one row more."""
+    cfg = dict(SHAPES[shape], **more)
+    nH, nKV, hd = cfg["n_heads"], cfg["n_kv_heads"], cfg["head_dim"]
+    qd, kvd = nH * hd, nKV * hd
+    q_rows = qd * (2 if cfg["gate"] else 1)
+    rows = q_rows + 2 * kvd
+    rng = np.random.default_rng(dim + qd)
+    w_qkv, s_qkv = _weights(kind, rows, dim, rng, scale=0.05)
+    w_o, s_o = _weights(kind, dim, qd, rng, scale=0.01)
+    nw = (1 + 0.1 * rng.standard_normal(dim)).astype(np.float32)
+    hw = (1 + 0.1 * rng.standard_normal(hd)).astype(np.float32)
+    x = rng.standard_normal(dim).astype(np.float32)
+    with PooledAttn(cfg, 640, n_layers=2, max_cols=640) as pa:
+        wq = pa.weight(kind, w_qkv, s_qkv); wo = pa.weight(kind, w_o, s_o)
+        dnw = pa.to_device(nw); dhw = pa.to_device(hw)
+        kraw, vraw = (pa.to_device(rng.standard_normal((640, kvd)).astype(np.float32)) for _ in range(2))
+        dqkv = pa.alloc(rows * 4); dat = pa.alloc(qd * 4)
+        for layer in (0, 1):
+            pa.layer_alloc(layer); pa.kv_store(layer, kraw, kvd, vraw, kvd, 0, 640)
+        for splits in (0, 3):                                         # 3: contiguous splits of several tiles a wave
+            pa.set_decode_splits(splits)
+            for pos in (0, 1, 127, 128, 129, 255, 256, 257, 384, 513, 639):
+                dx, dy = pa.to_device(x), pa.to_device(x)
+                pa.attn_layer_decode(0, wq, wo, dnw, dhw, dhw, dx, pos)
+                pa.gemv_norm(wq, dy, dnw, dqkv)
+                pa.L.pa_attn_decode_step(pa.ctx, 1, dqkv.ptr, dqkv.ptr + q_rows * 4, dqkv.ptr + (q_rows + kvd) * 4, dhw.ptr, dhw.ptr, pos, dat.ptr, 0)
+                pa.gemv(wo, dat, dy, acc=True)
+                pa.sync()
+                a, b = dx.download(np.float32, dim), dy.download(np.float32, dim)
+                assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32)), "pos %d splits %d" % (pos, splits)
