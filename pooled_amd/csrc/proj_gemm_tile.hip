@@ -8,14 +8,15 @@
 //   * both operands go to LDS by LDS-direct loads (no staging registers): K in stages of 32 KG, S buffers, so S - 1 stages
 //     are in flight.  Activation rows are staged with the 16-byte chunk order XORed by the row (conflict-free
 //     ds_read_b128 fragments: SQ_LDS_BANK_CONFLICT = 0), the weights as the 1 KB fragments they are kept in;
-//   * one barrier a stage, in the MIDDLE of its products: a stage is two k-steps a wave; the fragments of the next k-step are
+//   * one barrier a stage, in the MIDDLE of its products: a stage is two k-steps of 16 a wave, or, where a wave holds whole sums (KG = 1,
+//     the shapes of the power-limited sizes), one of 32 on 16 x 16 x 32 products (gt_whole_k); the next fragments are
 //     read, and the stage's loads issued, one at a time between the MFMAs, so that behind the barrier a wave's next MFMA
 //     has its operands.  (All reads and loads in front of the MFMAs: 8 % slower; the order left to the compiler: every
 //     k-step waits out its own LDS reads.)
 //   * a tile shape is picked per call, by the rule at pa_pick_tile.
 //
-// What bounds it: on full rounds of the chip the MFMA rate the power limit allows and the rounds' own ends (4096 columns:
-// 14336 x 5120 1090 - 1130 TFLOP/s, 9216 x 2048 1000); on one round or less the LDS-direct loads' latency (a tile's 96 - 120 KB
+// What bounds it: on full rounds of the chip the MFMA rate the power limit allows and the rounds' own ends (4096 columns, on 32 x 32 x 16
+// products: 14336 x 5120 1090 - 1130 TFLOP/s, 9216 x 2048 1000; the 16 x 16 x 32 ones are some 8 % faster there); on one round or less the LDS-direct loads' latency (a tile's 96 - 120 KB
 // in flight a CU).  Measured against the kernel it replaced (128 columns x 256 / 384 / 512 rows, four waves, weight fragments
 // from memory straight to registers) and the 64 x 64 kernel, Q8_0, five weights in rotation: 777 columns of 5120 x 6144 100 -> 64 us, of
 // 14336 x 5120 143 -> 133, of 9216 x 2048 59 -> 36; 2048 columns of 2048 x 4096 76 -> 40; 512 of 14336 x 5120 141 -> 92, of 4096 x 2048
@@ -195,6 +196,131 @@ static __device__ inline void finish_heads(const GlueParams& g, unsigned char* l
   }
 }
 
+// The main loop of the shapes whose waves each hold whole sums (KG = 1), on 16 x 16 x 32 products: at the power limit they run faster than 32 x 32 x 16
+// ones (half the accumulator traffic a product), and give the same bits.  Layer pass, 32 x 32 x 16 / so (us a layer): 4096 columns of the gated 16 / 2-head
+// shape 430 / 408, 2048 of it 231 / 226, 2048 of the 24 / 4-head shape 534 / 510; one round of few workgroups (777 of that shape) 297 / 297.  A stage is one k-step of 32: the products with the first half of a wave's column blocks, the barrier,
+// those with the second half; a fragment is read as soon as the products with the one in its registers are out, so a stage holds no more
+// fragments than the two k-steps of 16 did.  Weights are the first operand: a lane holds four consecutive rows of a column.
+template <int WM, int WN, int TM, int TN, int S, int EPI, int LPW, class Issue>
+static __device__ __attribute__((always_inline)) inline void gt_whole_k(const GemmTileParams& p, const GlueParams& gp, unsigned char* lds, uint32_t c0, uint32_t r0, uint32_t wm, uint32_t wn, uint32_t n_stages,
+                                              const unsigned char* const (&src)[LPW], const uint32_t (&step)[LPW], const uint32_t (&off)[LPW], const uint32_t (&dofs)[LPW], Issue issue) {
+  constexpr int BM = WM * TM * 32, BN = WN * TN * 32, ABYTES = BM * 64, STAGE = (BM + BN) * 64;
+  constexpr int NA = 2 * TM, NB = 2 * TN;                // 16-column and 16-row blocks of a wave
+  const uint32_t lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+  f4 acc[NA][NB];
+#pragma unroll
+  for (int a = 0; a < NA; a++)
+#pragma unroll
+    for (int b = 0; b < NB; b++) acc[a][b] = (f4){ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+  for (int j = 0; j < S; j++) issue(j, j);
+  // k 8 kq .. of a row: an activation row's chunk kq; of the weights' fragments, the half kq % 2 of k-step kq / 2
+  const uint32_t x_rd = (wm * TM * 32 + l16) * 64 + ((kq ^ ((l16 >> 2) & 3)) * 16), w_rd = ABYTES + wn * TN * 2048 + (kq >> 1) * 1024 + ((kq & 1) * 32 + l16) * 16;
+  h8 x0[TM], x1[TM], w[NB];
+  auto rd_x = [&](h8& f, const unsigned char* sb, int a) __attribute__((always_inline)) { f = *(const h8*)(sb + x_rd + a * 1024); };
+  auto rd_w = [&](h8& f, const unsigned char* sb, int b) __attribute__((always_inline)) { f = *(const h8*)(sb + w_rd + (b / 2) * 2048 + (b % 2) * 256); };
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(LPW * (S - 1)) : "memory");       // stage 0 (S stages were issued)
+  asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+  for (int a = 0; a < TM; a++) rd_x(x0[a], lds, a);
+#pragma unroll
+  for (int b = 0; b < NB; b++) rd_w(w[b], lds, b);
+  constexpr int NH = TM * NB;                            // products of half a stage
+  uint32_t buf = 0;
+  for (uint32_t st = 0; st < n_stages; st++) {
+    const uint32_t nbuf = buf + 1 == S ? 0 : buf + 1;
+    const unsigned char* sb = lds + buf * STAGE;
+    const unsigned char* sn = lds + nbuf * STAGE;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < NH; m++) {
+      acc[m % TM][m / TM] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[m / TM], x0[m % TM], acc[m % TM][m / TM], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (m < TM) { rd_x(x1[m], sb, TM + m); __builtin_amdgcn_sched_barrier(0); }
+    }
+    // stage st + 1 is in LDS behind this barrier, and every wave has read stage st: its buffer takes stage st + S
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(LPW * (S - 2)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t s_n = min(st + S, n_stages - 1);
+#pragma unroll
+    for (int m = 0; m < NH; m++) {
+      acc[TM + m % TM][m / TM] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[m / TM], x1[m % TM], acc[TM + m % TM][m / TM], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (m < TM) rd_x(x0[m], sn, m);
+      if (m % TM == TM - 1) rd_w(w[m / TM], sn, m / TM);
+#pragma unroll
+      for (int i = 0; i < LPW; i++)
+        if (i * (NH - 1) / LPW == m) PF_GLL_S(src[i] + (size_t)s_n * step[i], off[i], lds + buf * STAGE + dofs[i]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    buf = nbuf;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                       // (the stages past the end, never read)
+  if constexpr (EPI == GT_HEADS) {
+    float* hx = (float*)lds;
+    constexpr int LR = BN + 4;
+    lds_barrier();
+    heads_request<WM * 32, BN, BM>(gp, lds, c0);
+    auto dump = [&](auto A) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int b = 0; b < NB; b++) *(f4*)(hx + (wm * 32 + j * 16 + l16) * LR + (wn * NB + b) * 16 + 4 * kq) = acc[2 * decltype(A)::value + j][b];
+      asm volatile("; block %0" :: "n"(decltype(A)::value) : "memory");   // (the blocks' stores are not merged into one on selected registers)
+    };
+#pragma nounroll
+    for (int a = 0; a < TM; a++) {                                       // a phase: 32 of every wave's columns
+      static_assert(TM <= 7, "blocks of a wave");
+      if (a == 0) dump(std::integral_constant<int, 0>{});
+      if constexpr (TM > 1) if (a == 1) dump(std::integral_constant<int, 1>{});
+      if constexpr (TM > 2) if (a == 2) dump(std::integral_constant<int, 2>{});
+      if constexpr (TM > 3) if (a == 3) dump(std::integral_constant<int, 3>{});
+      if constexpr (TM > 4) if (a == 4) dump(std::integral_constant<int, 4>{});
+      if constexpr (TM > 5) if (a == 5) dump(std::integral_constant<int, 5>{});
+      if constexpr (TM > 6) if (a == 6) dump(std::integral_constant<int, 6>{});
+      if (a == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // what heads_request asked for
+      lds_barrier();
+      const auto col = [&](uint32_t c) { return c0 + (c / 32 * TM + a) * 32 + c % 32; };
+      if (gp.head_dim == 256) finish_heads<256, WM * 32, BN, BM>(gp, lds, c0, r0, p.d_out, col);
+      else finish_heads<128, WM * 32, BN, BM>(gp, lds, c0, r0, p.d_out, col);
+      lds_barrier();
+    }
+  } else {
+    // Accumulating calls: loads and stores share one counter, and a wait for a loaded value with stores pending waits for those as well, so the old
+    // values are fetched several blocks at a time, unconditionally (clamped addresses: a guarded load is a branch, one load a basic block), then added.
+    typedef f4 f4u __attribute__((aligned(4)));                           // (y is aligned to its elements)
+    constexpr int D = TN <= 5 ? 4 * TN : 16, NM = NA * NB;               // blocks of a phase: what fits next to the accumulators
+    auto col_of = [&](int a) { return c0 + (wm * NA + a) * 16 + l16; };
+    auto row_of = [&](int b) { return r0 + (wn * NB + b) * 16 + 4 * kq; };
+    const size_t last = (size_t)(p.n_cols - 1) * p.y_stride + p.d_out - 4;
+#pragma unroll
+    for (int m0 = 0; m0 < NM; m0 += D) {
+      f4 old[D];
+      if constexpr (EPI == GT_ACC) {
+#pragma unroll
+        for (int m = 0; m < D && m0 + m < NM; m++) {
+          const size_t at = (size_t)col_of((m0 + m) / NB) * p.y_stride + row_of((m0 + m) % NB);
+          old[m] = *(const f4u*)(p.y + (at < last ? at : last));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int m = 0; m < D && m0 + m < NM; m++) {
+        const int a = (m0 + m) / NB, b = (m0 + m) % NB;
+        const uint32_t col = col_of(a), row = row_of(b);
+        if (col < p.n_cols) {
+          float* y = p.y + (size_t)col * p.y_stride + row;
+          if (row + 4 <= p.d_out) *(f4u*)y = EPI == GT_ACC ? old[m] + acc[a][b] : acc[a][b];
+          else
+#pragma unroll
+            for (int i = 0; i < 3; i++) if (row + i < p.d_out) y[i] = EPI == GT_ACC ? y[i] + acc[a][b][i] : acc[a][b][i];
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
 template <int WM, int WN, int KG, int TM, int TN, int S, int EPI>
 __global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p, GlueParams gp) {
   constexpr bool ACC = EPI == GT_ACC;
@@ -246,6 +372,9 @@ __global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p, 
 #pragma unroll
     for (int i = 0; i < LPW; i++) PF_GLL_S(src[i] + (size_t)s * step[i], off[i], gt_lds + buf * STAGE + dofs[i]);
   };
+  if constexpr (KG == 1) {
+    gt_whole_k<WM, WN, TM, TN, S, EPI>(p, gp, gt_lds, c0, r0, wm, wn, n_stages, src, step, off, dofs, issue);
+  } else {
   auto col_of = [&](int a, int i) { return c0 + (wm * TM + a) * 32 + 8 * (i / 4) + 4 * fk + (i % 4); };
   auto row_of = [&](int b) { return r0 + (wn * TN + b) * 32 + fl; };
 
@@ -307,60 +436,6 @@ __global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p, 
     buf = nbuf;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                       // (the stages past the end, never read)
-  // accumulator i of a tile: column 8 (i / 4) + 4 fk + i % 4, row fl.  Accumulating calls: loads and stores share one counter,
-  // and a wait for a loaded value with stores pending waits for those as well, so the old values are fetched several
-  // tiles at a time, unconditionally (clamped addresses: a guarded load is a branch, one load a basic block), then added.
-  if constexpr (EPI == GT_HEADS && KG == 1) {
-    float* hx = (float*)gt_lds;
-    constexpr int LR = BN + 4;
-    lds_barrier();
-    heads_request<WM * 32, BN, BM>(gp, gt_lds, c0);
-    auto dump = [&](auto A) __attribute__((always_inline)) {
-#pragma unroll
-      for (int b = 0; b < TN; b++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) hx[(wm * 32 + 8 * (i / 4) + 4 * fk + (i % 4)) * LR + (wn * TN + b) * 32 + fl] = acc[decltype(A)::value][b][i];
-      asm volatile("; block %0" :: "n"(decltype(A)::value) : "memory");   // (the blocks' stores are not merged into one on selected registers)
-    };
-#pragma nounroll
-    for (int a = 0; a < TM; a++) {                                       // a phase: block a of every wave's columns
-      static_assert(TM <= 7, "blocks of a wave");
-      if (a == 0) dump(std::integral_constant<int, 0>{});
-      if constexpr (TM > 1) if (a == 1) dump(std::integral_constant<int, 1>{});
-      if constexpr (TM > 2) if (a == 2) dump(std::integral_constant<int, 2>{});
-      if constexpr (TM > 3) if (a == 3) dump(std::integral_constant<int, 3>{});
-      if constexpr (TM > 4) if (a == 4) dump(std::integral_constant<int, 4>{});
-      if constexpr (TM > 5) if (a == 5) dump(std::integral_constant<int, 5>{});
-      if constexpr (TM > 6) if (a == 6) dump(std::integral_constant<int, 6>{});
-      if (a == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // what heads_request asked for
-      lds_barrier();
-      const auto col = [&](uint32_t c) { return c0 + (c / 32 * TM + a) * 32 + c % 32; };
-      if (gp.head_dim == 256) finish_heads<256, WM * 32, BN, BM>(gp, gt_lds, c0, r0, p.d_out, col);
-      else finish_heads<128, WM * 32, BN, BM>(gp, gt_lds, c0, r0, p.d_out, col);
-      lds_barrier();
-    }
-  } else if constexpr (KG == 1) {
-    constexpr int D = TN <= 5 ? TN : 4;                                  // tiles of a phase: what fits next to the accumulators
-#pragma unroll
-    for (int m0 = 0; m0 < NM; m0 += D) {
-      float old[D][16];
-      if constexpr (ACC) {
-#pragma unroll
-        for (int m = 0; m < D && m0 + m < NM; m++)
-#pragma unroll
-          for (int i = 0; i < 16; i++) old[m][i] = p.y[(size_t)min(col_of((m0 + m) / TN, i), p.n_cols - 1) * p.y_stride + min(row_of((m0 + m) % TN), p.d_out - 1)];
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int m = 0; m < D && m0 + m < NM; m++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-          const int a = (m0 + m) / TN, b = (m0 + m) % TN;
-          if (row_of(b) < p.d_out && col_of(a, i) < p.n_cols) p.y[(size_t)col_of(a, i) * p.y_stride + row_of(b)] = ACC ? old[m][i] + acc[a][b][i] : acc[a][b][i];
-        }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  } else {
     constexpr int NT = TM * TN, SPW = NT * 16 / KG;
     const uint32_t wt = wave % (WM * WN);
     auto col_s = [&](int k) { const uint32_t sl = kgrp * SPW + k; return c0 + (wm * TM + sl / (16 * TN)) * 32 + 8 * (sl % 16 / 4) + 4 * fk + (sl % 4); };
@@ -485,7 +560,7 @@ float pa_gemm_tile_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, 
 }
 
 hipError_t pa_launch_gemm_tile(const GemmParams& p, const uint16_t* w16, int n_cu, hipStream_t s) {
-  if (p.d_out == 0 || p.d_in == 0 || p.d_in % 128 != 0 || p.n_cols == 0 || p.x_stride > (1u << 22)) return hipErrorInvalidValue;   // (32-bit row offsets inside a tile)
+  if (p.d_out == 0 || p.d_in == 0 || p.d_in % 128 != 0 || p.n_cols < 4 || p.x_stride > (1u << 22)) return hipErrorInvalidValue;   // (32-bit row offsets inside a tile)
   GemmTileParams q;
   q.x = p.x; q.w16 = w16; q.y = p.y; q.x_stride = p.x_stride; q.y_stride = p.y_stride; q.d_out = p.d_out; q.d_in = p.d_in; q.n_cols = p.n_cols;
   float us;

@@ -269,6 +269,25 @@ def test_gemm_tile_shapes(d_out, d_in, n):
         assert _rel(dy.download(np.float32, n * ys).reshape(n, ys)[:, :d_out], 2.0 * ref) < 2e-5, "accumulate"
 
 
+@pytest.mark.parametrize("d_out,d_in,n", [(9213, 128, 777), (8209, 256, 900), (446, 128, 25000), (4095, 256, 4095)])
+def test_gemm_tile_rows_four_at_a_time(d_out, d_in, n):
+    """Whole-sum tiles store four rows a lane, at any alignment of y: rows that are no multiple of four, columns back to back (a store past a column's last
+    row would land in the next one) and nothing past the last.  The bounds as above."""
+    rng = np.random.default_rng(d_out + n)
+    w, sc = _weights(PA_W_Q8_0, d_out, d_in, rng)
+    x16 = rng.standard_normal((n, d_in)).astype(np.float16)
+    ref = O.gemm_f16(PA_W_Q8_0, w, sc, x16.astype(np.float32))
+    with PooledAttn(SHAPES["qwen36_moe"], 64, n_layers=1, max_cols=1) as pa:
+        wh = pa.weight(PA_W_Q8_0, w, sc)
+        y0 = rng.standard_normal(n * d_out + 8).astype(np.float32)
+        dx = pa.to_device(x16.view(np.uint16)); dy = pa.to_device(y0)
+        for acc, scale in ((False, 1.0), (True, 2.0)):
+            pa.gemm(wh, dx, d_in, n, dy, d_out, acc=acc); pa.sync()
+            got = dy.download(np.float32, y0.size)
+            assert _rel(got[:-8].reshape(n, d_out), scale * ref) < 2e-5, acc
+            assert np.array_equal(got[-8:], y0[-8:]), "past the last column"
+
+
 @pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])
 def test_gemm_weight_cache_budget(kind):
     """The kept f16 copy and the per-call staging hold the same values: a context with no budget (every call widens into
