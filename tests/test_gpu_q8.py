@@ -223,3 +223,22 @@ def test_q8_short_verify_block_is_one_split_with_two_row_blocks():
         for out_dtype in (0, PA_OUT_F16):
             got = pa.run_attn("decode", 0, q, base, gate=gate, out_dtype=out_dtype).astype(np.float32)
             assert_parity(got, ref, "q8 short verify block out %d" % out_dtype)
+
+
+@pytest.mark.parametrize("base,n,splits,exact", [(12288, 1, 32, False), (12289, 1, 49, False), (12289, 1, 25, True), (12280, 8, 32, False), (12281, 8, 49, False),
+                                                 (16368, 16, 32, False), (16369, 16, 43, False)])
+def test_q8_head_dim_128_loop_at_two_workgroups_a_cu(base, n, splits, exact):
+    """Past three tiles a wave (four with two row blocks) the tile loop of int8 rows at head_dim 128 takes two workgroups a CU, in contexts that are not
+    column-exact: either side of the line, split counts of a 256-CU part, against the oracle on the de-quantised values."""
+    cfg = dict(_q8cfg("qwen3_1p7b"), verify_exact=exact)
+    rng = np.random.default_rng(base + n)
+    kq, ks, vq, vs, kf, vf = _quantised_cache(cfg, base + n, seed=41)
+    q = rng.standard_normal((n, cfg["n_heads"], cfg["head_dim"]), dtype=np.float32)
+    ref = O.attention_values(q, kf, vf, base)
+    with PooledAttn(cfg, base + n + 8, n_layers=1, max_cols=n) as pa:
+        pa.layer_alloc(0)
+        for w, a in enumerate((kq, vq, ks, vs)):
+            pa.kv_write(0, w, 0, a)
+        plan = pa.plan("decode", base, n)
+        assert plan["n_splits"] == splits, plan
+        assert_parity(pa.run_attn("decode", 0, q, base), ref, "q8 hd 128, %d columns at %d" % (n, base))
