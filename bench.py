@@ -212,7 +212,7 @@ def prefill_leg(steps, with_cpu, kv_q8=False):
                min_ms_per_step=round(min(step_ms), 4), max_ms_per_step=round(max(step_ms), 4), cold_first_ms=round(cold_first_ms, 4),
                step_ms=[round(x, 3) for x in step_ms], flops_per_step=flops, plan=pa.plan("prefill", base, n),
                roofline=dict(bound="mfma", achieved=round(tf_kernel, 1), peak=MFMA_F16_PEAK_TFLOPS, unit="TFLOP/s", frac=round(tf_kernel / MFMA_F16_PEAK_TFLOPS, 4),
-                             traffic=None, kernel="pa_prefill_kernel<256, 1, 8, false>", kernel_ms=round(k_ms, 4), kernel_ms_mean=round(k_mean, 4),
+                             traffic=None, kernel="pa_prefill_kernel<256, 8, false>", kernel_ms=round(k_ms, 4), kernel_ms_mean=round(k_mean, 4),
                              kernel_ms_min=round(min(kern_ms), 4), kernel_ms_max=round(max(kern_ms), 4), reported="median launch",
                              algorithmic_flops_per_launch=flops, launches=len(kern_ms)))
     if with_cpu:
@@ -569,8 +569,8 @@ def main():
 
 
 def pa_decode_kernel_name(plan, args):
-    """Template arguments: head_dim, row blocks, waves, fused pre-step, gather, int8 caches, single-round splits."""
-    return "pa_decode_kernel<256, 1, 4, %s, false, %s, %s>" % ("false" if args.unfused else "true", "true" if args.kv_q8 else "false",
+    """Template arguments: head_dim, row blocks, waves, fused pre-step, gather, int8 caches, single-round splits, two columns a workgroup."""
+    return "pa_decode_kernel<256, 1, 4, %s, false, %s, %s, false>" % ("false" if args.unfused else "true", "true" if args.kv_q8 else "false",
                                                                "true" if plan["split_len"] == 128 and plan["row_blocks"] == 1 else "false")
 
 
