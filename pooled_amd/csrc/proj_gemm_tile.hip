@@ -36,7 +36,7 @@ struct GemmTileParams {
 // in f64 in another order), and the f32 projections themselves are never stored: a launch less, and for 4096 columns of the gated 16 / 2-head
 // shape 150 MB less written and as much less read.  It is LDS, VALU and store work behind a tile's products, with nothing to hide under, so it is dealt
 // by what it is: columns on lanes for the sums of squares, rotation pairs on lanes for the rotation (both elements of a pair in one lane),
-// the other dims a column at a time, everything read before the first store.  Layer pass, apart / so (us a layer): 4096 columns
+// the other dims a column at a time, everything read before the first store.  Layer pass, apart / so (us a layer, both on 32 x 32 x 16 products): 4096 columns
 // of that shape 499 / 459, 2048 282 / 243, 300 71 / 66; 777 of the 24 / 4-head shape 292 / 280; 512 and 1024 of the 16 / 8-head shape 53 / 48 and 82 / 73.
 enum { GT_STORE = 0, GT_ACC = 1, GT_HEADS = 2 };
 
@@ -503,8 +503,8 @@ static hipError_t gt_launch(const GemmTileParams& q, int acc, const GlueParams* 
   return hipGetLastError();
 }
 
-// The tile shapes, with what a round of the chip costs: ns per k of d_in (measured on rounds of 200 - 256 workgroups) on top
-// of about 6 us for a round's first loads and last stores.
+// The tile shapes, with what a round of the chip costs: ns per k of d_in (measured on rounds of 200 - 256 workgroups, all on 32 x 32 x 16
+// products; several full rounds of a kg = 1 shape are some 5 % faster now) on top of about 6 us for a round's first loads and last stores.
 struct TileShape { uint16_t bm, bn, kg; float us, ns_k; hipError_t (*launch)(const GemmTileParams&, int, const GlueParams*, hipStream_t); };
 static const TileShape tile_shapes[] = {
   { 64, 128, 4, 6.f, 6.5f, gt_launch<1, 2, 4, 2, 2, 3, false> },
