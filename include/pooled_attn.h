@@ -41,7 +41,7 @@ extern "C" {
 
 #define PA_FLAG_VERIFY_EXACT 8u /* pa_attn_decode with n_cols > 1 runs every column as the one-column decode at its own position
                                  (its own splits, its own row block): column c then has the bits of pa_attn_decode(base_pos + c,
-                                 n_cols = 1) of a context with the flag, the invariant the reference states for its pair (engine/wgsl/attn_dec.js:12-16,
+                                 n_cols = 1), the invariant the reference states for its pair (engine/wgsl/attn_dec.js:12-16,
                                  tests/test_attn_dec.js:89-97) and its speculative decoding leans on (spec greedy == plain
                                  greedy).  Cost: every column streams the K/V rows through its own workgroups; a block whose
                                  columns share one one-column plan runs as one pass in which a split's columns sit side by

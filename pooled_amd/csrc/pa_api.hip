@@ -406,13 +406,14 @@ static int plan_decode(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa
     // workgroup: MoE shape, 4 columns at 4096 / 8192 / 16384 rows 20.5 -> 15.9, 20.7 -> 16.3, 21.1 -> 17.7 us; dense
     // hd-128 shape, 32 columns at 4096 / 8192 rows 26.6 -> 19.0, 26.6 -> 20.4 us).
     uint32_t target1 = std::max(1u, (uint32_t)ctx->n_cu / (c.n_kv_heads * groups));
-    // Int8 rows at head_dim 128 are a quarter of those bytes a wave, and two workgroups fit a CU (37 KB of staging, 162 - 230 registers): two of them, where
-    // a wave of one would have four tiles or more (five with two row blocks).  Measured, dense shape, one / two a CU: one column at 14500, 18000,
-    // 32000 rows 14.8 / 12.6, 17.5 / 15.2, 23.9 / 19.5 us, 8 columns 18.3 / 17.4, 20.8 / 19.5, 27.7 / 23.8, 16 columns at 18000 and 32000 26.4 / 23.0
-    // and 33.5 / 27.3; with three tiles 8 columns are 2 % slower, 12 columns 8 %.  F16 rows: 2 - 16 % slower on most; head_dim 256: 4 - 17 %.
-    // (One column: only one row block, so that the partials stay within those of the single-round plans.)  A column-exact context keeps one: its
-    // blocks run the plan of their one-column decodes, whose workgroups fill the chip already (2 - 8 columns at 13000 - 30000 rows 1 - 13 % slower with two).
-    if (kv_q8(ctx) && !(c.flags & PA_FLAG_VERIFY_EXACT) && c.head_dim == 128 && groups == 1 && (nb == 1 || (nb == 2 && n_cols > 1)) && ceil_div(tiles, target1 * W) >= 3 + nb)
+    // Blocks over int8 rows at head_dim 128, a quarter of those bytes a wave, and two workgroups fit a CU (37 KB of staging, 162 - 230 registers): two of them,
+    // where a wave of one would have four tiles or more (five with two row blocks).  Measured, dense shape, one / two a CU: 8 columns at 14500, 18000,
+    // 32000 rows 18.3 / 17.4, 20.8 / 19.5, 27.7 / 23.8 us, 16 columns at 18000 and 32000 26.4 / 23.0 and 33.5 / 27.3; with three tiles 8 columns
+    // are 2 % slower, 12 columns 8 %.  F16 rows: 2 - 16 % slower on most; head_dim 256: 4 - 17 %.  One column keeps one although two are faster
+    // there (13000, 18000, 32000 rows 14.6 / 12.1, 17.3 / 15.0, 24.1 / 19.1 us): a column-exact block (PA_FLAG_VERIFY_EXACT) runs the splits of the one-column decodes
+    // whose bits it repeats, whatever context made those, and its workgroups fill the chip already: with two, blocks of 2 - 16 columns at 13000 -
+    // 32000 rows are 2 - 14 % slower at 28 of 35 sizes.
+    if (kv_q8(ctx) && n_cols > 1 && c.head_dim == 128 && groups == 1 && nb <= 2 && ceil_div(tiles, target1 * W) >= 3 + nb)
       target1 = std::max(1u, 2 * (uint32_t)ctx->n_cu / c.n_kv_heads);
     ns = std::max(1u, std::min(target1, tiles / W));
     // ... and the fewest splits with that many tiles per wave: 2049 tiles over 256 waves are nine rounds for one wave

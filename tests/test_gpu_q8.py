@@ -225,11 +225,11 @@ def test_q8_short_verify_block_is_one_split_with_two_row_blocks():
             assert_parity(got, ref, "q8 short verify block out %d" % out_dtype)
 
 
-@pytest.mark.parametrize("base,n,splits,exact", [(12288, 1, 32, False), (12289, 1, 49, False), (12289, 1, 25, True), (12280, 8, 32, False), (12281, 8, 49, False),
+@pytest.mark.parametrize("base,n,splits,exact", [(12288, 1, 32, False), (12289, 1, 25, False), (12289, 1, 25, True), (12280, 8, 32, False), (12281, 8, 49, False),
                                                  (16368, 16, 32, False), (16369, 16, 43, False)])
 def test_q8_head_dim_128_loop_at_two_workgroups_a_cu(base, n, splits, exact):
-    """Past three tiles a wave (four with two row blocks) the tile loop of int8 rows at head_dim 128 takes two workgroups a CU, in contexts that are not
-    column-exact: either side of the line, split counts of a 256-CU part, against the oracle on the de-quantised values."""
+    """Past three tiles a wave (four with two row blocks) the tile loop of int8 rows at head_dim 128 takes two workgroups a CU for blocks, one for a
+    single column in any context: either side of the line, split counts of a 256-CU part, against the oracle on the de-quantised values."""
     cfg = dict(_q8cfg("qwen3_1p7b"), verify_exact=exact)
     rng = np.random.default_rng(base + n)
     kq, ks, vq, vs, kf, vf = _quantised_cache(cfg, base + n, seed=41)
@@ -242,3 +242,25 @@ def test_q8_head_dim_128_loop_at_two_workgroups_a_cu(base, n, splits, exact):
         plan = pa.plan("decode", base, n)
         assert plan["n_splits"] == splits, plan
         assert_parity(pa.run_attn("decode", 0, q, base), ref, "q8 hd 128, %d columns at %d" % (n, base))
+
+
+@pytest.mark.parametrize("base", [12289, 20001, 31000])
+def test_q8_exact_blocks_have_the_bits_of_another_contexts_decodes(base):
+    """A column-exact block repeats the one-column decode of any context of its shape, with the flag or without: int8 rows at head_dim 128 past
+    the single-round plans, through pa_attn_decode and through the fused step."""
+    n = 5
+    cfg = _q8cfg("qwen3_1p7b")
+    kq, ks, vq, vs, _, _ = _quantised_cache(cfg, base + n, seed=43)
+    q = np.random.default_rng(base).standard_normal((n, cfg["n_heads"], cfg["head_dim"]), dtype=np.float32)
+    got, steps = [], []
+    for exact in (True, False):
+        with PooledAttn(dict(cfg, verify_exact=exact), base + n, n_layers=1, max_cols=n) as pa:
+            pa.layer_alloc(0)
+            for w, a in enumerate((kq, vq, ks, vs)):
+                pa.kv_write(0, w, 0, a)
+            assert pa.plan("decode", base, 1)["split_len"] > 128
+            got.append(pa.run_attn("decode", 0, q, base) if exact else np.concatenate([pa.run_attn("decode", 0, q[c:c + 1], base + c) for c in range(n)]))
+            d = O.make_inputs(cfg, base, 1, seed=7)
+            steps.append(pa.run_decode_step(0, d["qraw"][0], d["kraw"][base], d["vraw"][base], d["qw"], d["kw"], base))
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    assert np.isfinite(steps[0]).all() and np.array_equal(steps[0].view(np.uint32), steps[1].view(np.uint32))
