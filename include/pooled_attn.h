@@ -150,7 +150,8 @@ float* pa_gate_buffer(pa_ctx* ctx);
  * engine that needs speculative greedy decoding to reproduce plain greedy decoding token for token sets the flag.
  *   d_q   : f32 [n_cols][q_stride], a column holds roped q [nH][hd]; NULL = pa_q_buffer
  *   d_gate: f32 [n_cols][gate_stride] gate pre-activations [nH][hd]; NULL = no gate
- *   d_out : [n_cols][out_stride] of out_dtype, a column holds [nH][hd]
+ *   d_out : [n_cols][out_stride] of out_dtype, a column holds [nH][hd].  With one column it may lie over d_q; otherwise it
+ *           must not share memory with the inputs.
  * pa_attn_prefill: the same contract for a causal prefill chunk of any width: the f16 MFMA kernel, or, for a chunk of
  * few columns (at most one 32- / 64-row block, or a few column groups over a long context, where the K/V stream and
  * not the matrix cores bound the pass), the split-K kernel; pa_plan_query tells which.
@@ -170,7 +171,7 @@ int pa_attn_prefill(pa_ctx* ctx, uint32_t layer, const float* d_q, uint32_t q_st
  * bits and the same output as pa_glue_kv followed by pa_attn_decode.
  *   d_q_in: f32 one column [nH][2*hd] (PA_FLAG_GATE: [q | gate] per head) or [nH][hd]
  *   d_k, d_v: f32 [nKV][hd];  d_qw, d_kw: f32 [hd] (ignored without PA_FLAG_QK_NORM)
- *   d_out : [nH][hd] of out_dtype
+ *   d_out : [nH][hd] of out_dtype; it may lie over d_k and d_v and, without PA_FLAG_GATE, over d_q_in
  * pa_q_buffer / pa_gate_buffer are not written by this call. */
 int pa_attn_decode_step(pa_ctx* ctx, uint32_t layer, const float* d_q_in, const float* d_k, const float* d_v,
                         const float* d_qw, const float* d_kw, uint32_t pos, void* d_out, int out_dtype);

@@ -1,4 +1,4 @@
-// Device-to-device copies of cache planes (checkpoint slots) on gfx950.
+// Device-to-device copies of cache planes (checkpoint slots) on gfx950; and of outputs that could not be written in place.
 //
 // A saved or restored session is rows [0, pos) of every layer's K and V (and scales): per tensor n_kv_heads contiguous
 // planes at one pitch on either side (the reference's copyBufferToBuffer calls: engine/dense.js:20-47).  One launch covers up
@@ -12,6 +12,7 @@
 #include "pa_internal.h"
 
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+typedef u4 u4d __attribute__((aligned(8)));       // (planes of an f16 output's columns are 8 bytes aligned)
 
 #define CP_PIECE 2048u      // 16-byte units of a workgroup's piece
 
@@ -23,7 +24,7 @@ __global__ __launch_bounds__(256) void pa_copy_planes_kernel(PaCopyParams p) {
   const uint32_t units = p.units[t], ppp = (units + CP_PIECE - 1) / CP_PIECE;
   const uint32_t plane = wg / ppp, u0 = (wg - plane * ppp) * CP_PIECE + threadIdx.x;
   const u4* src = (const u4*)((const unsigned char*)p.src[t] + (size_t)plane * p.src_pitch[t]);
-  u4* dst = (u4*)((unsigned char*)p.dst[t] + (size_t)plane * p.dst_pitch[t]);
+  u4d* dst = (u4d*)((unsigned char*)p.dst[t] + (size_t)plane * p.dst_pitch[t]);
   u4 v[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) v[i] = __builtin_nontemporal_load(src + min(u0 + 256u * i, units - 1));

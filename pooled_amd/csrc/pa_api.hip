@@ -555,6 +555,20 @@ static int prof_aux_pair(pa_ctx* ctx, const PaTiming& main, PaTiming* t) {
   return PA_OK;
 }
 
+// Where a kv head's one workgroup writes the output itself (plan_one_wg), other kv heads' workgroups may still be reading: an output that shares
+// memory with what the call reads (f16 results into the q buffer, results into the step's k or v) goes through the scratch of the split partials,
+// which that plan does not use, and is copied behind the kernel.
+static bool shares(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+  return b && (uintptr_t)a < (uintptr_t)b + b_bytes && (uintptr_t)b < (uintptr_t)a + a_bytes;
+}
+static size_t cols_bytes(uint32_t n_cols, uint32_t stride, uint32_t col, size_t elem) { return ((size_t)(n_cols - 1) * stride + col) * elem; }
+static int copy_out(pa_ctx* ctx, const float* staged, uint32_t col, void* out, uint32_t out_stride, uint32_t n_cols, size_t elem) {
+  PaCopyParams p; memset(&p, 0, sizeof p);
+  p.n = 1; p.src[0] = staged; p.dst[0] = out; p.src_pitch[0] = col * elem; p.dst_pitch[0] = out_stride * elem; p.units[0] = (uint32_t)(col * elem / 16);
+  HIPCHK(ctx, pa_launch_copy_planes(p, n_cols, ctx->stream));
+  return PA_OK;
+}
+
 static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, const float* d_q, uint32_t q_stride,
                        const float* d_gate, uint32_t gate_stride, uint32_t base_pos, uint32_t n_cols, void* d_out,
                        uint32_t out_stride, int out_dtype) {
@@ -600,12 +614,14 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
         if ((rc = attn_common(ctx, who, 0, layer, q_c, q_stride, gate_c, gate_stride, base_pos + col, 1, out_c, out_stride, out_dtype))) return rc;
       } else {
         const bool one = plan_one_wg(p0);
-        if (!one && (rc = ensure_partials(ctx, run, p0.slots))) return rc;
+        const bool staged = one && (shares(out_c, cols_bytes(run, out_stride, qd, osz), q_c, cols_bytes(run, q_stride, qd, 4)) ||
+                                    shares(out_c, cols_bytes(run, out_stride, qd, osz), gate_c, cols_bytes(run, gate_stride, qd, 4)));
+        if ((!one || staged) && (rc = ensure_partials(ctx, run, p0.slots))) return rc;
         AttnParams p; memset(&p, 0, sizeof p);
         p.q = q_c; p.gate = gate_c; p.k_cache = ctx->layers[layer].k; p.v_cache = ctx->layers[layer].v;
         p.k_scale = ctx->layers[layer].ks; p.v_scale = ctx->layers[layer].vs;
-        p.part_o = ctx->part_o; p.part_ml = ctx->part_ml; p.out = out_c;
-        p.q_stride = q_stride; p.gate_stride = gate_stride; p.out_stride = out_stride;
+        p.part_o = ctx->part_o; p.part_ml = ctx->part_ml; p.out = staged ? ctx->part_o : out_c;
+        p.q_stride = q_stride; p.gate_stride = gate_stride; p.out_stride = staged ? qd : out_stride;
         p.n_heads = c.n_heads; p.n_kv_heads = c.n_kv_heads; p.group = c.n_heads / c.n_kv_heads;
         p.base_pos = base_pos + col; p.n_cols = run;
         // On single-round plans a workgroup may take two columns (a row block each) of those splits that are whole for both: the columns of a
@@ -631,6 +647,7 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
           if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;
           HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream, &tm2));
         }
+        if (staged && (rc = copy_out(ctx, ctx->part_o, qd, out_c, out_stride, run, osz))) return rc;
       }
       col += run;
     }
@@ -643,10 +660,12 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
   // one split and no own-row partial: the kernel writes the output itself (the prefill kernel, or the split-K kernel's
   // tile loop: its single-round form always leaves a partial)
   const bool direct = plan_one_wg(pl) || (pl.n_splits == 1 && !plan_self_row(pl) && (pl.kernel == 1 || pl.split_len != 32 * pl.waves || pl.row_blocks > 1));
-  if (!direct && (rc = ensure_partials(ctx, n_cols, pl.slots))) return rc;
+  const size_t osz = out_dtype == PA_OUT_F16 ? 2 : 4;
+  const bool staged = plan_one_wg(pl) && (shares(d_out, qd * osz, d_q, qd * 4) || shares(d_out, qd * osz, d_gate, qd * 4));
+  if ((!direct || staged) && (rc = ensure_partials(ctx, n_cols, pl.slots))) return rc;
   AttnParams p; memset(&p, 0, sizeof p);
   p.q = d_q; p.gate = d_gate; p.k_cache = ctx->layers[layer].k; p.v_cache = ctx->layers[layer].v;
-  p.part_o = ctx->part_o; p.part_ml = ctx->part_ml; p.out = d_out;
+  p.part_o = ctx->part_o; p.part_ml = ctx->part_ml; p.out = staged ? ctx->part_o : d_out;
   p.q_stride = q_stride; p.gate_stride = gate_stride; p.out_stride = out_stride;
   p.n_heads = c.n_heads; p.n_kv_heads = c.n_kv_heads; p.group = c.n_heads / c.n_kv_heads;
   p.base_pos = base_pos; p.n_cols = n_cols;
@@ -688,7 +707,7 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
     if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;
     HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream, &tm2));
   }
-  return PA_OK;
+  return staged ? copy_out(ctx, ctx->part_o, qd, d_out, qd, 1, osz) : PA_OK;
 }
 
 extern "C" int pa_attn_decode(pa_ctx* ctx, uint32_t layer, const float* d_q, uint32_t q_stride, const float* d_gate,
@@ -737,7 +756,11 @@ static int decode_step_common(pa_ctx* ctx, const char* who, bool static_scratch,
   AttnParams p; memset(&p, 0, sizeof p);
   p.k_cache = ctx->layers[layer].k; p.v_cache = ctx->layers[layer].v;
   p.k_scale = ctx->layers[layer].ks; p.v_scale = ctx->layers[layer].vs;
-  p.part_o = part_o; p.part_ml = part_ml; p.out = d_out;
+  const uint32_t qd = c.n_heads * c.head_dim, kvd = c.n_kv_heads * c.head_dim;
+  const size_t osz = out_dtype == PA_OUT_F16 ? 2 : 4;
+  const bool staged = one && (shares(d_out, qd * osz, d_q_in, (size_t)qd * (gated ? 8 : 4)) || shares(d_out, qd * osz, d_k, kvd * 4) || shares(d_out, qd * osz, d_v, kvd * 4) ||
+                              (norm && (shares(d_out, qd * osz, d_qw, c.head_dim * 4) || shares(d_out, qd * osz, d_kw, c.head_dim * 4))));
+  p.part_o = part_o; p.part_ml = part_ml; p.out = staged ? (void*)part_o : d_out;
   p.n_heads = c.n_heads; p.n_kv_heads = c.n_kv_heads; p.group = c.n_heads / c.n_kv_heads;
   p.base_pos = pos; p.n_cols = 1;
   p.split_len = pl.split_len; p.n_splits = pl.n_splits; p.slots = pl.slots; p.cols_per_group = pl.cols_per_group;
@@ -754,7 +777,7 @@ static int decode_step_common(pa_ctx* ctx, const char* who, bool static_scratch,
   PaTiming tm;                                        // profiling may create events: not on the allocation-free path
   if (!static_scratch && (rc = prof_pair(ctx, &tm))) return rc;
   HIPCHK(ctx, pa_launch_decode_step(p, c.head_dim, ctx->stream, &tm));
-  if (one) return PA_OK;
+  if (one) return staged ? copy_out(ctx, part_o, qd, d_out, qd, 1, osz) : PA_OK;
   PaTiming tm2;
   if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;
   HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream, &tm2));

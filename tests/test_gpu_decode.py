@@ -265,6 +265,33 @@ def test_verify_exact_two_columns_a_workgroup(shape, n_cols, base, more):
             assert np.array_equal(single[0].view(np.uint32), multi[c].view(np.uint32)), "column %d differs from its decode" % c
 
 
+@pytest.mark.parametrize("shape,n_cols,base", [("qwen36_moe", 1, 200), ("qwen3_1p7b", 1, 256), ("qwen3_1p7b", 5, 120), ("qwen36_moe", 4, 250)])
+@pytest.mark.parametrize("into", ["q", "gate", "behind q"])
+def test_decode_output_over_its_inputs(shape, n_cols, base, into):
+    """Results written over the queries or the gate, f16 and f32, from their first byte or from a column's middle on, where one workgroup a kv head
+    writes the output itself (at most 256 rows, in column-exact blocks too): the bits of a call with a buffer of its own."""
+    cfg = dict(SHAPES[shape], verify_exact=True)
+    rng = np.random.default_rng(base + n_cols)
+    k16, v16 = random_cache(cfg, base + n_cols, seed=5)
+    with _ctx_with_cache(cfg, k16, v16, base + n_cols) as pa:
+        qd = pa.q_dim
+        q, gate = rng.standard_normal((2, n_cols, qd), dtype=np.float32)
+        for out_dtype, np_dtype, stride in ((0, np.float32, qd), (PA_OUT_F16, np.float16, qd), (PA_OUT_F16, np.float16, qd + 4)):
+            assert pa.plan("decode", base + n_cols - 1, 1)["waves"] == 8
+            room = np.zeros(n_cols * qd + 4 * stride, np.float32)
+            dq, dg, own = (pa.to_device(np.concatenate([a.ravel(), room])) for a in (q, gate, room))
+            pa.attn("decode", 0, dq, qd, dg, qd, base, n_cols, own, stride, out_dtype)
+            at = (dg if into == "gate" else dq).ptr + (qd * 2 if into == "behind q" else 0)
+            pa.sync()
+            want = own.download(np_dtype, n_cols * stride)
+            pa._chk(pa.L.pa_attn_decode(pa.ctx, 0, dq.ptr, qd, dg.ptr, qd, base, n_cols, at, stride, out_dtype))
+            pa.sync()
+            got = np.empty(n_cols * stride, np_dtype)
+            pa._chk(pa.L.pa_download(pa.ctx, got.ctypes.data, at, got.nbytes))
+            cols = lambda a: a.reshape(n_cols, stride)[:, :qd]
+            assert np.isfinite(cols(want).astype(np.float32)).all() and np.array_equal(cols(want), cols(got)), (out_dtype, stride)
+
+
 def test_decode_f16_output_and_strides():
     cfg = SHAPES["qwen36_moe"]
     rng = np.random.default_rng(14)

@@ -52,6 +52,34 @@ def test_decode_step_matches_oracle_and_unfused(shape, pos):
     assert np.array_equal(got.view(np.uint32), unf[0].view(np.uint32)), "fused output differs from pa_glue_kv + pa_attn_decode"
 
 
+@pytest.mark.parametrize("shape", ["qwen36_moe", "qwen3_1p7b"])
+def test_decode_step_output_over_its_inputs(shape):
+    """The output of a step of one workgroup a kv head may lie over anything that the step reads: over q, k and v (one buffer, as a fused projection
+    leaves them) from their first byte, from their middle and over the norm weights; the bits and the cache row of a call with an output of its own."""
+    cfg = SHAPES[shape]
+    pos = 200
+    d, k16, v16, K, V, _, max_seq = _case(cfg, pos, seed=3)
+    qkv = np.concatenate([d["qraw"][0].ravel(), d["kraw"][0].ravel(), d["vraw"][0].ravel(), d["qw"], d["kw"]]).astype(np.float32)
+    nq, hd, kvd = d["qraw"][0].size, cfg["head_dim"], cfg["n_kv_heads"] * cfg["head_dim"]
+    with PooledAttn(cfg, max_seq, n_layers=1, max_cols=1) as pa:
+        pa.layer_alloc(0)
+        pa.kv_write(0, 0, 0, k16); pa.kv_write(0, 1, 0, v16)
+        assert pa.plan("decode", pos, 1)["waves"] == 8
+        ins = [4 * x for x in (0, nq, nq + kvd, nq + 2 * kvd, nq + 2 * kvd + hd)]
+        for out_dtype, t in ((0, np.float32), (PA_OUT_F16, np.float16)):
+            want = pa.run_decode_step(0, *(d[n][0] for n in ("qraw", "kraw", "vraw")), d["qw"], d["kw"], pos, out_dtype).ravel()
+            for at in (0, nq * 2, nq * 4, (nq + kvd) * 4 - 16, (nq + 2 * kvd) * 4, (nq + 2 * kvd + hd) * 4 - 16):
+                for call in (pa.L.pa_attn_decode_step, pa.L.pa_attn_decode_step_noalloc):
+                    buf = pa.to_device(np.concatenate([qkv, np.zeros(want.size, np.float32)]))
+                    pa.kv_write(0, 0, pos, k16[pos:pos + 1]); pa.kv_write(0, 1, pos, v16[pos:pos + 1])
+                    pa._chk(call(pa.ctx, 0, *(buf.ptr + i for i in ins), pos, buf.ptr + at, out_dtype))
+                    pa.sync()
+                    got = np.empty(want.size, t)
+                    pa._chk(pa.L.pa_download(pa.ctx, got.ctypes.data, buf.ptr + at, got.nbytes))
+                    assert np.array_equal(got, want), (out_dtype, at)
+                    assert np.array_equal(pa.kv_read(0, 0, pos, 1).ravel(), K[pos].ravel()) and np.array_equal(pa.kv_read(0, 1, pos, 1).ravel(), V[pos].ravel())
+
+
 @pytest.mark.parametrize("shape,more", [("qwen36_moe", {}), ("qwen38_27b", {}), ("qwen3_1p7b", {}), ("qwen3_1p7b", dict(n_heads=13, n_kv_heads=1, gate=True)),
                                         ("qwen36_moe", dict(n_kv_heads=1, gate=False))])
 def test_decode_step_in_one_workgroup_and_past_it(shape, more):
