@@ -518,7 +518,8 @@ static const TileShape tile_shapes[] = {
   { 256, 256, 1, 6.f, 27.0f, gt_launch<2, 4, 1, 4, 2, 4, false> },
 };
 // ... and those that hold whole heads (128 rows: of head_dim 128) and can end with the pre-step, whose work is part of a round's start here.
-// Fitted to 75 sizes (the three model shapes, 33 to 4096 columns): of the shapes with the call's kg, the one taken is the fastest or within 0.6 % of it.
+// Fitted to 75 sizes (the three model shapes, 33 to 4096 columns) on 32 x 32 x 16 products.  As the kernels are now, on 16 sizes (257 to 1024 columns) timed on every
+// shape with the call's kg, the one taken is the fastest or within 1 % of it, but for 640 columns of the 24 / 4-head shape (205 us a layer, 199 on 192 columns).
 static const TileShape head_shapes[] = {
   { 64, 128, 4, 3.5f, 7.1f, gt_launch<1, 2, 4, 2, 2, 3, true> },
   { 128, 128, 2, 4.3f, 8.9f, gt_launch<2, 2, 2, 2, 2, 4, true> },
@@ -572,8 +573,13 @@ static int pick_heads(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t h
   int best = -1;
   *us = 1e30f;
   for (int i = 0; i < (int)(sizeof head_shapes / sizeof head_shapes[0]); i++) {
-    if (head_shapes[i].bn % head_dim || head_shapes[i].kg != kg) continue;
-    const float c = rounds_us(head_shapes[i], d_out, d_in, n_cols, n_cu);
+    const TileShape& t = head_shapes[i];
+    if (t.bn % head_dim || t.kg != kg) continue;
+    // 96 columns where 128 take as many blocks (65 - 96, 129 - 192, 257 - 288 columns): the wider tile is the faster one all the same, its last
+    // block is the emptier and brings the weights in for the others (us a layer of the 24 / 4-head shape, 96 / 128 columns a tile: 144 columns 116 / 107,
+    // 192 129 / 123, 257 133 / 118, 272 140 / 125, 288 143 / 133; 16 / 2-head shape, 257 66.8 / 64.1).
+    if (t.bm == 96 && (n_cols + 95) / 96 == (n_cols + 127) / 128) continue;
+    const float c = rounds_us(t, d_out, d_in, n_cols, n_cu);
     if (c < *us) { *us = c; best = i; }
   }
   return best;

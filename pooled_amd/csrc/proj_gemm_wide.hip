@@ -277,7 +277,9 @@ extern "C" uint32_t pa_rule_gemm_wide_tile(uint32_t d_out, uint32_t d_in, uint32
 // where the two apart are the faster form -- the tiles that hold whole heads are few, and below some 200 - 300 columns (64-column tiles of too
 // few workgroups) they cost more than the pre-step's launch, 3.5 us and the f32 projections through memory at 6 TB/s (16 columns 3.9 us, 512 of
 // the 16 / 8-head shape 6.5, 777 of the 24 / 4-head shape 19.6, 4096 of the 16 / 2-head shape 53.5).  Only tiles that split K as the call apart does:
-// the results are its bits.  On 75 sizes the choice is 4 % ahead of always apart (best 14 %), at no size more than 1 % behind.
+// a projection is its bits.  Taken where its estimate is 3 % ahead: closer than that the estimates do not tell which is faster (24 / 4-head shape, 214 - 256 columns,
+// estimates within 1.2 %: 118 - 126 us a layer apart, up to 1 % more so from position 0, up to 1 % less behind 1000 rows).  On 238 sizes (the three model
+// shapes, 33 to 4096 columns) the choice is 7 % ahead of always apart (best 22 %) and at no size behind it.
 extern "C" uint32_t pa_rule_gemm_heads(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t n_heads, uint32_t head_dim, int gated, int n_cu) {
   const uint32_t cus = n_cu > 0 ? (uint32_t)n_cu : 256u;
   uint32_t shape, kg, whole;
@@ -286,7 +288,7 @@ extern "C" uint32_t pa_rule_gemm_heads(uint32_t d_out, uint32_t d_in, uint32_t n
   const float mid = mid_tile_us(d_in, tiles64, cus);
   if (mid <= apart) { apart = mid; kg = 4; }                            // (the 64-column kernel's four waves: k-steps w and w + 4 of eight)
   apart += 3.5f + 0.166e-6f * 4.f * n_cols * ((float)d_out + n_heads * head_dim * (gated ? 2.f : 1.f));
-  return pa_gemm_heads_us(d_out, d_in, n_cols, head_dim, kg, n_cu, &whole) < apart ? kg << 28 | whole : 0;
+  return pa_gemm_heads_us(d_out, d_in, n_cols, head_dim, kg, n_cu, &whole) * 1.03f < apart ? kg << 28 | whole : 0;
 }
 // ... whose arithmetic takes rotation tables of a power of two of pairs, on int8 caches whole blocks of them
 bool pa_gemm_heads_serves(const GemmParams& p, const GlueParams& g, int n_cu) {

@@ -88,5 +88,8 @@ def test_pre_step_sizes_take_every_tile():
     every = {tile(heads, dim, n) for heads, d in models for dim in (d, 256, 1024, 8192) for n in range(33, 4097, 13)}
     assert every <= {size[3] for size in HEADS_SIZES} | {(0, 0, 0)}
     assert [tile(*models[0], 512), tile(*models[1], 4096), tile(*models[2], 777)] == [(4, 64, 128), (1, 320, 256), (1, 224, 256)]
+    # 24 / 4-head shape: apart where the estimates tell nothing (up to 256 columns); past them 96 columns a tile only where that is a block of columns more
+    assert {tile(*models[2], n) for n in range(200, 257)} == {(0, 0, 0)} and {tile(*models[2], n) for n in range(257, 289)} == {(1, 128, 256)}
+    assert {tile(*models[2], n) for n in range(289, 385)} == {(1, 96, 256)}
     # a few columns, and sizes whose sums are split as no tile of whole heads splits them: apart
     assert [tile(*models[0], 100), tile(*models[1], 100), tile(*models[1], 256)] == [(0, 0, 0)] * 3
