@@ -242,27 +242,34 @@ def test_verify_exact_two_columns_a_workgroup(shape, n_cols, base, more):
     """Column-exact blocks of more workgroups than the chip holds twice share their whole splits between two columns: odd and even
     numbers of columns, a last column that ends with a whole split (9216, 12160, 6144, 16384 rows) alone or before a change of plan, f16 and f32
     partials, more than eight heads a kv head, int8 caches; and short blocks of one workgroup a column and kv head up to 256 rows, splits past
-    them.  Rows behind a column are infinite: no column may see them."""
+    them.  Every column finite, with its decode's bits, and unchanged when all rows behind it are infinite (int8 caches: 3e4): no column may see them."""
     cfg = dict(SHAPES[shape], verify_exact=True, **more)
     rng = np.random.default_rng(base + n_cols)
     L = base + n_cols
+    far = 3e4 if cfg.get("kv_q8") else np.inf
     q = rng.standard_normal((n_cols, cfg["n_heads"], cfg["head_dim"]), dtype=np.float32)
     with PooledAttn(cfg, L + 5, n_layers=1, max_cols=2048) as pa:
         pa.layer_alloc(0)
         kvd = pa.kv_dim
-        for r in range(0, L, 2048):
-            n = min(2048, L - r)
-            k, v = rng.standard_normal((2, n, kvd), dtype=np.float32)
-            if not cfg.get("kv_q8"):
-                v[max(0, base + 1 - r):] = np.inf
+
+        def store(r, k, v):
             dk, dv = pa.to_device(k), pa.to_device(v)
-            pa.kv_store(0, dk, kvd, dv, kvd, r, n)
+            pa.kv_store(0, dk, kvd, dv, kvd, r, len(k))
             pa.sync()
+
+        for r in range(0, base, 2048):
+            store(r, *rng.standard_normal((2, min(2048, base - r), kvd), dtype=np.float32))
+        k, v = rng.standard_normal((2, n_cols + 5, kvd), dtype=np.float32)
+        behind = lambda c: np.where(np.arange(n_cols + 5)[:, None] > c, np.float32(far), v)   # noqa: E731
+        store(base, k, behind(n_cols - 1))
         multi = pa.run_attn("decode", 0, q, base)
-        assert np.isfinite(multi[0]).all()
+        assert np.isfinite(multi).all()
         for c in range(n_cols):
             single = pa.run_attn("decode", 0, q[c:c + 1], base + c)
             assert np.array_equal(single[0].view(np.uint32), multi[c].view(np.uint32)), "column %d differs from its decode" % c
+        for c in range(n_cols - 1):
+            store(base, k, behind(c))
+            assert np.array_equal(pa.run_attn("decode", 0, q, base)[c].view(np.uint32), multi[c].view(np.uint32)), "column %d sees rows behind it" % c
 
 
 @pytest.mark.parametrize("shape,n_cols,base", [("qwen36_moe", 1, 200), ("qwen3_1p7b", 1, 256), ("qwen3_1p7b", 5, 120), ("qwen36_moe", 4, 250)])
