@@ -434,20 +434,21 @@ static hipError_t launch_prefill_k(const AttnParams& p, uint32_t col_groups, uin
 // 614 / 587, at 16384 979 / 965, at 32768 1748 / 1733, at 124K 6286 / 6269; 2650 columns of the 24 / 4-head shape at 4096 370 / 356, at 8192 555 / 551, at
 // 16384 927 / 929; 158 workgroups, 2500 columns of the first at 8192 456 / 440, at 16384 763 / 754, at 32768 1387 / 1386, at 64K 2618 / 2646.
 // Head_dim 128 stays ahead (4096 columns at 28672 920 / 888).
-template <int HD>
-static bool pairs_pay(const AttnParams& p, uint32_t total, uint32_t n_cu) {
-  return HD == 128 || (uint64_t)p.base_pos * total <= 6ull * p.n_cols * n_cu;
+static bool pairs_pay(uint32_t hd, uint32_t base_pos, uint32_t n_cols, uint32_t total, uint32_t n_cu) {
+  return hd == 128 || (uint64_t)base_pos * total <= 6ull * n_cols * n_cu;
+}
+extern "C" int pa_rule_prefill_paired(uint32_t hd, uint32_t base_pos, uint32_t n_cols, uint32_t group, uint32_t n_kv_heads, uint32_t n_splits, uint32_t col_groups, uint32_t n_cu) {
+  const uint32_t half = PF_ROWS / 2 / group, total = col_groups * n_kv_heads * n_splits;
+  return n_splits == 1 && half > 0 && total <= n_cu && ((n_cols + half - 1) / half + 1) / 2 == col_groups && pairs_pay(hd, base_pos, n_cols, total, n_cu);
 }
 
 template <int HD, int W>
 static hipError_t launch_prefill_t(const AttnParams& p, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t) {
-  const uint32_t half = W / 2 * 32 / p.group;
-  const uint32_t total = col_groups * p.n_kv_heads * p.n_splits;
-  const bool one_round = total <= n_cu;
-  if (p.n_splits == 1 && half > 0 && one_round && ((p.n_cols + half - 1) / half + 1) / 2 == col_groups && pairs_pay<HD>(p, total, n_cu))
-    return launch_prefill_k<HD, W, true>(p, col_groups, half, 0, s, t);
+  static_assert(W * 32 == PF_ROWS, "the rule's rows of a workgroup");
+  if (pa_rule_prefill_paired(HD, p.base_pos, p.n_cols, p.group, p.n_kv_heads, p.n_splits, col_groups, n_cu))
+    return launch_prefill_k<HD, W, true>(p, col_groups, PF_ROWS / 2 / p.group, 0, s, t);
   // more workgroups than the chip holds at once: the longest blocks first
-  const uint32_t head_xcds = p.n_splits == 1 && !one_round && 8 % p.n_kv_heads == 0 ? 8 / p.n_kv_heads : 0;
+  const uint32_t head_xcds = p.n_splits == 1 && col_groups * p.n_kv_heads > n_cu && 8 % p.n_kv_heads == 0 ? 8 / p.n_kv_heads : 0;
   return launch_prefill_k<HD, W, false>(p, col_groups, 0, head_xcds, s, t);
 }
 

@@ -14,6 +14,7 @@ typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
 #define NEG_INF (-__builtin_inff())
 #define PF_TN 32                 // positions per step
+#define PF_ROWS 256              // stacked rows of a workgroup
 #ifndef PF_KD
 #define PF_KD 3                  // K fragments (two MFMAs each) fetched ahead
 #endif

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 from oracle import attn_oracle as O
 from oracle import c_oracle as C
+from pooled_amd import capi
 from pooled_amd.capi import PooledAttn, PA_OUT_F16
 from helpers import SHAPES, assert_parity, random_cache, oracle_cache
 
@@ -57,15 +58,16 @@ def test_prefill_paired_halves(shape, base, n):
     assert_parity(got, ref, "paired %s base %d n %d" % (shape, base, n))
 
 
-@pytest.mark.parametrize("base,n", [(3000, 1000), (3200, 1000), (3300, 1010), (9000, 1024)])
-def test_prefill_long_context_keeps_whole_blocks(base, n):
+@pytest.mark.parametrize("base,n,paired", [(3000, 1000, 1), (3200, 1000, 1), (3300, 1010, 1), (6107, 1010, 1), (6144, 1000, 1), (6145, 1000, 0), (6108, 1010, 0), (9000, 1024, 0)])
+def test_prefill_long_context_keeps_whole_blocks(base, n, paired):
     """At head_dim 256 an unsplit pass that fills the chip pairs half blocks only while base_pos x workgroups is within 6 x n_cols x
-    CUs (all but the last case on a 256-CU part); past that the blocks stay whole: either side of the line, a ragged last block."""
+    CUs (on a 256-CU part); past that the blocks stay whole: either side of the line, full and ragged last blocks on both."""
     cfg = dict(SHAPES["qwen36_moe"], n_heads=64, n_kv_heads=2)                      # 32 heads a kv head: blocks of eight columns
     rows = sorted(set(range(0, n, 50)) | set(range(5)) | set(range(n - 5, n)))
     got, ref, plan = _prefill(cfg, base, n, seed=base + n, check_rows=rows)
     assert plan["kernel"] == 1 and plan["n_splits"] == 1 and plan["col_groups"] * 2 == 2 * -(-n // 8) <= 256
-    assert_parity(got, ref, "whole blocks at base %d n %d" % (base, n))
+    assert capi.load().pa_rule_prefill_paired(256, base, n, 32, 2, 1, plan["col_groups"], 256) == paired
+    assert_parity(got, ref, "%s at base %d n %d" % ("pairs" if paired else "whole blocks", base, n))
 
 
 @pytest.mark.parametrize("shape,base,n", [("qwen36_moe", 0, 33), ("qwen36_moe", 31, 17), ("qwen36_moe", 64, 514), ("qwen38_27b", 10, 106),
