@@ -197,6 +197,34 @@ def test_c5_prefill_128k_row_sample():
     assert_parity(got, ref, "C5 prefill 128K, column sample", tight=True)
 
 
+@pytest.mark.parametrize("shape,base,n", [("qwen36_moe", 300, 40), ("qwen3_1p7b", 200, 120), ("qwen38_27b", 5000, 64)])
+@pytest.mark.parametrize("one_row", [False, True])
+@pytest.mark.parametrize("jump", [5.3, 5.5, 5.6, 6.0, 10.9, 11.2, 12.0])
+def test_prefill_jumps_around_the_raise(shape, base, n, one_row, jump):
+    """References are raised where a probability is past 2^8 (a score 5.55 above the reference) on its f16 value, which is infinite from 2^16 on (11.09):
+    a flat context whose scores jump once by a little less and a little more than either, for all rows of a wave and for one row among others that
+    must not notice; every row against the oracle, whole and split contexts."""
+    cfg = SHAPES[shape]
+    nH, nKV, hd = cfg["n_heads"], cfg["n_kv_heads"], cfg["head_dim"]
+    rng = np.random.default_rng(base + n)
+    rows = base + n
+    k = rng.standard_normal((rows, nKV, hd)).astype(np.float32) * 0.02
+    k[:, :, 0] = jump * (np.arange(rows) >= rows // 2)[:, None]   # q's first value is sqrt(hd) or 0: it adds the jump to a row's scores or not
+    k16 = k.astype(np.float16).view(np.uint16)
+    v16 = rng.standard_normal((rows, nKV, hd)).astype(np.float16).view(np.uint16)
+    q = rng.standard_normal((n, nH, hd)).astype(np.float16).astype(np.float32)
+    q[:, :, 0] = 0 if one_row else hd ** 0.5
+    q[n // 2, 0, 0] = hd ** 0.5
+    q = q.astype(np.float16).astype(np.float32)                   # f16 queries: the scores carry no rounding of q
+    ref = C.attention(q, k16, v16, base, gate=None, rows=list(range(n)))
+    with PooledAttn(cfg, rows + 3, n_layers=1, max_cols=n) as pa:
+        pa.layer_alloc(0); pa.kv_write(0, 0, 0, k16); pa.kv_write(0, 1, 0, v16)
+        pa.set_prefill_tile(1)
+        assert pa.plan("prefill", base, n)["kernel"] == 1
+        got = pa.run_attn("prefill", 0, q, base)
+    assert_parity(got.astype(np.float32), ref, "jump %g %s" % (jump, shape))
+
+
 @pytest.mark.parametrize("shape,base,n,tile", [("qwen36_moe", 0, 40, 1), ("qwen36_moe", 900, 33, 1), ("qwen3_1p7b", 70, 300, 1), ("qwen38_27b", 5000, 64, 1)])
 @pytest.mark.parametrize("trend", ["up", "down", "jump", "late"])
 def test_prefill_reference_maxima(shape, base, n, tile, trend):
