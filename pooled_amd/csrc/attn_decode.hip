@@ -99,6 +99,14 @@ static __device__ inline float quads_sum(float v) {
   return rows_sum(v);
 }
 
+// two splits' values and the own row's under their weights, rounded as the merge kernel rounds them (its group 0 holds the first split and the own
+// row, its group 1 the second)
+static __device__ inline float merge_two(float a, float wa, float b, float wb, float own, float wo) {
+#pragma clang fp contract(off)
+  const float g0 = __builtin_fmaf(own, wo, a * wa), g1 = b * wb;
+  return g0 + g1;
+}
+
 // 16 int8 values x scale -> 16 f16 (see the Q8 note at the kernel)
 static __device__ inline void dq16(const u4 raw, const float sc, h8& lo, h8& hi) {
   const h2 s2 = { (_Float16)sc, (_Float16)sc };
@@ -215,7 +223,8 @@ template <int HD> struct DecShape {
 // both -- the K/V tiles are loaded and staged once, everything behind them is done per block as the one-column decode does it, bit for bit.
 //
 // SR with eight waves (a one-column decode of at most 256 rows): the kv head's whole context in one workgroup, which also merges the column's own
-// row, normalises, gates and stores the output: no partials, no merge launch.
+// row, normalises, gates and stores the output: no partials, no merge launch.  Its waves are two splits of four, rows, sums and merge as two
+// workgroups and the merge kernel have them, so the bits are those of the two launches.
 //
 // SR (single-round splits; one 16-row block, or two of a verify block): splits are one tile per wave (split_len = W x
 // 32); the product O^T = V^T P^T of a split is divided over the waves by output dims, see the code.  Without SR every wave
@@ -235,6 +244,7 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
   static_assert(!EX2 || (SR && NB == 2 && !FUSED && !GATHER), "two columns of a column-exact block: two row blocks of single-round splits");
   p.f_q_in = a_f_q_in; p.group = a_group; p.f_q_head_stride = a_f_q_head_stride;
   const uint32_t grid_x = a_grid_x;
+  static_assert(!SR || W == 4 || ONE, "the waves of a split");
   static_assert(!SR || NB == 1 || (NB == 2 && W == 4 && !FUSED && !GATHER), "single-round splits: one 16-row block, or two of a verify block");
   static_assert(!FUSED || NB == 1, "the fused pre-step serves one column");
   static_assert(!GATHER || (NB == 1 && !FUSED), "the gather mode serves one column per workgroup");
@@ -340,9 +350,10 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
   uint32_t ilv_nw = 0, ilv_wv = 0;
   bool ilv = false;
   if constexpr (ILV) {
-    const uint32_t nfull = min(p.n_splits, seq_max / split_len);
-    ilv = sp < nfull;
-    ilv_nw = nfull * W;
+    // (ONE: its waves 0 - 3 and 4 - 7 are two such splits of four)
+    const uint32_t nfull = ONE ? seq_max / 128 : min(p.n_splits, seq_max / split_len);
+    ilv = (ONE ? (uint32_t)__builtin_amdgcn_readfirstlane(wave) / 4 : sp) < nfull;
+    ilv_nw = nfull * (ONE ? 4 : W);
     ilv_wv = sp * W + (threadIdx.x >> 6);
   }
   // cache row of row r (0 .. 31) of the tile at tile_pos
@@ -849,9 +860,20 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) *(h8*)(p_lds + ((wave * NB + nb) * 64 + lane) * 16) = pfs[nb];
       }
+      // ONE: the gate of the wave's slice of a row, requested ahead of the barrier
+      f4 gtv[ONE ? DBW : 1];
+      const uint32_t o_row = min(ln, G - 1);
+      if constexpr (ONE) {
+#pragma unroll
+        for (int j = 0; j < DBW; j++)
+          gtv[j] = p.gate ? *(const f4*)(p.gate + (size_t)c0 * p.gate_stride + (size_t)(g * G + o_row) * p.gate_head_stride + (wave * DBW + j) * 16 + 4 * kg) : (f4){0.f, 0.f, 0.f, 0.f};
+      }
       if (kg == 0) {
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) { mex[wave * 16 * NB + nb * 16 + ln] = mxs[nb]; lex[wave * 16 * NB + nb * 16 + ln] = pss[nb]; }
+        for (int nb = 0; nb < NB; nb++) {
+          const uint32_t at = ONE ? ln * W + wave : wave * 16 * NB + nb * 16 + ln;   // (ONE reads a row's eight values 16 bytes at a time)
+          mex[at] = mxs[nb]; lex[at] = pss[nb];
+        }
       }
       __syncthreads();
       {
@@ -868,6 +890,36 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
           lor[slot] = lds_read_tr16(vp);
           hir[slot] = lds_read_tr16(vp + 16 * S::VROW);
         };
+        // ONE: what the sums need besides the products -- two splits of four waves and the own row, merged as the merge kernel does it: the bits
+        // of the two launches.  Worked out here, under the reads of the products' operands, and with a row's eight (m, l) 16 bytes at a time (us a step, dense
+        // hd-128 shape at 203 rows: behind the products 5.59, here 5.51, wide reads 5.41; a one-level merge with other bits 5.50).
+        float cw[ONE ? W : 1], w0 = 0.f, w1 = 0.f, wo = 0.f, inv = 0.f;
+        bool dead1[ONE ? W : 1];
+        h4 v1[ONE ? DBW : 1];
+        if constexpr (ONE) {
+          float mw[W], lw[W], Ms[2], Ls[2];
+#pragma unroll
+          for (int h = 0; h < 2; h++) { *(f4*)(mw + 4 * h) = *(const f4*)(mex + ln * W + 4 * h); *(f4*)(lw + 4 * h) = *(const f4*)(lex + ln * W + 4 * h); }
+          const float own = own_s[o_row];
+#pragma unroll
+          for (int j = 0; j < DBW; j++) v1[j] = *(const h4*)(own_v + (wave * DBW + j) * 16 + 4 * kg);
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            Ms[h] = NEG_INF; Ls[h] = 0.f;
+#pragma unroll
+            for (int w2 = 4 * h; w2 < 4 * h + 4; w2++) Ms[h] = fmaxf(Ms[h], mw[w2]);
+            const float m_safe = Ms[h] == NEG_INF ? 0.f : Ms[h];
+#pragma unroll
+            for (int w2 = 4 * h; w2 < 4 * h + 4; w2++) {
+              dead1[w2] = mw[w2] == NEG_INF;                                   // a wave without a tile
+              cw[w2] = dead1[w2] ? 0.f : __expf(mw[w2] - m_safe);
+              Ls[h] += lw[w2] * cw[w2];
+            }
+          }
+          const float Mx = fmaxf(fmaxf(Ms[0], Ms[1]), own);
+          w0 = __expf(Ms[0] - Mx); w1 = __expf(Ms[1] - Mx); wo = __expf(own - Mx);
+          inv = __builtin_amdgcn_rcpf(merge_two(Ls[0], w0, Ls[1], w1, 1.f, wo));   // (v_rcp_f32, 1 ulp, as there)
+        }
 #pragma unroll
         for (int w2 = 0; w2 < W; w2++) {
           if constexpr (NB == 1) pfr[w2][0] = *(const h8*)(stage_all + w2 * S::STAGE + (lane >> 1) * S::VROW + HD * 2 + (lane & 1) * 16);
@@ -895,22 +947,33 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
           if (st + VD < NS) __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
           __builtin_amdgcn_sched_group_barrier(0x008, NB, 1);
         }
-        // ONE: the gate of the wave's slice of a row, requested ahead of the sums
-        f4 gtv[ONE ? DBW : 1];
-        const uint32_t o_row = min(ln, G - 1);
+        // a wave without a tile staged stale rows: its m is -inf, and its products must not reach O even as 0 x NaN
         if constexpr (ONE) {
 #pragma unroll
-          for (int j = 0; j < DBW; j++)
-            gtv[j] = p.gate ? *(const f4*)(p.gate + (size_t)c0 * p.gate_stride + (size_t)(g * G + o_row) * p.gate_head_stride + (wave * DBW + j) * 16 + 4 * kg) : (f4){0.f, 0.f, 0.f, 0.f};
+          for (int j = 0; j < DBW; j++) {
+            f4 o[2] = { (f4){0.f, 0.f, 0.f, 0.f}, (f4){0.f, 0.f, 0.f, 0.f} };
+#pragma unroll
+            for (int w2 = 0; w2 < W; w2++) o[w2 / 4] += (dead1[w2] ? (f4){0.f, 0.f, 0.f, 0.f} : pr[w2][j][0]) * cw[w2];
+            const uint32_t d = (wave * DBW + j) * 16 + 4 * kg;
+            f4 r;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              r[i] = merge_two(o[0][i], w0, o[1][i], w1, (float)v1[j][i], wo) * inv;
+              if (p.gate) r[i] *= __builtin_amdgcn_rcpf(1.f + __expf(-gtv[j][i]));
+            }
+            if (ln < G) {
+              const size_t at = (size_t)c0 * p.out_stride + (size_t)(g * G + ln) * HD + d;
+              if (p.out_f16) *(h4*)((_Float16*)p.out + at) = (h4){ (_Float16)r[0], (_Float16)r[1], (_Float16)r[2], (_Float16)r[3] };
+              else *(f4*)((float*)p.out + at) = r;
+            }
+          }
+          return;
         }
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) {
-          // a wave without a tile staged stale rows: its m is -inf, and its products must not reach O even as 0 x NaN
           float mw[W], lw[W], M = NEG_INF;
 #pragma unroll
           for (int w2 = 0; w2 < W; w2++) { mw[w2] = mex[w2 * 16 * NB + nb * 16 + ln]; lw[w2] = lex[w2 * 16 * NB + nb * 16 + ln]; M = fmaxf(M, mw[w2]); }
-          const float own = ONE ? own_s[o_row] : NEG_INF;
-          if constexpr (ONE) M = fmaxf(M, own);
           const float m_safe = M == NEG_INF ? 0.f : M;
           float Lr = 0.f;
           f4 o[DBW];
@@ -923,28 +986,6 @@ void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a
             Lr += lw[w2] * c;
 #pragma unroll
             for (int j = 0; j < DBW; j++) o[j] += (dead ? (f4){0.f, 0.f, 0.f, 0.f} : pr[w2][j][nb]) * c;
-          }
-          if constexpr (ONE) {
-            const float c = __expf(own - m_safe);
-            Lr += c;
-            const float inv = __builtin_amdgcn_rcpf(Lr);               // (v_rcp_f32, 1 ulp, as in the merge kernels)
-#pragma unroll
-            for (int j = 0; j < DBW; j++) {
-              const uint32_t d = (wave * DBW + j) * 16 + 4 * kg;
-              const h4 v = *(const h4*)(own_v + d);
-              f4 r;
-#pragma unroll
-              for (int i = 0; i < 4; i++) {
-                r[i] = (o[j][i] + (float)v[i] * c) * inv;
-                if (p.gate) r[i] *= __builtin_amdgcn_rcpf(1.f + __expf(-gtv[j][i]));
-              }
-              if (ln < G) {
-                const size_t at = (size_t)c0 * p.out_stride + (size_t)(g * G + ln) * HD + d;
-                if (p.out_f16) *(h4*)((_Float16*)p.out + at) = (h4){ (_Float16)r[0], (_Float16)r[1], (_Float16)r[2], (_Float16)r[3] };
-                else *(f4*)((float*)p.out + at) = r;
-              }
-            }
-            return;
           }
           const uint32_t r = nb * 16 + ln;
           if (EX2 ? ln < G && (uint32_t)nb < ncl : r < R) {

@@ -52,6 +52,34 @@ def test_decode_step_matches_oracle_and_unfused(shape, pos):
     assert np.array_equal(got.view(np.uint32), unf[0].view(np.uint32)), "fused output differs from pa_glue_kv + pa_attn_decode"
 
 
+@pytest.mark.parametrize("shape,more", [("qwen36_moe", {}), ("qwen36_moe", dict(kv_q8=True)), ("qwen38_27b", {}), ("qwen3_1p7b", {}), ("qwen3_1p7b", dict(kv_q8=True)),
+                                        ("qwen3_1p7b", dict(n_heads=13, n_kv_heads=1, gate=True))])
+def test_one_workgroup_has_the_bits_of_splits_and_a_merge(shape, more):
+    """One workgroup a kv head over at most 256 rows takes the rows, the sums and the merge of two splits of 128 in their order: the bits of the same
+    pass as splits behind a merge launch (a splits override of two), through the fused step and through pa_attn_decode, f32 and f16 output."""
+    cfg = dict(SHAPES[shape], **more)
+    rows = 260
+    rng = np.random.default_rng(rows)
+    kvd = cfg["n_kv_heads"] * cfg["head_dim"]
+    with PooledAttn(cfg, rows, n_layers=1, max_cols=rows) as pa:
+        pa.layer_alloc(0)
+        k, v = (pa.to_device(a) for a in rng.standard_normal((2, rows, kvd), dtype=np.float32))
+        pa.kv_store(0, k, kvd, v, kvd, 0, rows)
+        for pos in (0, 1, 32, 33, 96, 127, 128, 129, 160, 203, 224, 255, 256):
+            d = O.make_inputs(cfg, 0, 1, pos)
+            q = rng.standard_normal((1, cfg["n_heads"], cfg["head_dim"]), dtype=np.float32)
+            gate = rng.standard_normal(q.shape, dtype=np.float32) if cfg.get("gate") else None
+            got = []
+            for splits in (0, 2):
+                pa.set_decode_splits(splits)
+                pl = pa.plan("decode", pos, 1)
+                assert (pl["waves"], pl["split_len"]) == ((4, 128) if splits else (8, 256)), pl
+                got.append([pa.run_decode_step(0, d["qraw"][0], d["kraw"][0], d["vraw"][0], d["qw"], d["kw"], pos, t) for t in (0, PA_OUT_F16)] +
+                           [pa.run_attn("decode", 0, q, pos, gate=gate, out_dtype=t) for t in (0, PA_OUT_F16)])
+            for a, b in zip(*got):
+                assert np.isfinite(a.astype(np.float32)).all() and np.array_equal(a, b), (pos, a.dtype)
+
+
 @pytest.mark.parametrize("shape", ["qwen36_moe", "qwen3_1p7b"])
 def test_decode_step_output_over_its_inputs(shape):
     """The output of a step of one workgroup a kv head may lie over anything that the step reads: over q, k and v (one buffer, as a fused projection
