@@ -43,10 +43,13 @@ extern "C" {
                                  (its own splits, its own row block): column c then has the bits of pa_attn_decode(base_pos + c,
                                  n_cols = 1), the invariant the reference states for its pair (engine/wgsl/attn_dec.js:12-16,
                                  tests/test_attn_dec.js:89-97) and its speculative decoding leans on (spec greedy == plain
-                                 greedy).  Cost: every column streams the K/V rows through its own workgroups; a block whose
-                                 columns share one one-column plan runs as one pass in which a split's columns sit side by
-                                 side on one L2 (about 2.3x the default block's time), a block that straddles a change of
-                                 plan as one pass per column.  Off by default: see the note at pa_attn_decode. */
+                                 greedy), whether the decodes ran in a context with the flag or without.  Cost: a block whose columns
+                                 share one one-column plan runs as one pass in which a split's columns sit side by side on one
+                                 L2, each with workgroups of its own or, in larger blocks, two columns to a workgroup; a
+                                 block that straddles a change of plan as one pass per run of columns.  Up to 2.3x the default block's
+                                 time (attention of the 16 / 2-head shape, us a call without / with the flag: 8 columns at 12000
+                                 rows 16.4 / 19.2; 2, 8 and 16 columns at 30000 16.4 / 17.5, 22.3 / 41.9, 32.3 / 74.7).
+                                 Off by default: see the note at pa_attn_decode. */
 
 /* output element types */
 #define PA_OUT_F32 0          /* the engine's attnOut feeding wo (engine/qwen35.js:881) */
@@ -74,15 +77,16 @@ typedef struct pa_ctx pa_ctx;
  * formulas: engine/autotune.js:10-68, engine/wgsl/attn_dec.js:40-48, engine/wgsl/attn_tile.js:43-56). */
 typedef struct pa_plan {
   uint32_t kernel;       /* 0 = split-K decode/verify kernel, 1 = MFMA prefill kernel */
-  uint32_t split_len;    /* cache rows per split (split-K kernel with more than 128 rows a split: the rows of a split's
-                            32-row tiles, which are dealt round robin to the splits of a kv head, not one contiguous range) */
+  uint32_t split_len;    /* cache rows per split (split-K kernel with more than 128 rows a split and more than one split: the rows of
+                            a split's 32-row tiles, which are dealt round robin to the splits of a kv head, not one contiguous range;
+                            a one-column decode of at most 256 rows is one split of 256) */
   uint32_t n_splits;     /* splits over the streamed rows; a one-column decode streams rows 0 .. base_pos - 1 */
   uint32_t col_groups;   /* column groups (workgroups = n_splits x kv heads x col_groups) */
   uint32_t cols_per_group;
   uint32_t waves;        /* wavefronts per workgroup */
   uint32_t row_blocks;   /* 16-row (decode) or 32-row (prefill) query blocks per workgroup */
-  uint32_t slots;        /* partial slots per (column, head) the pass needs: n_splits, + 1 for a one-column decode, whose
-                            own row base_pos is a partial of its own */
+  uint32_t slots;        /* partial slots per (column, head) of the pass: n_splits, + 1 for a one-column decode, whose own row base_pos
+                            is a partial of its own (a pass of one split that writes its output itself uses none of them) */
 } pa_plan;
 
 /* ---- life cycle (replaces Qwen35Engine / DenseEngine buffer creation, engine/qwen35.js:871-890,
@@ -289,7 +293,7 @@ int pa_gemv_norm(pa_ctx* ctx, const pa_weight* w, const float* d_x_raw, const fl
  * attention -> merge + gate -> output projection accumulated into the residual.  w_qkv: rows [q (n_heads x head_dim,
  * x 2 with PA_FLAG_GATE: q | gate interleaved per head) | k | v] x dim, one fused weight (the reference fuses k | v,
  * engine/qwen35.js:1109-1114); w_o: dim x (n_heads x head_dim).  d_x [dim] is read and updated in place.  Four
- * launches: normed GEMV, fused decode step (2), accumulating GEMV.  f16 or int8 caches. */
+ * launches: normed GEMV, fused decode step (2; 1 over at most 256 rows), accumulating GEMV.  f16 or int8 caches. */
 int pa_attn_layer_decode(pa_ctx* ctx, uint32_t layer, const pa_weight* w_qkv, const pa_weight* w_o, const float* d_attn_norm_w,
                          const float* d_qw, const float* d_kw, float* d_x, uint32_t pos);
 
@@ -316,8 +320,8 @@ int pa_set_weight_cache(pa_ctx* ctx, size_t max_bytes);
 /* n_cols tokens at positions base_pos .. through the attention half of a full-attention layer, as
  * _encodeLayerBatch / _encodeLayerWide record it (engine/qwen35.js:2416-2425, :2827): rmsnorm -> [q | k | v] GEMM ->
  * pre-step + cache write -> causal attention -> gate -> wo GEMM accumulated into the residual columns d_x
- * [n_cols][x_stride] (f32, read and updated in place).  Weights as pa_attn_layer_decode.  Five launches (six when
- * the attention pass is split).  n_cols <= max_cols.  On int8 caches one more launch widens the visible rows for the
+ * [n_cols][x_stride] (f32, read and updated in place).  Weights as pa_attn_layer_decode.  Five launches (one more when
+ * the attention pass is split, one less where a wide chunk's [q | k | v] GEMM ends with the pre-step and the cache write).  n_cols <= max_cols.  On int8 caches one more launch widens the visible rows for the
  * prefill kernel (as pa_attn_prefill on such caches). */
 int pa_attn_layer_prefill(pa_ctx* ctx, uint32_t layer, const pa_weight* w_qkv, const pa_weight* w_o, const float* d_attn_norm_w,
                           const float* d_qw, const float* d_kw, float* d_x, uint32_t x_stride, uint32_t base_pos, uint32_t n_cols);

@@ -277,7 +277,7 @@ extern "C" uint32_t pa_rule_gemm_wide_tile(uint32_t d_out, uint32_t d_in, uint32
 // where the two apart are the faster form -- the tiles that hold whole heads are few, and below some 200 - 300 columns (64-column tiles of too
 // few workgroups) they cost more than the pre-step's launch, 3.5 us and the f32 projections through memory at 6 TB/s (16 columns 3.9 us, 512 of
 // the 16 / 8-head shape 6.5, 777 of the 24 / 4-head shape 19.6, 4096 of the 16 / 2-head shape 53.5).  Only tiles that split K as the call apart does:
-// a projection is its bits.  Taken where its estimate is 3 % ahead: closer than that the estimates do not tell which is faster (24 / 4-head shape, 214 - 256 columns,
+// a projection has its bits.  Taken where its estimate is 3 % ahead: closer than that the estimates do not tell which is faster (24 / 4-head shape, 214 - 256 columns,
 // estimates within 1.2 %: 118 - 126 us a layer apart, up to 1 % more so from position 0, up to 1 % less behind 1000 rows).  On 238 sizes (the three model
 // shapes, 33 to 4096 columns) the choice is 7 % ahead of always apart (best 22 %) and at no size behind it.
 extern "C" uint32_t pa_rule_gemm_heads(uint32_t d_out, uint32_t d_in, uint32_t n_cols, uint32_t n_heads, uint32_t head_dim, int gated, int n_cu) {

@@ -40,7 +40,7 @@ class HipAttention {
     this.kvQ8 = !!opts.kvQ8;                                       // int8 caches (engine option kvQ8)
     // verifyExact: every column of a verify block is run as the one-column decode at its position, so it has the bits
     // of a sequential decode (the reference's invariant, engine/wgsl/attn_dec.js:12-16); every column then does a
-    // one-column decode's work (about 2.3x the default block's time).  Off by default: a block's columns then agree with sequential decodes to rounding only.
+    // one-column decode's work (up to 2.3x the default block's time).  Off by default: a block's columns then agree with sequential decodes to rounding only.
     this.verifyExact = !!opts.verifyExact;
     const flags = (this.qkNorm ? PA_FLAG_QK_NORM : 0) | (this.gate ? PA_FLAG_GATE : 0) | (this.kvQ8 ? PA_FLAG_KV_Q8 : 0) | (this.verifyExact ? PA_FLAG_VERIFY_EXACT : 0);
     // a readable throw at create, like the engine's KV binding check (engine/qwen35.js:378-383)
