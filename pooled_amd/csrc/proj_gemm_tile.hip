@@ -197,6 +197,11 @@ static __device__ inline void finish_heads(const GlueParams& g, unsigned char* l
   }
 }
 
+// The swizzle of 64-byte activation rows (KG = 1): chunk c of row r sits at c ^ (0, 2, 3, 1)[r / 4 % 4].  A 128-bit LDS read takes 16 lanes a clock, of a 16-row fragment rows 0 - 3 and
+// 12 - 15 of one k quarter with rows 4 - 11 of the next: the four of r / 4 have to differ over those too, which (0, 1, 2, 3) does not give (rows 0 - 3 of
+// quarter 0 and 4 - 7 of quarter 1 on the same banks: every activation read twice as long).
+static __device__ inline uint32_t gt_swz64(uint32_t r) { return ((r >> 3) & 1) | (((r >> 2 ^ r >> 3) & 1) << 1); }
+
 // The main loop of the shapes whose waves each hold whole sums (KG = 1), on 16 x 16 x 32 products: at the power limit they run faster than 32 x 32 x 16
 // ones (half the accumulator traffic a product), and give the same bits.  Layer pass, 32 x 32 x 16 / so (us a layer): 4096 columns of the gated 16 / 2-head
 // shape 430 / 408, 2048 of it 231 / 226, 2048 of the 24 / 4-head shape 534 / 510; one round of few workgroups (777 of that shape) 297 / 297.  A stage is one k-step of 32: the products with the first half of a wave's column blocks, the barrier,
@@ -216,7 +221,7 @@ static __device__ __attribute__((always_inline)) inline void gt_whole_k(const Ge
 #pragma unroll
   for (int j = 0; j < S; j++) issue(j, j);
   // k 8 kq .. of a row: an activation row's chunk kq; of the weights' fragments, the half kq % 2 of k-step kq / 2
-  const uint32_t x_rd = (wm * TM * 32 + l16) * 64 + ((kq ^ ((l16 >> 2) & 3)) * 16), w_rd = ABYTES + wn * TN * 2048 + (kq >> 1) * 1024 + ((kq & 1) * 32 + l16) * 16;
+  const uint32_t x_rd = (wm * TM * 32 + l16) * 64 + ((kq ^ gt_swz64(l16)) * 16), w_rd = ABYTES + wn * TN * 2048 + (kq >> 1) * 1024 + ((kq & 1) * 32 + l16) * 16;
   h8 x0[TM], x1[TM], w[NB];
   auto rd_x = [&](h8& f, const unsigned char* sb, int a) __attribute__((always_inline)) { f = *(const h8*)(sb + x_rd + a * 1024); };
   auto rd_w = [&](h8& f, const unsigned char* sb, int b) __attribute__((always_inline)) { f = *(const h8*)(sb + w_rd + (b / 2) * 2048 + (b % 2) * 256); };
@@ -346,7 +351,7 @@ __global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p, 
   }
   const uint32_t c0 = cb * BM, r0 = rb_ * BN;
   const uint32_t n_stages = p.d_in / BK, n_rb32 = (p.d_out + 31) / 32;
-  auto swz = [](uint32_t r) __attribute__((always_inline)) -> uint32_t { return BK >= 128 ? r & 15 : BK == 64 ? (r >> 1) & 7 : (r >> 2) & 3; };
+  auto swz = [](uint32_t r) __attribute__((always_inline)) -> uint32_t { return BK >= 128 ? r & 15 : BK == 64 ? (r >> 1) & 7 : gt_swz64(r); };
 
   const unsigned char* xb = (const unsigned char*)(p.x + (size_t)c0 * p.x_stride);
   // load q of a stage fills the q-th KB of its buffer: ALD pieces of activations, then BLD weight fragments.  Wave w takes
