@@ -142,6 +142,7 @@ hipError_t pa_launch_gemm_heads(const GemmParams& p, const uint16_t* w16, const 
 // its kernel for larger tiles (proj_gemm_tile.hip), and what a call would take there, on which tile (columns << 16 | rows)
 float pa_gemm_tile_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, uint32_t* shape, uint32_t* kg);
 // the rules that pick an instance by size, in plain C: the tests ask them which instances their sizes take
+extern "C" uint32_t pa_rule_gemv_resident(int kind, uint32_t d_out, int norm, int n_cu);
 extern "C" uint32_t pa_rule_gemv_wide_rows(int kind, uint32_t d_out, uint32_t d_in, int norm, int n_cu);
 extern "C" int pa_rule_gemm_few_groups(int kind, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu);
 extern "C" int pa_rule_gemm_few_dot(int kind, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu);

@@ -18,6 +18,7 @@
 // the additions differs from the reference's workgroup tree (the parity tests use a tolerance, as the reference's do).
 #include "pa_internal.h"
 #include "glue_math.h"
+#include <algorithm>
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
@@ -95,9 +96,19 @@ void pa_gemv_kernel(const float* a_x, const float* a_norm_w, const void* a_w, co
   // batch of scalar loads (the compiler would fetch each where it is first used, a dependent round trip each).
   GemvParams p = p_in;
   p.x = a_x; p.norm_w = a_norm_w; p.w = a_w; p.scales = a_scales; p.y = a_y; p.d_out = a_d_out; p.d_in = a_d_in;
+  // Up to 4096 inputs, and for up to three rows, a wave's rows are all requested at once; past that it keeps two or three in flight and asks for the next when
+  // one is consumed.  With everything requested in front, a wave sat in the issue of its loads while the memory pipeline was full (of 14336 x 5120 Q4_0, seven rows a wave:
+  // until 4.3 us after the first wave's entry on average, 7.4 at the latest), staged x behind that and did all of its arithmetic, 3 us, behind the last
+  // byte; so the arithmetic runs under the stream (12.5 -> 10.8 us; 16384 x 5120 14.1 -> 11.9, 14336 x 8192 18.5 -> 14.3; one row in flight 13.3, three 11.0;
+  // without the norm three are ahead, 12288 x 6144 10.35 / 10.15).  The rows of a wave are then dealt one of every 4 x gridDim.x: at any time the chip reads one
+  // range of the matrix (10.8 -> 10.5 us), and the waves' counts differ by one at most.
+  constexpr int AHEAD = BPL < 3 || KIND == PA_W_F32 || RW <= 3 ? RW : KIND == PA_W_Q4_0 && BPL == 3 && !NORM && RW >= 5 ? 3 : 2;
+  constexpr bool STREAM = RW > AHEAD;
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t nb = p.d_in / 32;
-  const size_t row0 = ((size_t)blockIdx.x * 4 + wave) * RW;
+  // rows of a wave: consecutive ones, or, where it streams them, one of every 4 x gridDim.x
+  const size_t row0 = STREAM ? (size_t)__builtin_amdgcn_readfirstlane(wave) * gridDim.x + blockIdx.x : ((size_t)blockIdx.x * 4 + wave) * RW;
+  const size_t row_step = STREAM ? 4 * (size_t)gridDim.x : 1;
   const unsigned char* wbase = (const unsigned char*)p.w;
   // x (and the norm weights) are requested FIRST, the wave's weight rows right behind them: the loads of a wave complete
   // in order, x comes from L2 in a fraction of the time the weight stream takes from HBM, and everything that depends
@@ -121,22 +132,23 @@ void pa_gemv_kernel(const float* a_x, const float* a_norm_w, const void* a_w, co
   __builtin_amdgcn_sched_barrier(0);
   BlockRegs<KIND> wr[RW][BPL];
   uint16_t sc[RW][BPL];
-#pragma unroll
-  for (int r = 0; r < RW; r++) {
-    const size_t row = min(row0 + r, (size_t)p.d_out - 1);            // rows past the end repeat the last one (not stored)
+  auto request = [&](int r, int pass) __attribute__((always_inline)) {
+    const size_t row = min(row0 + r * row_step, (size_t)p.d_out - 1);            // rows past the end repeat the last one (not stored)
 #pragma unroll
     for (int i = 0; i < BPL; i++) {
-      const uint32_t b = min(lane + 64 * i, nb - 1);                   // blocks past the end likewise (weighted by x = 0)
+      const uint32_t b = min(lane + 64 * (i + BPL * pass), nb - 1);    // blocks past the end likewise (weighted by x = 0)
       load_block<KIND>(wr[r][i], wbase, row, nb, b);
       if constexpr (KIND != PA_W_F32) sc[r][i] = p.scales[row * nb + b];
     }
-  }
+  };
+#pragma unroll
+  for (int r = 0; r < (RW < AHEAD ? RW : AHEAD); r++) request(r, 0);
   // accumulating calls: the old values of the wave's rows are requested here, with everything else, instead of in a
   // round trip of their own behind the reduction
   asm volatile("" :: "s"(p.xn_out), "s"(p.eps), "s"(p.acc));
   float yold[RW];
 #pragma unroll
-  for (int r = 0; r < RW; r++) yold[r] = p.acc ? p.y[min(row0 + r, (size_t)p.d_out - 1)] : 0.f;
+  for (int r = 0; r < RW; r++) yold[r] = p.acc ? p.y[min(row0 + r * row_step, (size_t)p.d_out - 1)] : 0.f;
   __builtin_amdgcn_sched_barrier(0);
   // x -> LDS (a lane's own slice is 32 consecutive floats: loaded directly, a wave-wide load would touch 64 cache lines
   // for 1 KB), normed on the way when asked; block b sits at xs[b * 36]: the 4-float pad makes the 8 lanes of a 128-bit
@@ -176,15 +188,7 @@ void pa_gemv_kernel(const float* a_x, const float* a_norm_w, const void* a_w, co
   for (int pass = 0; pass < PASSES; pass++) {
   if (pass > 0) {                                                      // the next pass's weight rows
 #pragma unroll
-    for (int r = 0; r < RW; r++) {
-      const size_t row = min(row0 + r, (size_t)p.d_out - 1);
-#pragma unroll
-      for (int i = 0; i < BPL; i++) {
-        const uint32_t b = min(lane + 64 * (i + BPL * pass), nb - 1);
-        load_block<KIND>(wr[r][i], wbase, row, nb, b);
-        if constexpr (KIND != PA_W_F32) sc[r][i] = p.scales[row * nb + b];
-      }
-    }
+    for (int r = 0; r < (RW < AHEAD ? RW : AHEAD); r++) request(r, pass);
   }
   float x[BPL][32], sx[BPL];
 #pragma unroll
@@ -221,6 +225,11 @@ void pa_gemv_kernel(const float* a_x, const float* a_norm_w, const void* a_w, co
       else a = __builtin_fmaf((float)__ushort_as_half(sc[r][i]), d, a);
     }
     part[r] = a;
+    if constexpr (RW > AHEAD) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (r + AHEAD < RW) request(r + AHEAD, pass);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
   }
 #pragma unroll
@@ -228,28 +237,28 @@ void pa_gemv_kernel(const float* a_x, const float* a_norm_w, const void* a_w, co
   if (lane == 0) {
 #pragma unroll
     for (int r = 0; r < RW; r++) {
-      const size_t row = row0 + r;
+      const size_t row = row0 + r * row_step;
       if (row < p.d_out) p.y[row] = p.acc ? yold[r] + part[r] : part[r];
     }
   }
 }
 
 template <int KIND, int BPL, int RW, bool NORM, int PASSES = 1>
-static hipError_t launch_k(const GemvParams& p, hipStream_t s) {
-  const uint32_t rows_wg = 4 * RW;
+static hipError_t launch_k(const GemvParams& p, hipStream_t s, uint32_t wgs = 0) {
+  if (wgs == 0) wgs = (p.d_out + 4 * RW - 1) / (4 * RW);
   const size_t lds = (size_t)(p.d_in / 32) * 36 * sizeof(float);
-  hipLaunchKernelGGL((pa_gemv_kernel<KIND, BPL, RW, NORM, PASSES>), dim3((p.d_out + rows_wg - 1) / rows_wg), dim3(256), lds, s, p.x, p.norm_w, p.w, p.scales, p.y, p.d_out, p.d_in, p);
+  hipLaunchKernelGGL((pa_gemv_kernel<KIND, BPL, RW, NORM, PASSES>), dim3(wgs), dim3(256), lds, s, p.x, p.norm_w, p.w, p.scales, p.y, p.d_out, p.d_in, p);
   return hipGetLastError();
 }
 
 // rw of 1 .. R rows per wave
 template <int KIND, int BPL, bool NORM, int R>
-static hipError_t launch_rows(uint32_t rw, const GemvParams& p, hipStream_t s) {
-  if constexpr (R > 1) { if (rw < (uint32_t)R) return launch_rows<KIND, BPL, NORM, R - 1>(rw, p, s); }
-  return launch_k<KIND, BPL, R, NORM>(p, s);
+static hipError_t launch_rows(uint32_t rw, const GemvParams& p, hipStream_t s, uint32_t wgs = 0) {
+  if constexpr (R > 1) { if (rw < (uint32_t)R) return launch_rows<KIND, BPL, NORM, R - 1>(rw, p, s, wgs); }
+  return launch_k<KIND, BPL, R, NORM>(p, s, wgs);
 }
 
-// Rows per wave past 4096 inputs (quantised weights).  Every workgroup fetches, norms and stages all of x -- 20 KB and the norm's
+// Rows per wave past 4096 inputs (quantised weights) of the calls that pa_rule_gemv_resident leaves.  Every workgroup fetches, norms and stages all of x -- 20 KB and the norm's
 // 20 KB at 5120 inputs, twice the Q4_0 weights of its eight rows at two rows a wave -- so few large workgroups are faster as long as
 // every SIMD keeps two waves and they come out even.  Time follows the rows of the busiest SIMD plus about 1.6 rows' worth for every
 // wave it is dealt; measured at 1 .. 7 rows a wave with the norm (us, cold weights, Q4_0): 14336 x 5120 18.5 13.5 13.3 13.1 12.9 13.6 12.3;
@@ -277,9 +286,25 @@ extern "C" uint32_t pa_rule_gemv_wide_rows(int kind, uint32_t d_out, uint32_t d_
   return best;
 }
 
+// One or two workgroups a CU that stay for the whole call (<< 16 | the rows a wave; 0: neither): past 4096 inputs, quantised weights.  Every workgroup stages all of x and every
+// wave reads it from LDS into its registers (10 waves a CU of 5120 x 6144: 240 KB, 0.8 us), so as few of them as keep the stream going are ahead.  One a CU with the norm
+// in front up to eight rows a wave (Q4_0 2048 x 6144 5.6 -> 4.4 us, 3072 x 5120 6.5 -> 4.6, 5120 x 5120 7.4 -> 6.7, 6144 x 6144 8.1 -> 7.5, 8192 x 8192 12.0 -> 10.4; Q8_0
+// 5120 x 6144 10.1 -> 8.7, 7168 x 5120 10.6 -> 9.7); without it up to three rows and at five, where the rule below comes to 2.5 workgroups a CU (5120 x 6144 7.06 -> 6.70,
+// Q8_0 8.9 -> 8.5), but not at four or six (4096 x 6144 5.9, one a CU 6.3; 6144 x 6144 7.2 and 7.7; Q8_0 three rows 6.0 and 6.3).  Two a CU from there to eight rows
+// (Q4_0 14336 x 5120 12.5 -> 10.5, 9500 x 7168 14.5 -> 11.3; Q8_0 14336 x 5120 17.5 -> 15.2, 9216 x 5120 without the norm 11.6 -> 10.8; at four rows Q8_0 6144 x 6144
+// 9.1 -> 9.7).  More rows a wave were not built.
+extern "C" uint32_t pa_rule_gemv_resident(int kind, uint32_t d_out, int norm, int n_cu) {
+  const uint32_t one = (d_out + 4 * n_cu - 1) / (4 * n_cu), two = (d_out + 8 * n_cu - 1) / (8 * n_cu);
+  if (norm ? one <= 8 : one <= 2 || one == 5 || (one == 3 && kind == PA_W_Q4_0)) return 1u << 16 | one;
+  if (two >= 5 && two <= 8) return 2u << 16 | two;
+  return 0;
+}
+
 template <int KIND, int BPL, bool NORM>
 static hipError_t launch_rw(const GemvParams& p, int n_cu, hipStream_t s) {
   if constexpr (BPL >= 3) {
+    const uint32_t resident = pa_rule_gemv_resident(KIND, p.d_out, NORM, n_cu), rows = resident & 0xffff;
+    if (resident) return launch_rows<KIND, BPL, NORM, 8>(rows, p, s, std::min((resident >> 16) * (uint32_t)n_cu, (p.d_out + 3) / 4));
     return launch_rows<KIND, BPL, NORM, wide_rows_max(KIND, BPL, NORM)>(pa_rule_gemv_wide_rows(KIND, p.d_out, p.d_in, NORM, n_cu), p, s);
   } else {
     // rows per wave: as many as still leave about two 4-wave workgroups per CU, within the registers that RW x BPL

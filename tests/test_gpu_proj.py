@@ -79,6 +79,34 @@ def test_gemv_many_rows_a_wave(kind, d_out, d_in):
         assert got[d_out] == 7 and _rel(got[rows], ref_n) < 2e-5
 
 
+# one or two workgroups a CU that stay for the whole call, one to eight rows a wave (test_proj_rules.py asks the rule): counts that come out
+# even, one row more or less, and the first size that is left to the rows above
+GEMV_RESIDENT_SIZES = [(1024, 4128), (1025, 8192), (2047, 4160), (2049, 5120), (3071, 7008), (3073, 6144), (4001, 7008), (4097, 6400), (5120, 6144), (5121, 8192), (6145, 6208), (7169, 8192),
+                       (8192, 4160), (8193, 8160), (10241, 6144), (10241, 7008), (12289, 8192), (14337, 6208), (16384, 6144), (16385, 4128)]
+
+
+@pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])
+@pytest.mark.parametrize("d_out,d_in", GEMV_RESIDENT_SIZES)
+def test_gemv_resident_workgroups(kind, d_out, d_in):
+    """Every row against the f64 product of the dequantised weights, with the norm, without it and accumulating: rows dealt to waves whose counts
+    differ by one.  2e-5 of the largest output, the bound of the tests above: f32 sums of up to 8192 products, 4 to 8e-7 measured there."""
+    rng = np.random.default_rng(d_out + 3 * d_in + kind)
+    w, sc = _weights(kind, d_out, d_in, rng)
+    x = rng.standard_normal(d_in).astype(np.float32)
+    nw = (1 + 0.1 * rng.standard_normal(d_in)).astype(np.float32)
+    y0 = rng.standard_normal(d_out).astype(np.float32)
+    cfg = SHAPES["qwen36_moe"]
+    ref = O.gemv(kind, w, sc, x)
+    ref_n = O.gemv(kind, w, sc, O.rmsnorm(x, nw, cfg["eps"]).astype(np.float32))
+    with PooledAttn(cfg, 64, n_layers=1, max_cols=1) as pa:
+        wh = pa.weight(kind, w, sc)
+        dx = pa.to_device(x); dn = pa.to_device(nw); dy = pa.to_device(np.r_[y0, np.float32(7)])
+        for call, want in ((lambda: pa.gemv(wh, dx, dy, acc=True), ref + y0), (lambda: pa.gemv(wh, dx, dy), ref), (lambda: pa.gemv_norm(wh, dx, dn, dy), ref_n)):
+            call(); pa.sync()
+            got = dy.download(np.float32, d_out + 1)
+            assert got[d_out] == 7 and _rel(got[:d_out], want) < 2e-5
+
+
 @pytest.mark.parametrize("kind", [PA_W_F32, PA_W_Q4_0])
 def test_gemv_norm_matches_rmsnorm_then_gemv(kind):
     cfg = SHAPES["qwen36_moe"]

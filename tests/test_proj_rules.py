@@ -3,7 +3,7 @@ the sizes that the GPU tests run.  A change of a rule that leaves an instance wi
 import ctypes
 from pooled_amd import capi
 from pooled_amd.capi import PA_W_Q4_0, PA_W_Q8_0
-from test_gpu_proj import GEMM_FEW_SIZES, GEMM_TILE_SIZES, GEMV_WIDE_SIZES, HEADS_SIZES
+from test_gpu_proj import GEMM_FEW_SIZES, GEMM_TILE_SIZES, GEMV_RESIDENT_SIZES, GEMV_WIDE_SIZES, HEADS_SIZES
 
 CUS = 256
 u32 = ctypes.c_uint32
@@ -31,6 +31,21 @@ def test_gemv_sizes_take_every_number_of_rows():
     assert all(b == 3 and r == 3 for _, b, _, r in {g for g in got if g[3] > 1} - ragged)
     # Q8_0: two rows without the norm, and on tall weights
     assert _gemv(PA_W_Q8_0, 14336, 5120, False)[3] == 2 and _gemv(PA_W_Q8_0, 14336, 5120, True)[3] == 2 and _gemv(PA_W_Q8_0, 7168, 5120, True)[3] == 4
+
+
+def test_gemv_resident_sizes_take_every_form():
+    def form(kind, d_out, d_in, norm):
+        v = _rule("pa_rule_gemv_resident", ctypes.c_int(kind), d_out, ctypes.c_int(norm), ctypes.c_int(CUS))
+        return (kind, 3 if d_in <= 6144 else 4, norm, v >> 16, v & 0xffff) if v else None
+    forms = [(k, norm) for k in (PA_W_Q4_0, PA_W_Q8_0) for norm in (0, 1)]
+    sizes = GEMV_RESIDENT_SIZES + GEMV_WIDE_SIZES
+    tested = {form(k, d_out, d_in, norm) for k, norm in forms for d_out, d_in in sizes}
+    reached = {form(k, d_out, d_in, norm) for k, norm in forms for d_out in range(1, 20000, 7) for d_in in (4128, 8192)}
+    assert {f[3:] for f in reached - {None}} == {(1, r) for r in range(1, 9)} | {(2, r) for r in range(5, 9)}
+    assert reached <= tested
+    # the line without the norm: not at four rows a wave, nor at six to eight of one workgroup a CU
+    assert [form(PA_W_Q4_0, d_out, 6144, 0) for d_out in (4096, 5121, 8192)] == [None] * 3 and form(PA_W_Q8_0, 3072, 6144, 0) is None
+    assert form(PA_W_Q4_0, 5120, 6144, 0)[3:] == (1, 5) and form(PA_W_Q4_0, 14336, 5120, 1)[3:] == (2, 7)
 
 
 def _few(kind, d_out, d_in, n):
