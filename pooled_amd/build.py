@@ -13,7 +13,7 @@ LIBDIR = os.path.join(ROOT, "pooled_amd", "lib")
 LIB = os.path.join(LIBDIR, "libpooled_attn.so")
 ADDON = os.path.join(LIBDIR, "pooled_attn.node")
 
-HIP_SOURCES = ["pa_api.hip", "glue_kv.hip", "kv_copy.hip", "attn_decode.hip", "attn_prefill.hip", "proj_gemv.hip", "proj_gemm.hip", "proj_gemm_skinny.hip", "proj_gemm_dot.hip", "proj_gemm_wide.hip", "proj_gemm_tile.hip"]
+HIP_SOURCES = ["pa_api.hip", "glue_kv.hip", "kv_copy.hip", "attn_decode.hip", "attn_block.hip", "attn_prefill.hip", "proj_gemv.hip", "proj_gemm.hip", "proj_gemm_skinny.hip", "proj_gemm_dot.hip", "proj_gemm_wide.hip", "proj_gemm_tile.hip"]
 HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
                # packed-FP32 VALU forms are kept off for all device code
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

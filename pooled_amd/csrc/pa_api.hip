@@ -335,6 +335,21 @@ static bool plan_self_row(const pa_plan& pl) { return pl.kernel == 0 && pl.slots
 static bool plan_single_round2(const pa_plan& pl) {
   return pl.kernel == 0 && pl.row_blocks == 2 && pl.waves == 4 && pl.split_len == 32 * pl.waves && pl.n_splits > 1;
 }
+// Two row blocks or more over several splits: the kernel whose waves share one softmax and divide O by output dims (attn_block.hip) where nothing
+// outweighs its shorter end, the single-round kernel or the tile loop elsewhere.  Measured (us a call, that kernel / the other): one column group, two tiles a wave or more: 16 / 2-head
+// shape, 4 columns at 30000 rows 19.1 / 20.6, 24 / 4-head, 5 at 12001 and 20000 16.5 / 17.9 and 21.0 / 22.1, 8 at 65536 53.4 / 55.9, 16 / 8-head, 16 at 20000 22.9 / 24.3.  Several
+// column groups: two tiles a wave, 16 / 2-head, 8 columns at 12001 15.9 / 17.1, 24 / 4-head, 10 at 8000 15.4 / 16.9; from three on the waves of the tile loop, which meet
+// only at its end, share the L2's rows better (24 / 4-head, 10 columns at 20000 26.2 / 25.0, at 65536 67.3 / 57.6).  One tile a wave: where several groups or the small
+// heads fill more than half the chip but not twice (16 / 2-head, 6 at 8000 13.4 / 14.0, 24 / 4-head, 10 at 4000 13.3 / 14.3, 16 / 8-head, 9 at 4000 9.6 / 10.8; one
+// group, 16 / 2-head, 4 at 600 and 12001 11.0 / 10.6 and 14.4 / 14.2; 16 / 8-head, 12 at 8000 12.9 / 12.5).
+static bool plan_block(const pa_ctx* ctx, const pa_plan& pl) {
+  if (pl.kernel != 0 || pl.waves != 4 || pl.row_blocks < 2 || pl.n_splits == 1) return false;
+  if (ctx->decode_splits_override) return true;
+  const uint32_t tiles = pl.split_len / 128, n_cu = (uint32_t)ctx->n_cu;
+  const uint64_t wgs = (uint64_t)pl.n_splits * ctx->cfg.n_kv_heads * pl.col_groups;
+  if (tiles == 1) return wgs * 2 > n_cu && wgs <= n_cu && (pl.col_groups > 1 || ctx->cfg.head_dim == 128);
+  return pl.col_groups == 1 || tiles == 2;
+}
 static uint32_t plan_tile_ilv(const pa_plan& pl) {
   return pl.kernel == 0 && pl.split_len != 32 * pl.waves && pl.n_splits > 1 ? 32 * pl.waves : 0;
 }
@@ -700,7 +715,8 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
   p.gate_head_stride = c.head_dim;
   PaTiming tm;
   if ((rc = prof_pair(ctx, &tm))) return rc;
-  if (pl.kernel == 0) HIPCHK(ctx, pa_launch_decode(p, c.head_dim, pl.row_blocks, pl.waves, pl.col_groups, ctx->stream, &tm));
+  if (plan_block(ctx, pl)) HIPCHK(ctx, pa_launch_block(p, c.head_dim, pl.row_blocks, pl.col_groups, ctx->stream, &tm));
+  else if (pl.kernel == 0) HIPCHK(ctx, pa_launch_decode(p, c.head_dim, pl.row_blocks, pl.waves, pl.col_groups, ctx->stream, &tm));
   else HIPCHK(ctx, pa_launch_prefill(p, c.head_dim, pl.row_blocks, pl.col_groups, ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u, ctx->stream, &tm));
   if (!direct) {
     PaTiming tm2;

@@ -448,3 +448,56 @@ def test_decode_growing_maximum(shape, n_cols, base, blocks):
         plan = pa.plan("decode", base, n_cols)
         assert plan["row_blocks"] == blocks and plan["split_len"] >= 3 * 128, plan     # the tile loop, three tiles a wave or more
         assert_parity(pa.run_attn("decode", 0, q, base), ref, "jumping maximum, %d row blocks" % blocks)
+
+
+@pytest.mark.parametrize("shape,kv_q8,n_cols,base,blocks,groups,tiles", [
+    ("qwen36_moe", False, 5, 8191, 2, 2, 2), ("qwen36_moe", False, 6, 8100, 2, 2, 1), ("qwen36_moe", False, 4, 16385, 2, 1, 2), ("qwen36_moe", False, 3, 36000, 2, 1, 3),
+    ("qwen38_27b", False, 8, 50000, 3, 1, 7), ("qwen38_27b", False, 10, 4000, 2, 2, 1), ("qwen3_1p7b", False, 9, 4000, 2, 1, 1), ("qwen3_1p7b", False, 24, 4200, 3, 1, 2),
+    ("qwen3_1p7b", False, 32, 12345, 4, 1, 4), ("qwen36_moe", True, 16, 8000, 2, 4, 2), ("qwen38_27b", True, 5, 20001, 2, 1, 3), ("qwen3_1p7b", True, 32, 9000, 4, 1, 3)])
+def test_blocks_whose_waves_share_one_softmax(shape, kv_q8, n_cols, base, blocks, groups, tiles):
+    """Blocks of two row blocks or more over several splits on the kernel that divides O by output dims, either side of the turns and column groups its
+    rule knows: against the oracle, with low and high keys in turn (a raised reference), rows past the context poisoned, f32 and f16 out.  Budget of the
+    decode tests.  Then value rows that are all alike: that vector comes back, whatever the rounding of P (f32 sums of the same weights above and below the
+    fraction bar, a reciprocal of 1 ulp: a few 1e-7), also on contiguous splits."""
+    cfg = dict(SHAPES[shape], kv_q8=kv_q8)
+    rng = np.random.default_rng(base + n_cols)
+    rows, tail = base + n_cols, 40
+    nKV, hd = cfg["n_kv_heads"], cfg["head_dim"]
+    scale = np.where((np.arange(rows) // max(rows // 9, 1)) % 2 == 0, 0.2, 2.0).astype(np.float32)[:, None, None]
+    k = rng.standard_normal((rows, nKV, hd), dtype=np.float32) * scale
+    v = rng.standard_normal((rows, nKV, hd), dtype=np.float32)
+    q = rng.standard_normal((n_cols, cfg["n_heads"], hd), dtype=np.float32)
+    gate = rng.standard_normal(q.shape, dtype=np.float32) if cfg["gate"] else None
+    same = np.ascontiguousarray(np.broadcast_to(v[:1], v.shape))
+    with PooledAttn(cfg, rows + tail, n_layers=1, max_cols=n_cols) as pa:
+        pa.layer_alloc(0)
+        pl = pa.plan("decode", base, n_cols)
+        assert (pl["row_blocks"], pl["col_groups"], pl["split_len"]) == (blocks, groups, 128 * tiles) and pl["n_splits"] > 1, pl
+
+        first_v = []                     # int8 rows: the first value row as the kernels widen it, f16 value x f16 scale
+
+        def fill(k, v):
+            pa.kv_write(0, 2 if kv_q8 else 0, rows, np.full((tail, nKV, hd // 32), np.nan, np.float32) if kv_q8 else np.full((tail, nKV, hd), 0x7e00, np.uint16))
+            pa.kv_write(0, 3 if kv_q8 else 1, rows, np.full((tail, nKV, hd // 32), np.nan, np.float32) if kv_q8 else np.full((tail, nKV, hd), 0x7e00, np.uint16))
+            if not kv_q8:
+                k16, v16 = k.astype(np.float16).view(np.uint16), v.astype(np.float16).view(np.uint16)
+                pa.kv_write(0, 0, 0, k16); pa.kv_write(0, 1, 0, v16)
+                return k16, v16
+            kq, ks = O.q8_quantize(k); vq, vs = O.q8_quantize(v)
+            for which, a in enumerate((kq, vq, ks, vs)):
+                pa.kv_write(0, which, 0, a)
+            first_v[:] = [(vq[:1].reshape(1, nKV, hd // 32, 32).astype(np.float16) * vs[:1].reshape(1, nKV, hd // 32, 1).astype(np.float16)).reshape(1, nKV, hd)]
+            return O.q8_dequantize(kq, ks), O.q8_dequantize(vq, vs)
+
+        kk, vv = fill(k, v)
+        ref = O.attention_values(q, kk, vv, base, gate=gate) if kv_q8 else C.attention(q, kk, vv, base, gate=gate)
+        for out_dtype in (0, PA_OUT_F16):
+            assert_parity(pa.run_attn("decode", 0, q, base, gate=gate, out_dtype=out_dtype).astype(np.float32), ref, "one softmax, %s %d columns at %d" % (shape, n_cols, base))
+        first = pa.run_attn("decode", 0, q, base, gate=gate)
+        assert np.array_equal(first, pa.run_attn("decode", 0, q, base, gate=gate))          # no atomics, fixed orders
+        _, vv = fill(k, same)
+        vec = (first_v[0] if kv_q8 else vv.view(np.float16))[0].astype(np.float32)
+        want = np.repeat(vec, cfg["n_heads"] // nKV, axis=0)[None]
+        for splits in (0, max(2, pl["n_splits"] // 3)):
+            pa.set_decode_splits(splits)
+            assert np.abs(pa.run_attn("decode", 0, q, base) - want).max() <= 2e-6
