@@ -1459,11 +1459,15 @@ hipError_t pa_launch_decode_gather(const AttnParams& p, uint32_t hd, hipStream_t
   return hipErrorInvalidValue;
 }
 
-hipError_t pa_launch_combine(const AttnParams& p, uint32_t hd, hipStream_t s, const PaTiming* t) {
-  // many columns, few splits: one thread per (column, head, 4 dims)
-  if (p.n_cols >= 16 && p.n_splits <= 32 && (hd == 256 || hd == 128) && !p.exact_cols && !p.self_row) {
-    const size_t threads = (size_t)p.n_cols * p.n_heads * (hd / 4);
-    const dim3 grid((unsigned)((threads + 255) / 256));
+hipError_t pa_launch_combine(const AttnParams& p, uint32_t hd, int n_cu, hipStream_t s, const PaTiming* t) {
+  // many columns, few splits: one thread per (column, head, 4 dims).  Its workgroups walk a column's splits, eight a round trip, so with few of them (two fifths of the CUs)
+  // and more splits than one round trip has, the wavefront kernel is ahead although every one of its waves is a launch of its own (us a call, this / that: 16 / 2-head shape, 16
+  // columns at 8000 and 12345 rows 18.9 / 15.9 and 22.3 / 19.3 (64 workgroups here; 32 and 25 splits), 24 at 12345 23.7 / 22.3, 32 at 8000 (128 workgroups) 21.8 / 22.2, 48 at 12345
+  // 31.4 / 32.4; 16 / 8-head, 32 at 12345 21.3 / 18.4; 24 / 4-head, 16 at 600 (five splits) 11.7 / 12.7 and at 4200 (eleven) 19.2 / 18.3).
+  const uint64_t wide_wgs = ((uint64_t)p.n_cols * p.n_heads * (hd / 4) + 255) / 256;
+  const bool few = p.n_splits > 6 && wide_wgs * 5 <= 2 * (uint64_t)n_cu;
+  if (p.n_cols >= 16 && p.n_splits <= 32 && !few && (hd == 256 || hd == 128) && !p.exact_cols && !p.self_row) {
+    const dim3 grid((unsigned)wide_wgs);
     if (hd == 256) hipLaunchKernelGGL(pa_combine_wide_kernel<256>, grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL(pa_combine_wide_kernel<128>, grid, dim3(256), 0, s, p);
     return hipGetLastError();

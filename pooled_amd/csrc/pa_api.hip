@@ -660,7 +660,7 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
         HIPCHK(ctx, pa_launch_decode(p, c.head_dim, two ? 2 : 1, p0.waves, two ? pairs : run, ctx->stream, &tm));
         if (!one) {
           if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;
-          HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream, &tm2));
+          HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->n_cu, ctx->stream, &tm2));
         }
         if (staged && (rc = copy_out(ctx, ctx->part_o, qd, out_c, out_stride, run, osz))) return rc;
       }
@@ -721,7 +721,7 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
   if (!direct) {
     PaTiming tm2;
     if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;
-    HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream, &tm2));
+    HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->n_cu, ctx->stream, &tm2));
   }
   return staged ? copy_out(ctx, ctx->part_o, qd, d_out, qd, 1, osz) : PA_OK;
 }
@@ -796,7 +796,7 @@ static int decode_step_common(pa_ctx* ctx, const char* who, bool static_scratch,
   if (one) return staged ? copy_out(ctx, part_o, qd, d_out, qd, 1, osz) : PA_OK;
   PaTiming tm2;
   if ((rc = prof_aux_pair(ctx, tm, &tm2))) return rc;
-  HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream, &tm2));
+  HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->n_cu, ctx->stream, &tm2));
   return PA_OK;
 }
 
@@ -1100,7 +1100,7 @@ extern "C" int pa_attn_decode_gather(pa_ctx* ctx, uint32_t layer, const float* d
   PaTiming tm;
   if ((rc = prof_pair(ctx, &tm))) return rc;
   HIPCHK(ctx, pa_launch_decode_gather(p, c.head_dim, ctx->stream, &tm));
-  HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->stream));
+  HIPCHK(ctx, pa_launch_combine(p, c.head_dim, ctx->n_cu, ctx->stream));
   return PA_OK;
 }
 

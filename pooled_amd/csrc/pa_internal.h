@@ -103,7 +103,7 @@ hipError_t pa_launch_decode_gather(const AttnParams& p, uint32_t hd, hipStream_t
 // the same with the pre-step of the one column fused in (p.f_* set; one 16-row block, n_cols == 1)
 hipError_t pa_launch_decode_step(const AttnParams& p, uint32_t hd, hipStream_t s, const PaTiming* t = nullptr);
 hipError_t pa_prepare_decode_step(uint32_t hd, bool q8);
-hipError_t pa_launch_combine(const AttnParams& p, uint32_t hd, hipStream_t s, const PaTiming* t = nullptr);
+hipError_t pa_launch_combine(const AttnParams& p, uint32_t hd, int n_cu, hipStream_t s, const PaTiming* t = nullptr);
 // MFMA prefill; returns hipErrorNotSupported for shapes it does not cover
 hipError_t pa_launch_prefill(const AttnParams& p, uint32_t hd, uint32_t row_blocks, uint32_t col_groups, uint32_t n_cu, hipStream_t s, const PaTiming* t = nullptr);
 

@@ -501,3 +501,19 @@ def test_blocks_whose_waves_share_one_softmax(shape, kv_q8, n_cols, base, blocks
         for splits in (0, max(2, pl["n_splits"] // 3)):
             pa.set_decode_splits(splits)
             assert np.abs(pa.run_attn("decode", 0, q, base) - want).max() <= 2e-6
+
+
+@pytest.mark.parametrize("shape,n_cols,base", [("qwen36_moe", 16, 700), ("qwen36_moe", 16, 760), ("qwen36_moe", 25, 4500), ("qwen36_moe", 26, 4500), ("qwen3_1p7b", 51, 4300),
+                                               ("qwen3_1p7b", 52, 4300), ("qwen38_27b", 17, 5000)])
+def test_merge_of_sixteen_columns_and_more(shape, n_cols, base):
+    """Either merge kernel behind a pass of 16 columns or more: up to six splits and past them, two fifths of the CUs' worth of workgroups and past that."""
+    cfg = SHAPES[shape]
+    rng = np.random.default_rng(base + n_cols)
+    k16, v16 = random_cache(cfg, base + n_cols, seed=base)
+    q = rng.standard_normal((n_cols, cfg["n_heads"], cfg["head_dim"]), dtype=np.float32)
+    gate = rng.standard_normal(q.shape, dtype=np.float32) if cfg["gate"] else None
+    ref = C.attention(q, k16, v16, base, gate=gate)
+    with _ctx_with_cache(cfg, k16, v16, base + n_cols, max_cols=n_cols) as pa:
+        assert pa.plan("decode", base, n_cols)["n_splits"] > 1
+        for out_dtype in (0, PA_OUT_F16):
+            assert_parity(pa.run_attn("decode", 0, q, base, gate=gate, out_dtype=out_dtype).astype(np.float32), ref, "merge of %d columns at %d" % (n_cols, base), tight=True)
