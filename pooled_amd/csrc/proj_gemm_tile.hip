@@ -159,7 +159,7 @@ static __device__ inline void finish_heads(const GlueParams& g, unsigned char* l
         const uint32_t c = lw + (e >> lgU), col = col_of(c);
         const bool on = col < g.n_cols;
         f4 t0, t1;
-        if (cs_lds) { const f4* t = (const f4*)(lds + H::cs + ((col - c0) * half + da) * 8); t0 = t[0]; t1 = t[1]; }
+        if (cs_lds) { const f4* t = (const f4*)(lds + H::cs + (min(col - c0, (uint32_t)BM - 1) * half + da) * 8); t0 = t[0]; t1 = t[1]; }
         else { const f4* t = (const f4*)(g.rope_tab + (size_t)(g.base_pos + (on ? col : c0)) * half + da); t0 = t[0]; t1 = t[1]; }
         const float cs[4] = { t0[0], t0[2], t1[0], t1[2] }, sn[4] = { t0[1], t0[3], t1[1], t1[3] };
         const f4 va = *(const f4*)(hx0 + c * LR + da), vb = *(const f4*)(hx0 + c * LR + db);
@@ -207,11 +207,11 @@ static __device__ inline uint32_t gt_swz64(uint32_t r) { return ((r >> 3) & 1) |
 // shape 430 / 408, 2048 of it 231 / 226, 2048 of the 24 / 4-head shape 534 / 510; one round of few workgroups (777 of that shape) 297 / 297.  A stage is one k-step of 32: the products with the first half of a wave's column blocks, the barrier,
 // those with the second half; a fragment is read as soon as the products with the one in its registers are out, so a stage holds no more
 // fragments than the two k-steps of 16 did.  Weights are the first operand: a lane holds four consecutive rows of a column.
-template <int WM, int WN, int TM, int TN, int S, int EPI, int LPW, class Issue>
+template <int WM, int WN, int NA, int NB, int S, int EPI, int LPW, class Issue>
 static __device__ __attribute__((always_inline)) inline void gt_whole_k(const GemmTileParams& p, const GlueParams& gp, unsigned char* lds, uint32_t c0, uint32_t r0, uint32_t wm, uint32_t wn, uint32_t n_stages,
                                               const unsigned char* const (&src)[LPW], const uint32_t (&step)[LPW], const uint32_t (&off)[LPW], const uint32_t (&dofs)[LPW], Issue issue) {
-  constexpr int BM = WM * TM * 32, BN = WN * TN * 32, ABYTES = BM * 64, STAGE = (BM + BN) * 64;
-  constexpr int NA = 2 * TM, NB = 2 * TN;                // 16-column and 16-row blocks of a wave
+  constexpr int BM = WM * NA * 16, BN = WN * NB * 16, ABYTES = BM * 64, STAGE = (BM + BN) * 64;
+  constexpr int N0 = (NA + 1) / 2, N1 = NA / 2;          // 16-column blocks of a wave in either half of a stage
   const uint32_t lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
   f4 acc[NA][NB];
 #pragma unroll
@@ -221,17 +221,21 @@ static __device__ __attribute__((always_inline)) inline void gt_whole_k(const Ge
 #pragma unroll
   for (int j = 0; j < S; j++) issue(j, j);
   // k 8 kq .. of a row: an activation row's chunk kq; of the weights' fragments, the half kq % 2 of k-step kq / 2
-  const uint32_t x_rd = (wm * TM * 32 + l16) * 64 + ((kq ^ gt_swz64(l16)) * 16), w_rd = ABYTES + wn * TN * 2048 + (kq >> 1) * 1024 + ((kq & 1) * 32 + l16) * 16;
-  h8 x0[TM], x1[TM], w[NB];
+  const uint32_t x_rd = (wm * NA * 16 + l16) * 64 + ((kq ^ gt_swz64(l16)) * 16);
+  // ... of a wave's 16-row block b, block wn NB + b of the tile: the half of a 32-row fragment that its parity says
+  const uint32_t w_l = ABYTES + (kq >> 1) * 1024 + ((kq & 1) * 32 + l16) * 16, wb0 = wn * NB, wb1 = wb0 + 1;
+  const uint32_t w_rd[2] = { w_l + (wb0 >> 1) * 2048 + (wb0 & 1) * 256, w_l + (wb1 >> 1) * 2048 + (wb1 & 1) * 256 };
+  h8 x0[N0], x1[N1 > 0 ? N1 : 1], w[NB];
   auto rd_x = [&](h8& f, const unsigned char* sb, int a) __attribute__((always_inline)) { f = *(const h8*)(sb + x_rd + a * 1024); };
-  auto rd_w = [&](h8& f, const unsigned char* sb, int b) __attribute__((always_inline)) { f = *(const h8*)(sb + w_rd + (b / 2) * 2048 + (b % 2) * 256); };
+  auto rd_w = [&](h8& f, const unsigned char* sb, int b) __attribute__((always_inline)) { f = *(const h8*)(sb + w_rd[b % 2] + (b / 2) * 2048); };
   asm volatile("s_waitcnt vmcnt(%0)" :: "n"(LPW * (S - 1)) : "memory");       // stage 0 (S stages were issued)
   asm volatile("s_barrier" ::: "memory");
 #pragma unroll
-  for (int a = 0; a < TM; a++) rd_x(x0[a], lds, a);
+  for (int a = 0; a < N0; a++) rd_x(x0[a], lds, a);
 #pragma unroll
   for (int b = 0; b < NB; b++) rd_w(w[b], lds, b);
-  constexpr int NH = TM * NB;                            // products of half a stage
+  constexpr int H0 = N0 * NB, H1 = N1 * NB;              // products of either half of a stage
+  static_assert(H1 >= N0 && N1 > 0, "a read behind each product of the second half");
   uint32_t buf = 0;
   for (uint32_t st = 0; st < n_stages; st++) {
     const uint32_t nbuf = buf + 1 == S ? 0 : buf + 1;
@@ -239,24 +243,24 @@ static __device__ __attribute__((always_inline)) inline void gt_whole_k(const Ge
     const unsigned char* sn = lds + nbuf * STAGE;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int m = 0; m < NH; m++) {
-      acc[m % TM][m / TM] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[m / TM], x0[m % TM], acc[m % TM][m / TM], 0, 0, 0);
+    for (int m = 0; m < H0; m++) {
+      acc[m % N0][m / N0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[m / N0], x0[m % N0], acc[m % N0][m / N0], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
-      if (m < TM) { rd_x(x1[m], sb, TM + m); __builtin_amdgcn_sched_barrier(0); }
+      if (m < N1) { rd_x(x1[m], sb, N0 + m); __builtin_amdgcn_sched_barrier(0); }
     }
     // stage st + 1 is in LDS behind this barrier, and every wave has read stage st: its buffer takes stage st + S
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(LPW * (S - 2)) : "memory");
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t s_n = min(st + S, n_stages - 1);
 #pragma unroll
-    for (int m = 0; m < NH; m++) {
-      acc[TM + m % TM][m / TM] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[m / TM], x1[m % TM], acc[TM + m % TM][m / TM], 0, 0, 0);
+    for (int m = 0; m < H1; m++) {
+      acc[N0 + m % N1][m / N1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[m / N1], x1[m % N1], acc[N0 + m % N1][m / N1], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
-      if (m < TM) rd_x(x0[m], sn, m);
-      if (m % TM == TM - 1) rd_w(w[m / TM], sn, m / TM);
+      if (m < N0) rd_x(x0[m], sn, m);
+      if (m % N1 == N1 - 1) rd_w(w[m / N1], sn, m / N1);
 #pragma unroll
       for (int i = 0; i < LPW; i++)
-        if (i * (NH - 1) / LPW == m) PF_GLL_S(src[i] + (size_t)s_n * step[i], off[i], lds + buf * STAGE + dofs[i]);
+        if (i * (H1 - 1) / LPW == m) PF_GLL_S(src[i] + (size_t)s_n * step[i], off[i], lds + buf * STAGE + dofs[i]);
       __builtin_amdgcn_sched_barrier(0);
     }
     buf = nbuf;
@@ -270,23 +274,26 @@ static __device__ __attribute__((always_inline)) inline void gt_whole_k(const Ge
     auto dump = [&](auto A) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < 2; j++)
+        if constexpr (2 * decltype(A)::value < NA)
+          if (2 * decltype(A)::value + j < NA)
 #pragma unroll
-        for (int b = 0; b < NB; b++) *(f4*)(hx + (wm * 32 + j * 16 + l16) * LR + (wn * NB + b) * 16 + 4 * kq) = acc[2 * decltype(A)::value + j][b];
+            for (int b = 0; b < NB; b++) *(f4*)(hx + (wm * 32 + j * 16 + l16) * LR + (wn * NB + b) * 16 + 4 * kq) = acc[2 * decltype(A)::value + j < NA ? 2 * decltype(A)::value + j : 0][b];
       asm volatile("; block %0" :: "n"(decltype(A)::value) : "memory");   // (the blocks' stores are not merged into one on selected registers)
     };
 #pragma nounroll
-    for (int a = 0; a < TM; a++) {                                       // a phase: 32 of every wave's columns
-      static_assert(TM <= 7, "blocks of a wave");
+    for (int a = 0; a < N0; a++) {                                       // a phase: 32 of every wave's columns (the last one of an odd number of blocks: 16)
+      static_assert(N0 <= 5, "blocks of a wave");
       if (a == 0) dump(std::integral_constant<int, 0>{});
-      if constexpr (TM > 1) if (a == 1) dump(std::integral_constant<int, 1>{});
-      if constexpr (TM > 2) if (a == 2) dump(std::integral_constant<int, 2>{});
-      if constexpr (TM > 3) if (a == 3) dump(std::integral_constant<int, 3>{});
-      if constexpr (TM > 4) if (a == 4) dump(std::integral_constant<int, 4>{});
-      if constexpr (TM > 5) if (a == 5) dump(std::integral_constant<int, 5>{});
-      if constexpr (TM > 6) if (a == 6) dump(std::integral_constant<int, 6>{});
+      if constexpr (N0 > 1) if (a == 1) dump(std::integral_constant<int, 1>{});
+      if constexpr (N0 > 2) if (a == 2) dump(std::integral_constant<int, 2>{});
+      if constexpr (N0 > 3) if (a == 3) dump(std::integral_constant<int, 3>{});
+      if constexpr (N0 > 4) if (a == 4) dump(std::integral_constant<int, 4>{});
       if (a == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // what heads_request asked for
       lds_barrier();
-      const auto col = [&](uint32_t c) { return c0 + (c / 32 * TM + a) * 32 + c % 32; };
+      const auto col = [&](uint32_t c) -> uint32_t {
+        if (NA % 2 && a * 32 + c % 32 >= NA * 16) return 0xffffffffu;      // no column: its row of LDS is an earlier phase's
+        return c0 + c / 32 * (NA * 16) + a * 32 + c % 32;
+      };
       if (gp.head_dim == 256) finish_heads<256, WM * 32, BN, BM>(gp, lds, c0, r0, p.d_out, col);
       else finish_heads<128, WM * 32, BN, BM>(gp, lds, c0, r0, p.d_out, col);
       lds_barrier();
@@ -295,7 +302,7 @@ static __device__ __attribute__((always_inline)) inline void gt_whole_k(const Ge
     // Accumulating calls: loads and stores share one counter, and a wait for a loaded value with stores pending waits for those as well, so the old
     // values are fetched several blocks at a time, unconditionally (clamped addresses: a guarded load is a branch, one load a basic block), then added.
     typedef f4 f4u __attribute__((aligned(4)));                           // (y is aligned to its elements)
-    constexpr int D = TN <= 5 ? 4 * TN : 16, NM = NA * NB;               // blocks of a phase: what fits next to the accumulators
+    constexpr int D = NB <= 10 ? 2 * NB : 16, NM = NA * NB;               // blocks of a phase: what fits next to the accumulators
     auto col_of = [&](int a) { return c0 + (wm * NA + a) * 16 + l16; };
     auto row_of = [&](int b) { return r0 + (wn * NB + b) * 16 + 4 * kq; };
     const size_t last = (size_t)(p.n_cols - 1) * p.y_stride + p.d_out - 4;
@@ -332,7 +339,9 @@ __global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p, 
   constexpr bool ACC = EPI == GT_ACC;
   static_assert(WM * WN * KG == 8, "eight waves");
   constexpr int KS = 2;                                  // k-steps of a stage per wave
-  constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BK = 16 * KG * KS;
+  constexpr int U = KG == 1 ? 16 : 32;                   // columns and rows of a wave's blocks
+  constexpr int BM = WM * TM * U, BN = WN * TN * U, BK = 16 * KG * KS;
+  static_assert(BN % 32 == 0, "whole fragments of weights");
   constexpr int CH = BK / 8;                             // 16-byte chunks of a staged activation row
   constexpr int RPL = 64 / CH;                           // rows of a 1 KB load
   constexpr int ALD = BM * BK / 512, BLD = BN * BK / 512, LPW = (ALD + BLD + 7) / 8;
@@ -492,7 +501,7 @@ __global__ __launch_bounds__(512, 2) void pa_gemm_tile_kernel(GemmTileParams p, 
 
 template <int WM, int WN, int KG, int TM, int TN, int S, bool HEADS>
 static hipError_t gt_launch(const GemmTileParams& q, int acc, const GlueParams* heads, hipStream_t s) {
-  constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BK = 32 * KG;
+  constexpr int U = KG == 1 ? 16 : 32, BM = WM * TM * U, BN = WN * TN * U, BK = 32 * KG;
   constexpr int lds_st = S * (BM + BN) * BK * 2, lds_red = KG > 1 ? KG * BM * BN * 4 : 0, lds_fixed = lds_st > lds_red ? lds_st : lds_red;
   typedef HeadsLds<(KG > 1 ? BM : WM * 32), BN> H;
   static_assert(lds_fixed <= GT_LDS && (!HEADS || H::cs <= GT_LDS), "LDS");
@@ -516,12 +525,12 @@ static const TileShape tile_shapes[] = {
   { 64, 128, 4, 6.f, 6.5f, gt_launch<1, 2, 4, 2, 2, 3, false> },
   { 128, 128, 2, 6.f, 10.3f, gt_launch<2, 2, 2, 2, 2, 4, false> },
   { 128, 160, 2, 6.f, 11.8f, gt_launch<4, 1, 2, 1, 5, 4, false> },
-  { 128, 192, 1, 6.f, 14.0f, gt_launch<4, 2, 1, 1, 3, 6, false> },
-  { 128, 256, 1, 6.f, 15.5f, gt_launch<2, 4, 1, 2, 2, 6, false> },
-  { 128, 320, 1, 6.f, 19.0f, gt_launch<4, 2, 1, 1, 5, 5, false> },
-  { 128, 384, 1, 6.f, 21.5f, gt_launch<2, 4, 1, 2, 3, 4, false> },
-  { 128, 448, 1, 6.f, 25.0f, gt_launch<4, 2, 1, 1, 7, 4, false> },
-  { 256, 256, 1, 6.f, 27.0f, gt_launch<2, 4, 1, 4, 2, 4, false> },
+  { 128, 192, 1, 6.f, 14.0f, gt_launch<2, 4, 1, 4, 3, 6, false> },
+  { 128, 256, 1, 6.f, 15.5f, gt_launch<2, 4, 1, 4, 4, 6, false> },
+  { 128, 320, 1, 6.f, 19.0f, gt_launch<2, 4, 1, 4, 5, 5, false> },
+  { 128, 384, 1, 6.f, 21.5f, gt_launch<2, 4, 1, 4, 6, 4, false> },
+  { 128, 448, 1, 6.f, 25.0f, gt_launch<2, 4, 1, 4, 7, 4, false> },
+  { 256, 256, 1, 6.f, 27.0f, gt_launch<2, 4, 1, 8, 4, 4, false> },
 };
 // ... and those that hold whole heads (128 rows: of head_dim 128) and can end with the pre-step, whose work is part of a round's start here.
 // Fitted to 75 sizes (the three model shapes, 33 to 4096 columns) on 32 x 32 x 16 products.  As the kernels are now, on 16 sizes (257 to 1024 columns) timed on every
@@ -530,13 +539,13 @@ static const TileShape head_shapes[] = {
   { 64, 128, 4, 3.5f, 7.1f, gt_launch<1, 2, 4, 2, 2, 3, true> },
   { 128, 128, 2, 4.3f, 8.9f, gt_launch<2, 2, 2, 2, 2, 4, true> },
   { 64, 256, 2, 5.6f, 11.8f, gt_launch<1, 4, 2, 2, 2, 3, true> },
-  { 96, 256, 1, 5.f, 12.8f, gt_launch<1, 8, 1, 3, 1, 6, true> },
-  { 128, 256, 1, 3.7f, 14.5f, gt_launch<2, 4, 1, 2, 2, 6, true> },
-  { 160, 256, 1, 9.2f, 15.9f, gt_launch<1, 8, 1, 5, 1, 5, true> },
-  { 192, 256, 1, 10.3f, 16.1f, gt_launch<2, 4, 1, 3, 2, 5, true> },
-  { 224, 256, 1, 17.2f, 17.4f, gt_launch<1, 8, 1, 7, 1, 4, true> },
-  { 256, 256, 1, 16.5f, 17.8f, gt_launch<2, 4, 1, 4, 2, 4, true> },
-  { 320, 256, 1, 24.2f, 20.7f, gt_launch<2, 4, 1, 5, 2, 4, true> },
+  { 96, 256, 1, 5.f, 12.8f, gt_launch<2, 4, 1, 3, 4, 6, true> },
+  { 128, 256, 1, 3.7f, 14.5f, gt_launch<2, 4, 1, 4, 4, 6, true> },
+  { 160, 256, 1, 9.2f, 15.9f, gt_launch<2, 4, 1, 5, 4, 5, true> },
+  { 192, 256, 1, 10.3f, 16.1f, gt_launch<2, 4, 1, 6, 4, 5, true> },
+  { 224, 256, 1, 17.2f, 17.4f, gt_launch<2, 4, 1, 7, 4, 4, true> },
+  { 256, 256, 1, 16.5f, 17.8f, gt_launch<2, 4, 1, 8, 4, 4, true> },
+  { 320, 256, 1, 24.2f, 20.7f, gt_launch<2, 4, 1, 10, 4, 4, true> },
 };
 
 // One workgroup is resident per CU, so a call costs whole rounds of n_cu workgroups: the shape with the cheapest rounds, and
