@@ -41,6 +41,8 @@ struct GemmTileParams {
 // of that shape 499 / 459, 2048 282 / 243, 300 71 / 66; 777 of the 24 / 4-head shape 292 / 280; 512 and 1024 of the 16 / 8-head shape 53 / 48 and 82 / 73.
 enum { GT_STORE = 0, GT_ACC = 1, GT_HEADS = 2 };
 
+#define GT_OLD 16                // old blocks of an accumulating call that a wave requests under its last products
+
 // what a block of head_dim weight rows is: [q | gate] or q heads, then k, then v heads
 enum { HB_Q = 0, HB_GATE = 1, HB_K = 2, HB_V = 3 };
 static __device__ inline uint32_t head_block(const GlueParams& g, uint32_t b, uint32_t& h) {
@@ -236,11 +238,21 @@ static __device__ __attribute__((always_inline)) inline void gt_whole_k(const Ge
   for (int b = 0; b < NB; b++) rd_w(w[b], lds, b);
   constexpr int H0 = N0 * NB, H1 = N1 * NB;              // products of either half of a stage
   static_assert(H1 >= N0 && N1 > 0, "a read behind each product of the second half");
-  uint32_t buf = 0;
-  for (uint32_t st = 0; st < n_stages; st++) {
-    const uint32_t nbuf = buf + 1 == S ? 0 : buf + 1;
-    const unsigned char* sb = lds + buf * STAGE;
-    const unsigned char* sn = lds + nbuf * STAGE;
+  // Accumulating calls: the first NOLD of the wave's old blocks are requested behind the last stage's loads, under the products of the last S stages (addresses clamped
+  // instead of guarded: a guarded load is a branch, one load a basic block, and the compiler waits for each).  Behind the loop, where every CU asks at once, they and the
+  // stores took 7.4 of 61 us (4096 columns of 2048 x 4096): 69.8 -> 67.8 us a call, 4096 of 2048 x 2048 45.4 -> 44.2, 1300 of 5120 x 6144 86.5 -> 84.9.  Not on the 256 x 256 tile, whose
+  // accumulators leave no room for a useful part of them (3000 of 5120 x 6144 160.0, with 16 of its 32 blocks 164.0, with 8 161.9).
+  constexpr int NM = NA * NB, PHASE = NM > 28 ? 8 : NM < GT_OLD ? NM : GT_OLD, NOLD = EPI == GT_ACC && NM <= 28 ? PHASE : 0;
+  typedef f4 f4u __attribute__((aligned(4)));                             // (y is aligned to its elements)
+  auto col_of = [&](int a) { return c0 + (wm * NA + a) * 16 + l16; };
+  auto row_of = [&](int b) { return r0 + (wn * NB + b) * 16 + 4 * kq; };
+  const size_t last = EPI == GT_ACC ? (size_t)(p.n_cols - 1) * p.y_stride + p.d_out - 4 : 0;
+  f4 old[EPI == GT_ACC ? PHASE : 1];
+  auto request_old = [&](f4& o, int m) __attribute__((always_inline)) {
+    const size_t at = (size_t)col_of(m / NB) * p.y_stride + row_of(m % NB);
+    o = *(const f4u*)(p.y + (at < last ? at : last));
+  };
+  auto first_half = [&](const unsigned char* sb) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int m = 0; m < H0; m++) {
@@ -248,24 +260,57 @@ static __device__ __attribute__((always_inline)) inline void gt_whole_k(const Ge
       __builtin_amdgcn_sched_barrier(0);
       if (m < N1) { rd_x(x1[m], sb, N0 + m); __builtin_amdgcn_sched_barrier(0); }
     }
-    // stage st + 1 is in LDS behind this barrier, and every wave has read stage st: its buffer takes stage st + S
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(LPW * (S - 2)) : "memory");
+  };
+  auto second_half = [&](const unsigned char* sn, auto READ, auto load) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
-    const uint32_t s_n = min(st + S, n_stages - 1);
 #pragma unroll
     for (int m = 0; m < H1; m++) {
       acc[N0 + m % N1][m / N1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[m / N1], x1[m % N1], acc[N0 + m % N1][m / N1], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
-      if (m < N0) rd_x(x0[m], sn, m);
-      if (m % N1 == N1 - 1) rd_w(w[m / N1], sn, m / N1);
-#pragma unroll
-      for (int i = 0; i < LPW; i++)
-        if (i * (H1 - 1) / LPW == m) PF_GLL_S(src[i] + (size_t)s_n * step[i], off[i], lds + buf * STAGE + dofs[i]);
+      if constexpr (decltype(READ)::value) {
+        if (m < N0) rd_x(x0[m], sn, m);
+        if (m % N1 == N1 - 1) rd_w(w[m / N1], sn, m / N1);
+      }
+      load(m);
       __builtin_amdgcn_sched_barrier(0);
     }
+  };
+  uint32_t buf = 0;
+  const uint32_t n_main = n_stages > S ? n_stages - S : 0;
+  for (uint32_t st = 0; st < n_main; st++) {
+    const uint32_t nbuf = buf + 1 == S ? 0 : buf + 1;
+    first_half(lds + buf * STAGE);
+    // stage st + 1 is in LDS behind this barrier, and every wave has read stage st: its buffer takes stage st + S
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(LPW * (S - 2)) : "memory");
+    second_half(lds + nbuf * STAGE, std::true_type{}, [&](int m) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < LPW; i++)
+        if (i * (H1 - 1) / LPW == m) PF_GLL_S(src[i] + (size_t)(st + S) * step[i], off[i], lds + buf * STAGE + dofs[i]);
+    });
     buf = nbuf;
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                       // (the stages past the end, never read)
+  // the last S stages, whose loads are all on their way (fewer stages than S: the ones past the end were requested as copies of the last, never read)
+  auto tail = [&](auto J) __attribute__((always_inline)) {
+    constexpr int j = decltype(J)::value;
+    if (n_main + j >= n_stages) return;
+    const uint32_t nbuf = buf + 1 == S ? 0 : buf + 1;
+    first_half(lds + buf * STAGE);
+    if constexpr (j < S - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(LPW * (S - 2 - j) + (j > 0 ? NOLD : 0)) : "memory");
+    second_half(lds + nbuf * STAGE, std::integral_constant<bool, (j < S - 1)>{}, [&](int m) __attribute__((always_inline)) {
+      if constexpr (j == 0) {
+#pragma unroll
+        for (int i = 0; i < NOLD; i++) if (i * H1 / (NOLD > 0 ? NOLD : 1) == m) request_old(old[i], i);
+      }
+    });
+    buf = nbuf;
+  };
+  static_assert(S >= 2 && S <= 6, "buffers");
+  tail(std::integral_constant<int, 0>{}); tail(std::integral_constant<int, 1>{});
+  if constexpr (S > 2) tail(std::integral_constant<int, 2>{});
+  if constexpr (S > 3) tail(std::integral_constant<int, 3>{});
+  if constexpr (S > 4) tail(std::integral_constant<int, 4>{});
+  if constexpr (S > 5) tail(std::integral_constant<int, 5>{});
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NOLD) : "memory");              // (copies past the end)
   if constexpr (EPI == GT_HEADS) {
     float* hx = (float*)lds;
     constexpr int LR = BN + 4;
@@ -299,37 +344,40 @@ static __device__ __attribute__((always_inline)) inline void gt_whole_k(const Ge
       lds_barrier();
     }
   } else {
-    // Accumulating calls: loads and stores share one counter, and a wait for a loaded value with stores pending waits for those as well, so the old
-    // values are fetched several blocks at a time, unconditionally (clamped addresses: a guarded load is a branch, one load a basic block), then added.
-    typedef f4 f4u __attribute__((aligned(4)));                           // (y is aligned to its elements)
-    constexpr int D = NB <= 10 ? 2 * NB : 16, NM = NA * NB;               // blocks of a phase: what fits next to the accumulators
-    auto col_of = [&](int a) { return c0 + (wm * NA + a) * 16 + l16; };
-    auto row_of = [&](int b) { return r0 + (wn * NB + b) * 16 + 4 * kq; };
-    const size_t last = (size_t)(p.n_cols - 1) * p.y_stride + p.d_out - 4;
+    // Accumulating calls: loads and stores share one counter, and a wait for a loaded value waits for the stores in front of it as well, so the old values past the first
+    // PHASE are requested, PHASE at a time, between the sums with those that are there and their stores.
+    auto store = [&](int m) __attribute__((always_inline)) {
+      const int a = m / NB, b = m % NB;
+      const uint32_t col = col_of(a), row = row_of(b);
+      if (col < p.n_cols) {
+        float* y = p.y + (size_t)col * p.y_stride + row;
+        if (row + 4 <= p.d_out) *(f4u*)y = acc[a][b];
+        else
 #pragma unroll
-    for (int m0 = 0; m0 < NM; m0 += D) {
-      f4 old[D];
-      if constexpr (EPI == GT_ACC) {
+          for (int i = 0; i < 3; i++) if (row + i < p.d_out) y[i] = EPI == GT_ACC ? y[i] + acc[a][b][i] : acc[a][b][i];
+      }
+    };
+    if constexpr (EPI != GT_ACC) {
 #pragma unroll
-        for (int m = 0; m < D && m0 + m < NM; m++) {
-          const size_t at = (size_t)col_of((m0 + m) / NB) * p.y_stride + row_of((m0 + m) % NB);
-          old[m] = *(const f4u*)(p.y + (at < last ? at : last));
+      for (int m = 0; m < NM; m++) store(m);
+    } else {
+#pragma unroll
+      for (int m0 = 0; m0 < NM; m0 += PHASE) {
+        if (NOLD == 0 && m0 == 0) {
+#pragma unroll
+          for (int m = 0; m < PHASE; m++) request_old(old[m], m);
+          __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int m = m0; m < m0 + PHASE && m < NM; m++) if (row_of(m % NB) + 4 <= p.d_out) acc[m / NB][m % NB] = old[m - m0] + acc[m / NB][m % NB];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = m0 + PHASE; m < m0 + 2 * PHASE && m < NM; m++) request_old(old[m - m0 - PHASE], m);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = m0; m < m0 + PHASE && m < NM; m++) store(m);
         __builtin_amdgcn_sched_barrier(0);
       }
-#pragma unroll
-      for (int m = 0; m < D && m0 + m < NM; m++) {
-        const int a = (m0 + m) / NB, b = (m0 + m) % NB;
-        const uint32_t col = col_of(a), row = row_of(b);
-        if (col < p.n_cols) {
-          float* y = p.y + (size_t)col * p.y_stride + row;
-          if (row + 4 <= p.d_out) *(f4u*)y = EPI == GT_ACC ? old[m] + acc[a][b] : acc[a][b];
-          else
-#pragma unroll
-            for (int i = 0; i < 3; i++) if (row + i < p.d_out) y[i] = EPI == GT_ACC ? y[i] + acc[a][b][i] : acc[a][b][i];
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
