@@ -156,9 +156,9 @@ float* pa_gate_buffer(pa_ctx* ctx);
  *   d_gate: f32 [n_cols][gate_stride] gate pre-activations [nH][hd]; NULL = no gate
  *   d_out : [n_cols][out_stride] of out_dtype, a column holds [nH][hd].  With one column it may lie over d_q; otherwise it
  *           must not share memory with the inputs.
- * pa_attn_prefill: the same contract for a causal prefill chunk of any width: the f16 MFMA kernel, or, for a chunk of
- * few columns (at most one 32- / 64-row block, or a few column groups over a long context, where the K/V stream and
- * not the matrix cores bound the pass), the split-K kernel; pa_plan_query tells which.
+ * pa_attn_prefill: the same contract for a causal prefill chunk of any width: the f16 MFMA kernel, or the split-K kernel
+ * in column groups, with a merge launch or, over a short context, in one launch, whichever an estimate of the three finds
+ * cheapest; pa_plan_query tells which.  Under stream capture, where scratch cannot grow, it is the cheapest that fits.
  * Replaces attn_flash_tile + attn_combine_tile + sigmoid_mul_mc (engine/wgsl/attn_tile.js:108-193;
  * call site engine/qwen35.js:2489-2493, :2516); one call covers what the reference runs as
  * ceil(n_cols / 16) consecutive 16-column passes (engine/qwen35.js:3843-3860). */

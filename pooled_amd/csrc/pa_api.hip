@@ -359,6 +359,9 @@ static bool plan_one_wg(const pa_plan& pl) { return plan_self_row(pl) && pl.row_
 static bool plan_f16_partials(const pa_plan& pl, uint32_t n_cols) {
   return pl.kernel == 0 && pl.row_blocks == 1 && pl.split_len == 32 * pl.waves && n_cols < 16 && pl.n_splits >= PA_F16_PARTIALS_MIN_SPLITS;
 }
+// The context up to which one workgroup per column group, in one launch, beats splits and a merge.  Int8 rows keep the plans that they had: the sums of a
+// short context in another order move an output by up to 4e-4, and with it up to 2 % of the int8 values that a chain of ten layers stores by a step.
+static uint32_t one_launch_rows(const pa_ctx* ctx) { return kv_q8(ctx) ? 0u : 256u; }
 // rows_cap (optional): at most this many stacked rows per workgroup (16 or 32) instead of the table's choice;
 // one_split: the whole context as one split per workgroup -- with no own-row partial the kernel then writes the
 // output itself (no partials, no merge launch).  Both are what plan_prefill asks for on small chunks.
@@ -397,9 +400,15 @@ static int plan_decode(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa
     // 250 rows 7.5 / 5.9, 7.4 / 5.8, 7.4 / 6.0, MoE shape 9.5 / 8.2, 9.2 / 8.3, 9.1 / 8.1, 27B shape 9.5 / 8.1, 9.5 / 8.3, 9.3 / 8.1.  (Eight tiles are what a
     // CU's LDS holds at hd 256.)
     waves = 8; sl = 256; ns = 1;
+  } else if (!self && nb == 1 && !one_split && !ctx->decode_splits_override && seq_max <= one_launch_rows(ctx)) {
+    // ... and several columns in one row block on the tile loop's four waves (us a call, two launches / one; 2 columns at 40 and 200: 16 / 2-head shape 9.9 / 7.1, 9.7 / 9.0, 24 / 4-head
+    // 9.4 / 6.7, 9.2 / 8.7, 16 / 8-head 6.8 / 4.8, 6.8 / 5.6)
+    sl = 256; ns = 1;
   } else if (one_split || ctx->decode_splits_override) {
     // a given number of splits (a tuning override; its splits are contiguous ranges, the last one open-ended), or one
-    const uint32_t tpw = one_split ? std::max(ceil_div(tiles, W), 1u) : std::max(ceil_div(tiles, target * W), 1u);
+    // (one: two tiles a wave at least on f16 rows, since only the tile loop writes the output itself; 20 - 100 columns over up to 128 rows, us a call with the
+    // single-round kernel and a merge of its one split / without: 16 / 2-head shape 10.1 / 8.6, 16 / 8-head shape 8.7 / 6.0)
+    const uint32_t tpw = one_split ? std::max(ceil_div(tiles, W), kv_q8(ctx) ? 1u : 2u) : std::max(ceil_div(tiles, target * W), 1u);
     sl = 32 * W * tpw; ns = ceil_div(seq_max, sl);
   } else if ((nb == 1 || (nb == 2 && W == 4 && seq_max > 32 * W)) &&
              ceil_div(seq_max, 32 * W) <= (nb == 2 && c.head_dim == 128 ? 2 * target : target)) {
@@ -444,61 +453,115 @@ static int plan_decode(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa
   return PA_OK;
 }
 
-// Prefill (MFMA kernel): a workgroup is 8 wavefronts x 32 query rows = 256 rows of one kv head, i.e.
-// floor(256 / G) columns x G heads.  Chunks wide enough to give every CU a workgroup run unsplit and write the
-// output directly; narrower chunks are also split over the context (partials + merge kernel) until every CU has a
-// workgroup (one is resident per CU; a second round of a few workgroups costs more than longer splits).  Chunks of fewer rows than one wavefront tile go to the split-K decode kernel.
-static int plan_prefill(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa_plan* pl) {
+// Bytes of the partials of n_cols columns in `slots` slots: O rows and (m, l) pairs
+static size_t partial_o_bytes(const pa_ctx* ctx, uint32_t n_cols, uint32_t slots) { return (size_t)n_cols * ctx->cfg.n_heads * slots * ctx->cfg.head_dim * sizeof(float); }
+static size_t partial_ml_bytes(const pa_ctx* ctx, uint32_t n_cols, uint32_t slots) { return (size_t)n_cols * ctx->cfg.n_heads * slots * 2 * sizeof(float); }
+
+// What the three ways to serve a chunk take, in us, fitted to 750 timed calls (16 / 2-, 24 / 4- and 16 / 8-head shapes, 5 - 1024 columns at 0 - 60000 rows, f16 and
+// int8 rows; mean error 4 - 10 %; over 890 more with sizes by their logarithm the plans come to 92 % of the time of fixed lines between the three and to 100.4 % of the best choice on f16 rows).  u counts 16-row blocks times 128-row steps of a CU; x a cache's values, in millions; `at` is a context in thousands of rows.
+// Split-K kernel with its merge launch: the two launches' fixed time, then a workgroup's chain of tiles (which is the average over the CUs only if its
+// splits fill them), whose rate rises once the chip is busy; not less than the cache's stream.
+static double chunk_us_split(const pa_ctx* ctx, const pa_plan& pl, uint32_t rows) {
   const pa_config& c = ctx->cfg;
-  const uint32_t G = c.n_heads / c.n_kv_heads;
+  const double wgs = (double)pl.col_groups * c.n_kv_heads * pl.n_splits / ctx->n_cu, steps = pl.split_len / 128, x = 1e-6 * c.n_kv_heads * rows * c.head_dim;
+  const double mean = (double)pl.col_groups * pl.row_blocks * c.n_kv_heads * ceil_div(rows, 32) / (4.0 * ctx->n_cu);
+  const double chain = steps > 1.0 ? pl.row_blocks * steps * std::max(1.0, wgs) : mean;
+  const auto bend = [](double u, double k, double lo, double hi) { return lo * std::min(u, k) + hi * std::max(u - k, 0.0); };
+  double us;
+  if (c.head_dim == 256) us = kv_q8(ctx) ? 11.4 + bend(chain, 15.0, 1.46, 0.95) : 11.2 + bend(chain, 8.5, 1.26, 0.75);
+  else us = kv_q8(ctx) ? 10.6 + bend(0.5 * (mean + chain), 14.5, 0.82, 0.56) : 11.1 + bend(0.7 * mean + 0.3 * chain, 14.0, 0.65, 0.42);
+  return std::max(us, (kv_q8(ctx) ? 0.4 : 0.8) * x);
+}
+// Split-K kernel, the whole context in one workgroup per column group: one launch, the chain of a workgroup's tiles; past one workgroup a CU they share it.
+// From two a CU on their number counts: at head_dim 256, where a CU holds one workgroup of two row blocks, in whole rounds, at 128 by the CU that has one more where
+// every workgroup has the whole context, and on average where their contexts differ (1360 columns at 35 of the 16 / 8-head shape, 680 workgroups, 29 us).
+static double chunk_us_one(const pa_ctx* ctx, const pa_plan& pl, uint32_t base_pos, uint32_t rows) {
+  const double wgs = (double)pl.col_groups * ctx->cfg.n_kv_heads / ctx->n_cu;
+  double load = 1.0;
+  if (ctx->cfg.head_dim == 256 && pl.row_blocks > 1) load = 0.5 * std::ceil(wgs);
+  else load = 0.5 * (wgs + (std::ceil(wgs) - wgs) * base_pos / rows);
+  const double at = 1e-3 * rows * std::max(load, 1.0);
+  const bool over = wgs > 1.0, wide = pl.row_blocks > 2;
+  if (ctx->cfg.head_dim == 256) {
+    if (kv_q8(ctx)) return wide ? 13.0 + (over ? 55.0 : 23.6) * at : pl.row_blocks == 2 ? 11.2 + (over ? 48.0 : 20.0) * at : 6.4 + (over ? 30.0 : 18.4) * at;
+    return wide ? 14.0 + (over ? 40.0 : 17.3) * at : pl.row_blocks == 2 ? (over ? 14.0 + 31.5 * at : 10.8 + 13.6 * at) : (over ? 7.0 + 21.1 * at : 8.0 + 10.8 * at);
+  }
+  if (kv_q8(ctx)) return wide ? 9.0 + (over ? 32.0 : 17.0) * at : pl.row_blocks == 2 ? (over ? 5.2 + 20.0 * at : 6.2 + 13.0 * at) : 4.7 + (over ? 15.5 : 10.6) * at;
+  return wide ? 8.8 + (over ? 25.0 : 13.5) * at : pl.row_blocks == 2 ? (over ? 5.2 + 13.0 * at : 6.4 + 7.1 * at) : (over ? 4.8 + 10.3 * at : 6.0 + 5.7 * at);
+}
+// Matrix-core kernel (int8 rows: the widening of the cache before it): staging of up to 256 query rows, the work, the cache's stream.
+static double chunk_us_mfma(const pa_ctx* ctx, uint32_t n_cols, uint32_t rows) {
+  const pa_config& c = ctx->cfg;
+  const uint32_t stacked = n_cols * (c.n_heads / c.n_kv_heads);
+  const double u = stacked / 16.0 * c.n_kv_heads * ceil_div(rows, 32) / (4.0 * ctx->n_cu), x = 1e-6 * c.n_kv_heads * rows * c.head_dim;
+  const double wg = std::min(stacked, 256u) / 256.0;
+  if (c.head_dim == 256) return kv_q8(ctx) ? 18.0 + 18.5 * wg + 0.32 * u + 0.82 * x : std::max(14.0 + 20.0 * wg + 0.30 * u + 0.26 * x, 12.0 + 0.8 * x);
+  return kv_q8(ctx) ? 14.0 + 9.0 * wg + 0.24 * u + 0.92 * x : 8.5 + 16.0 * std::min(wg, 0.78) + 0.17 * u + 0.47 * x;
+}
+
+static bool chunk_would_allocate(const pa_ctx* ctx, uint32_t n_cols, const pa_plan& pl) {
+  return (pl.n_splits > 1 && (partial_o_bytes(ctx, n_cols, pl.slots) > ctx->part_o_bytes || partial_ml_bytes(ctx, n_cols, pl.slots) > ctx->part_ml_bytes)) ||
+         (pl.kernel == 1 && kv_q8(ctx) && !(ctx->wide_k && ctx->wide_v));
+}
+
+// Prefill.  Chunks of up to two (head_dim 256) or four 16-row blocks go to the split-K kernel as a verify block does.  The others take the cheapest of three by
+// the estimates above.  Matrix-core kernel: a workgroup is 8 wavefronts x 32 query rows = 256 rows of one kv head, i.e. floor(256 / G) columns x G heads; chunks wide
+// enough to give every CU a workgroup run unsplit and write the output directly, narrower ones are also split over the context (partials + merge
+// kernel) until every CU has a workgroup (one is resident per CU; a second round of a few workgroups costs more than longer splits).  Split-K kernel in column
+// groups: its workgroups of 16 - 64 rows fill the chip from a few columns on.  The same in one launch, each workgroup over the whole context of its columns,
+// where the column groups alone fill half the chip.  Measured (us a call: matrix-core kernel / split-K / one launch): 16 / 2-head shape, 16 columns at 2000
+// 22.8 / 12.8 / -, 64 at 2000 34.8 / 19.0 / -, 128 at 2000 38.0 / 22.1 / 32.1, 256 at 3000 42.2 / 44.4 / -, 64 at 30000 50.8 / 63.6 / -; 24 / 4-head shape, 64 at 3000 38.2 / 24.4 / 42.4; 16 / 8-head
+// shape, 256 at 0 16.8 / 14.5 / 6.3, 512 at 1500 30.0 / 28.9 / 20.7, 96 at 600 19.0 / 14.1 / 21.1, 192 at 12000 37.3 / 45.3 / -, 256 at 30000 69.7 / 112.7 / -.
+// fits_scratch: only plans whose partials (and, for int8 rows, whose widened cache) the context already holds (a call under capture cannot allocate).
+static int plan_prefill(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa_plan* pl, bool fits_scratch = false) {
+  const pa_config& c = ctx->cfg;
+  const uint32_t G = c.n_heads / c.n_kv_heads, rows = base_pos + n_cols;
   const uint32_t max_rows_sk = c.head_dim == 256 ? 32u : 64u;
-  if (n_cols * G <= max_rows_sk) return plan_decode(ctx, base_pos, n_cols, pl, true);
-  // pa_set_prefill_tile: 2 = never the matrix-core kernel (where the split-K kernel can hold a column's heads),
-  // 1 = always (the two table rules below are skipped), 0 = the table
+  if (n_cols * G <= max_rows_sk) {
+    // (over a short context in groups of one row block, in one launch: 4 columns at 40 and 200, 24 / 4-head shape 9.6 / 6.9 and 10.4 / 8.7 us; 32 at 40, 16 / 8-head shape 9.9 / 5.1)
+    if (n_cols > 1 && rows <= one_launch_rows(ctx) && G <= 16 && !ctx->decode_splits_override) return plan_decode(ctx, base_pos, n_cols, pl, true, 16, true);
+    return plan_decode(ctx, base_pos, n_cols, pl, true);
+  }
+  // pa_set_prefill_tile: 2 = never the matrix-core kernel (where the split-K kernel can hold a column's heads), 1 = always, 0 = by the estimates
   if (ctx->prefill_tile_mode == 2 && max_rows_sk >= G) return plan_decode(ctx, base_pos, n_cols, pl, true);
   const bool table = ctx->prefill_tile_mode == 0;
-  // A chunk of a few column groups over a long context (the reference's own prefill passes are 16 columns wide) is
-  // bound by the K/V stream, not by the matrix cores: the split-K kernel serves it in column groups, whose workgroups
-  // share the stream through L2, for as long as groups x K/V bytes stays below what the MFMA kernel's fixed costs
-  // (Q staging, one partial per split and row, the merge) amount to.  Measured crossover on the MoE and 27B shapes
-  // at 32K - 64K rows: about 1.4 GB of L2-level K/V traffic; below 4096 rows both kernels take 25 - 40 us.
-  if (table && n_cols * G <= 512 && base_pos + n_cols >= 4096 && max_rows_sk >= G) {
-    pa_plan sk;
-    const uint64_t kv_bytes = 2ull * (base_pos + n_cols) * c.n_kv_heads * c.head_dim * (kv_q8(ctx) ? 1 : 2);
-    if (plan_decode(ctx, base_pos, n_cols, &sk, true) == PA_OK && (uint64_t)sk.col_groups * kv_bytes <= 1400000000ull) {
-      *pl = sk;
-      return PA_OK;
-    }
+  const uint32_t cw = 256 / G;
+  pa_plan best; memset(&best, 0, sizeof best);
+  double best_us = -1.0;
+  const auto offer = [&](const pa_plan& q, double us) {
+    if (fits_scratch && chunk_would_allocate(ctx, n_cols, q)) return;
+    if (best_us < 0.0 || us < best_us) { best = q; best_us = us; }
+  };
+  if (cw) {
+    const uint32_t groups = ceil_div(n_cols, cw), base_wgs = groups * c.n_kv_heads;
+    uint32_t splits = 1;
+    if (base_wgs < (uint32_t)ctx->n_cu) splits = std::min(std::max(1u, (uint32_t)ctx->n_cu / base_wgs), std::max(1u, rows / 256));
+    const uint32_t sl = ceil_div(ceil_div(rows, splits), 32) * 32;
+    pa_plan q; memset(&q, 0, sizeof q);
+    q.kernel = 1; q.split_len = sl; q.n_splits = ceil_div(rows, sl);
+    q.col_groups = groups; q.cols_per_group = cw; q.waves = 8; q.row_blocks = 8; q.slots = q.n_splits;
+    // (up to two of its workgroups' rows and within the estimates' error: the split-K kernel, whose fewer splits keep smaller partials)
+    offer(q, (n_cols * G <= 512 ? 1.05 : 1.0) * chunk_us_mfma(ctx, n_cols, rows));
   }
-  // A small chunk (the first chunks of a prompt, a 512-column chunk over a 2K context): the matrix-core kernel's
-  // 256-row workgroups leave most CUs idle unless the chunk is also split over the context, and then the partials
-  // (a row of head_dim floats per split and stacked row) and the merge launch cost more than the attention itself.
-  // Below about 8 GFLOP of causal work the split-K kernel serves the chunk in one launch instead: 16- or 32-row
-  // workgroups (the larger that still gives every CU a workgroup), each over the whole context of its columns,
-  // writing the normalised, gated output itself -- for contexts below 4096 rows (longer ones are the rule above) and
-  // chunks whose column groups fill at least half the chip.  Measured crossover (us per call, this path vs the matrix-core
-  // kernel): dense shape 256 columns from position 0: 6.3 vs 16.8, 512 columns at 1536: 25 vs 32, 2048 from 0: 48 vs
-  // 47; MoE shape 256 from 0: 11 vs 33, 512 from 0: 21 vs 36, 1024 from 0: 52 vs 44.
-  {
+  if (table && max_rows_sk >= G) {
+    pa_plan q; memset(&q, 0, sizeof q);
+    // Int8 rows over contexts this short: the matrix-core kernel or, up to 8 GFLOP, 16 or 32 rows in one launch (one_launch_rows tells why; 40 columns at 700,
+    // 100 at 300 of the 16 / 8-head shape move 1.2 and 2.1 % of the twelfth layer's values, 40 at 3000 0.7 %; 10 layers of the 16 / 2-head shape 0.8 % at 700).
+    const bool keep = kv_q8(ctx) && rows < (c.head_dim == 256 ? 1000u : 2000u);
     const double flops = 4.0 * c.n_heads * c.head_dim * ((double)n_cols * base_pos + 0.5 * (double)n_cols * (n_cols + 1));
-    if (table && flops <= 8.0e9 && G <= 16 && base_pos + n_cols < 4096 && !ctx->decode_splits_override) {
-      const uint32_t rows = (uint64_t)ceil_div(n_cols, 32 / G) * c.n_kv_heads >= (uint64_t)ctx->n_cu ? 32u : 16u;
-      // one split per workgroup only pays when the column groups alone occupy the chip (or the context is a few tiles)
-      if ((uint64_t)ceil_div(n_cols, rows / G) * c.n_kv_heads * 2 >= (uint64_t)ctx->n_cu || base_pos + n_cols <= 256)
-        return plan_decode(ctx, base_pos, n_cols, pl, true, rows, true);
+    const uint64_t n_cu = (uint64_t)ctx->n_cu;
+    const bool full32 = 32 >= G && (uint64_t)ceil_div(n_cols, 32 / G) * c.n_kv_heads >= n_cu;      // 32 rows a workgroup fill the chip
+    if (!keep && plan_decode(ctx, base_pos, n_cols, &q, true) == PA_OK && q.n_splits > 1) offer(q, chunk_us_split(ctx, q, rows));
+    // one launch: 16, 32 or, at a workgroup a CU at most, more stacked rows in a workgroup, where the groups alone occupy half the chip (or the context is a few tiles)
+    for (uint32_t cap = 16; !ctx->decode_splits_override && cap <= (c.head_dim == 256 ? 48u : 64u); cap = cap == 32 && c.head_dim == 128 ? 64 : cap + 16) {
+      if ((cap == 16 && full32) || (keep && (cap != (full32 ? 32u : 16u) || flops > 8.0e9))) continue;
+      if (cap < G || plan_decode(ctx, base_pos, n_cols, &q, true, cap, true) != PA_OK || q.n_splits != 1) continue;
+      const uint64_t wgs = (uint64_t)q.col_groups * c.n_kv_heads;
+      if ((wgs * 2 >= n_cu || rows <= 256) && (cap <= 32 || wgs <= n_cu)) offer(q, keep ? 0.0 : chunk_us_one(ctx, q, base_pos, rows));
     }
   }
-  const uint32_t rows_wg = 256;
-  const uint32_t cw = rows_wg / G;
-  if (cw == 0) return PA_ERR_UNSUPPORTED;
-  const uint32_t groups = ceil_div(n_cols, cw);
-  const uint32_t seq_max = base_pos + n_cols;
-  const uint32_t base_wgs = groups * c.n_kv_heads;
-  uint32_t splits = 1;
-  if (base_wgs < (uint32_t)ctx->n_cu) splits = std::min(std::max(1u, (uint32_t)ctx->n_cu / base_wgs), std::max(1u, seq_max / 256));
-  uint32_t sl = ceil_div(ceil_div(seq_max, splits), 32) * 32;
-  pl->kernel = 1; pl->split_len = sl; pl->n_splits = ceil_div(seq_max, sl);
-  pl->col_groups = groups; pl->cols_per_group = cw; pl->waves = 8; pl->row_blocks = 8; pl->slots = pl->n_splits;
+  if (best_us < 0.0) return PA_ERR_UNSUPPORTED;
+  *pl = best;
   return PA_OK;
 }
 
@@ -535,12 +598,9 @@ static int grow_scratch(pa_ctx* ctx, void** buf, size_t* have, size_t need) {
 }
 
 static int ensure_partials(pa_ctx* ctx, uint32_t n_cols, uint32_t slots) {
-  const pa_config& c = ctx->cfg;
-  const size_t need_o = (size_t)n_cols * c.n_heads * slots * c.head_dim * sizeof(float);
-  const size_t need_ml = (size_t)n_cols * c.n_heads * slots * 2 * sizeof(float);
-  int rc = grow_scratch(ctx, (void**)&ctx->part_o, &ctx->part_o_bytes, need_o);
+  int rc = grow_scratch(ctx, (void**)&ctx->part_o, &ctx->part_o_bytes, partial_o_bytes(ctx, n_cols, slots));
   if (rc) return rc;
-  return grow_scratch(ctx, (void**)&ctx->part_ml, &ctx->part_ml_bytes, need_ml);
+  return grow_scratch(ctx, (void**)&ctx->part_ml, &ctx->part_ml_bytes, partial_ml_bytes(ctx, n_cols, slots));
 }
 
 // an event pair for a kernel-exact timing of the next main-kernel launch (profiling on), else an empty PaTiming
@@ -670,6 +730,12 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
   }
   pa_plan pl;
   rc = kind == 0 ? plan_decode(ctx, base_pos, n_cols, &pl, true) : plan_prefill(ctx, base_pos, n_cols, &pl);
+  if (kind == 1 && rc == PA_OK && chunk_would_allocate(ctx, n_cols, pl)) {
+    // under capture nothing can grow: the cheapest plan that the context's scratch already holds, if there is one
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    pa_plan held;
+    if (hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st == hipStreamCaptureStatusActive && plan_prefill(ctx, base_pos, n_cols, &held, true) == PA_OK) pl = held;
+  }
   if (rc) return fail(ctx, rc, std::string(who) + ": shape outside the gfx950 table");
   if (pl.slots > 8192) return fail(ctx, PA_ERR_UNSUPPORTED, std::string(who) + ": too many splits");
   // one split and no own-row partial: the kernel writes the output itself (the prefill kernel, or the split-K kernel's

@@ -6,7 +6,8 @@ import ctypes
 import numpy as np
 import pytest
 from pooled_amd.capi import PooledAttn, PA_OUT_F32, PA_W_Q4_0
-from helpers import SHAPES
+from helpers import SHAPES, assert_parity, random_cache
+from oracle import c_oracle as C
 
 pytestmark = pytest.mark.gpu
 vp = ctypes.c_void_p
@@ -83,6 +84,46 @@ def test_decode_steps_replayed_from_a_graph():
             _ok(hip.hipStreamSynchronize(stream), "hipStreamSynchronize")
             for a, b in zip(results(), eager):
                 assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), "replay %d differs from the eager run" % rep
+        _ok(hip.hipGraphExecDestroy(gexec), "hipGraphExecDestroy"); _ok(hip.hipGraphDestroy(graph), "hipGraphDestroy")
+        pa._chk(pa.L.pa_set_stream(pa.ctx, None))
+    _ok(hip.hipStreamDestroy(stream), "hipStreamDestroy")
+
+
+def test_chunk_captured_before_any_eager_call_takes_a_plan_without_scratch():
+    """A chunk whose cheapest plan needs partials that the context has not allocated yet: under capture it takes the
+    cheapest plan that needs none, and every replay gives that plan's result; eager calls take the cheapest plan."""
+    cfg = SHAPES["qwen38_27b"]
+    nH, nKV, hd = cfg["n_heads"], cfg["n_kv_heads"], cfg["head_dim"]
+    qd, base, n = nH * hd, 300, 144
+    rng = np.random.default_rng(15)
+    k16, v16 = random_cache(cfg, base + n, seed=16)
+    q = rng.standard_normal((n, nH, hd), dtype=np.float32); gate = rng.standard_normal(q.shape, dtype=np.float32)
+    ref = C.attention(q, k16, v16, base, gate=gate)
+    hip = _hip()
+    stream = vp()
+    _ok(hip.hipStreamCreate(ctypes.byref(stream)), "hipStreamCreate")
+    with PooledAttn(cfg, base + n, n_layers=1, max_cols=n) as pa:
+        pa._chk(pa.L.pa_set_stream(pa.ctx, stream))
+        pa.layer_alloc(0)
+        pa.kv_write(0, 0, 0, k16); pa.kv_write(0, 1, 0, v16)
+        assert pa.plan("prefill", base, n)["n_splits"] > 1
+        dq, dg, dout = pa.to_device(q), pa.to_device(gate), pa.alloc(n * qd * 4)
+        graph, gexec = vp(), vp()
+        pa.sync()
+        _ok(hip.hipStreamBeginCapture(stream, 0), "hipStreamBeginCapture")
+        pa.attn("prefill", 0, dq, qd, dg, qd, base, n, dout, qd, PA_OUT_F32)
+        _ok(hip.hipStreamEndCapture(stream, ctypes.byref(graph)), "hipStreamEndCapture")
+        _ok(hip.hipGraphInstantiate(ctypes.byref(gexec), graph, None, None, 0), "hipGraphInstantiate")
+        first = None
+        for rep in range(3):
+            dout.upload(np.zeros(n * qd, np.float32)); pa.sync()
+            _ok(hip.hipGraphLaunch(gexec, stream), "hipGraphLaunch")
+            _ok(hip.hipStreamSynchronize(stream), "hipStreamSynchronize")
+            got = dout.download(np.float32, n * qd).copy().reshape(ref.shape)
+            assert_parity(got, ref, "captured chunk, replay %d" % rep)
+            first = got if first is None else first
+            assert np.array_equal(got, first)
+            assert_parity(pa.run_attn("prefill", 0, q, base, gate=gate), ref, "eager chunk between replays")
         _ok(hip.hipGraphExecDestroy(gexec), "hipGraphExecDestroy"); _ok(hip.hipGraphDestroy(graph), "hipGraphDestroy")
         pa._chk(pa.L.pa_set_stream(pa.ctx, None))
     _ok(hip.hipStreamDestroy(stream), "hipStreamDestroy")

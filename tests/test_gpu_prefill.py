@@ -142,6 +142,42 @@ def test_prefill_small_chunk_takes_the_stream_kernel_in_one_launch(shape, base, 
         assert_parity(got, ref, "small chunk %s base %d n %d" % (shape, base, n))
 
 
+@pytest.mark.parametrize("shape,base,n,kernel,split,blocks", [
+    ("qwen36_moe", 0, 33, 0, False, 1), ("qwen36_moe", 1000, 5, 0, True, 2), ("qwen36_moe", 450, 320, 0, False, 2), ("qwen36_moe", 2000, 100, 0, True, 2),
+    ("qwen36_moe", 3500, 256, 1, True, 8), ("qwen38_27b", 300, 512, 0, False, 3), ("qwen38_27b", 1500, 40, 0, True, 2), ("qwen38_27b", 3500, 200, 1, True, 8),
+    ("qwen3_1p7b", 2000, 128, 0, True, 4), ("qwen3_1p7b", 300, 1000, 0, False, 2), ("qwen3_1p7b", 500, 400, 0, False, 2), ("qwen3_1p7b", 3000, 33, 1, True, 8),
+])
+def test_prefill_chunk_takes_the_cheapest_of_three(shape, base, n, kernel, split, blocks):
+    """Both sides of the lines between the matrix-core kernel, the split-K kernel with its merge and the one-launch split-K
+    kernel of one, two and more row blocks; rows past the chunk are NaN."""
+    rows = sorted({0, 1, n // 3, n // 2, n - 2, n - 1})
+    got, ref, plan = _prefill(SHAPES[shape], base, n, seed=base + n + 9, tile=0, check_rows=rows)
+    assert (plan["kernel"], plan["n_splits"] > 1, plan["row_blocks"]) == (kernel, split, blocks), plan
+    assert_parity(got, ref, "chunk %s base %d n %d" % (shape, base, n))
+
+
+@pytest.mark.parametrize("shape", ["qwen36_moe", "qwen38_27b", "qwen3_1p7b"])
+@pytest.mark.parametrize("total", [3, 32, 33, 128, 129, 256, 257])
+def test_a_few_columns_over_a_short_context(shape, total):
+    """Blocks of one row block (prefill and decode calls) and chunks of several, either side of the context that one
+    launch serves: no column has more rows than one before the last, the first block starts at position 0."""
+    cfg = SHAPES[shape]
+    G = cfg["n_heads"] // cfg["n_kv_heads"]
+    for n in sorted({min(total, 2), min(total, 16 // G), min(total, 32 // G + 1)}):
+        got, ref, plan = _prefill(cfg, total - n, n, seed=total + n, tile=0)
+        assert plan["kernel"] == 0 and ((plan["n_splits"] == 1) == (total <= 256)) and (total > 256 or plan["row_blocks"] == 1), plan
+        assert_parity(got, ref, "short %s %d columns of %d" % (shape, n, total))
+    n = min(total, 16 // G)
+    rng = np.random.default_rng(total)
+    k16, v16 = random_cache(cfg, total, seed=total)
+    q = rng.standard_normal((n, cfg["n_heads"], cfg["head_dim"]), dtype=np.float32)
+    with PooledAttn(cfg, total, n_layers=1, max_cols=n) as pa:
+        pa.layer_alloc(0)
+        pa.kv_write(0, 0, 0, k16.copy()); pa.kv_write(0, 1, 0, v16.copy())
+        assert pa.plan("decode", total - n, n)["n_splits"] == (1 if total <= 256 else 3)
+        assert_parity(pa.run_attn("decode", 0, q, total - n), C.attention(q, k16, v16, total - n), "short decode block %s of %d" % (shape, total))
+
+
 def test_prefill_tile_override():
     """pa_set_prefill_tile (the reference's attnPrefillTile option, engine/qwen35.js:389-401): 1 forces the matrix-core
     kernel, 2 the split-K kernel, 0 is the table; all three give the same result within tolerance."""

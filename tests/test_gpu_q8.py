@@ -202,6 +202,28 @@ def test_q8_small_chunk_in_one_launch_writes_the_output_itself(base, n, rows):
             assert_parity(got, ref, "q8 small chunk base %d n %d out %d" % (base, n, out_dtype))
 
 
+@pytest.mark.parametrize("shape,base,n,kernel,split,blocks", [
+    ("qwen36_moe", 900, 130, 0, True, 2), ("qwen36_moe", 400, 640, 0, False, 3), ("qwen36_moe", 2500, 256, 1, True, 8), ("qwen38_27b", 900, 192, 0, False, 2),
+    ("qwen38_27b", 500, 192, 0, False, 1), ("qwen3_1p7b", 700, 40, 1, True, 8), ("qwen3_1p7b", 2000, 40, 0, True, 4), ("qwen3_1p7b", 1750, 300, 0, True, 4), ("qwen3_1p7b", 2500, 512, 1, True, 8),
+])
+def test_q8_chunk_takes_the_cheapest_of_three(shape, base, n, kernel, split, blocks):
+    """The plans of int8 chunks on both sides of the lines between the three ways to serve one, and of the context below
+    which they keep the two that round as before."""
+    cfg = _q8cfg(shape)
+    rng = np.random.default_rng(300 + base + n)
+    kq, ks, vq, vs, kf, vf = _quantised_cache(cfg, base + n, seed=400 + n)
+    q = rng.standard_normal((n, cfg["n_heads"], cfg["head_dim"]), dtype=np.float32)
+    gate = rng.standard_normal(q.shape, dtype=np.float32) if cfg["gate"] else None
+    ref = O.attention_values(q, kf, vf, base, gate=gate)
+    with PooledAttn(cfg, base + n, n_layers=1, max_cols=n) as pa:
+        pa.layer_alloc(0)
+        for w, a in enumerate((kq, vq, ks, vs)):
+            pa.kv_write(0, w, 0, a)
+        plan = pa.plan("prefill", base, n)
+        assert (plan["kernel"], plan["n_splits"] > 1, plan["row_blocks"]) == (kernel, split, blocks), plan
+        assert_parity(pa.run_attn("prefill", 0, q, base, gate=gate), ref, "q8 chunk %s base %d n %d" % (shape, base, n))
+
+
 def test_q8_short_verify_block_is_one_split_with_two_row_blocks():
     """A verify block over a few tiles on an int8 cache: one split, two row blocks (4 columns x 8 heads), output written
     by the split-K kernel's own epilogue."""
