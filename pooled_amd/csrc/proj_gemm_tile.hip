@@ -7,8 +7,8 @@
 //     their copies of the tile meet in LDS at the end, added up in group order (no partial sums in memory);
 //   * both operands go to LDS by LDS-direct loads (no staging registers): K in stages of 32 KG, S buffers, so S - 1 stages
 //     are in flight.  Activation rows are staged with the 16-byte chunk order XORed by the row, the weights as the 1 KB fragments they
-//     are kept in: fragments without bank conflicts where KG groups split K (SQ_LDS_BANK_CONFLICT = 0); the 16-row fragments of gt_whole_k lose
-//     14 - 44 % of the LDS's cycles to them (conflicts / active, by tile: 128 x 320 0.14, 128 x 256 0.33, 320 x 256 0.40, 224 x 256 0.44);
+//     are kept in: fragments without bank conflicts where KG groups split K (SQ_LDS_BANK_CONFLICT = 0); the 16-row fragments of gt_whole_k have a swizzle of their
+//     own (gt_swz64; under the other one 14 - 44 % of the LDS's active cycles were conflicts);
 //   * one barrier a stage, in the MIDDLE of its products: a stage is two k-steps of 16 a wave, or, where a wave holds whole sums (KG = 1,
 //     the shapes of the power-limited sizes), one of 32 on 16 x 16 x 32 products (gt_whole_k); the next fragments are
 //     read, and the stage's loads issued, one at a time between the MFMAs, so that behind the barrier a wave's next MFMA
