@@ -6,6 +6,11 @@
 // tiles instead of all dims of its own tile's:
 //   * a wave scores its own tile (q fragments in registers: the K tile is all that the product reads from LDS) and publishes its row maxima; behind a
 //     barrier every wave knows the workgroup's, so all of them work relative to one lazily updated reference and P of the four tiles can be added up by the MFMA;
+//   * with one reference for four tiles only one of their largest weights is 1, and exact in f16, where a wave of its own has one in every tile: P's rounding alone would
+//     make an output's error 1 - 2 % larger over several tiles a wave and 6 % over one (relative, against 64 bits; tile loop and single-round kernel 2.5 - 2.9e-4).  The scores
+//     therefore see the first quarter of q's dims at f32 precision (f16 + f16, q_lo_row of attn_decode.hip), which takes a quarter of q's rounding out: 0.92 - 0.98 of
+//     the others' error for 0.2 - 0.4 us a call (16 / 2-head shape, 5 columns at 8191 rows 14.3 -> 14.7, 24 / 4-head, 8 at 65536 54.0 -> 54.3; half of the dims 0.87 - 0.89
+//     for 0.4 - 0.9 us, all of them spill; P in two halves 0.73 - 0.82 for 0.5 - 3 us);
 //   * P goes to LDS, V to the wave's V region; behind a second barrier each wave multiplies the four tiles' V^T by their P for its dims.
 // Nothing is merged at the end: the waves of the tile loop meet in LDS there, 1.9 / 2.6 / 4.3 us with two / two / three row blocks (in-kernel stamps: 16 / 2-head shape, 5
 // columns at 8191 rows and 16 at 12345; 24 / 4-head shape, 8 at 65536), which no stream hides.  The price is two barriers a turn, so that the workgroup's
@@ -23,7 +28,9 @@ template <int HD, int NB> struct BlockLds {
   typedef DecShape<HD> S;
   static constexpr int W = 4;
   static constexpr int v = W * TILE * S::KROW, p = v + W * S::STAGE, mx = p + W * NB * 1024, l = mx + W * 16 * NB * 4, bytes = l + W * 16 * NB * 4;
-  static_assert(16 * NB * S::QROW <= W * S::STAGE, "the q rows pass through the V regions");
+  // the low halves of q's first HD / 4 dims (k-steps 0 .. QL - 1), rows of LROW bytes behind the q rows
+  static constexpr int QL = S::KS / 4, LROW = QL * 64 + 16;
+  static_assert(16 * NB * (S::QROW + LROW) <= W * S::STAGE, "the q rows and their low halves pass through the V regions");
 };
 
 template <int HD, int NB, bool Q8>
@@ -119,6 +126,14 @@ void pa_block_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a_
     const uint32_t e = tid + j * 256, r = min(e / (HD / 4), R - 1), d4 = e % (HD / 4), qc = div_g(r);      // padding rows copy the last live one (masked below)
     qv[j] = *(const f4*)(p.q + (size_t)(c0 + qc) * p.q_stride + (size_t)(g * G + r - qc * G) * HD + 4 * d4);
   }
+  // (a quarter of the rows' dims once more: in the threads that have them already, the low halves cost four times the instructions; 0.2 us a call)
+  constexpr int QL = L::QL, QL4 = QL * 8, LPT = (16 * NB * QL4 + 255) / 256;
+  f4 qlv[LPT];
+#pragma unroll
+  for (int j = 0; j < LPT; j++) {
+    const uint32_t e = min(tid + j * 256, 16u * NB * QL4 - 1), r = min(e / QL4, R - 1), qc = div_g(r);
+    qlv[j] = *(const f4*)(p.q + (size_t)(c0 + qc) * p.q_stride + (size_t)(g * G + r - qc * G) * HD + 4 * (e % QL4));
+  }
   uint32_t tp = t_begin + wave * TILE;
   load_tile(kr, ksr, kbase, ksbase, min(tp, lim - TILE));
   load_tile(vr, vsr, vbase, vsbase, min(tp, lim - TILE));
@@ -127,6 +142,15 @@ void pa_block_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a_
   for (int j = 0; j < QPT; j++) {
     const uint32_t e = tid + j * 256;
     *(h4*)(smem + L::v + e / (HD / 4) * S::QROW + e % (HD / 4) * 8) = (h4){ (_Float16)qv[j][0], (_Float16)qv[j][1], (_Float16)qv[j][2], (_Float16)qv[j][3] };
+  }
+  unsigned char* qlo = smem + L::v + 16 * NB * S::QROW;
+#pragma unroll
+  for (int j = 0; j < LPT; j++) {
+    const uint32_t e = min(tid + j * 256, 16u * NB * QL4 - 1);
+    float lo[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) lo[i] = qlv[j][i] - (float)(_Float16)qlv[j][i];
+    *(h4*)(qlo + e / QL4 * L::LROW + e % QL4 * 8) = (h4){ (_Float16)lo[0], (_Float16)lo[1], (_Float16)lo[2], (_Float16)lo[3] };
   }
   uint32_t end_pos[NB];                                              // a row sees cache rows below this; 0 for padding rows
 #pragma unroll
@@ -138,6 +162,11 @@ void pa_block_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a_
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) qf[ks][nb] = *(const h8*)(smem + L::v + (nb * 16 + ln) * S::QROW + ks * 64 + kg * 16);     // (the V tiles go there, behind the loop's first barrier)
 
+  h8 ql[QL][NB];
+#pragma unroll
+  for (int ks = 0; ks < QL; ks++)
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) ql[ks][nb] = *(const h8*)(qlo + (nb * 16 + ln) * L::LROW + ks * 64 + kg * 16);
   f4 acc[DBW][NB];
 #pragma unroll
   for (int j = 0; j < DBW; j++)
@@ -175,12 +204,20 @@ void pa_block_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a_
           s[0][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qf[ks][nb], s[0][nb], 0, 0, 0);
           s[1][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qf[ks][nb], s[1][nb], 0, 0, 0);
         }
+        if (ks < QL) {
+#pragma unroll
+          for (int nb = 0; nb < NB; nb++) {
+            s[0][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, ql[ks < QL ? ks : 0][nb], s[0][nb], 0, 0, 0);
+            s[1][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, ql[ks < QL ? ks : 0][nb], s[1][nb], 0, 0, 0);
+          }
+        }
       }
       __builtin_amdgcn_sched_group_barrier(0x100, 2 * FD, 0);
 #pragma unroll
       for (int ks = 0; ks < S::KS; ks++) {
         if (ks + FD < S::KS) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 2 * NB, 0);
+        if (ks < QL) __builtin_amdgcn_sched_group_barrier(0x008, 4 * NB, 0);
+        else __builtin_amdgcn_sched_group_barrier(0x008, 2 * NB, 0);
       }
     }
     // a lane holds row nb 16 + ln, positions tp + pb 16 + 4 kg + i (a wave past the last tile: none, end_pos is below tp)

@@ -337,11 +337,11 @@ static bool plan_single_round2(const pa_plan& pl) {
 }
 // Two row blocks or more over several splits: the kernel whose waves share one softmax and divide O by output dims (attn_block.hip) where nothing
 // outweighs its shorter end, the single-round kernel or the tile loop elsewhere.  Measured (us a call, that kernel / the other): one column group, two tiles a wave or more: 16 / 2-head
-// shape, 4 columns at 30000 rows 19.1 / 20.6, 24 / 4-head, 5 at 12001 and 20000 16.5 / 17.9 and 21.0 / 22.1, 8 at 65536 53.4 / 55.9, 16 / 8-head, 16 at 20000 22.9 / 24.3.  Several
-// column groups: two tiles a wave, 16 / 2-head, 8 columns at 12001 15.9 / 17.1, 24 / 4-head, 10 at 8000 15.4 / 16.9; from three on the waves of the tile loop, which meet
-// only at its end, share the L2's rows better (24 / 4-head, 10 columns at 20000 26.2 / 25.0, at 65536 67.3 / 57.6).  One tile a wave: where several groups or the small
-// heads fill more than half the chip but not twice (16 / 2-head, 6 at 8000 13.4 / 14.0, 24 / 4-head, 10 at 4000 13.3 / 14.3, 16 / 8-head, 9 at 4000 9.6 / 10.8; one
-// group, 16 / 2-head, 4 at 600 and 12001 11.0 / 10.6 and 14.4 / 14.2; 16 / 8-head, 12 at 8000 12.9 / 12.5).
+// shape, 4 columns at 30000 rows 19.8 / 21.2, 24 / 4-head, 5 at 12001 and 20000 18.5 / 19.4 and 23.1 / 24.1, 8 at 65536 54.3 / 57.1.  Several
+// column groups: two tiles a wave, 16 / 2-head, 8 columns at 12001 16.6 / 17.7, 24 / 4-head, 10 at 8000 17.1 / 18.5; from three on the waves of the tile loop, which meet
+// only at its end, share the L2's rows better (24 / 4-head, 10 columns at 20000 26.2 / 25.0, at 65536 67.3 / 57.6, both without the low halves of q).  One tile a wave: where several
+// groups or the small heads fill more than half the chip but not twice (16 / 2-head, 6 at 8000 13.9 / 14.6, 24 / 4-head, 10 at 4000 13.8 / 15.1, 16 / 8-head, 9 at 4000 9.0 / 10.5; one
+// group, 16 / 2-head, 4 at 600 and 12001 11.0 / 10.6 and 14.4 / 14.2; 16 / 8-head, 12 at 8000 12.9 / 12.5, as before).
 static bool plan_block(const pa_ctx* ctx, const pa_plan& pl) {
   if (pl.kernel != 0 || pl.waves != 4 || pl.row_blocks < 2 || pl.n_splits == 1) return false;
   if (ctx->decode_splits_override) return true;
