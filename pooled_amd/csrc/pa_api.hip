@@ -342,8 +342,9 @@ static bool plan_single_round2(const pa_plan& pl) {
 // only at its end, share the L2's rows better (24 / 4-head, 10 columns at 20000 26.2 / 25.0, at 65536 67.3 / 57.6, both without the low halves of q).  One tile a wave: where several
 // groups or the small heads fill more than half the chip but not twice (16 / 2-head, 6 at 8000 13.9 / 14.6, 24 / 4-head, 10 at 4000 13.8 / 15.1, 16 / 8-head, 9 at 4000 9.0 / 10.5; one
 // group, 16 / 2-head, 4 at 600 and 12001 11.0 / 10.6 and 14.4 / 14.2; 16 / 8-head, 12 at 8000 12.9 / 12.5, as before).
+// Not one column of more than 16 query heads a kv head: its own row is a partial of its own, which that kernel does not make.
 static bool plan_block(const pa_ctx* ctx, const pa_plan& pl) {
-  if (pl.kernel != 0 || pl.waves != 4 || pl.row_blocks < 2 || pl.n_splits == 1) return false;
+  if (pl.kernel != 0 || pl.waves != 4 || pl.row_blocks < 2 || pl.n_splits == 1 || plan_self_row(pl)) return false;
   if (ctx->decode_splits_override) return true;
   const uint32_t tiles = pl.split_len / 128, n_cu = (uint32_t)ctx->n_cu;
   const uint64_t wgs = (uint64_t)pl.n_splits * ctx->cfg.n_kv_heads * pl.col_groups;
@@ -355,6 +356,14 @@ static uint32_t plan_tile_ilv(const pa_plan& pl) {
 }
 // a one-column decode of at most 256 rows: one workgroup a kv head, which writes the output itself
 static bool plan_one_wg(const pa_plan& pl) { return plan_self_row(pl) && pl.row_blocks == 1 && pl.waves == 8 && pl.n_splits == 1 && pl.split_len == 256; }
+// the kernel that serves a plan
+enum { ATTN_MFMA = 0, ATTN_LOOP = 1, ATTN_SINGLE_ROUND = 2, ATTN_ONE_WG = 3, ATTN_BLOCK = 4 };
+static int plan_kernel(const pa_ctx* ctx, const pa_plan& pl) {
+  if (pl.kernel != 0) return ATTN_MFMA;
+  if (plan_one_wg(pl)) return ATTN_ONE_WG;
+  if (plan_block(ctx, pl)) return ATTN_BLOCK;
+  return (pl.row_blocks == 1 && pl.split_len == 32 * pl.waves) || plan_single_round2(pl) ? ATTN_SINGLE_ROUND : ATTN_LOOP;
+}
 #define PA_F16_PARTIALS_MIN_SPLITS 64u
 static bool plan_f16_partials(const pa_plan& pl, uint32_t n_cols) {
   return pl.kernel == 0 && pl.row_blocks == 1 && pl.split_len == 32 * pl.waves && n_cols < 16 && pl.n_splits >= PA_F16_PARTIALS_MIN_SPLITS;
@@ -569,6 +578,12 @@ extern "C" int pa_plan_query(const pa_ctx* ctx, int kind, uint32_t base_pos, uin
   if (!ctx || !out || n_cols == 0) return PA_ERR_INVALID;
   return kind == 0 ? plan_decode(ctx, base_pos, n_cols, out) : plan_prefill(ctx, base_pos, n_cols, out);
 }
+extern "C" int pa_rule_attn(const pa_config* cfg, int n_cu, int kind, uint32_t base_pos, uint32_t n_cols, uint32_t splits, pa_plan* out) {
+  pa_ctx ctx;
+  ctx.cfg = *cfg; ctx.n_cu = n_cu; ctx.decode_splits_override = splits;
+  const int rc = kind == 0 ? plan_decode(&ctx, base_pos, n_cols, out) : plan_prefill(&ctx, base_pos, n_cols, out);
+  return rc == PA_OK ? plan_kernel(&ctx, *out) : -1;
+}
 extern "C" int pa_set_prefill_tile(pa_ctx* ctx, int mode) {
   if (!ctx) return PA_ERR_INVALID;
   if (mode < 0 || mode > 2) return fail(ctx, PA_ERR_INVALID, "pa_set_prefill_tile: mode must be 0 (table), 1 (always) or 2 (never)");
@@ -781,7 +796,7 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
   p.gate_head_stride = c.head_dim;
   PaTiming tm;
   if ((rc = prof_pair(ctx, &tm))) return rc;
-  if (plan_block(ctx, pl)) HIPCHK(ctx, pa_launch_block(p, c.head_dim, pl.row_blocks, pl.col_groups, ctx->stream, &tm));
+  if (plan_kernel(ctx, pl) == ATTN_BLOCK) HIPCHK(ctx, pa_launch_block(p, c.head_dim, pl.row_blocks, pl.col_groups, ctx->stream, &tm));
   else if (pl.kernel == 0) HIPCHK(ctx, pa_launch_decode(p, c.head_dim, pl.row_blocks, pl.waves, pl.col_groups, ctx->stream, &tm));
   else HIPCHK(ctx, pa_launch_prefill(p, c.head_dim, pl.row_blocks, pl.col_groups, ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u, ctx->stream, &tm));
   if (!direct) {

@@ -568,3 +568,57 @@ def test_one_softmax_for_four_waves_is_as_exact_as_four(shape, n_cols, base, blo
     err = (((got - exact) ** 2).sum() / (exact ** 2).sum()) ** 0.5
     print("error %.4e, own references %.4e, ratio %.4f" % (err, limit, err / limit))
     assert err <= limit
+
+
+WIDE_GROUPS = [(256, 34, 2, False, (0, 100, 128, 129, 300, 16384, 16390)), (256, 64, 2, True, (127, 2000, 16390, 33000)), (256, 24, 1, False, (200, 33000)),
+               (128, 33, 1, False, (0, 127, 200, 300, 400, 2000, 4097)), (128, 64, 1, True, (130, 260, 300, 2000)), (128, 64, 2, False, (100, 2000, 10000, 33000)), (128, 20, 1, False, (128, 700, 33000))]
+
+
+@pytest.mark.parametrize("kv_q8", [False, True])
+@pytest.mark.parametrize("head_dim,n_heads,n_kv,gate,bases", WIDE_GROUPS)
+def test_one_column_of_more_than_sixteen_heads_a_kv_head(head_dim, n_heads, n_kv, gate, bases, kv_q8):
+    """Two to four row blocks whose own row is a partial of its own, either side of the lengths where the plan changes its kernel or its tiles a wave, with rows past the
+    column poisoned; the same through the prefill entry point, under a splits override, and as the columns of a column-exact block (bit for bit)."""
+    cfg = dict(n_heads=n_heads, n_kv_heads=n_kv, head_dim=head_dim, n_rot=64, rope_theta=1e6, eps=1e-6, qk_norm=True, gate=gate, kv_q8=kv_q8)
+    rng = np.random.default_rng(n_heads + head_dim)
+    rows = max(bases) + 40
+    k, v = rng.standard_normal((2, rows, n_kv, head_dim), dtype=np.float32)
+    q = rng.standard_normal((3, n_heads, head_dim), dtype=np.float32)
+    g = rng.standard_normal(q.shape, dtype=np.float32) if gate else None
+    if kv_q8:
+        kq, ks = O.q8_quantize(k); vq, vs = O.q8_quantize(v)
+        parts, bad = [kq, vq, ks, vs], {2: np.nan, 3: np.nan}
+        kf, vf = O.q8_dequantize(kq, ks), O.q8_dequantize(vq, vs)
+    else:
+        parts, bad = [x.astype(np.float16).view(np.uint16) for x in (k, v)], {0: NAN16, 1: NAN16}
+    def ref(base, n):
+        return O.attention_values(q[:n], kf[:base + n], vf[:base + n], base, gate=None if g is None else g[:n]) if kv_q8 else \
+            C.attention(q[:n], parts[0][:base + n], parts[1][:base + n], base, gate=None if g is None else g[:n])
+    def fill(pa, live):
+        for w, x in enumerate(parts):
+            x = x.copy()
+            if w in bad:
+                x[live:] = bad[w]
+            pa.kv_write(0, w, 0, x)
+    one = lambda pa, c, base, kind="decode": pa.run_attn(kind, 0, q[c:c + 1], base, gate=None if g is None else g[c:c + 1])  # noqa: E731
+    with PooledAttn(cfg, rows, n_layers=1, max_cols=4) as pa:
+        pa.layer_alloc(0)
+        for base in bases:
+            fill(pa, base + 1)
+            want = ref(base, 1)
+            what = "%d / %d heads of %d, %s, at %d" % (n_heads, n_kv, head_dim, "q8" if kv_q8 else "f16", base)
+            got = one(pa, 0, base)
+            assert_parity(got, want, what)
+            assert np.array_equal(got, one(pa, 0, base, "prefill"))
+            for splits in (2, 5):
+                pa.set_decode_splits(splits)
+                assert_parity(one(pa, 0, base), want, what + ", splits %d" % splits)
+            pa.set_decode_splits(0)
+    with PooledAttn(dict(cfg, verify_exact=True), rows, n_layers=1, max_cols=4) as pa:
+        pa.layer_alloc(0)
+        base = bases[-2]
+        fill(pa, base + 3)
+        got = pa.run_attn("decode", 0, q, base, gate=g)
+        assert_parity(got, ref(base, 3), "column-exact block of %d / %d heads" % (n_heads, n_kv))
+        for c in range(3):
+            assert np.array_equal(got[c], one(pa, c, base + c)[0])

@@ -1,0 +1,18 @@
+"""No-GPU checks of which kernel serves an attention call: the library's own plan rules, asked on a 256-CU part."""
+import pytest
+from helpers import attn_rule, BLOCK
+
+
+@pytest.mark.parametrize("kv_q8", [False, True])
+@pytest.mark.parametrize("head_dim,most", [(256, 32), (128, 64)])
+def test_one_column_never_goes_to_the_kernel_without_an_own_row(head_dim, most, kv_q8):
+    """One column of any group size over any context, with and without a splits override: its own row is a partial of its own (slots = splits + 1), which the
+    kernel of verify blocks does not make."""
+    for n_kv in (1, 2, 8):
+        for group in sorted({1, 8, 16, 17, 24, most // 2 + 1, most}):
+            cfg = dict(n_heads=group * n_kv, n_kv_heads=n_kv, head_dim=head_dim, n_rot=64, rope_theta=1e6, eps=1e-6, kv_q8=kv_q8)
+            for base in (0, 1, 127, 128, 129, 255, 256, 257, 1000, 2048, 4100, 8192, 10001, 16400, 20000, 32768, 65536, 120000):
+                for splits in (0, 1, 2, 7, 64):
+                    for kind in ("decode", "prefill"):
+                        kernel, pl = attn_rule(cfg, kind, base, 1, splits)
+                        assert kernel >= 0 and pl["slots"] == pl["n_splits"] + 1 and kernel != BLOCK, (cfg, base, splits, kind, pl)
