@@ -158,7 +158,8 @@ float* pa_gate_buffer(pa_ctx* ctx);
  *           must not share memory with the inputs.
  * pa_attn_prefill: the same contract for a causal prefill chunk of any width: the f16 MFMA kernel, or the split-K kernel
  * in column groups, with a merge launch or, over a short context, in one launch, whichever an estimate of the three finds
- * cheapest; pa_plan_query tells which.  Under stream capture, where scratch cannot grow, it is the cheapest that fits.
+ * cheapest; pa_plan_query tells which.  Under stream capture, where scratch cannot grow, it is the cheapest that fits the
+ * scratch of the context's earlier calls, or else one launch that needs none (slower: an eager call of the same shape first avoids it).
  * Replaces attn_flash_tile + attn_combine_tile + sigmoid_mul_mc (engine/wgsl/attn_tile.js:108-193;
  * call site engine/qwen35.js:2489-2493, :2516); one call covers what the reference runs as
  * ceil(n_cols / 16) consecutive 16-column passes (engine/qwen35.js:3843-3860). */

@@ -356,6 +356,10 @@ static uint32_t plan_tile_ilv(const pa_plan& pl) {
 }
 // a one-column decode of at most 256 rows: one workgroup a kv head, which writes the output itself
 static bool plan_one_wg(const pa_plan& pl) { return plan_self_row(pl) && pl.row_blocks == 1 && pl.waves == 8 && pl.n_splits == 1 && pl.split_len == 256; }
+// one split and no own-row partial: the kernel writes the output itself (the prefill kernel, or the split-K kernel's tile loop: its single-round form always leaves a partial)
+static bool plan_direct(const pa_plan& pl) {
+  return plan_one_wg(pl) || (pl.n_splits == 1 && !plan_self_row(pl) && (pl.kernel == 1 || pl.split_len != 32 * pl.waves || pl.row_blocks > 1));
+}
 // the kernel that serves a plan
 enum { ATTN_MFMA = 0, ATTN_LOOP = 1, ATTN_SINGLE_ROUND = 2, ATTN_ONE_WG = 3, ATTN_BLOCK = 4 };
 static int plan_kernel(const pa_ctx* ctx, const pa_plan& pl) {
@@ -509,8 +513,30 @@ static double chunk_us_mfma(const pa_ctx* ctx, uint32_t n_cols, uint32_t rows) {
 }
 
 static bool chunk_would_allocate(const pa_ctx* ctx, uint32_t n_cols, const pa_plan& pl) {
-  return (pl.n_splits > 1 && (partial_o_bytes(ctx, n_cols, pl.slots) > ctx->part_o_bytes || partial_ml_bytes(ctx, n_cols, pl.slots) > ctx->part_ml_bytes)) ||
+  return (!plan_direct(pl) && (partial_o_bytes(ctx, n_cols, pl.slots) > ctx->part_o_bytes || partial_ml_bytes(ctx, n_cols, pl.slots) > ctx->part_ml_bytes)) ||
          (pl.kernel == 1 && kv_q8(ctx) && !(ctx->wide_k && ctx->wide_v));
+}
+
+// Under capture, where nothing that the context holds is enough for another plan: one launch of the tile loop, which writes the output itself, however few
+// workgroups that is (one column streams its own row with the others); mode 1 of pa_set_prefill_tile: the matrix-core kernel unsplit.
+static int plan_no_scratch(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa_plan* pl) {
+  const pa_config& c = ctx->cfg;
+  const uint32_t G = c.n_heads / c.n_kv_heads, rows = base_pos + n_cols;
+  pa_plan q; memset(&q, 0, sizeof q);
+  if (ctx->prefill_tile_mode == 1 && n_cols * G > (c.head_dim == 256 ? 32u : 64u)) {
+    q.kernel = 1; q.split_len = ceil_div(rows, 32) * 32; q.n_splits = q.slots = 1;
+    q.cols_per_group = 256 / G; q.col_groups = ceil_div(n_cols, q.cols_per_group); q.waves = 8; q.row_blocks = 8;
+    *pl = q;
+    return chunk_would_allocate(ctx, n_cols, q) ? PA_ERR_UNSUPPORTED : PA_OK;
+  }
+  double best_us = -1.0;
+  for (uint32_t cap = 16; cap <= (c.head_dim == 256 ? 48u : 64u); cap = cap == 32 && c.head_dim == 128 ? 64 : cap + 16) {
+    if (cap < G || plan_decode(ctx, base_pos, n_cols, &q, false, cap, true) != PA_OK || q.n_splits != 1) continue;
+    if (!plan_direct(q)) q.split_len *= 2;
+    const double us = chunk_us_one(ctx, q, base_pos, rows);
+    if (best_us < 0.0 || us < best_us) { *pl = q; best_us = us; }
+  }
+  return best_us < 0.0 ? PA_ERR_UNSUPPORTED : PA_OK;
 }
 
 // Prefill.  Chunks of up to two (head_dim 256) or four 16-row blocks go to the split-K kernel as a verify block does.  The others take the cheapest of three by
@@ -528,11 +554,15 @@ static int plan_prefill(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, p
   const uint32_t max_rows_sk = c.head_dim == 256 ? 32u : 64u;
   if (n_cols * G <= max_rows_sk) {
     // (over a short context in groups of one row block, in one launch: 4 columns at 40 and 200, 24 / 4-head shape 9.6 / 6.9 and 10.4 / 8.7 us; 32 at 40, 16 / 8-head shape 9.9 / 5.1)
-    if (n_cols > 1 && rows <= one_launch_rows(ctx) && G <= 16 && !ctx->decode_splits_override) return plan_decode(ctx, base_pos, n_cols, pl, true, 16, true);
-    return plan_decode(ctx, base_pos, n_cols, pl, true);
+    const bool one = n_cols > 1 && rows <= one_launch_rows(ctx) && G <= 16 && !ctx->decode_splits_override;
+    const int rc = plan_decode(ctx, base_pos, n_cols, pl, true, one ? 16 : 0, one);
+    return fits_scratch && rc == PA_OK && chunk_would_allocate(ctx, n_cols, *pl) ? plan_no_scratch(ctx, base_pos, n_cols, pl) : rc;
   }
   // pa_set_prefill_tile: 2 = never the matrix-core kernel (where the split-K kernel can hold a column's heads), 1 = always, 0 = by the estimates
-  if (ctx->prefill_tile_mode == 2 && max_rows_sk >= G) return plan_decode(ctx, base_pos, n_cols, pl, true);
+  if (ctx->prefill_tile_mode == 2 && max_rows_sk >= G) {
+    const int rc = plan_decode(ctx, base_pos, n_cols, pl, true);
+    return fits_scratch && rc == PA_OK && chunk_would_allocate(ctx, n_cols, *pl) ? plan_no_scratch(ctx, base_pos, n_cols, pl) : rc;
+  }
   const bool table = ctx->prefill_tile_mode == 0;
   const uint32_t cw = 256 / G;
   pa_plan best; memset(&best, 0, sizeof best);
@@ -569,7 +599,7 @@ static int plan_prefill(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, p
       if ((wgs * 2 >= n_cu || rows <= 256) && (cap <= 32 || wgs <= n_cu)) offer(q, keep ? 0.0 : chunk_us_one(ctx, q, base_pos, rows));
     }
   }
-  if (best_us < 0.0) return PA_ERR_UNSUPPORTED;
+  if (best_us < 0.0) return fits_scratch ? plan_no_scratch(ctx, base_pos, n_cols, pl) : PA_ERR_UNSUPPORTED;
   *pl = best;
   return PA_OK;
 }
@@ -578,11 +608,11 @@ extern "C" int pa_plan_query(const pa_ctx* ctx, int kind, uint32_t base_pos, uin
   if (!ctx || !out || n_cols == 0) return PA_ERR_INVALID;
   return kind == 0 ? plan_decode(ctx, base_pos, n_cols, out) : plan_prefill(ctx, base_pos, n_cols, out);
 }
-extern "C" int pa_rule_attn(const pa_config* cfg, int n_cu, int kind, uint32_t base_pos, uint32_t n_cols, uint32_t splits, pa_plan* out) {
+extern "C" int pa_rule_attn(const pa_config* cfg, int n_cu, int kind, uint32_t base_pos, uint32_t n_cols, uint32_t splits, int tile_mode, pa_plan* out) {
   pa_ctx ctx;
-  ctx.cfg = *cfg; ctx.n_cu = n_cu; ctx.decode_splits_override = splits;
-  const int rc = kind == 0 ? plan_decode(&ctx, base_pos, n_cols, out) : plan_prefill(&ctx, base_pos, n_cols, out);
-  return rc == PA_OK ? plan_kernel(&ctx, *out) : -1;
+  ctx.cfg = *cfg; ctx.n_cu = n_cu; ctx.decode_splits_override = splits; ctx.prefill_tile_mode = tile_mode;
+  const int rc = kind == 0 ? plan_decode(&ctx, base_pos, n_cols, out) : plan_prefill(&ctx, base_pos, n_cols, out, kind == 2);
+  return rc != PA_OK ? -1 : kind == 2 && chunk_would_allocate(&ctx, n_cols, *out) ? -2 : plan_kernel(&ctx, *out);
 }
 extern "C" int pa_set_prefill_tile(pa_ctx* ctx, int mode) {
   if (!ctx) return PA_ERR_INVALID;
@@ -602,7 +632,8 @@ extern "C" int pa_set_decode_splits(pa_ctx* ctx, uint32_t splits) {
 // freed or moved while the context lives: launches recorded into a HIP graph by the caller carry the address they
 // were recorded with, and a later, larger pass must not pull that memory from under a replay.  The outgrown block is
 // kept until pa_destroy.  (Growth itself allocates, so a pass that grows a buffer cannot be captured; one eager call
-// of the same or a larger shape before the capture is enough.)
+// of the same shape at the same position before the capture is enough.  A larger one need not be: a wide chunk may be a plan without
+// partials.  A prefill call then still runs, on a plan that fits what there is, but not on its cheapest.)
 static int grow_scratch(pa_ctx* ctx, void** buf, size_t* have, size_t need) {
   if (need <= *have) return PA_OK;
   void* mem = nullptr;
@@ -746,16 +777,14 @@ static int attn_common(pa_ctx* ctx, const char* who, int kind, uint32_t layer, c
   pa_plan pl;
   rc = kind == 0 ? plan_decode(ctx, base_pos, n_cols, &pl, true) : plan_prefill(ctx, base_pos, n_cols, &pl);
   if (kind == 1 && rc == PA_OK && chunk_would_allocate(ctx, n_cols, pl)) {
-    // under capture nothing can grow: the cheapest plan that the context's scratch already holds, if there is one
+    // under capture nothing can grow: the cheapest plan that the context's scratch already holds
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     pa_plan held;
     if (hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st == hipStreamCaptureStatusActive && plan_prefill(ctx, base_pos, n_cols, &held, true) == PA_OK) pl = held;
   }
   if (rc) return fail(ctx, rc, std::string(who) + ": shape outside the gfx950 table");
   if (pl.slots > 8192) return fail(ctx, PA_ERR_UNSUPPORTED, std::string(who) + ": too many splits");
-  // one split and no own-row partial: the kernel writes the output itself (the prefill kernel, or the split-K kernel's
-  // tile loop: its single-round form always leaves a partial)
-  const bool direct = plan_one_wg(pl) || (pl.n_splits == 1 && !plan_self_row(pl) && (pl.kernel == 1 || pl.split_len != 32 * pl.waves || pl.row_blocks > 1));
+  const bool direct = plan_direct(pl);
   const size_t osz = out_dtype == PA_OUT_F16 ? 2 : 4;
   const bool staged = plan_one_wg(pl) && (shares(d_out, qd * osz, d_q, qd * 4) || shares(d_out, qd * osz, d_gate, qd * 4));
   if ((!direct || staged) && (rc = ensure_partials(ctx, n_cols, pl.slots))) return rc;

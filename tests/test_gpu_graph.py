@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 from pooled_amd.capi import PooledAttn, PA_OUT_F32, PA_W_Q4_0
 from helpers import SHAPES, assert_parity, random_cache
+from oracle import attn_oracle as O
 from oracle import c_oracle as C
 
 pytestmark = pytest.mark.gpu
@@ -124,6 +125,60 @@ def test_chunk_captured_before_any_eager_call_takes_a_plan_without_scratch():
             first = got if first is None else first
             assert np.array_equal(got, first)
             assert_parity(pa.run_attn("prefill", 0, q, base, gate=gate), ref, "eager chunk between replays")
+        _ok(hip.hipGraphExecDestroy(gexec), "hipGraphExecDestroy"); _ok(hip.hipGraphDestroy(graph), "hipGraphDestroy")
+        pa._chk(pa.L.pa_set_stream(pa.ctx, None))
+    _ok(hip.hipStreamDestroy(stream), "hipStreamDestroy")
+
+
+@pytest.mark.parametrize("shape,kv_q8,base,n,tile,warm", [
+    ("qwen36_moe", False, 2000, 64, 0, (900, 512)), ("qwen38_27b", False, 300, 4, 0, None), ("qwen36_moe", False, 5000, 1, 0, None), ("qwen36_moe", False, 2000, 64, 2, None),
+    ("qwen38_27b", False, 300, 144, 1, None), ("qwen3_1p7b", True, 0, 40, 0, None), ("qwen36_moe", True, 3000, 256, 0, None), ("qwen36_moe", True, 90, 2, 0, None)])
+def test_any_chunk_is_captured_with_the_scratch_there_is(shape, kv_q8, base, n, tile, warm):
+    """A prefill call captured in a context that has allocated nothing for it, or behind an eager call of a larger chunk whose plan had no partials: it takes a plan that
+    fits, and every replay gives the same result; eager calls between the replays take the cheapest plan and grow the scratch.  (An int8 chunk over at most 128 rows
+    has one split whose workgroups do not write the output themselves; a few columns and the tile overrides have no estimates to choose by.)"""
+    cfg = dict(SHAPES[shape], kv_q8=kv_q8)
+    nH, nKV, hd = cfg["n_heads"], cfg["n_kv_heads"], cfg["head_dim"]
+    qd, rows = nH * hd, max(base + n, sum(warm) if warm else 0)
+    rng = np.random.default_rng(base + n)
+    k, v = rng.standard_normal((2, rows, nKV, hd), dtype=np.float32)
+    q = rng.standard_normal((n, nH, hd), dtype=np.float32); gate = rng.standard_normal(q.shape, dtype=np.float32) if cfg["gate"] else None
+    if kv_q8:
+        kq, ks = O.q8_quantize(k); vq, vs = O.q8_quantize(v)
+        parts = [kq, vq, ks, vs]
+        ref = O.attention_values(q, O.q8_dequantize(kq, ks)[:base + n], O.q8_dequantize(vq, vs)[:base + n], base, gate=gate)
+    else:
+        parts = [x.astype(np.float16).view(np.uint16) for x in (k, v)]
+        ref = C.attention(q, parts[0][:base + n], parts[1][:base + n], base, gate=gate)
+    hip = _hip()
+    stream = vp()
+    _ok(hip.hipStreamCreate(ctypes.byref(stream)), "hipStreamCreate")
+    with PooledAttn(cfg, rows, n_layers=1, max_cols=max(n, warm[1] if warm else 0)) as pa:
+        pa._chk(pa.L.pa_set_stream(pa.ctx, stream))
+        pa.set_prefill_tile(tile)
+        pa.layer_alloc(0)
+        for w, x in enumerate(parts):
+            pa.kv_write(0, w, 0, x)
+        if warm:
+            assert pa.plan("prefill", warm[0], warm[1])["n_splits"] == 1 and pa.plan("prefill", base, n)["n_splits"] > 1
+            pa.run_attn("prefill", 0, rng.standard_normal((warm[1], nH, hd), dtype=np.float32), warm[0])
+        dq, dg, dout = pa.to_device(q), pa.to_device(gate) if cfg["gate"] else None, pa.alloc(n * qd * 4)
+        graph, gexec = vp(), vp()
+        pa.sync()
+        _ok(hip.hipStreamBeginCapture(stream, 0), "hipStreamBeginCapture")
+        pa.attn("prefill", 0, dq, qd, dg, qd if dg else 0, base, n, dout, qd, PA_OUT_F32)
+        _ok(hip.hipStreamEndCapture(stream, ctypes.byref(graph)), "hipStreamEndCapture")
+        _ok(hip.hipGraphInstantiate(ctypes.byref(gexec), graph, None, None, 0), "hipGraphInstantiate")
+        first = None
+        for rep in range(3):
+            dout.upload(np.zeros(n * qd, np.float32)); pa.sync()
+            _ok(hip.hipGraphLaunch(gexec, stream), "hipGraphLaunch")
+            _ok(hip.hipStreamSynchronize(stream), "hipStreamSynchronize")
+            got = dout.download(np.float32, n * qd).copy().reshape(ref.shape)
+            assert_parity(got, ref, "captured %s %d columns at %d, replay %d" % (shape, n, base, rep))
+            first = got if first is None else first
+            assert np.array_equal(got, first)
+            assert_parity(pa.run_attn("prefill", 0, q, base, gate=gate), ref, "eager call between replays")
         _ok(hip.hipGraphExecDestroy(gexec), "hipGraphExecDestroy"); _ok(hip.hipGraphDestroy(graph), "hipGraphDestroy")
         pa._chk(pa.L.pa_set_stream(pa.ctx, None))
     _ok(hip.hipStreamDestroy(stream), "hipStreamDestroy")

@@ -1,6 +1,6 @@
 """No-GPU checks of which kernel serves an attention call: the library's own plan rules, asked on a 256-CU part."""
 import pytest
-from helpers import attn_rule, BLOCK
+from helpers import attn_rule, BLOCK, ONE_WG
 
 
 @pytest.mark.parametrize("kv_q8", [False, True])
@@ -16,3 +16,21 @@ def test_one_column_never_goes_to_the_kernel_without_an_own_row(head_dim, most, 
                     for kind in ("decode", "prefill"):
                         kernel, pl = attn_rule(cfg, kind, base, 1, splits)
                         assert kernel >= 0 and pl["slots"] == pl["n_splits"] + 1 and kernel != BLOCK, (cfg, base, splits, kind, pl)
+
+
+@pytest.mark.parametrize("kv_q8", [False, True])
+@pytest.mark.parametrize("n_heads,n_kv,head_dim", [(16, 2, 256), (24, 4, 256), (16, 8, 128), (64, 2, 256), (64, 1, 128), (8, 8, 128)])
+def test_a_chunk_under_capture_has_a_plan_without_scratch(n_heads, n_kv, head_dim, kv_q8):
+    """Prefill calls captured in a context that holds no scratch, from one column to thousands, with the tile override and a splits override too: none is left with a plan
+    that would allocate.  (Always the matrix-core kernel over int8 rows needs its widened cache.)"""
+    cfg = dict(n_heads=n_heads, n_kv_heads=n_kv, head_dim=head_dim, n_rot=64, rope_theta=1e6, eps=1e-6, kv_q8=kv_q8)
+    for n in (1, 2, 4, 9, 16, 33, 40, 64, 100, 144, 300, 777, 2048):
+        for base in (0, 20, 88, 200, 300, 900, 2000, 5000, 30000):
+            for splits in (0, 3):
+                for tile in (0, 1, 2):
+                    kernel, pl = attn_rule(cfg, "cold", base, n, splits, tile)
+                    if tile == 1 and kv_q8 and n * n_heads // n_kv > (32 if head_dim == 256 else 64):
+                        continue
+                    assert kernel >= 0 and pl["n_splits"] == 1, (cfg, base, n, splits, tile, kernel, pl)
+                    rows = pl["split_len"]
+                    assert kernel == ONE_WG or (rows >= base + n and (pl["kernel"] == 1 or rows > 32 * pl["waves"] or pl["row_blocks"] > 1))
