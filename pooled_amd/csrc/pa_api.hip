@@ -413,7 +413,7 @@ static int plan_decode(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa
     // 250 rows 7.5 / 5.9, 7.4 / 5.8, 7.4 / 6.0, MoE shape 9.5 / 8.2, 9.2 / 8.3, 9.1 / 8.1, 27B shape 9.5 / 8.1, 9.5 / 8.3, 9.3 / 8.1.  (Eight tiles are what a
     // CU's LDS holds at hd 256.)
     waves = 8; sl = 256; ns = 1;
-  } else if (!self && nb == 1 && !one_split && !ctx->decode_splits_override && seq_max <= one_launch_rows(ctx)) {
+  } else if (n_cols > 1 && nb == 1 && !one_split && !ctx->decode_splits_override && seq_max <= one_launch_rows(ctx)) {
     // ... and several columns in one row block on the tile loop's four waves (us a call, two launches / one; 2 columns at 40 and 200: 16 / 2-head shape 9.9 / 7.1, 9.7 / 9.0, 24 / 4-head
     // 9.4 / 6.7, 9.2 / 8.7, 16 / 8-head 6.8 / 4.8, 6.8 / 5.6)
     sl = 256; ns = 1;
@@ -604,6 +604,21 @@ static int plan_prefill(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, p
   return PA_OK;
 }
 
+// Gather: splits over list positions, the table's choice for one column of max_rows streamed rows (there is no own row), thinned when several columns share the
+// chip.  Always partials and a merge: also up to 256 rows, where one or two workgroups a kv head with a tile a wave are ahead of one with two tiles a wave in
+// one (us a call, one column of 200 rows, splits of 128 / of 256: 16 / 2-head shape 7.5 / 10.8, 24 / 4-head 7.8 / 10.9, 16 / 8-head 6.5 / 8.0; of 40 7.7 / 8.2, 7.9 / 8.4, 6.5 / 6.7).
+static int plan_gather(const pa_ctx* ctx, uint32_t max_rows, uint32_t n_cols, pa_plan* pl) {
+  const int rc = plan_decode(ctx, max_rows - 1, 1, pl, false);
+  if (rc) return rc;
+  if (n_cols > 1 && pl->n_splits > 1) {
+    const uint32_t want = std::max(1u, pl->n_splits / n_cols);
+    pl->split_len = ceil_div(ceil_div(max_rows, want), 128) * 128;
+    pl->n_splits = ceil_div(max_rows, pl->split_len);
+  }
+  pl->slots = pl->n_splits;
+  return PA_OK;
+}
+
 extern "C" int pa_plan_query(const pa_ctx* ctx, int kind, uint32_t base_pos, uint32_t n_cols, pa_plan* out) {
   if (!ctx || !out || n_cols == 0) return PA_ERR_INVALID;
   return kind == 0 ? plan_decode(ctx, base_pos, n_cols, out) : plan_prefill(ctx, base_pos, n_cols, out);
@@ -611,7 +626,7 @@ extern "C" int pa_plan_query(const pa_ctx* ctx, int kind, uint32_t base_pos, uin
 extern "C" int pa_rule_attn(const pa_config* cfg, int n_cu, int kind, uint32_t base_pos, uint32_t n_cols, uint32_t splits, int tile_mode, pa_plan* out) {
   pa_ctx ctx;
   ctx.cfg = *cfg; ctx.n_cu = n_cu; ctx.decode_splits_override = splits; ctx.prefill_tile_mode = tile_mode;
-  const int rc = kind == 0 ? plan_decode(&ctx, base_pos, n_cols, out) : plan_prefill(&ctx, base_pos, n_cols, out, kind == 2);
+  const int rc = kind == 0 ? plan_decode(&ctx, base_pos, n_cols, out) : kind == 3 ? plan_gather(&ctx, base_pos, n_cols, out) : plan_prefill(&ctx, base_pos, n_cols, out, kind == 2);
   return rc != PA_OK ? -1 : kind == 2 && chunk_would_allocate(&ctx, n_cols, *out) ? -2 : plan_kernel(&ctx, *out);
 }
 extern "C" int pa_set_prefill_tile(pa_ctx* ctx, int mode) {
@@ -1183,17 +1198,8 @@ extern "C" int pa_attn_decode_gather(pa_ctx* ctx, uint32_t layer, const float* d
   if ((q_stride & 3) || (out_stride & 3) || (d_gate && (gate_stride & 3)) || ((uintptr_t)d_q & 15) || ((uintptr_t)d_out & 15) || ((uintptr_t)d_gate & 15) || ((uintptr_t)d_sel & 3))
     return fail(ctx, PA_ERR_INVALID, std::string(who) + ": buffers must be 16-byte aligned with strides a multiple of 4 elements");
   if (c.n_heads / c.n_kv_heads > 16) return fail(ctx, PA_ERR_UNSUPPORTED, std::string(who) + ": more than 16 query heads per kv head");
-  // splits over list positions: the table's choice for one column of max_rows rows (an identity list then runs
-  // exactly the dense decode), thinned when several columns share the chip
   pa_plan pl;
-  rc = plan_decode(ctx, max_rows - 1, 1, &pl, false);
-  if (rc) return fail(ctx, rc, std::string(who) + ": shape outside the gfx950 table");
-  if (n_cols > 1 && pl.n_splits > 1) {
-    const uint32_t want = std::max(1u, pl.n_splits / n_cols);
-    pl.split_len = ceil_div(ceil_div(max_rows, want), 128) * 128;
-    pl.n_splits = ceil_div(max_rows, pl.split_len);
-  }
-  pl.slots = pl.n_splits;
+  if ((rc = plan_gather(ctx, max_rows, n_cols, &pl))) return fail(ctx, rc, std::string(who) + ": shape outside the gfx950 table");
   if ((rc = ensure_partials(ctx, n_cols, pl.slots))) return rc;
   AttnParams p; memset(&p, 0, sizeof p);
   p.q = d_q; p.gate = d_gate; p.k_cache = ctx->layers[layer].k; p.v_cache = ctx->layers[layer].v;

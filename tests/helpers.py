@@ -82,13 +82,13 @@ MFMA, LOOP, SINGLE_ROUND, ONE_WG, BLOCK = range(5)
 
 def attn_rule(cfg, kind, base, n_cols, splits=0, tile=0):
     """(kernel, plan) that a decode or prefill call takes on a part of 256 CUs, by the library's own rules; no GPU needed.  "cold": a prefill call under
-    stream capture in a context without scratch (kernel -2: its plan would allocate)."""
+    stream capture in a context without scratch (kernel -2: its plan would allocate).  "gather": base is the longest list."""
     L = capi.load()
     flags = ((capi.PA_FLAG_QK_NORM if cfg.get("qk_norm", True) else 0) | (capi.PA_FLAG_GATE if cfg.get("gate", False) else 0)
              | (capi.PA_FLAG_KV_Q8 if cfg.get("kv_q8", False) else 0))
     c = capi.PaConfig(cfg["n_heads"], cfg["n_kv_heads"], cfg["head_dim"], cfg["n_rot"], cfg["rope_theta"], cfg["eps"], base + n_cols, 1, n_cols, flags)
     pl = capi.PaPlan()
     u32 = ctypes.c_uint32
-    kernel = L.pa_rule_attn(ctypes.byref(c), ctypes.c_int(256), ctypes.c_int({"decode": 0, "prefill": 1, "cold": 2}[kind]), u32(base), u32(n_cols), u32(splits), ctypes.c_int(tile),
+    kernel = L.pa_rule_attn(ctypes.byref(c), ctypes.c_int(256), ctypes.c_int({"decode": 0, "prefill": 1, "cold": 2, "gather": 3}[kind]), u32(base), u32(n_cols), u32(splits), ctypes.c_int(tile),
                             ctypes.byref(pl))
     return kernel, {n: getattr(pl, n) for n, _ in pl._fields_}

@@ -1,6 +1,6 @@
 """No-GPU checks of which kernel serves an attention call: the library's own plan rules, asked on a 256-CU part."""
 import pytest
-from helpers import attn_rule, BLOCK, ONE_WG
+from helpers import attn_rule, BLOCK, ONE_WG, SINGLE_ROUND
 
 
 @pytest.mark.parametrize("kv_q8", [False, True])
@@ -34,3 +34,13 @@ def test_a_chunk_under_capture_has_a_plan_without_scratch(n_heads, n_kv, head_di
                     assert kernel >= 0 and pl["n_splits"] == 1, (cfg, base, n, splits, tile, kernel, pl)
                     rows = pl["split_len"]
                     assert kernel == ONE_WG or (rows >= base + n and (pl["kernel"] == 1 or rows > 32 * pl["waves"] or pl["row_blocks"] > 1))
+
+
+@pytest.mark.parametrize("n_heads,n_kv,head_dim", [(16, 2, 256), (24, 4, 256), (16, 8, 128)])
+def test_a_gather_over_a_short_list_keeps_splits_of_one_tile_a_wave(n_heads, n_kv, head_dim):
+    """Gather calls always have partials and a merge: lists of up to 256 rows are splits of 128, one tile a wave, on the single-round kernel, as longer ones are
+    (not the one split that a block of columns over as many rows takes to write its output itself)."""
+    cfg = dict(n_heads=n_heads, n_kv_heads=n_kv, head_dim=head_dim, n_rot=64, rope_theta=1e6, eps=1e-6)
+    for rows in (1, 31, 32, 33, 127, 128, 129, 200, 255, 256, 257, 400, 2051):
+        kernel, pl = attn_rule(cfg, "gather", rows, 1)
+        assert (kernel, pl["split_len"], pl["n_splits"], pl["slots"]) == (SINGLE_ROUND, 128, -(-rows // 128), -(-rows // 128)), (rows, pl)
