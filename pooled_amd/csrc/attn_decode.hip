@@ -1390,6 +1390,7 @@ static hipError_t launch_decode_hd(const AttnParams& p, uint32_t nb, uint32_t wa
   // eight waves: the one-launch path for small chunks at head_dim 128 with two row blocks (its 250 registers a wave
   // leave room for two waves a SIMD, and a tile's softmax and LDS work is what the loop waits for)
   if (waves == 8) {
+    if (nb == 1 && p.direct_out && !p.self_row) return p.k_scale ? hipErrorInvalidValue : launch_decode_k<HD, 1, 8, false, false, false, false>(p, col_groups, s, t);
     if (nb == 1 && p.direct_out) return p.k_scale ? launch_decode_k<HD, 1, 8, false, false, true, true>(p, col_groups, s, t) : launch_decode_k<HD, 1, 8, false, false, false, true>(p, col_groups, s, t);
     if constexpr (HD == 128) { if (nb == 2 && !p.k_scale) return launch_decode_t<HD, 2, 8, false>(p, col_groups, s, t); }
     return hipErrorInvalidValue;

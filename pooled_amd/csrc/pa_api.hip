@@ -351,6 +351,8 @@ static bool plan_block(const pa_ctx* ctx, const pa_plan& pl) {
   if (tiles == 1) return wgs * 2 > n_cu && wgs <= n_cu && (pl.col_groups > 1 || ctx->cfg.head_dim == 128);
   return pl.col_groups == 1 || tiles == 2;
 }
+// one row block on the single-round kernel (eight waves of one row block are the tile loop, or plan_one_wg)
+static bool plan_single_round1(const pa_plan& pl) { return pl.kernel == 0 && pl.row_blocks == 1 && pl.waves == 4 && pl.split_len == 128; }
 static uint32_t plan_tile_ilv(const pa_plan& pl) {
   return pl.kernel == 0 && pl.split_len != 32 * pl.waves && pl.n_splits > 1 ? 32 * pl.waves : 0;
 }
@@ -358,7 +360,7 @@ static uint32_t plan_tile_ilv(const pa_plan& pl) {
 static bool plan_one_wg(const pa_plan& pl) { return plan_self_row(pl) && pl.row_blocks == 1 && pl.waves == 8 && pl.n_splits == 1 && pl.split_len == 256; }
 // one split and no own-row partial: the kernel writes the output itself (the prefill kernel, or the split-K kernel's tile loop: its single-round form always leaves a partial)
 static bool plan_direct(const pa_plan& pl) {
-  return plan_one_wg(pl) || (pl.n_splits == 1 && !plan_self_row(pl) && (pl.kernel == 1 || pl.split_len != 32 * pl.waves || pl.row_blocks > 1));
+  return plan_one_wg(pl) || (pl.n_splits == 1 && !plan_self_row(pl) && (pl.kernel == 1 || !plan_single_round1(pl)));
 }
 // the kernel that serves a plan
 enum { ATTN_MFMA = 0, ATTN_LOOP = 1, ATTN_SINGLE_ROUND = 2, ATTN_ONE_WG = 3, ATTN_BLOCK = 4 };
@@ -366,7 +368,7 @@ static int plan_kernel(const pa_ctx* ctx, const pa_plan& pl) {
   if (pl.kernel != 0) return ATTN_MFMA;
   if (plan_one_wg(pl)) return ATTN_ONE_WG;
   if (plan_block(ctx, pl)) return ATTN_BLOCK;
-  return (pl.row_blocks == 1 && pl.split_len == 32 * pl.waves) || plan_single_round2(pl) ? ATTN_SINGLE_ROUND : ATTN_LOOP;
+  return plan_single_round1(pl) || plan_single_round2(pl) ? ATTN_SINGLE_ROUND : ATTN_LOOP;
 }
 #define PA_F16_PARTIALS_MIN_SPLITS 64u
 static bool plan_f16_partials(const pa_plan& pl, uint32_t n_cols) {
@@ -413,10 +415,14 @@ static int plan_decode(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa
     // 250 rows 7.5 / 5.9, 7.4 / 5.8, 7.4 / 6.0, MoE shape 9.5 / 8.2, 9.2 / 8.3, 9.1 / 8.1, 27B shape 9.5 / 8.1, 9.5 / 8.3, 9.3 / 8.1.  (Eight tiles are what a
     // CU's LDS holds at hd 256.)
     waves = 8; sl = 256; ns = 1;
-  } else if (n_cols > 1 && nb == 1 && !one_split && !ctx->decode_splits_override && seq_max <= one_launch_rows(ctx)) {
-    // ... and several columns in one row block on the tile loop's four waves (us a call, two launches / one; 2 columns at 40 and 200: 16 / 2-head shape 9.9 / 7.1, 9.7 / 9.0, 24 / 4-head
-    // 9.4 / 6.7, 9.2 / 8.7, 16 / 8-head 6.8 / 4.8, 6.8 / 5.6)
+  } else if (n_cols > 1 && nb == 1 && !one_split && !ctx->decode_splits_override && seq_max <= (c.head_dim == 256 && groups == 1 ? 128u : 256u) && seq_max <= one_launch_rows(ctx)) {
+    // ... and several columns in row blocks of 16, on the tile loop, a tile a wave: four waves up to 128 rows, eight past that.  (Two tiles a wave, one reference for both:
+    // 3 - 20 % more error against 64 bits.)  One row block at head_dim 256 only up to 128: there the splits fill no more CUs but finish sooner than eight
+    // waves that merge in LDS.  us a call, two launches / one: 16 / 2-head shape, 2 columns at 40, 140 and 250 7.9 / 6.9, 8.0 / 8.4, 7.8 / 9.1, 4 (two blocks) at 140 and 200
+    // 9.4 / 8.5, 9.3 / 9.0; 24 / 4-head, 2 at 40, 140 and 250 8.0 / 6.6, 8.1 / 8.3, 8.0 / 9.0, 4 at 240 9.5 / 9.0; 16 / 8-head, 2 at 40 and 250 7.6 / 4.4, 6.6 / 5.7, 8 at 240 6.7 / 5.8,
+    // 24 at 200 9.6 / 5.7.
     sl = 256; ns = 1;
+    if (seq_max > 128) waves = 8;
   } else if (one_split || ctx->decode_splits_override) {
     // a given number of splits (a tuning override; its splits are contiguous ranges, the last one open-ended), or one
     // (one: two tiles a wave at least on f16 rows, since only the tile loop writes the output itself; 20 - 100 columns over up to 128 rows, us a call with the
@@ -553,9 +559,9 @@ static int plan_prefill(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, p
   const uint32_t G = c.n_heads / c.n_kv_heads, rows = base_pos + n_cols;
   const uint32_t max_rows_sk = c.head_dim == 256 ? 32u : 64u;
   if (n_cols * G <= max_rows_sk) {
-    // (over a short context in groups of one row block, in one launch: 4 columns at 40 and 200, 24 / 4-head shape 9.6 / 6.9 and 10.4 / 8.7 us; 32 at 40, 16 / 8-head shape 9.9 / 5.1)
+    // (over a short context in groups of one row block, in one launch: plan_decode has the figures)
     const bool one = n_cols > 1 && rows <= one_launch_rows(ctx) && G <= 16 && !ctx->decode_splits_override;
-    const int rc = plan_decode(ctx, base_pos, n_cols, pl, true, one ? 16 : 0, one);
+    const int rc = plan_decode(ctx, base_pos, n_cols, pl, true, one ? 16 : 0);
     return fits_scratch && rc == PA_OK && chunk_would_allocate(ctx, n_cols, *pl) ? plan_no_scratch(ctx, base_pos, n_cols, pl) : rc;
   }
   // pa_set_prefill_tile: 2 = never the matrix-core kernel (where the split-K kernel can hold a column's heads), 1 = always, 0 = by the estimates

@@ -519,9 +519,9 @@ def test_merge_of_sixteen_columns_and_more(shape, n_cols, base):
             assert_parity(pa.run_attn("decode", 0, q, base, gate=gate, out_dtype=out_dtype).astype(np.float32), ref, "merge of %d columns at %d" % (n_cols, base), tight=True)
 
 
-def _own_reference_error(q, k, v, base, waves):
-    """Relative error against 64 bits of attention whose waves keep a softmax reference of their own: q and P rounded to f16, all else exact; wave w of `waves`
-    takes the 32-row tiles w, w + waves, ... and raises its reference when a row's maximum passes it by 8."""
+def _own_reference_error(q, k, v, base, waves, q_f32=False):
+    """Relative error against 64 bits of attention whose waves keep a softmax reference of their own: q (unless q_f32) and P rounded to f16, all else exact; wave w
+    of `waves` takes the 32-row tiles w, w + waves, ... and raises its reference when a row's maximum passes it by 8."""
     n, nH, hd = q.shape
     rows, G = k.shape[0], nH // k.shape[1]
     k, v = k.astype(np.float64), v.astype(np.float64)
@@ -533,7 +533,7 @@ def _own_reference_error(q, k, v, base, waves):
         s = np.where(vis, q[:, h].astype(np.float64) @ kh.T / hd ** 0.5, -np.inf)
         w = np.exp(s - s.max(1, keepdims=True))
         exact[:, h] = w @ vh / w.sum(1, keepdims=True)
-        s = np.where(vis, q[:, h].astype(np.float16).astype(np.float64) @ kh.T / hd ** 0.5, -np.inf)
+        s = np.where(vis, q[:, h].astype(np.float32 if q_f32 else np.float16).astype(np.float64) @ kh.T / hd ** 0.5, -np.inf)
         M, L, O_ = np.full((waves, n), -np.inf), np.zeros((waves, n)), np.zeros((waves, n, hd))
         for t in range(-(-rows // 32)):
             i, sl = t % waves, slice(32 * t, 32 * t + 32)
@@ -622,3 +622,24 @@ def test_one_column_of_more_than_sixteen_heads_a_kv_head(head_dim, n_heads, n_kv
         assert_parity(got, ref(base, 3), "column-exact block of %d / %d heads" % (n_heads, n_kv))
         for c in range(3):
             assert np.array_equal(got[c], one(pa, c, base + c)[0])
+
+
+@pytest.mark.parametrize("kind,shape,n_cols,rows", [("decode", "qwen3_1p7b", 2, 256), ("decode", "qwen3_1p7b", 4, 200), ("decode", "qwen3_1p7b", 8, 240), ("decode", "qwen36_moe", 2, 256),
+                                                    ("decode", "qwen38_27b", 2, 200), ("prefill", "qwen36_moe", 4, 250), ("prefill", "qwen38_27b", 4, 256), ("prefill", "qwen3_1p7b", 16, 256)])
+def test_a_few_columns_over_a_short_context_are_as_exact_as_a_tile_a_wave(kind, shape, n_cols, rows):
+    """Blocks of a few columns over 129 to 256 rows, in one launch or two: the error against 64 bits is that of tiles with softmax references of their own.  (Which rows
+    are a tile differs between the two, which moves it by 1 % at most; with two tiles a wave it is 1.06 to 1.2 times as large.)"""
+    cfg = SHAPES[shape]
+    rng = np.random.default_rng(rows + n_cols)
+    base = rows - n_cols
+    err2 = lim2 = 0.0
+    for seed in range(8):
+        k16, v16 = random_cache(cfg, rows, seed=seed)
+        q = rng.standard_normal((n_cols, cfg["n_heads"], cfg["head_dim"]), dtype=np.float32)
+        with _ctx_with_cache(cfg, k16, v16, rows, max_cols=n_cols) as pa:
+            got = pa.run_attn(kind, 0, q, base)
+        k, v = [x.view(np.float16).reshape(rows, cfg["n_kv_heads"], -1) for x in (k16, v16)]
+        lim, exact = _own_reference_error(q, k, v, base, 8, n_cols * cfg["n_heads"] // cfg["n_kv_heads"] <= 8)
+        err2 += ((got - exact) ** 2).sum() / (exact ** 2).sum(); lim2 += lim ** 2
+    print("error %.4e, a tile a wave %.4e, ratio %.4f" % ((err2 / 8) ** 0.5, (lim2 / 8) ** 0.5, (err2 / lim2) ** 0.5))
+    assert err2 <= lim2 * 1.02 ** 2

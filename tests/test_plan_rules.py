@@ -1,6 +1,6 @@
 """No-GPU checks of which kernel serves an attention call: the library's own plan rules, asked on a 256-CU part."""
 import pytest
-from helpers import attn_rule, BLOCK, ONE_WG, SINGLE_ROUND
+from helpers import attn_rule, BLOCK, LOOP, MFMA, ONE_WG, SINGLE_ROUND
 
 
 @pytest.mark.parametrize("kv_q8", [False, True])
@@ -33,7 +33,7 @@ def test_a_chunk_under_capture_has_a_plan_without_scratch(n_heads, n_kv, head_di
                         continue
                     assert kernel >= 0 and pl["n_splits"] == 1, (cfg, base, n, splits, tile, kernel, pl)
                     rows = pl["split_len"]
-                    assert kernel == ONE_WG or (rows >= base + n and (pl["kernel"] == 1 or rows > 32 * pl["waves"] or pl["row_blocks"] > 1))
+                    assert kernel == ONE_WG or (rows >= base + n and kernel in (MFMA, LOOP))
 
 
 @pytest.mark.parametrize("n_heads,n_kv,head_dim", [(16, 2, 256), (24, 4, 256), (16, 8, 128)])
@@ -44,3 +44,19 @@ def test_a_gather_over_a_short_list_keeps_splits_of_one_tile_a_wave(n_heads, n_k
     for rows in (1, 31, 32, 33, 127, 128, 129, 200, 255, 256, 257, 400, 2051):
         kernel, pl = attn_rule(cfg, "gather", rows, 1)
         assert (kernel, pl["split_len"], pl["n_splits"], pl["slots"]) == (SINGLE_ROUND, 128, -(-rows // 128), -(-rows // 128)), (rows, pl)
+
+
+@pytest.mark.parametrize("n_heads,n_kv,head_dim", [(16, 2, 256), (24, 4, 256), (16, 8, 128), (32, 4, 128)])
+def test_a_few_columns_over_a_short_context_keep_a_tile_a_wave(n_heads, n_kv, head_dim):
+    """Up to 256 rows no wave of a block of columns takes two tiles: one launch of four or eight waves, or, one row block at head_dim 256 past 128 rows, two splits."""
+    cfg = dict(n_heads=n_heads, n_kv_heads=n_kv, head_dim=head_dim, n_rot=64, rope_theta=1e6, eps=1e-6)
+    group = n_heads // n_kv
+    for rows in (3, 32, 33, 127, 128, 129, 130, 200, 255, 256, 257):
+        for kind, n in [("decode", 2), ("decode", 16 // group), ("prefill", 2), ("prefill", 16 // group), ("prefill", 32 // group)]:
+            if n > rows or n < 2:
+                continue
+            kernel, pl = attn_rule(cfg, kind, rows - n, n)
+            assert pl["row_blocks"] <= 2 and pl["waves"] * pl["n_splits"] * 32 >= rows, (kind, n, rows, pl)
+            one = rows <= (128 if head_dim == 256 and n * group <= 16 else 256)
+            assert (pl["n_splits"] == 1) == one and (kernel == LOOP) == one, (kind, n, rows, kernel, pl)
+            assert not one or pl["waves"] == (8 if rows > 128 else 4)
