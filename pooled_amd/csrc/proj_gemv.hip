@@ -87,8 +87,8 @@ static __device__ inline float dot_block(const BlockRegs<KIND>& r, const float (
 
 // BPL: blocks per lane and pass; PASSES: passes over the input (d_in <= 2048 * BPL * PASSES; two for f32 weights past
 // 4096 inputs, whose 32 registers a block leave no room for four blocks a lane: the second pass's weight rows are
-// requested when the first pass's are consumed); RW: rows per wave
-template <int KIND, int BPL, int RW, bool NORM, int PASSES = 1>
+// requested when the first pass's are consumed); RW: rows per wave; AT_ONCE: all of them requested in front
+template <int KIND, int BPL, int RW, bool NORM, int PASSES, bool AT_ONCE>
 __global__ __launch_bounds__(256)
 void pa_gemv_kernel(const float* a_x, const float* a_norm_w, const void* a_w, const uint16_t* a_scales, float* a_y, uint32_t a_d_out, uint32_t a_d_in, GemvParams p_in) {
   // The leading arguments repeat fields of p_in: the first twelve dwords of the arguments are preloaded into scalar
@@ -96,13 +96,13 @@ void pa_gemv_kernel(const float* a_x, const float* a_norm_w, const void* a_w, co
   // batch of scalar loads (the compiler would fetch each where it is first used, a dependent round trip each).
   GemvParams p = p_in;
   p.x = a_x; p.norm_w = a_norm_w; p.w = a_w; p.scales = a_scales; p.y = a_y; p.d_out = a_d_out; p.d_in = a_d_in;
-  // Up to 4096 inputs, and for up to three rows, a wave's rows are all requested at once; past that it keeps two or three in flight and asks for the next when
+  // Up to 4096 inputs, for up to three rows, and with AT_ONCE (pa_rule_gemv_at_once) a wave's rows are all requested at once; past that it keeps two or three in flight and asks for the next when
   // one is consumed.  With everything requested in front, a wave sat in the issue of its loads while the memory pipeline was full (of 14336 x 5120 Q4_0, seven rows a wave:
   // until 4.3 us after the first wave's entry on average, 7.4 at the latest), staged x behind that and did all of its arithmetic, 3 us, behind the last
   // byte; so the arithmetic runs under the stream (12.5 -> 10.8 us; 16384 x 5120 14.1 -> 11.9, 14336 x 8192 18.5 -> 14.3; one row in flight 13.3, three 11.0;
   // without the norm three are ahead, 12288 x 6144 10.35 / 10.15).  The rows of a wave are then dealt one of every 4 x gridDim.x: at any time the chip reads one
   // range of the matrix (10.8 -> 10.5 us), and the waves' counts differ by one at most.
-  constexpr int AHEAD = BPL < 3 || KIND == PA_W_F32 || RW <= 3 ? RW : KIND == PA_W_Q4_0 && BPL == 3 && !NORM && RW >= 5 ? 3 : 2;
+  constexpr int AHEAD = AT_ONCE || BPL < 3 || KIND == PA_W_F32 || RW <= 3 ? RW : KIND == PA_W_Q4_0 && BPL == 3 && !NORM && RW >= 5 ? 3 : 2;
   constexpr bool STREAM = RW > AHEAD;
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t nb = p.d_in / 32;
@@ -243,11 +243,11 @@ void pa_gemv_kernel(const float* a_x, const float* a_norm_w, const void* a_w, co
   }
 }
 
-template <int KIND, int BPL, int RW, bool NORM, int PASSES = 1>
+template <int KIND, int BPL, int RW, bool NORM, int PASSES = 1, bool AT_ONCE = false>
 static hipError_t launch_k(const GemvParams& p, hipStream_t s, uint32_t wgs = 0) {
   if (wgs == 0) wgs = (p.d_out + 4 * RW - 1) / (4 * RW);
   const size_t lds = (size_t)(p.d_in / 32) * 36 * sizeof(float);
-  hipLaunchKernelGGL((pa_gemv_kernel<KIND, BPL, RW, NORM, PASSES>), dim3(wgs), dim3(256), lds, s, p.x, p.norm_w, p.w, p.scales, p.y, p.d_out, p.d_in, p);
+  hipLaunchKernelGGL((pa_gemv_kernel<KIND, BPL, RW, NORM, PASSES, AT_ONCE>), dim3(wgs), dim3(256), lds, s, p.x, p.norm_w, p.w, p.scales, p.y, p.d_out, p.d_in, p);
   return hipGetLastError();
 }
 
@@ -289,23 +289,42 @@ extern "C" uint32_t pa_rule_gemv_wide_rows(int kind, uint32_t d_out, uint32_t d_
 // One or two workgroups a CU that stay for the whole call (<< 16 | the rows a wave; 0: neither): past 4096 inputs, quantised weights.  Every workgroup stages all of x and every
 // wave reads it from LDS into its registers (10 waves a CU of 5120 x 6144: 240 KB, 0.8 us), so as few of them as keep the stream going are ahead.  One a CU with the norm
 // in front up to eight rows a wave (Q4_0 2048 x 6144 5.6 -> 4.4 us, 3072 x 5120 6.5 -> 4.6, 5120 x 5120 7.4 -> 6.7, 6144 x 6144 8.1 -> 7.5, 8192 x 8192 12.0 -> 10.4; Q8_0
-// 5120 x 6144 10.1 -> 8.7, 7168 x 5120 10.6 -> 9.7); without it up to three rows and at five, where the rule below comes to 2.5 workgroups a CU (5120 x 6144 7.06 -> 6.70,
-// Q8_0 8.9 -> 8.5), but not at four or six (4096 x 6144 5.9, one a CU 6.3; 6144 x 6144 7.2 and 7.7; Q8_0 three rows 6.0 and 6.3).  Two a CU from there to eight rows
+// 5120 x 6144 10.1 -> 8.7, 7168 x 5120 10.6 -> 9.7), but up to five for Q4_0 rows of at most 5120 inputs, whose arithmetic four waves a CU do not hide under so few bytes (5600 x 4128 7.3,
+// one a CU 7.6; 7600 x 4128 8.2 and 8.8, x 5120 8.4 and 8.9, x 5632 8.9 and 9.0, x 6144 9.3 and 9.1).  Without the norm up to three rows and at five, where the rule above
+// comes to 2.0 - 2.5 workgroups of two rows a wave a CU (Q4_0 4200, 4700 and 5120 rows of 6144 7.2 -> 7.0, 7.3 -> 6.9, 7.4 -> 7.1, of 8192 8.7 -> 8.2, 8.9 -> 8.3, 9.1 -> 8.4; Q8_0 of 6144 8.9 -> 8.1,
+// 9.0 -> 8.4, 9.0 -> 8.7; the few workgroups of 4097 - 4112 rows past two a CU are not worth it: 4104 x 6144 6.65, one a CU 6.87, 4120 x 6144 6.96 and 6.88), but not at
+// four or six (4096 x 6144 5.9, one a CU 6.3; 6144 x 6144 7.2 and 7.7; Q8_0 three rows 6.0 and 6.3).  Two a CU from there to eight rows
 // (Q4_0 14336 x 5120 12.5 -> 10.5, 9500 x 7168 14.5 -> 11.3; Q8_0 14336 x 5120 17.5 -> 15.2, 9216 x 5120 without the norm 11.6 -> 10.8; at four rows Q8_0 6144 x 6144
-// 9.1 -> 9.7).  More rows a wave were not built.
-extern "C" uint32_t pa_rule_gemv_resident(int kind, uint32_t d_out, int norm, int n_cu) {
+// 9.1 -> 9.7), from six for Q4_0 rows of less than 5120 inputs without the norm (9000 x 4128 8.6, two a CU 9.0, x 5120 9.2 and 9.2).  More rows a wave were not built.
+// (Up to three rows a wave do not stream and stay consecutive, so the last CUs may have none: 1025 rows of 5120 on 129 workgroups 4.2 us, dealt over all of them one
+// row of every 1024 4.7; 2049 x 8192 with the norm 6.5 and 7.3.)
+extern "C" uint32_t pa_rule_gemv_resident(int kind, uint32_t d_out, uint32_t d_in, int norm, int n_cu) {
   const uint32_t one = (d_out + 4 * n_cu - 1) / (4 * n_cu), two = (d_out + 8 * n_cu - 1) / (8 * n_cu);
-  if (norm ? one <= 8 : one <= 2 || one == 5 || (one == 3 && kind == PA_W_Q4_0)) return 1u << 16 | one;
-  if (two >= 5 && two <= 8) return 2u << 16 | two;
+  const bool q4 = kind == PA_W_Q4_0;
+  if (norm ? one <= (q4 && d_in <= 5120 ? 5 : 8) : one <= 2 || (one == 3 && q4) || (one == 5 && d_out > 16u * n_cu + n_cu / 16)) return 1u << 16 | one;
+  if (two >= (q4 && !norm && d_in < 5120 ? 6 : 5) && two <= 8) return 2u << 16 | two;
   return 0;
+}
+// Q4_0 calls of four or five rows a wave that the rule above leaves, without the norm: all rows requested in front where that is ahead of two or three in flight, over short rows and on
+// tall weights, whose five waves a SIMD keep the stream going by themselves (us, in front / streamed: 7200 x 4128 7.3 / 7.7, x 4608 7.5 / 7.7, x 5120 7.7 / 7.8, x 6144 8.2 / 8.1, x 8192 11.0 / 10.4; 9000 x 4128
+// 8.6 / 9.0; 19000 x 6400 19.0 / 21.0, x 8192 21.6 / 22.5).
+extern "C" int pa_rule_gemv_at_once(int kind, uint32_t d_out, uint32_t d_in, int norm, uint32_t rows, int n_cu) {
+  return kind == PA_W_Q4_0 && !norm && ((rows == 4 && (d_in <= 5120 || d_out > 64u * n_cu)) || (rows == 5 && d_in <= 5120));
 }
 
 template <int KIND, int BPL, bool NORM>
 static hipError_t launch_rw(const GemvParams& p, int n_cu, hipStream_t s) {
   if constexpr (BPL >= 3) {
-    const uint32_t resident = pa_rule_gemv_resident(KIND, p.d_out, NORM, n_cu), rows = resident & 0xffff;
-    if (resident) return launch_rows<KIND, BPL, NORM, 8>(rows, p, s, std::min((resident >> 16) * (uint32_t)n_cu, (p.d_out + 3) / 4));
-    return launch_rows<KIND, BPL, NORM, wide_rows_max(KIND, BPL, NORM)>(pa_rule_gemv_wide_rows(KIND, p.d_out, p.d_in, NORM, n_cu), p, s);
+    const uint32_t resident = pa_rule_gemv_resident(KIND, p.d_out, p.d_in, NORM, n_cu);
+    if (resident) return launch_rows<KIND, BPL, NORM, 8>(resident & 0xffff, p, s, std::min((resident >> 16) * (uint32_t)n_cu, (p.d_out + 3) / 4));
+    const uint32_t rows = pa_rule_gemv_wide_rows(KIND, p.d_out, p.d_in, NORM, n_cu);
+    if constexpr (KIND == PA_W_Q4_0 && !NORM) {
+      if (pa_rule_gemv_at_once(KIND, p.d_out, p.d_in, NORM, rows, n_cu)) {
+        if constexpr (BPL == 3) { if (rows == 5) return launch_k<KIND, BPL, 5, NORM, 1, true>(p, s); }
+        return launch_k<KIND, BPL, 4, NORM, 1, true>(p, s);
+      }
+    }
+    return launch_rows<KIND, BPL, NORM, wide_rows_max(KIND, BPL, NORM)>(rows, p, s);
   } else {
     // rows per wave: as many as still leave about two 4-wave workgroups per CU, within the registers that RW x BPL
     // blocks of weights take (f32: 32 registers a block, Q8_0: 8, Q4_0: 4)

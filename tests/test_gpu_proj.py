@@ -51,7 +51,8 @@ def test_gemv_matches_oracle(kind, d_out, d_in):
 
 # sizes past 4096 inputs that take every number of rows a wave with and without the norm (test_proj_rules.py asks the rule)
 GEMV_WIDE_SIZES = [(6143, 4128), (6145, 4128), (8191, 5120), (11265, 4160), (14337, 6144), (9001, 6176), (6150, 8192),
-                   (14335, 5120), (4000, 4128), (6144, 4128), (4111, 8192), (1000, 7968), (9003, 6016)]
+                   (14335, 5120), (4000, 4128), (6144, 4128), (4111, 8192), (1000, 7968), (9003, 6016),
+                   (7001, 6144), (7001, 4128), (8603, 4128), (18753, 7168)]
 
 
 @pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])
@@ -82,7 +83,8 @@ def test_gemv_many_rows_a_wave(kind, d_out, d_in):
 # one or two workgroups a CU that stay for the whole call, one to eight rows a wave (test_proj_rules.py asks the rule): counts that come out
 # even, one row more or less, and the first size that is left to the rows above
 GEMV_RESIDENT_SIZES = [(1024, 4128), (1025, 8192), (2047, 4160), (2049, 5120), (3071, 7008), (3073, 6144), (4001, 7008), (4097, 6400), (5120, 6144), (5121, 8192), (6145, 6208), (7169, 8192),
-                       (8192, 4160), (8193, 8160), (10241, 6144), (10241, 7008), (12289, 8192), (14337, 6208), (16384, 6144), (16385, 4128)]
+                       (8192, 4160), (8193, 8160), (10241, 6144), (10241, 7008), (12289, 8192), (14337, 6208), (16384, 6144), (16385, 4128),
+                       (4112, 5120), (4113, 6400), (5501, 5152), (6803, 5632), (7901, 5152), (9001, 5120)]
 
 
 @pytest.mark.parametrize("kind", [PA_W_Q8_0, PA_W_Q4_0])

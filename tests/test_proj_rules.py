@@ -35,17 +35,36 @@ def test_gemv_sizes_take_every_number_of_rows():
 
 def test_gemv_resident_sizes_take_every_form():
     def form(kind, d_out, d_in, norm):
-        v = _rule("pa_rule_gemv_resident", ctypes.c_int(kind), d_out, ctypes.c_int(norm), ctypes.c_int(CUS))
+        v = _rule("pa_rule_gemv_resident", ctypes.c_int(kind), d_out, d_in, ctypes.c_int(norm), ctypes.c_int(CUS))
         return (kind, 3 if d_in <= 6144 else 4, norm, v >> 16, v & 0xffff) if v else None
     forms = [(k, norm) for k in (PA_W_Q4_0, PA_W_Q8_0) for norm in (0, 1)]
     sizes = GEMV_RESIDENT_SIZES + GEMV_WIDE_SIZES
     tested = {form(k, d_out, d_in, norm) for k, norm in forms for d_out, d_in in sizes}
-    reached = {form(k, d_out, d_in, norm) for k, norm in forms for d_out in range(1, 20000, 7) for d_in in (4128, 8192)}
+    reached = {form(k, d_out, d_in, norm) for k, norm in forms for d_out in range(1, 20000, 7) for d_in in (4128, 5152, 8192)}
     assert {f[3:] for f in reached - {None}} == {(1, r) for r in range(1, 9)} | {(2, r) for r in range(5, 9)}
     assert reached <= tested
     # the line without the norm: not at four rows a wave, nor at six to eight of one workgroup a CU
     assert [form(PA_W_Q4_0, d_out, 6144, 0) for d_out in (4096, 5121, 8192)] == [None] * 3 and form(PA_W_Q8_0, 3072, 6144, 0) is None
     assert form(PA_W_Q4_0, 5120, 6144, 0)[3:] == (1, 5) and form(PA_W_Q4_0, 14336, 5120, 1)[3:] == (2, 7)
+    # ... nor at five for a handful of rows past 4096
+    assert [form(k, d_out, 6144, 0) for k in (PA_W_Q4_0, PA_W_Q8_0) for d_out in (4097, 4112)] == [None] * 4 and form(PA_W_Q4_0, 4113, 4128, 0)[3:] == (1, 5)
+    # Q4_0 rows of at most 5120 inputs: six to eight rows a wave not with the norm, two workgroups a CU of five not without
+    assert [form(PA_W_Q4_0, 7168, d_in, 1) for d_in in (4128, 5120)] == [None] * 2 and form(PA_W_Q4_0, 7168, 5152, 1)[3:] == (1, 7) and form(PA_W_Q8_0, 7168, 4128, 1)[3:] == (1, 7)
+    assert form(PA_W_Q4_0, 9000, 5088, 0) is None and form(PA_W_Q4_0, 9000, 5120, 0)[3:] == (2, 5) and form(PA_W_Q4_0, 9000, 4128, 1)[3:] == (2, 5)
+
+
+def test_gemv_sizes_take_every_instance():
+    """Every kernel instance that some size reaches (kind, blocks a lane, norm, rows a wave, requested at once), ragged last rows among them where it has more than one."""
+    def instance(kind, d_out, d_in, norm):
+        v = _rule("pa_rule_gemv_resident", ctypes.c_int(kind), d_out, d_in, ctypes.c_int(norm), ctypes.c_int(CUS)) & 0xffff
+        rows = v or _gemv(kind, d_out, d_in, norm)[3]
+        once = not v and _rule("pa_rule_gemv_at_once", ctypes.c_int(kind), d_out, d_in, ctypes.c_int(norm), rows, ctypes.c_int(CUS))
+        return kind, 3 if d_in <= 6144 else 4, norm, rows, bool(once)
+    forms = [(k, norm) for k in (PA_W_Q4_0, PA_W_Q8_0) for norm in (0, 1)]
+    tested = {instance(k, d_out, d_in, norm) for k, norm in forms for d_out, d_in in GEMV_RESIDENT_SIZES + GEMV_WIDE_SIZES}
+    reached = {instance(k, d_out, d_in, norm) for k, norm in forms for d_out in range(1, 36000, 7) for d_in in (4128, 5120, 5152, 6144, 6176, 8192)}
+    assert reached <= tested, reached - tested
+    assert {i[1:] for i in reached if i[4]} == {(3, 0, 4, True), (3, 0, 5, True), (4, 0, 4, True)}
 
 
 def _few(kind, d_out, d_in, n):
