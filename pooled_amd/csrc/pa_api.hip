@@ -345,7 +345,6 @@ static bool plan_single_round2(const pa_plan& pl) {
 // Not one column of more than 16 query heads a kv head: its own row is a partial of its own, which that kernel does not make.
 static bool plan_block(const pa_ctx* ctx, const pa_plan& pl) {
   if (pl.kernel != 0 || pl.waves != 4 || pl.row_blocks < 2 || pl.n_splits == 1 || plan_self_row(pl)) return false;
-  if (ctx->decode_splits_override) return true;
   const uint32_t tiles = pl.split_len / 128, n_cu = (uint32_t)ctx->n_cu;
   const uint64_t wgs = (uint64_t)pl.n_splits * ctx->cfg.n_kv_heads * pl.col_groups;
   if (tiles == 1) return wgs * 2 > n_cu && wgs <= n_cu && (pl.col_groups > 1 || ctx->cfg.head_dim == 128);
@@ -424,7 +423,7 @@ static int plan_decode(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa
     sl = 256; ns = 1;
     if (seq_max > 128) waves = 8;
   } else if (one_split || ctx->decode_splits_override) {
-    // a given number of splits (a tuning override; its splits are contiguous ranges, the last one open-ended), or one
+    // a given number of splits (a tuning override: at most that many, of whole rounds of tiles a wave), or one
     // (one: two tiles a wave at least on f16 rows, since only the tile loop writes the output itself; 20 - 100 columns over up to 128 rows, us a call with the
     // single-round kernel and a merge of its one split / without: 16 / 2-head shape 10.1 / 8.6, 16 / 8-head shape 8.7 / 6.0)
     const uint32_t tpw = one_split ? std::max(ceil_div(tiles, W), kv_q8(ctx) ? 1u : 2u) : std::max(ceil_div(tiles, target * W), 1u);

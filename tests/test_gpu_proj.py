@@ -588,7 +588,7 @@ def test_layer_decode_equals_its_stages(shape, more, kind, dim):
         dqkv = pa.alloc(rows * 4); dat = pa.alloc(qd * 4)
         for layer in (0, 1):
             pa.layer_alloc(layer); pa.kv_store(layer, kraw, kvd, vraw, kvd, 0, 640)
-        for splits in (0, 3):                                         # 3: contiguous splits of several tiles a wave
+        for splits in (0, 3):                                         # 3: the tile loop, several tiles a wave
             pa.set_decode_splits(splits)
             for pos in (0, 1, 127, 128, 129, 255, 256, 257, 384, 513, 639):
                 dx, dy = pa.to_device(x), pa.to_device(x)

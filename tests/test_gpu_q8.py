@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 from oracle import attn_oracle as O
 from pooled_amd.capi import PooledAttn, PaError, PA_ERR_UNSUPPORTED, PA_OUT_F16
-from helpers import SHAPES, assert_parity
+from helpers import LOOP, SHAPES, SINGLE_ROUND, assert_parity, attn_rule
 
 pytestmark = pytest.mark.gpu
 
@@ -86,7 +86,7 @@ def test_q8_verify_block_prefill_chunk_and_slots():
         assert pl["row_blocks"] == 2 and pl["split_len"] == 128 and pl["n_splits"] == -(-(base + 8) // 128) and pl["col_groups"] == 2, pl
         assert_parity(pa.run_attn("decode", 0, q[:8], base, gate=gate[:8]), ref[:8], "q8 verify block")
         pa.set_decode_splits(4)              # the same block on the tile loop
-        assert pa.plan("decode", base, 8)["split_len"] > 128
+        assert attn_rule(cfg, "decode", base, 8) == (SINGLE_ROUND, pl) and attn_rule(cfg, "decode", base, 8, 4) == (LOOP, pa.plan("decode", base, 8))
         assert_parity(pa.run_attn("decode", 0, q[:8], base, gate=gate[:8]), ref[:8], "q8 verify block, tile loop")
         pa.set_decode_splits(0)
         # a narrow chunk runs on the split-K kernel, a wide one on the MFMA prefill kernel over rows widened to f16 (forced:
@@ -250,7 +250,7 @@ def test_q8_short_verify_block_is_one_split_with_two_row_blocks():
 @pytest.mark.parametrize("base,n,splits,exact", [(12288, 1, 32, False), (12289, 1, 25, False), (12289, 1, 25, True), (12280, 8, 32, False), (12281, 8, 49, False),
                                                  (16368, 16, 32, False), (16369, 16, 43, False)])
 def test_q8_head_dim_128_loop_at_two_workgroups_a_cu(base, n, splits, exact):
-    """Past three tiles a wave (four with two row blocks) the tile loop of int8 rows at head_dim 128 takes two workgroups a CU for blocks, one for a
+    """Past three tiles a wave (four with two row blocks, whose waves share one softmax) int8 rows at head_dim 128 take two workgroups a CU for blocks, one for a
     single column in any context: either side of the line, split counts of a 256-CU part, against the oracle on the de-quantised values."""
     cfg = dict(_q8cfg("qwen3_1p7b"), verify_exact=exact)
     rng = np.random.default_rng(base + n)

@@ -1,6 +1,6 @@
 """No-GPU checks of which kernel serves an attention call: the library's own plan rules, asked on a 256-CU part."""
 import pytest
-from helpers import attn_rule, BLOCK, LOOP, MFMA, ONE_WG, SINGLE_ROUND
+from helpers import attn_rule, BLOCK, LOOP, MFMA, ONE_WG, SHAPES, SINGLE_ROUND
 
 
 @pytest.mark.parametrize("kv_q8", [False, True])
@@ -60,3 +60,19 @@ def test_a_few_columns_over_a_short_context_keep_a_tile_a_wave(n_heads, n_kv, he
             one = rows <= (128 if head_dim == 256 and n * group <= 16 else 256)
             assert (pl["n_splits"] == 1) == one and (kernel == LOOP) == one, (kind, n, rows, kernel, pl)
             assert not one or pl["waves"] == (8 if rows > 128 else 4)
+
+
+@pytest.mark.parametrize("shape,n,base,splits,kernel", [
+    # one column group: from two tiles a wave on (three row blocks and more: also where few workgroups are made), not with one at head_dim 256, nor on less than half the chip
+    ("qwen36_moe", 4, 16377, 0, SINGLE_ROUND), ("qwen36_moe", 4, 16385, 0, BLOCK), ("qwen36_moe", 4, 60000, 0, BLOCK), ("qwen38_27b", 5, 8180, 0, SINGLE_ROUND), ("qwen38_27b", 5, 8190, 0, BLOCK),
+    ("qwen3_1p7b", 12, 2030, 0, SINGLE_ROUND), ("qwen3_1p7b", 12, 2040, 0, BLOCK), ("qwen3_1p7b", 12, 4080, 0, BLOCK), ("qwen3_1p7b", 12, 4090, 0, SINGLE_ROUND), ("qwen3_1p7b", 12, 8170, 0, SINGLE_ROUND),
+    ("qwen3_1p7b", 12, 8190, 0, BLOCK), ("qwen3_1p7b", 24, 200, 0, LOOP), ("qwen3_1p7b", 24, 250, 0, BLOCK),
+    # several: two tiles a wave, or one on more than half the chip and not twice
+    ("qwen36_moe", 8, 4080, 0, SINGLE_ROUND), ("qwen36_moe", 8, 4090, 0, BLOCK), ("qwen36_moe", 8, 8180, 0, BLOCK), ("qwen36_moe", 8, 8190, 0, BLOCK), ("qwen36_moe", 8, 16370, 0, BLOCK),
+    ("qwen36_moe", 8, 16380, 0, LOOP), ("qwen36_moe", 8, 60000, 0, LOOP), ("qwen38_27b", 10, 8170, 0, BLOCK), ("qwen38_27b", 10, 8190, 0, LOOP),
+    # one split, one row block, and overrides by the same lines
+    ("qwen36_moe", 4, 100, 0, LOOP), ("qwen36_moe", 2, 40000, 0, LOOP), ("qwen36_moe", 4, 8000, 10, BLOCK), ("qwen36_moe", 8, 8000, 10, LOOP), ("qwen36_moe", 8, 8000, 32, BLOCK), ("qwen36_moe", 4, 8000, 1, LOOP)])
+def test_which_kernel_serves_a_verify_block(shape, n, base, splits, kernel):
+    """Both sides of each line between the single-round kernel, the tile loop and the kernel whose waves share one softmax."""
+    got, pl = attn_rule(SHAPES[shape], "decode", base, n, splits)
+    assert got == kernel, (got, pl)
