@@ -58,11 +58,9 @@ void pa_block_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a_
   auto div_g = [&](uint32_t r) __attribute__((always_inline)) -> uint32_t { return (r * g_magic) >> 16; };      // row r is (column r / G, head r % G)
   const uint32_t c0 = cg * p.cols_per_group, ncl = min(p.cols_per_group, p.n_cols - c0), R = ncl * G;
   const uint32_t seq_max = p.base_pos + c0 + ncl;                    // rows visible to the group's last column
-  const bool tilv = p.tile_ilv != 0;
-  const uint32_t t_begin = sp * (tilv ? (uint32_t)(W * TILE) : p.split_len);
+  const uint32_t t_begin = sp * (uint32_t)(W * TILE);                // a split's first round of tiles; one tile a wave is one round
   if (t_begin >= seq_max) return;
-  const uint32_t t_end = sp + 1 == p.n_splits || tilv ? seq_max : min(t_begin + p.split_len, seq_max);
-  const uint32_t lim = t_begin + (t_end - t_begin + TILE - 1) / TILE * TILE, step = tilv ? p.n_splits * (uint32_t)(W * TILE) : (uint32_t)(W * TILE);
+  const uint32_t lim = t_begin + (seq_max - t_begin + TILE - 1) / TILE * TILE, step = p.n_splits * (uint32_t)(W * TILE);
   const size_t head_rows = (size_t)p.max_seq + TILE;                 // rows of one kv head's plane, padding included
   const size_t row_bytes = (size_t)HD * 2;
   const uint32_t lrow = lane / S::LPR, voff = lrow * (uint32_t)row_bytes + (lane % S::LPR) * 16;
@@ -115,10 +113,10 @@ void pa_block_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a_
       }
     }
   };
-  asm volatile("" :: "s"(p.q), "s"(p.v_cache), "s"(p.q_stride), "s"(p.n_heads), "s"(p.split_len), "s"(p.tile_ilv));
+  asm volatile("" :: "s"(p.q), "s"(p.v_cache), "s"(p.q_stride), "s"(p.n_heads));
   if constexpr (Q8) asm volatile("" :: "s"(p.k_scale), "s"(p.v_scale));
   // q first (it returns first), then the first tile.  Loads are unconditional: the caches carry TILE rows of padding past max_seq; a wave without a tile
-  // of its own reads the split's last one, whose scores are masked and whose rows are staged as zeros.
+  // of its own reads the last one, whose scores are masked and whose rows are staged as zeros.
   constexpr int QPT = 16 * NB * (HD / 4) / 256;
   f4 qv[QPT];
 #pragma unroll
@@ -268,7 +266,7 @@ void pa_block_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a_
       l_run[nb] = sum_f16(pf, l_run[nb]);
       *(h8*)(smem + L::p + ((wave * NB + nb) * 64 + lane) * 16) = pf;
     }
-    store_tile(vr, vsr, vst, S::VROW, (int)t_end - (int)min(tp, t_end));
+    store_tile(vr, vsr, vst, S::VROW, (int)seq_max - (int)min(tp, seq_max));
     if (more) load_tile(vr, vsr, vbase, vsbase, tpn);
     lds_barrier();
     // O^T += V^T P^T over the four tiles, dims [wave HD / 4, + HD / 4); V^T fragments (two transpose reads each) VD steps ahead
@@ -356,7 +354,7 @@ static hipError_t launch_block_nb(const AttnParams& p, uint32_t nb, uint32_t col
 }
 
 hipError_t pa_launch_block(const AttnParams& p, uint32_t hd, uint32_t nb, uint32_t col_groups, hipStream_t s, const PaTiming* t) {
-  if (p.self_row || p.sel || p.part_f16 || p.direct_out || p.exact_cols) return hipErrorInvalidValue;
+  if (p.self_row || p.sel || p.part_f16 || p.direct_out || p.exact_cols || (p.split_len != 128 && p.tile_ilv != 128)) return hipErrorInvalidValue;
   if (hd == 256) return p.k_scale ? launch_block_nb<256, true>(p, nb, col_groups, s, t) : launch_block_nb<256, false>(p, nb, col_groups, s, t);
   if (hd == 128) return p.k_scale ? launch_block_nb<128, true>(p, nb, col_groups, s, t) : launch_block_nb<128, false>(p, nb, col_groups, s, t);
   return hipErrorInvalidValue;

@@ -550,7 +550,7 @@ def _own_reference_error(q, k, v, base, waves, q_f32=False):
             i, sl = t % waves, slice(32 * t, 32 * t + 32)
             top = s[:, sl].max(1)
             m = np.where(top > M[i] + 8, top, M[i])
-            a = np.where(np.isneginf(m), 1.0, np.exp(np.where(np.isneginf(m), 0.0, M[i] - m)))
+            a = np.exp(np.subtract(M[i], m, out=np.zeros(n), where=~np.isneginf(m)))
             p = np.exp(s[:, sl] - np.where(np.isneginf(m), 0.0, m)[:, None]).astype(np.float16).astype(np.float64)
             M[i], L[i], O_[i] = m, L[i] * a + p.sum(1), O_[i] * a[:, None] + p @ vh[sl]
         c = np.exp(M - M.max(0))
