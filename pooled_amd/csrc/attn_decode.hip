@@ -139,8 +139,8 @@ static __device__ inline void fused_q_rows(const float (&xq)[16 / W][4], const f
 //
 // SR (single-round splits; one 16-row block, or two of a verify block): splits are one tile per wave (split_len = W x
 // 32); the product O^T = V^T P^T of a split is divided over the waves by output dims, see the code.  Without SR every wave
-// loops over its own tiles: contiguous splits of any length, or (AttnParams::tile_ilv) a kv head's tiles dealt round robin
-// to the waves of all its splits.
+// loops over its own tiles: those of one split, of contiguous splits (a gather list), or (AttnParams::tile_ilv) a kv head's tiles dealt round
+// robin to the waves of all its splits.
 template <int HD, int NB, int W, bool FUSED, bool GATHER, bool Q8, bool SR, bool EX2>
 __global__ __launch_bounds__(W * 64, ((NB == 1 && !GATHER && W <= 4) || (SR && NB == 2 && HD == 128) || EX2 ? 2 : 1))
 void pa_decode_kernel(const uint16_t* a_k_cache, uint32_t a_base_pos, uint32_t a_max_seq, uint32_t a_n_splits, uint32_t a_self_row,
@@ -1387,8 +1387,8 @@ static hipError_t launch_decode_t(const AttnParams& p, uint32_t col_groups, hipS
 
 template <int HD>
 static hipError_t launch_decode_hd(const AttnParams& p, uint32_t nb, uint32_t waves, uint32_t col_groups, hipStream_t s, const PaTiming* t) {
-  // eight waves: the one-launch path for small chunks at head_dim 128 with two row blocks (its 250 registers a wave
-  // leave room for two waves a SIMD, and a tile's softmax and LDS work is what the loop waits for)
+  // eight waves: one column over at most 256 rows (plan_one_wg); a few columns over 129 - 256 rows, a tile a wave; and the one-launch path for small chunks at head_dim 128
+  // with two row blocks (its 250 registers a wave leave room for two waves a SIMD, and a tile's softmax and LDS work is what the loop waits for)
   if (waves == 8) {
     if (nb == 1 && p.direct_out && !p.self_row) return p.k_scale ? hipErrorInvalidValue : launch_decode_k<HD, 1, 8, false, false, false, false>(p, col_groups, s, t);
     if (nb == 1 && p.direct_out) return p.k_scale ? launch_decode_k<HD, 1, 8, false, false, true, true>(p, col_groups, s, t) : launch_decode_k<HD, 1, 8, false, false, false, true>(p, col_groups, s, t);

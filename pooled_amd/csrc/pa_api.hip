@@ -323,13 +323,6 @@ extern "C" int pa_kv_store(pa_ctx* ctx, uint32_t layer, const float* d_k, uint32
 // self_ok: a one-column decode keeps the column's own row out of the streamed rows (the kernel turns it
 // into one more partial: slots = n_splits + 1), so a token at a multiple of the split length streams whole tiles only.
 static bool plan_self_row(const pa_plan& pl) { return pl.kernel == 0 && pl.slots == pl.n_splits + 1; }
-// f16 O partials: the single-round split-K kernel (one row block, one tile per wave) merged by the wavefront kernel
-// (pa_launch_combine takes the other merge kernel from 16 columns on), from 64 splits on: each partial's rounding
-// (2^-12 of a 128-row average of V) then enters the output with a weight of a sixty-fourth or less, an order of
-// magnitude under what the f16 probabilities of the MFMA path already cost; shorter contexts, where a partial IS most
-// of the output, and every other pass keep f32 partials.
-// round-robin tiles: the tile loop of the split-K kernel (every plan of that kernel but the single-round one) with more
-// than one split; the value is the distance between the first rows of two splits
 // two row blocks on the single-round kernel: what plan_decode picks when a verify block's context fits
 // one round of one-tile-per-wave splits at one workgroup a CU (a pass of a single split stays on the tile loop)
 static bool plan_single_round2(const pa_plan& pl) {
@@ -352,6 +345,7 @@ static bool plan_block(const pa_ctx* ctx, const pa_plan& pl) {
 }
 // one row block on the single-round kernel (eight waves of one row block are the tile loop, or plan_one_wg)
 static bool plan_single_round1(const pa_plan& pl) { return pl.kernel == 0 && pl.row_blocks == 1 && pl.waves == 4 && pl.split_len == 128; }
+// round-robin tiles: more than one split of several tiles a wave; the value is the distance between the first rows of two splits
 static uint32_t plan_tile_ilv(const pa_plan& pl) {
   return pl.kernel == 0 && pl.split_len != 32 * pl.waves && pl.n_splits > 1 ? 32 * pl.waves : 0;
 }
@@ -370,15 +364,20 @@ static int plan_kernel(const pa_ctx* ctx, const pa_plan& pl) {
   return plan_single_round1(pl) || plan_single_round2(pl) ? ATTN_SINGLE_ROUND : ATTN_LOOP;
 }
 #define PA_F16_PARTIALS_MIN_SPLITS 64u
+// f16 O partials: the single-round split-K kernel (one row block, one tile per wave) merged by the wavefront kernel
+// (from 16 columns on a pass may take the other merge kernel, which reads f32 rows), from 64 splits on: each partial's rounding
+// (2^-12 of a 128-row average of V) then enters the output with a weight of a sixty-fourth or less, an order of
+// magnitude under what the f16 probabilities of the MFMA path already cost; shorter contexts, where a partial IS most
+// of the output, and every other pass keep f32 partials.
 static bool plan_f16_partials(const pa_plan& pl, uint32_t n_cols) {
   return pl.kernel == 0 && pl.row_blocks == 1 && pl.split_len == 32 * pl.waves && n_cols < 16 && pl.n_splits >= PA_F16_PARTIALS_MIN_SPLITS;
 }
-// The context up to which one workgroup per column group, in one launch, beats splits and a merge.  Int8 rows keep the plans that they had: the sums of a
+// The context up to which one workgroup per column group, in one launch, beats splits and a merge (plan_decode has a shorter one for one row block at head_dim 256).  Int8 rows keep the plans that they had: the sums of a
 // short context in another order move an output by up to 4e-4, and with it up to 2 % of the int8 values that a chain of ten layers stores by a step.
 static uint32_t one_launch_rows(const pa_ctx* ctx) { return kv_q8(ctx) ? 0u : 256u; }
-// rows_cap (optional): at most this many stacked rows per workgroup (16 or 32) instead of the table's choice;
-// one_split: the whole context as one split per workgroup -- with no own-row partial the kernel then writes the
-// output itself (no partials, no merge launch).  Both are what plan_prefill asks for on small chunks.
+// rows_cap (optional): at most this many stacked rows per workgroup (16, 32, 48 or 64) instead of the table's choice;
+// one_split: the whole context as one split per workgroup -- with no own-row partial the tile loop then writes the
+// output itself (no partials, no merge launch).  Both are what plan_prefill asks for on chunks, the first also on a few columns over a short context.
 static int plan_decode(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, pa_plan* pl, bool self_ok = true,
                        uint32_t rows_cap = 0, bool one_split = false) {
   const pa_config& c = ctx->cfg;

@@ -94,9 +94,9 @@ inline hipError_t pa_lds_limit(PaPerDevice& set, const void* kernel, size_t byte
 
 hipError_t pa_launch_glue(const GlueParams& p, hipStream_t s);
 hipError_t pa_launch_rope_table(float2* tab, const float* inv_freq, uint32_t half, uint32_t n_pos, hipStream_t s);
-// waves per workgroup W in {4, 8}; NB = 16-row query blocks per workgroup (1..4); hd in {128, 256}
 // blocks of two to four row blocks a workgroup over more than one split (attn_block.hip)
 hipError_t pa_launch_block(const AttnParams& p, uint32_t hd, uint32_t nb, uint32_t col_groups, hipStream_t s, const PaTiming* t = nullptr);
+// waves per workgroup W in {4, 8}; NB = 16-row query blocks per workgroup (1..4); hd in {128, 256}
 hipError_t pa_launch_decode(const AttnParams& p, uint32_t hd, uint32_t nb, uint32_t waves, uint32_t col_groups, hipStream_t s, const PaTiming* t = nullptr);
 // gather mode: every column attends to its own list of cache rows (p.sel set; cols_per_group == 1, grid z = column)
 hipError_t pa_launch_decode_gather(const AttnParams& p, uint32_t hd, hipStream_t s, const PaTiming* t = nullptr);

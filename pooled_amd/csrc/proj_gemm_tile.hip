@@ -566,8 +566,8 @@ static hipError_t gt_launch(const GemmTileParams& q, int acc, const GlueParams* 
   return hipGetLastError();
 }
 
-// The tile shapes, with what a round of the chip costs: ns per k of d_in (measured on rounds of 200 - 256 workgroups, all on 32 x 32 x 16
-// products; several full rounds of a kg = 1 shape are some 5 % faster now) on top of about 6 us for a round's first loads and last stores.
+// The tile shapes, with what a round of the chip costs: ns per k of d_in (measured on rounds of 200 - 256 workgroups on 32 x 32 x 16 products; those of the kg = 1
+// shapes are from before gt_whole_k, which takes some 5 % off several full rounds of them) on top of about 6 us for a round's first loads and last stores.
 struct TileShape { uint16_t bm, bn, kg; float us, ns_k; hipError_t (*launch)(const GemmTileParams&, int, const GlueParams*, hipStream_t); };
 static const TileShape tile_shapes[] = {
   { 64, 128, 4, 6.f, 6.5f, gt_launch<1, 2, 4, 2, 2, 3, false> },
@@ -599,9 +599,9 @@ static const TileShape head_shapes[] = {
 // One workgroup is resident per CU, so a call costs whole rounds of n_cu workgroups: the shape with the cheapest rounds, and
 // its estimate in us.  Larger tiles pay less traffic per product but are coarser: which one wins changes with every
 // multiple of a tile edge (777 columns of 5120 x 6144: 128 x 160, 224 workgroups, 63 us; 128 x 128, 280 workgroups, 87 us).  Of
-// 104 sizes measured on every tile and on the 64 x 64 kernel (8 weight shapes x 13 column counts, cold weights) the choice between
-// all of them is the fastest at 84 and within 6 % at 8; it is 9 - 33 % behind at 12, most where one round of few workgroups (which
-// costs less than a full one) is set against the 64 x 64 kernel: 9216 x 2048, 200 columns 27.9 us, on 128 x 128 21.1.
+// 104 sizes measured on every tile as they are and on the 64 x 64 kernel (8 weight shapes x 13 column counts, cold weights) the choice between
+// all of them is the fastest at 90 and within 6 % at 2; it is 7 - 27 % behind at 12, most where one round of few workgroups (which
+// costs less than a full one) is set against the 64 x 64 kernel: 9216 x 2048, 200 columns 27 % over 128 x 128.
 static float rounds_us(const TileShape& t, uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu) {
   const uint64_t wgs = (uint64_t)((n_cols + t.bm - 1) / t.bm) * ((d_out + t.bn - 1) / t.bn), cus = n_cu > 0 ? n_cu : 256;
   return (float)((wgs + cus - 1) / cus) * (t.us + t.ns_k * 1e-3f * d_in);
