@@ -596,12 +596,19 @@ static int plan_prefill(const pa_ctx* ctx, uint32_t base_pos, uint32_t n_cols, p
     const bool full32 = 32 >= G && (uint64_t)ceil_div(n_cols, 32 / G) * c.n_kv_heads >= n_cu;      // 32 rows a workgroup fill the chip
     if (!keep && plan_decode(ctx, base_pos, n_cols, &q, true) == PA_OK && q.n_splits > 1) offer(q, chunk_us_split(ctx, q, rows));
     // one launch: 16, 32 or, at a workgroup a CU at most, more stacked rows in a workgroup, where the groups alone occupy half the chip (or the context is a few tiles)
+    pa_plan one; memset(&one, 0, sizeof one);
+    double one_us = -1.0;
     for (uint32_t cap = 16; !ctx->decode_splits_override && cap <= (c.head_dim == 256 ? 48u : 64u); cap = cap == 32 && c.head_dim == 128 ? 64 : cap + 16) {
       if ((cap == 16 && full32) || (keep && (cap != (full32 ? 32u : 16u) || flops > 8.0e9))) continue;
       if (cap < G || plan_decode(ctx, base_pos, n_cols, &q, true, cap, true) != PA_OK || q.n_splits != 1) continue;
       const uint64_t wgs = (uint64_t)q.col_groups * c.n_kv_heads;
-      if ((wgs * 2 >= n_cu || rows <= 256) && (cap <= 32 || wgs <= n_cu)) offer(q, keep ? 0.0 : chunk_us_one(ctx, q, base_pos, rows));
+      const double us = keep ? 0.0 : chunk_us_one(ctx, q, base_pos, rows);
+      if ((wgs * 2 >= n_cu || rows <= 256) && (cap <= 32 || wgs <= n_cu) && (one_us < 0.0 || us < one_us)) { one = q; one_us = us; }
     }
+    // (against the matrix-core kernel on f16 rows it is taken within 3 %: that close the estimates favour the other too often -- 46 calls between the two lines, us: 16 / 8-head shape, 655 columns at
+    // 1093 32.5 / 28.6, 1463 at 86 44.0 / 34.2, 16 / 2-head, 854 at 10 43.4 / 42.0, 877 at 38 44.0 / 44.7, 24 / 4-head, 606 at 275 45.4 / 42.4 -- and its error against 64 bits is the smaller
+    // one on such chunks, 2.56 and 2.69e-4)
+    if (one_us >= 0.0) offer(one, best.kernel == 1 && !kv_q8(ctx) ? 0.97 * one_us : one_us);
   }
   if (best_us < 0.0) return fits_scratch ? plan_no_scratch(ctx, base_pos, n_cols, pl) : PA_ERR_UNSUPPORTED;
   *pl = best;

@@ -76,3 +76,12 @@ def test_which_kernel_serves_a_verify_block(shape, n, base, splits, kernel):
     """Both sides of each line between the single-round kernel, the tile loop and the kernel whose waves share one softmax."""
     got, pl = attn_rule(SHAPES[shape], "decode", base, n, splits)
     assert got == kernel, (got, pl)
+
+
+@pytest.mark.parametrize("shape,q8,n,base,kernel", [
+    ("qwen36_moe", False, 854, 10, LOOP), ("qwen36_moe", False, 807, 44, LOOP), ("qwen3_1p7b", False, 655, 1093, LOOP), ("qwen3_1p7b", False, 1463, 86, LOOP), ("qwen38_27b", False, 606, 275, LOOP),
+    ("qwen38_27b", False, 660, 0, MFMA), ("qwen36_moe", False, 1024, 0, MFMA), ("qwen3_1p7b", False, 2048, 0, MFMA), ("qwen36_moe", True, 585, 844, MFMA), ("qwen36_moe", True, 446, 1265, MFMA)])
+def test_a_chunk_runs_in_one_launch_where_it_is_close(shape, q8, n, base, kernel):
+    """One launch is taken within 3 % of the matrix-core kernel's estimate on f16 rows, not on int8 rows, whose plans stay what they were that close."""
+    got, pl = attn_rule(dict(SHAPES[shape], kv_q8=q8), "prefill", base, n)
+    assert got == kernel and (kernel == MFMA or pl["n_splits"] == 1), (got, pl)
