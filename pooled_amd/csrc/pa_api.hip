@@ -335,12 +335,16 @@ static bool plan_single_round2(const pa_plan& pl) {
 // only at its end, share the L2's rows better (24 / 4-head, 10 columns at 20000 26.2 / 25.0, at 65536 67.3 / 57.6, both without the low halves of q).  One tile a wave: where several
 // groups or the small heads fill more than half the chip but not twice (16 / 2-head, 6 at 8000 13.9 / 14.6, 24 / 4-head, 10 at 4000 13.8 / 15.1, 16 / 8-head, 9 at 4000 9.0 / 10.5; one
 // group, 16 / 2-head, 4 at 600 and 12001 11.0 / 10.6 and 14.4 / 14.2; 16 / 8-head, 12 at 8000 12.9 / 12.5, as before).
+// Int8 rows at head_dim 256 up to three tiles a wave: widening a tile is work that waves in step do not hide under each other's loads (one group, 24 / 4-head, 3 columns at 9000, 21000, 25000,
+// 37000 and 64000 14.6 / 16.0, 20.3 / 20.3, 23.5 / 22.7, 28.2 / 26.2, 40.5 / 36.1, 8 at 65000 47.3 / 42.3; 16 / 2-head, 4 at 25000 and 57000 16.8 / 18.5, 25.3 / 24.6; at head_dim 128 it stays
+// ahead: 16 / 8-head, 16 at 30000 22.6 / 23.2).
 // Not one column of more than 16 query heads a kv head: its own row is a partial of its own, which that kernel does not make.
 static bool plan_block(const pa_ctx* ctx, const pa_plan& pl) {
   if (pl.kernel != 0 || pl.waves != 4 || pl.row_blocks < 2 || pl.n_splits == 1 || plan_self_row(pl)) return false;
   const uint32_t tiles = pl.split_len / 128, n_cu = (uint32_t)ctx->n_cu;
   const uint64_t wgs = (uint64_t)pl.n_splits * ctx->cfg.n_kv_heads * pl.col_groups;
   if (tiles == 1) return wgs * 2 > n_cu && wgs <= n_cu && (pl.col_groups > 1 || ctx->cfg.head_dim == 128);
+  if (tiles > 3 && kv_q8(ctx) && ctx->cfg.head_dim == 256) return false;
   return pl.col_groups == 1 || tiles == 2;
 }
 // one row block on the single-round kernel (eight waves of one row block are the tile loop, or plan_one_wg)

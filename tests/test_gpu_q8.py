@@ -286,3 +286,28 @@ def test_q8_exact_blocks_have_the_bits_of_another_contexts_decodes(base):
             steps.append(pa.run_decode_step(0, d["qraw"][0], d["kraw"][base], d["vraw"][base], d["qw"], d["kw"], base))
     assert np.isfinite(got[0]).all() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
     assert np.isfinite(steps[0]).all() and np.array_equal(steps[0].view(np.uint32), steps[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("shape,n,base,blocks", [("qwen38_27b", 5, 26000, 2), ("qwen38_27b", 8, 50000, 3), ("qwen36_moe", 4, 50000, 2)])
+def test_q8_verify_block_past_three_tiles_a_wave(shape, n, base, blocks):
+    """One column group of two and three row blocks over int8 rows at head_dim 256, four tiles a wave and more: the tile loop, with low and high keys in turn (a raised
+    reference), scales past the context poisoned, both output types.  Budget of the decode tests."""
+    cfg = _q8cfg(shape)
+    rng = np.random.default_rng(base + n)
+    rows, nKV, hd = base + n, cfg["n_kv_heads"], cfg["head_dim"]
+    scale = np.where((np.arange(rows) // (rows // 9)) % 2 == 0, 0.2, 2.0).astype(np.float32)[:, None, None]
+    kq, ks = O.q8_quantize(rng.standard_normal((rows, nKV, hd), dtype=np.float32) * scale)
+    vq, vs = O.q8_quantize(rng.standard_normal((rows, nKV, hd), dtype=np.float32))
+    q = rng.standard_normal((n, cfg["n_heads"], hd), dtype=np.float32)
+    gate = rng.standard_normal(q.shape, dtype=np.float32)
+    ref = O.attention_values(q, O.q8_dequantize(kq, ks), O.q8_dequantize(vq, vs), base, gate=gate)
+    with PooledAttn(cfg, rows + 40, n_layers=1, max_cols=n) as pa:
+        pa.layer_alloc(0)
+        for w, a in enumerate((kq, vq, ks, vs)):
+            pa.kv_write(0, w, 0, a)
+        for w in (2, 3):
+            pa.kv_write(0, w, rows, np.full((40, nKV, hd // 32), np.nan, np.float32))
+        kernel, plan = attn_rule(cfg, "decode", base, n)
+        assert kernel == LOOP and plan == pa.plan("decode", base, n) and plan["row_blocks"] == blocks and plan["col_groups"] == 1 and plan["split_len"] >= 4 * 128, (kernel, plan)
+        for out_dtype in (0, PA_OUT_F16):
+            assert_parity(pa.run_attn("decode", 0, q, base, gate=gate, out_dtype=out_dtype).astype(np.float32), ref, "q8 verify block of %d at %d" % (n, base))

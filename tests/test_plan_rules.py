@@ -85,3 +85,12 @@ def test_a_chunk_runs_in_one_launch_where_it_is_close(shape, q8, n, base, kernel
     """One launch is taken within 3 % of the matrix-core kernel's estimate on f16 rows, not on int8 rows, whose plans stay what they were that close."""
     got, pl = attn_rule(dict(SHAPES[shape], kv_q8=q8), "prefill", base, n)
     assert got == kernel and (kernel == MFMA or pl["n_splits"] == 1), (got, pl)
+
+
+@pytest.mark.parametrize("shape,n,base,kernel", [
+    ("qwen38_27b", 5, 9000, BLOCK), ("qwen38_27b", 5, 24560, BLOCK), ("qwen38_27b", 5, 24580, LOOP), ("qwen38_27b", 5, 60000, LOOP), ("qwen38_27b", 8, 65000, LOOP), ("qwen36_moe", 3, 49140, BLOCK),
+    ("qwen36_moe", 3, 49160, LOOP), ("qwen36_moe", 16, 8000, BLOCK), ("qwen3_1p7b", 16, 30000, BLOCK), ("qwen3_1p7b", 32, 30000, BLOCK)])
+def test_which_kernel_serves_a_verify_block_over_int8_rows(shape, n, base, kernel):
+    """Int8 rows at head_dim 256 leave the kernel with one softmax a workgroup past three tiles a wave; at head_dim 128 they do not."""
+    got, pl = attn_rule(dict(SHAPES[shape], kv_q8=True), "decode", base, n)
+    assert got == kernel, (got, pl)
