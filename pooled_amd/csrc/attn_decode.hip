@@ -1460,15 +1460,19 @@ hipError_t pa_launch_decode_gather(const AttnParams& p, uint32_t hd, hipStream_t
   return hipErrorInvalidValue;
 }
 
+// Many columns, few splits: one thread per (column, head, 4 dims).  Its workgroups walk a column's splits, eight a round trip, so with few of them (two fifths of the CUs)
+// and more splits than one round trip has, the wavefront kernel is ahead although every one of its waves is a launch of its own (us a call, this / that: 16 / 2-head shape, 16
+// columns at 8000 and 12345 rows 18.9 / 15.9 and 22.3 / 19.3 (64 workgroups here; 32 and 25 splits), 24 at 12345 23.7 / 22.3, 32 at 8000 (128 workgroups) 21.8 / 22.2, 48 at 12345
+// 31.4 / 32.4; 16 / 8-head, 32 at 12345 21.3 / 18.4; 24 / 4-head, 16 at 850 and 1000 (seven and eight splits) 11.5 / 12.2, 11.9 / 12.6, at 1100 and 1400 (nine and twelve)
+// 12.9 / 12.2, 13.3 / 12.4, at 4200 (eleven) 19.2 / 18.3).
+extern "C" int pa_rule_merge_wide(uint32_t n_cols, uint32_t n_heads, uint32_t hd, uint32_t n_splits, int n_cu) {
+  const uint64_t wgs = ((uint64_t)n_cols * n_heads * (hd / 4) + 255) / 256;
+  return n_cols >= 16 && n_splits <= 32 && !(n_splits > 8 && wgs * 5 <= 2 * (uint64_t)n_cu);
+}
+
 hipError_t pa_launch_combine(const AttnParams& p, uint32_t hd, int n_cu, hipStream_t s, const PaTiming* t) {
-  // many columns, few splits: one thread per (column, head, 4 dims).  Its workgroups walk a column's splits, eight a round trip, so with few of them (two fifths of the CUs)
-  // and more splits than one round trip has, the wavefront kernel is ahead although every one of its waves is a launch of its own (us a call, this / that: 16 / 2-head shape, 16
-  // columns at 8000 and 12345 rows 18.9 / 15.9 and 22.3 / 19.3 (64 workgroups here; 32 and 25 splits), 24 at 12345 23.7 / 22.3, 32 at 8000 (128 workgroups) 21.8 / 22.2, 48 at 12345
-  // 31.4 / 32.4; 16 / 8-head, 32 at 12345 21.3 / 18.4; 24 / 4-head, 16 at 600 (five splits) 11.7 / 12.7 and at 4200 (eleven) 19.2 / 18.3).
-  const uint64_t wide_wgs = ((uint64_t)p.n_cols * p.n_heads * (hd / 4) + 255) / 256;
-  const bool few = p.n_splits > 6 && wide_wgs * 5 <= 2 * (uint64_t)n_cu;
-  if (p.n_cols >= 16 && p.n_splits <= 32 && !few && (hd == 256 || hd == 128) && !p.exact_cols && !p.self_row) {
-    const dim3 grid((unsigned)wide_wgs);
+  if (pa_rule_merge_wide(p.n_cols, p.n_heads, hd, p.n_splits, n_cu) && (hd == 256 || hd == 128) && !p.exact_cols && !p.self_row) {
+    const dim3 grid((unsigned)(((size_t)p.n_cols * p.n_heads * (hd / 4) + 255) / 256));
     if (hd == 256) hipLaunchKernelGGL(pa_combine_wide_kernel<256>, grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL(pa_combine_wide_kernel<128>, grid, dim3(256), 0, s, p);
     return hipGetLastError();

@@ -147,6 +147,7 @@ float pa_gemm_tile_us(uint32_t d_out, uint32_t d_in, uint32_t n_cols, int n_cu, 
 // (attention: the plan of a decode (kind 0) or prefill call (1; 2: under capture in a context that holds no scratch), or of a gather call (3; base_pos: its max_rows), on n_cu CUs, under a splits override or 0 and a mode of
 // pa_set_prefill_tile, and its kernel: 0 matrix cores, 1 tile loop, 2 single round, 3 one workgroup a kv head, 4 waves that share one softmax; -1: none, -2: under capture one that allocates)
 extern "C" int pa_rule_attn(const pa_config* cfg, int n_cu, int kind, uint32_t base_pos, uint32_t n_cols, uint32_t splits, int tile_mode, pa_plan* out);
+extern "C" int pa_rule_merge_wide(uint32_t n_cols, uint32_t n_heads, uint32_t hd, uint32_t n_splits, int n_cu);      // 0: the wavefront merge kernel
 extern "C" uint32_t pa_rule_gemv_resident(int kind, uint32_t d_out, uint32_t d_in, int norm, int n_cu);
 extern "C" int pa_rule_gemv_at_once(int kind, uint32_t d_out, uint32_t d_in, int norm, uint32_t rows, int n_cu);
 extern "C" uint32_t pa_rule_gemv_wide_rows(int kind, uint32_t d_out, uint32_t d_in, int norm, int n_cu);

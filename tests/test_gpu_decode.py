@@ -514,10 +514,10 @@ def test_blocks_whose_waves_share_one_softmax(shape, kv_q8, n_cols, base, blocks
             assert np.abs(pa.run_attn("decode", 0, q, base) - want).max() <= 2e-6
 
 
-@pytest.mark.parametrize("shape,n_cols,base", [("qwen36_moe", 16, 700), ("qwen36_moe", 16, 760), ("qwen36_moe", 25, 4500), ("qwen36_moe", 26, 4500), ("qwen3_1p7b", 51, 4300),
+@pytest.mark.parametrize("shape,n_cols,base", [("qwen36_moe", 16, 700), ("qwen36_moe", 16, 760), ("qwen36_moe", 16, 1000), ("qwen36_moe", 16, 1010), ("qwen36_moe", 25, 4500), ("qwen36_moe", 26, 4500), ("qwen3_1p7b", 51, 4300),
                                                ("qwen3_1p7b", 52, 4300), ("qwen38_27b", 17, 5000)])
 def test_merge_of_sixteen_columns_and_more(shape, n_cols, base):
-    """Either merge kernel behind a pass of 16 columns or more: up to six splits and past them, two fifths of the CUs' worth of workgroups and past that."""
+    """Either merge kernel behind a pass of 16 columns or more: up to eight splits and past them, two fifths of the CUs' worth of workgroups and past that."""
     cfg = SHAPES[shape]
     rng = np.random.default_rng(base + n_cols)
     k16, v16 = random_cache(cfg, base + n_cols, seed=base)

@@ -1,5 +1,7 @@
 """No-GPU checks of which kernel serves an attention call: the library's own plan rules, asked on a 256-CU part."""
+import ctypes
 import pytest
+from pooled_amd import capi
 from helpers import attn_rule, BLOCK, LOOP, MFMA, ONE_WG, SHAPES, SINGLE_ROUND
 
 
@@ -94,3 +96,10 @@ def test_which_kernel_serves_a_verify_block_over_int8_rows(shape, n, base, kerne
     """Int8 rows at head_dim 256 leave the kernel with one softmax a workgroup past three tiles a wave; at head_dim 128 they do not."""
     got, pl = attn_rule(dict(SHAPES[shape], kv_q8=True), "decode", base, n)
     assert got == kernel, (got, pl)
+
+
+@pytest.mark.parametrize("n_cols,n_heads,head_dim,n_splits,wide", [(15, 16, 256, 4, 0), (16, 16, 256, 4, 1), (16, 24, 256, 7, 1), (16, 24, 256, 8, 1), (16, 24, 256, 9, 0), (16, 16, 256, 32, 0),
+                                                                   (25, 16, 256, 9, 0), (26, 16, 256, 9, 1), (51, 16, 128, 9, 0), (52, 16, 128, 9, 1), (64, 16, 256, 32, 1), (64, 16, 256, 33, 0)])
+def test_which_kernel_merges_the_splits(n_cols, n_heads, head_dim, n_splits, wide):
+    """From 16 columns on one thread a (column, head, 4 dims) merges up to 32 splits, but past the eight of one round trip only with more than two fifths of the CUs' worth of workgroups."""
+    assert capi.load().pa_rule_merge_wide(*(ctypes.c_uint32(v) for v in (n_cols, n_heads, head_dim, n_splits)), ctypes.c_int(256)) == wide
